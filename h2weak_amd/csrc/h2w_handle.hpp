@@ -244,7 +244,7 @@ struct h2w_handle {
     double memory = 0.0;
     double assembly_seconds = 0.0;
     int aca_reruns = 0;
-    int aca_batches = 0;                // k_aca launch batches of the last assembly
+    int aca_batches = 0;                // cross approximation batches of the last assembly
     int64_t aca_pool_bytes = 0;         // largest ACA workspace of the last assembly
     h2w::DevBuf<uint16_t> rank_model;   // BF16 rank-predictor parameters (empty: heuristic estimates)
     int rank_pred_blocks = 0, rank_pred_under = 0;  // predicted blocks / blocks whose rank exceeded the estimate

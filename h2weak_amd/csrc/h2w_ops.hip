@@ -172,6 +172,13 @@ struct AcaPool {
     DevBuf<double> ws;
     DevBuf<unsigned long long> top;
     int64_t cap = 0;  // doubles
+    // the wide cross: tiles, states and partials of a batch, kept over the batches of an assembly
+    DevBuf<WideState> wstate;
+    DevBuf<WideBlk> wblk;
+    DevBuf<int2> wtiles;
+    DevBuf<double> wpart, wdot;
+    DevBuf<uint32_t> warrived;
+    DevBuf<int32_t> wdone;
 };
 
 // The workspace holds the U and V columns of every block of a batch.  It is sized
@@ -241,7 +248,7 @@ void block_features(const Handle &h, int fam, int j, int b, const std::vector<in
     B.has_feat = true;
 }
 
-// The wide cross of the first nh jobs of a batch (device copies at djobs).  Blocks with a
+// The cross of a batch's blocks (device copies of the jobs at djobs).  Blocks with a
 // fixed-rank phase (AcaJob.pad = kfix > 1, from the rank model) first take kfix pivot steps
 // without the normS update and stopping test -- every launch enqueued at once, no host reads
 // in between -- and are then judged by the reference's own stopping rule, applied to all their
@@ -252,30 +259,55 @@ void block_features(const Handle &h, int fam, int j, int b, const std::vector<in
 // steps are enqueued 16 at a time; between groups the host reads how many blocks are done.
 // Every step advances a block's rank, moves its first-row search on, or finishes it, so the
 // loop ends within max(m) + max(tcap) + 1 steps.
-void run_wide(Handle &h, const std::vector<AcaJob> &jobs, size_t nh, const AcaJob *djobs, const int32_t *didx,
-              AcaPool &pool, int64_t *dtab, uint8_t *dflags, int32_t *drank, int32_t *dstat, int32_t *drp,
+void run_wide(Handle &h, const std::vector<AcaJob> &jobs, const std::vector<int> &est, const AcaJob *djobs,
+              const int32_t *didx, AcaPool &pool, int64_t *dtab, uint8_t *dflags, int32_t *drank, int32_t *dstat, int32_t *drp,
               int32_t *dcp, double *dhist, double tol) {
     hipStream_t s = h.stream;
-    const int nb = (int)nh;
-    int maxm = 0, maxn = 0, maxt = 0, maxfix = 0;
-    for (size_t q = 0; q < nh; ++q) {
-        maxm = std::max(maxm, jobs[q].m);
-        maxn = std::max(maxn, jobs[q].n);
-        maxt = std::max(maxt, jobs[q].tcap);
-        maxfix = std::max(maxfix, jobs[q].pad);
+    const int nb = (int)jobs.size();
+    int maxm = 0, maxt = 0, maxfix = 0;
+    // tiles of every block, and room for the inner products of twice its estimated rank and more
+    const int T = wide_tile();
+    std::vector<WideBlk> wb(nb);
+    std::vector<int2> rt, ct;
+    int64_t pd = 0;
+    for (int q = 0; q < nb; ++q) {
+        const AcaJob &J = jobs[q];
+        maxm = std::max(maxm, J.m);
+        maxt = std::max(maxt, J.tcap);
+        maxfix = std::max(maxfix, J.pad);
+        WideBlk &W = wb[q];
+        W.nrt = (J.n + T - 1) / T;
+        W.nct = (J.m + T - 1) / T;
+        W.cap = std::min(J.tcap, std::max(4 * est[q], 256));
+        W.pad = 0;
+        W.rt0 = (int)rt.size();
+        W.ct0 = (int)ct.size();
+        W.pd = pd;
+        pd += (int64_t)(W.nrt + W.nct) * W.cap;
+        for (int t = 0; t < W.nrt; ++t) rt.push_back(int2{q, t});
+        for (int t = 0; t < W.nct; ++t) ct.push_back(int2{q, t});
     }
-    const int pstride = std::max(1, std::max((maxm + 2047) / 2048, (maxn + 2047) / 2048));
-    const int dstride = std::max(maxt, 1);
-    DevBuf<WideState> st;
-    DevBuf<WidePart> part;
-    DevBuf<double> dots;
-    DevBuf<int32_t> ndone;
-    st.alloc(nb);
-    part.alloc((size_t)nb * pstride);
-    dots.alloc((size_t)nb * dstride);
-    ndone.alloc(1);
-    launch_wide_init(djobs, nb, maxm + maxn, st.p, dflags, dtab, pool.top.p, pool.cap, s);
-    const int64_t limit = (int64_t)maxm + maxt + 1;
+    const int nrow = (int)rt.size(), ncol = (int)ct.size();
+    for (WideBlk &W : wb) W.ct0 += nrow;
+    rt.insert(rt.end(), ct.begin(), ct.end());
+    pool.wblk.upload(wb, s);
+    pool.wtiles.upload(rt, s);
+    pool.wstate.ensure(nb);
+    pool.wpart.ensure(std::max<size_t>(4 * rt.size(), 1));
+    pool.wdot.ensure(std::max<int64_t>(pd, 1));
+    pool.wdone.ensure(1);
+    pool.warrived.ensure(nb);
+    H2W_HIP(hipMemsetAsync(pool.warrived.p, 0, nb * sizeof(uint32_t), s));
+    const WideArgs W{pool.wblk.p, pool.wtiles.p, nrow, ncol, pool.wpart.p, pool.wdot.p, pool.warrived.p};
+    DevBuf<WideState> &st = pool.wstate;
+    launch_wide_init(djobs, pool.wblk.p, nb, st.p, dflags, dtab, pool.top.p, pool.cap, s);
+    auto step = [&]() {
+        if (nrow > 0 && ncol > 0)
+            launch_wide_step(djobs, W, didx, pool.ws.p, dtab, dflags, st.p, drp, dcp, dhist, pool.top.p, pool.cap, h.kp,
+                             tol, s);
+    };
+    // (the step after the last accepted one is taken beside its inner products)
+    const int64_t limit = (int64_t)maxm + maxt + 2;
     int64_t steps = 0;
     if (maxfix > 1) {
         // ---- fixed phase (a block whose first rows are zero spends steps on its first-row search:
@@ -283,9 +315,7 @@ void run_wide(Handle &h, const std::vector<AcaJob> &jobs, size_t nh, const AcaJo
         std::vector<WideState> hs(nb);
         int64_t todo = maxfix;
         while (true) {
-            for (int64_t c = 0; c < todo; ++c, ++steps)
-                launch_wide_fixed_step(djobs, nb, maxm, maxn, didx, pool.ws.p, dtab, dflags, st.p, part.p, pstride,
-                                       drp, dcp, dhist, pool.top.p, pool.cap, h.kp, tol, s);
+            for (int64_t c = 0; c < todo; ++c, ++steps) step();
             H2W_HIP(hipGetLastError());
             H2W_HIP(hipMemcpyAsync(hs.data(), st.p, (size_t)nb * sizeof(WideState), hipMemcpyDeviceToHost, s));
             H2W_HIP(hipStreamSynchronize(s));
@@ -363,23 +393,20 @@ void run_wide(Handle &h, const std::vector<AcaJob> &jobs, size_t nh, const AcaJo
             DevBuf<double> dnrm;
             dfin.upload(fin, s);
             dnrm.upload(nrm, s);
-            launch_wide_judge(djobs, nb, st.p, dfin.p, dnrm.p, dtab, pool.top.p, pool.cap, s);
+            launch_wide_judge(djobs, pool.wblk.p, nb, st.p, dfin.p, dnrm.p, dtab, pool.top.p, pool.cap, s);
             H2W_HIP(hipGetLastError());
             H2W_HIP(hipStreamSynchronize(s));
         }
     }
     while (true) {
-        launch_wide_finish(st.p, nb, drank, dstat, ndone.p, s);
+        launch_wide_finish(st.p, nb, drank, dstat, pool.wdone.p, s);
         H2W_HIP(hipGetLastError());
         int nd = 0;
-        H2W_HIP(hipMemcpyAsync(&nd, ndone.p, 4, hipMemcpyDeviceToHost, s));
+        H2W_HIP(hipMemcpyAsync(&nd, pool.wdone.p, 4, hipMemcpyDeviceToHost, s));
         H2W_HIP(hipStreamSynchronize(s));
         if (nd == nb) break;
         if (steps > limit) throw Error{H2W_EHIP, "wide cross did not finish within its step bound"};
-        for (int c = 0; c < 16; ++c, ++steps)
-            launch_wide_step(djobs, nb, maxm, maxn, (int)std::min<int64_t>(steps + 1, dstride), didx, pool.ws.p, dtab,
-                             dflags, st.p, part.p, pstride, dots.p, dstride, drp, dcp, dhist, pool.top.p, pool.cap,
-                             h.kp, tol, s);
+        for (int c = 0; c < 16; ++c, ++steps) step();
     }
     // sampled entries of the fixed-rank blocks against their cross approximation
     if (maxfix > 1) {
@@ -452,7 +479,12 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
     const bool cx = h.cplx;
     const int esz = cx ? 2 : 1;
     int64_t need = 0;
-    for (size_t b = 0; b < blocks.size(); ++b) need += (int64_t)(blocks[b].rows.size() + blocks[b].cols.size()) * est[b];
+    // a block's workspace: a column pair (each padded to an even length) per term, and the step ahead
+    auto space_of = [&](size_t b) {
+        const int64_t mp = (blocks[b].rows.size() + 1) / 2 * 2, np = (blocks[b].cols.size() + 1) / 2 * 2;
+        return (mp + np) * (int64_t)(est[b] + 1);
+    };
+    for (size_t b = 0; b < blocks.size(); ++b) need += space_of(b);
     ensure_pool(h, pool, need * esz);
     h.aca_pool_bytes = std::max<int64_t>(h.aca_pool_bytes, pool.cap * 8);
     DevBuf<uint8_t> flags;
@@ -462,8 +494,9 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
     DevBuf<AcaJob> djobs;
     DevBuf<LrJob> dlr;
     DevBuf<double> dlrout;
-    const size_t kBig = 16384;    // m + n above which a block gets a 1024-thread workgroup
-    // m + n above which a block's cross is spread over many workgroups (H2W_WIDE_MIN overrides)
+    const size_t kBig = 16384;    // complex kernels: m + n above which a block gets a 1024-thread workgroup
+    // m + n above which a block with a predicted rank takes a fixed-rank phase (H2W_WIDE_MIN overrides):
+    // its judgement costs host work per block, which small blocks do not repay
     const size_t kHuge = cx ? SIZE_MAX
                             : std::getenv("H2W_WIDE_MIN") ? (size_t)std::atoll(std::getenv("H2W_WIDE_MIN")) : 8192;
     while (!todo.empty()) {
@@ -475,7 +508,7 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
             while (pos < todo.size()) {
                 size_t b = todo[pos];
                 const AcaBlock &B = blocks[b];
-                int64_t nb = (int64_t)(B.rows.size() + B.cols.size()) * est[b];
+                const int64_t nb = space_of(b);
                 if (!batch.empty() && need + nb > pool.cap / esz) break;
                 batch.push_back(b);
                 need += nb;
@@ -483,7 +516,7 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
                 ++pos;
                 if (batch.size() >= 65535) break;
             }
-            // huge blocks first (wide cross), then big ones (1024-thread workgroups), each group contiguous
+            // the largest blocks first
             auto mn_of = [&](size_t b) { return blocks[b].rows.size() + blocks[b].cols.size(); };
             std::stable_partition(batch.begin(), batch.end(), [&](size_t b) { return mn_of(b) > kBig; });
             std::stable_partition(batch.begin(), batch.end(), [&](size_t b) { return mn_of(b) > kHuge; });
@@ -501,7 +534,7 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
                 J.m = (int32_t)B.rows.size();
                 J.n = (int32_t)B.cols.size();
                 J.tcap = std::min(std::min(J.m, J.n), 8192);
-                // wide blocks with a predicted rank: a fixed-rank phase of about that many steps
+                // large blocks with a predicted rank: a fixed-rank phase of about that many steps
                 J.pad = (pred && q < nhuge && !fixed_off) ? std::min(J.tcap, kfix_of(batch[q])) : 0;
                 J.rows = (int64_t)idx.size();
                 idx.insert(idx.end(), B.rows.begin(), B.rows.end());
@@ -535,15 +568,10 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
                     launch_aca_c(djobs.p + nbig, (int)(batch.size() - nbig), didx.p, wsc, pool.cap / 2, pool.top.p,
                                  dtab.p, flags.p, drank.p + nbig, dstat.p + nbig, drp.p, dcp.p, h.kpc, tol, dhist.p, 0, s);
             } else {
-                if (nhuge > 0)
-                    run_wide(h, jobs, nhuge, djobs.p, didx.p, pool, dtab.p, flags.p, drank.p, dstat.p, drp.p, dcp.p,
-                             dhist.p, tol);
-                if (nbig > nhuge)
-                    launch_aca(djobs.p + nhuge, (int)(nbig - nhuge), didx.p, pool.ws.p, pool.cap, pool.top.p, dtab.p,
-                               flags.p, drank.p + nhuge, dstat.p + nhuge, drp.p, dcp.p, h.kp, tol, dhist.p, 1, s);
-                if (batch.size() > nbig)
-                    launch_aca(djobs.p + nbig, (int)(batch.size() - nbig), didx.p, pool.ws.p, pool.cap, pool.top.p,
-                               dtab.p, flags.p, drank.p + nbig, dstat.p + nbig, drp.p, dcp.p, h.kp, tol, dhist.p, 0, s);
+                std::vector<int> best(batch.size());
+                for (size_t q = 0; q < batch.size(); ++q) best[q] = est[batch[q]];
+                run_wide(h, jobs, best, djobs.p, didx.p, pool, dtab.p, flags.p, drank.p, dstat.p, drp.p, dcp.p, dhist.p,
+                         tol);
             }
             H2W_HIP(hipGetLastError());
             std::vector<int32_t> rk(batch.size()), st(batch.size()), rp(po), cp(po);
@@ -628,7 +656,7 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
         if (!todo.empty()) {
             // re-runs go with larger estimates: let the workspace grow to hold them
             int64_t need2 = 0;
-            for (size_t b : todo) need2 += (int64_t)(blocks[b].rows.size() + blocks[b].cols.size()) * est[b];
+            for (size_t b : todo) need2 += space_of(b);
             ensure_pool(h, pool, need2 * esz);
         }
     }

@@ -138,10 +138,63 @@ __device__ __forceinline__ void block_reduce(BlockRed<NT> &sh, double &s0, doubl
     }
 }
 
+// Value of lane (lane ^ O) for a power of two O < 64: quad permutes (DPP) for 1 and 2,
+// ds_swizzle in its bit-mask mode for 4 .. 16, ds_bpermute for 32.  Every lane of the
+// aligned group of 2 O lanes must be active.
+template <int O>
+__device__ __forceinline__ int xor_lane(int v) {
+    if constexpr (O == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false);
+    else if constexpr (O == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false);
+    else if constexpr (O < 32) return __builtin_amdgcn_ds_swizzle(v, 0x1F | (O << 10));
+    else return __builtin_amdgcn_ds_bpermute((int)(((threadIdx.x & 63) ^ O) << 2), v);
+}
+template <int O>
+__device__ __forceinline__ float xor_lane(float v) {
+    return __int_as_float(xor_lane<O>(__float_as_int(v)));
+}
+template <int O>
+__device__ __forceinline__ double xor_lane(double v) {
+    const int64_t b = __double_as_longlong(v);
+    const int lo = xor_lane<O>((int)(uint32_t)b), hi = xor_lane<O>((int)(b >> 32));
+    return __longlong_as_double((int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo));
+}
+// Value of a lane that differs in bit O (1, 2: lane ^ O; 4, 8: rotation by O within a row of 16 lanes,
+// which flips bit O and keeps the bits below): enough for sums over whole rows, without the LDS crossbar.
+template <int O>
+__device__ __forceinline__ double fold_lane(double v) {
+    constexpr int ctrl = O == 1 ? 0xB1 : O == 2 ? 0x4E : 0x120 + O;
+    const int64_t b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)(uint32_t)b, ctrl, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), ctrl, 0xF, 0xF, false);
+    return __longlong_as_double((int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo));
+}
+// sum of a value's four copies at lanes equal modulo 16
+__device__ __forceinline__ double sum_halves(double v) {
+    auto fold = [](double x, auto swap) {
+        const int64_t b = __double_as_longlong(x);
+        const auto lo = swap((uint32_t)b), hi = swap((uint32_t)(b >> 32));
+        return __longlong_as_double((int64_t)(((uint64_t)hi[0] << 32) | lo[0])) +
+               __longlong_as_double((int64_t)(((uint64_t)hi[1] << 32) | lo[1]));
+    };
+    v = fold(v, [](uint32_t w) { return __builtin_amdgcn_permlane16_swap(w, w, false, false); });
+    return fold(v, [](uint32_t w) { return __builtin_amdgcn_permlane32_swap(w, w, false, false); });
+}
+// the same with O known only after unrolling
+template <typename T>
+__device__ __forceinline__ T xor_lane_n(T v, int o) {
+    switch (o) {
+    case 1: return xor_lane<1>(v);
+    case 2: return xor_lane<2>(v);
+    case 4: return xor_lane<4>(v);
+    case 8: return xor_lane<8>(v);
+    case 16: return xor_lane<16>(v);
+    default: return xor_lane<32>(v);
+    }
+}
+
 // ------------------------------------------------------------------ batched ACA
-// One workgroup per block.  Restates LowRank::ACA_only_nodes / ACA_only_nodesCUR
-// (2D/codes/aca.hpp:158-446) and ACA_only_nodesUV (1D/codes/aca.hpp:40-156),
-// which share the pivot loop:
+// Restates LowRank::ACA_only_nodes / ACA_only_nodesCUR (2D/codes/aca.hpp:158-446)
+// and ACA_only_nodesUV (1D/codes/aca.hpp:40-156), which share the pivot loop:
 //   - first row (in order) whose max |entry| exceeds 1e-36 starts the cross,
 //   - pivot column = first argmax of |residual row| over unused columns,
 //   - u = residual column / pivot, next row = first argmax of |residual column|
@@ -152,378 +205,95 @@ __device__ __forceinline__ void block_reduce(BlockRed<NT> &sh, double &s0, doubl
 //     the newest term, as the reference's loop does, 2D/codes/aca.hpp:404-409).
 // Residual rows/columns subtract the previous terms one by one in rank order
 // with separate multiply and subtract, as the reference does.
-// U and V columns live in a workspace pool shared by the batch: before each
-// step the workgroup's leader reserves m + n doubles with an atomic bump; the
-// column offsets go to the job's table.  status = 1 when the table or the pool
-// is full before the cross converged (the host re-runs the block alone).
+// One pivot step of every block of a batch is two launches, a row pass and a
+// column pass over tiles of all of them: a cross reads the (m + n) k entries of
+// its earlier terms at step k, and a level has few blocks near the root and small
+// ones near the leaves, so only all blocks together fill the chip at every level.
+// (One workgroup per block, with only the blocks of m + n > 8192 spread: the vertex
+// level of 64 blocks of m + n up to 8192 took 208 ms at N = 20011, now 13 ms for its
+// 272 steps; assemblies 572 -> 180 ms there, 32^3 grid at tol 1e-10 2440 -> 560 ms.
+// With a workgroup per block kept below m + n = 512, 2048, 8192: 194, 280, 478 ms at
+// N = 20011; 2D N = 40000 95, 102, 136 ms; 1D N = 65536 57, 63, 80 ms against 60 ms
+// with every block spread: the one-workgroup form is gone.)
+// U and V columns live in a workspace pool shared by the batch: each step reserves
+// a column pair with an atomic bump; the column offsets go to the job's table.
+// Per-block state lives in WideState; a finished block (converged, exhausted, or out
+// of workspace: status 1, re-run by the host) is skipped by every later launch.
 constexpr int kChunk = 512;
 
-template <int NT>
-__device__ __forceinline__ bool aca_reserve(int64_t *tab, int k, int m, int n, int tcap,
-                                            unsigned long long *ws_top, int64_t ws_cap, int64_t *sh_off) {
-    if (threadIdx.x == 0) {
-        int64_t off = -1;
-        if (k < tcap) {
-            unsigned long long o = atomicAdd(ws_top, (unsigned long long)(m + n));
-            if ((int64_t)o + m + n <= ws_cap) off = (int64_t)o;
-        }
-        *sh_off = off;
-        if (off >= 0) {
-            tab[2 * k] = off;
-            tab[2 * k + 1] = off + m;
-        }
-    }
-    __syncthreads();
-    return *sh_off >= 0;
-}
+// A tile of the wide passes: 256 threads x 2 consecutive entries (one 16-byte load per earlier term),
+// kWideU terms in flight twice over: 64 KB of loads outstanding per workgroup.  Large levels are bound by
+// the bytes of the earlier terms (a row pass over 1617 tiles at rank 150 reads 1.0 GB in 195 us, 5.1 TB/s;
+// that level of 64 blocks takes 28 ms, with 2048 entries per workgroup and eight loads in flight it took
+// 121 ms), small ones by the 10 us that a pass's chain of dependent accesses takes.  (Four waves per SIMD by a register limit spilled: 45 ms; the offsets and
+// weights through LDS instead of lane broadcasts, and the sums through the LDS crossbar: 31 ms.)
+constexpr int kWideTile = 512;
+constexpr int kWideU = 8;
 
-template <int NT>
-__global__ __launch_bounds__(NT) void k_aca(const AcaJob *__restrict__ jobs, const int32_t *__restrict__ idx,
-                                            double *__restrict__ ws, int64_t ws_cap, unsigned long long *ws_top,
-                                            int64_t *__restrict__ tab_all, uint8_t *__restrict__ flags,
-                                            int32_t *__restrict__ rank_out, int32_t *__restrict__ status_out,
-                                            int32_t *__restrict__ rowpiv, int32_t *__restrict__ colpiv, KParams kp,
-                                            double tol, double *__restrict__ hist_all) {
-    const AcaJob jb = jobs[blockIdx.x];
-    const int m = jb.m, n = jb.n, tcap = jb.tcap;
-    double *hist = hist_all + 2 * jb.piv;  // per accepted step: |u||v|, normS after the step
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    constexpr int NW = NT / 64;
-    const int32_t *rows = idx + jb.rows;
-    const int32_t *cols = idx + jb.cols;
-    int64_t *tab = tab_all + jb.tab;
-    uint8_t *ru = flags + jb.wsF;
-    uint8_t *cu = ru + m;
-    int32_t *rp_out = rowpiv + jb.piv;
-    int32_t *cp_out = colpiv + jb.piv;
-    __shared__ double coef[kChunk];
-    __shared__ int64_t cofs[kChunk];
-    __shared__ BlockRed<NT> red;
-    __shared__ double dacc[NW];
-    __shared__ int64_t sh_off;
-
-    if (m == 0 || n == 0 || tcap == 0) {
-        if (tid == 0) {
-            rank_out[blockIdx.x] = 0;
-            status_out[blockIdx.x] = 0;
-        }
-        return;
-    }
-    for (int i = tid; i < m; i += NT) ru[i] = 0;
-    for (int s = tid; s < n; s += NT) cu[s] = 0;
-    const int mn = min(m, n);
-    if (!aca_reserve<NT>(tab, 0, m, n, tcap, ws_top, ws_cap, &sh_off)) {
-        if (tid == 0) {
-            rank_out[blockIdx.x] = 0;
-            status_out[blockIdx.x] = 1;
-        }
-        return;
-    }
-    double *U0 = ws + sh_off;
-    double *V0 = U0 + m;
-
-    // ---- first row with a nonzero entry
-    int l = 0, cp = -1;
-    double piv = 0.0;
-    for (l = 0; l < m; ++l) {
-        PointI pr = load_point(kp, rows[l]);
-        AMax am{-1.0, INT_MAX, 0.0};
-        for (int s = tid; s < n; s += NT) {
-            double v = kentry(kp, pr, cols[s]);
-            V0[s] = v;
-            amax_update(am, v, s);
-        }
-        double d0 = 0.0, d1 = 0.0;
-        block_reduce<NT>(red, d0, d1, am);
-        if (am.idx != INT_MAX && am.a > 1e-36) {
-            cp = am.idx;
-            piv = am.sv;
-            break;
-        }
-    }
-    if (l == m) {
-        if (tid == 0) {
-            rank_out[blockIdx.x] = 0;
-            status_out[blockIdx.x] = 0;
-        }
-        return;
-    }
-    int rp = l;
-    // ---- first column
-    double un2 = 0.0, vn2 = 0.0;
-    AMax an{-1.0, INT_MAX, 0.0};
-    {
-        PointI pc = load_point(kp, cols[cp]);
-        for (int t = tid; t < m; t += NT) {
-            double c = kentry(kp, pc, rows[t]);  // A(rows[t], cols[cp]) (symmetric entry)
-            double u = c / piv;
-            U0[t] = u;
-            un2 += u * u;
-            if (t != rp) amax_update(an, c, t);
-        }
-        for (int s = tid; s < n; s += NT) vn2 += V0[s] * V0[s];
-    }
-    block_reduce<NT>(red, un2, vn2, an);
-    if (tid == 0) {
-        rp_out[0] = rp;
-        cp_out[0] = cp;
-        ru[rp] = 1;
-        cu[cp] = 1;
-    }
-    int rank = 1;
-    int status = 0;
-    double normS = 0.0;
-    double un = sqrt(un2), vn = sqrt(vn2);
-    int next_rp = an.idx;
-    if (tid == 0) {
-        hist[0] = un * vn;
-        hist[1] = 0.0;
-    }
-    __syncthreads();
-
-    while (un * vn > tol * normS && rank < mn) {
-        rp = next_rp;
-        if (rp == INT_MAX) break;
-        if (!aca_reserve<NT>(tab, rank, m, n, tcap, ws_top, ws_cap, &sh_off)) {
-            status = 1;
-            break;
-        }
-        double *Ur = ws + sh_off;
-        double *Vr = Ur + m;
-        const int nch = (rank + kChunk - 1) / kChunk;
-        // ---- residual row -> V column `rank`
-        PointI pr = load_point(kp, rows[rp]);
-        AMax am{-1.0, INT_MAX, 0.0};
-        vn2 = 0.0;
-        for (int ch = 0; ch < nch; ++ch) {
-            const int l0 = ch * kChunk, l1 = min(rank, l0 + kChunk);
-            for (int q = l0 + tid; q < l1; q += NT) {
-                coef[q - l0] = ws[tab[2 * q] + rp];
-                cofs[q - l0] = tab[2 * q + 1];
-            }
-            __syncthreads();
-            for (int s = tid; s < n; s += NT) {
-                double r = ch == 0 ? kentry(kp, pr, cols[s]) : Vr[s];
-                for (int q = l0; q < l1; ++q) r -= coef[q - l0] * ws[cofs[q - l0] + s];
-                Vr[s] = r;
-                if (ch == nch - 1) {
-                    vn2 += r * r;
-                    if (!cu[s]) amax_update(am, r, s);
-                }
-            }
-            __syncthreads();
-        }
-        double dummy = 0.0;
-        block_reduce<NT>(red, vn2, dummy, am);
-        if (am.idx == INT_MAX) break;
-        cp = am.idx;
-        piv = am.sv;
-        // ---- residual column -> U column `rank`
-        PointI pc = load_point(kp, cols[cp]);
-        an = AMax{-1.0, INT_MAX, 0.0};
-        un2 = 0.0;
-        for (int ch = 0; ch < nch; ++ch) {
-            const int l0 = ch * kChunk, l1 = min(rank, l0 + kChunk);
-            for (int q = l0 + tid; q < l1; q += NT) {
-                coef[q - l0] = ws[tab[2 * q + 1] + cp];
-                cofs[q - l0] = tab[2 * q];
-            }
-            __syncthreads();
-            for (int t = tid; t < m; t += NT) {
-                double c = ch == 0 ? kentry(kp, pc, rows[t]) : Ur[t];
-                for (int q = l0; q < l1; ++q) c -= coef[q - l0] * ws[cofs[q - l0] + t];
-                if (ch == nch - 1) {
-                    double u = c / piv;
-                    Ur[t] = u;
-                    un2 += u * u;
-                    if (t != rp && !ru[t]) amax_update(an, c, t);
-                } else {
-                    Ur[t] = c;
-                }
-            }
-            __syncthreads();
-        }
-        block_reduce<NT>(red, un2, dummy, an);
-        un = sqrt(un2);
-        vn = sqrt(vn2);
-        if (un < 1e-36 || vn < 1e-36) break;
-        if (tid == 0) {
-            rp_out[rank] = rp;
-            cp_out[rank] = cp;
-            ru[rp] = 1;
-            cu[cp] = 1;
-        }
-        ++rank;
-        next_rp = an.idx;
-        // ---- normS update: dots of the new term with every term
-        double acc = 0.0;
-        for (int q = wv; q < rank; q += NW) {
-            const double *Uq = ws + tab[2 * q];
-            const double *Vq = ws + tab[2 * q + 1];
-            double du = 0.0, dv = 0.0;
-            for (int t = lane; t < m; t += 64) du += Uq[t] * Ur[t];
-            for (int s = lane; s < n; s += 64) dv += Vq[s] * Vr[s];
-            du = wave_sum(du);
-            dv = wave_sum(dv);
-            acc += fabs(du * dv);
-        }
-        if (lane == 0) dacc[wv] = acc;
-        __syncthreads();
-        double S = 0.0;
-        for (int q = 0; q < NW; ++q) S += dacc[q];
-        double uv = un * vn;
-        normS = sqrt(normS * normS + uv * uv + 2.0 * S);
-        if (tid == 0) {
-            hist[2 * (rank - 1)] = uv;
-            hist[2 * (rank - 1) + 1] = normS;
-        }
-        __syncthreads();
-    }
-    if (tid == 0) {
-        rank_out[blockIdx.x] = rank;
-        status_out[blockIdx.x] = status;
-    }
-}
-
-// ------------------------------------------------------------------ wide ACA
-// The cross of k_aca for a few very large blocks, each spread over many
-// workgroups: one pivot step is a sequence of launches over all such blocks --
-// residual row (wide), row reduction, residual column (wide), column reduction
-// and acceptance, normS dot products (wide), normS update and the next step's
-// reservation.  Residual entries subtract the earlier terms in rank order as in
-// k_aca, so rows, columns and pivots are the same numbers; only the sums of
-// squares and dot products are reduced in another order.  Per-block state lives
-// in WideState; a finished block (converged, exhausted, or out of workspace:
-// status 1) is skipped by every later launch.
-constexpr int kWideCols = 2048;  // row / column entries one workgroup of the wide passes covers
-constexpr int kWidePT = kWideCols / 256;  // of them per thread
-
-__device__ __forceinline__ void wide_reserve(WideState &st, const AcaJob &jb, int64_t *tab,
-                                             unsigned long long *ws_top, int64_t ws_cap) {
-    int64_t off = -1;
-    if (st.rank < jb.tcap) {
-        unsigned long long o = atomicAdd(ws_top, (unsigned long long)(jb.m + jb.n));
-        if ((int64_t)o + jb.m + jb.n <= ws_cap) off = (int64_t)o;
-    }
-    if (off < 0) {
-        st.status = 1;
-        st.done = 1;
-        return;
-    }
+// space for one (U, V) pair; both columns start 16-byte aligned and hold an even number of entries
+__device__ __forceinline__ bool wide_take(WideState &st, const AcaJob &jb, int cap, int64_t *tab,
+                                          unsigned long long *ws_top, int64_t ws_cap) {
+    const int64_t mp = (jb.m + 1) & ~1, np = (jb.n + 1) & ~1;
+    if (st.rank >= cap) return false;
+    const int64_t off = (int64_t)atomicAdd(ws_top, (unsigned long long)(mp + np));
+    if (off + mp + np > ws_cap) return false;
     st.off = off;
     tab[2 * st.rank] = off;
-    tab[2 * st.rank + 1] = off + jb.m;
+    tab[2 * st.rank + 1] = off + mp;
+    return true;
+}
+__device__ __forceinline__ void wide_reserve(WideState &st, const AcaJob &jb, int cap, int64_t *tab,
+                                             unsigned long long *ws_top, int64_t ws_cap) {
+    if (!wide_take(st, jb, cap, tab, ws_top, ws_cap)) {
+        st.status = 1;
+        st.done = 1;
+    }
 }
 
 // first launch: clear the used-row/column flags, reserve step 0, start the first-row search
-__global__ __launch_bounds__(256) void k_wide_init(const AcaJob *__restrict__ jobs, WideState *__restrict__ state,
-                                                   uint8_t *__restrict__ flags, int64_t *__restrict__ tab_all,
-                                                   unsigned long long *ws_top, int64_t ws_cap) {
-    const AcaJob jb = jobs[blockIdx.y];
-    const int64_t tot = (int64_t)jb.m + jb.n;
-    for (int64_t e = blockIdx.x * 256 + threadIdx.x; e < tot; e += (int64_t)gridDim.x * 256) flags[jb.wsF + e] = 0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+__global__ __launch_bounds__(256) void k_wide_init(const AcaJob *__restrict__ jobs, const WideBlk *__restrict__ blk,
+                                                   WideState *__restrict__ state, uint8_t *__restrict__ flags,
+                                                   int64_t *__restrict__ tab_all, unsigned long long *ws_top,
+                                                   int64_t ws_cap) {
+    const AcaJob jb = jobs[blockIdx.x];
+    const int tot = jb.m + jb.n;
+    for (int e = threadIdx.x; e < tot; e += 256) flags[jb.wsF + e] = 0;
+    if (threadIdx.x == 0) {
         WideState st{};
-        st.rank = 0;
-        st.rp = 0;
-        st.l = 0;
         st.next_rp = INT_MAX;
         st.done = (jb.m == 0 || jb.n == 0 || jb.tcap == 0);
         st.kfix = jb.pad;
-        if (!st.done) wide_reserve(st, jb, tab_all + jb.tab, ws_top, ws_cap);
-        state[blockIdx.y] = st;
+        if (!st.done) wide_reserve(st, jb, blk[blockIdx.x].cap, tab_all + jb.tab, ws_top, ws_cap);
+        state[blockIdx.x] = st;
     }
 }
 
-// residual row rp -> V slot of the current step; partial sum of squares and argmax over unused columns
-__global__ __launch_bounds__(256) void k_wide_row(const AcaJob *__restrict__ jobs, const int32_t *__restrict__ idx,
-                                                  const double *__restrict__ wsr, double *__restrict__ ws,
-                                                  const int64_t *__restrict__ tab_all, const uint8_t *__restrict__ flags,
-                                                  const WideState *__restrict__ state, WidePart *__restrict__ part,
-                                                  int pstride, KParams kp) {
-    const AcaJob jb = jobs[blockIdx.y];
-    const WideState st = state[blockIdx.y];
-    const int s0 = blockIdx.x * kWideCols;
-    if (st.done || s0 >= jb.n) return;
-    const int s1 = min(jb.n, s0 + kWideCols);
-    const int rank = st.rank, rp = st.rp;
-    const int32_t *rows = idx + jb.rows, *cols = idx + jb.cols;
-    const int64_t *tab = tab_all + jb.tab;
-    const uint8_t *cu = flags + jb.wsF + jb.m;
-    double *Vr = ws + st.off + jb.m;
-    __shared__ double coef[kChunk];
-    __shared__ int64_t cofs[kChunk];
-    __shared__ BlockRed<256> red;
-    PointI pr = load_point(kp, rows[rp]);
-    AMax am{-1.0, INT_MAX, 0.0};
-    double vn2 = 0.0;
-    // a thread's kWidePT columns s0 + threadIdx.x + 256 i stay in registers over the residual's terms,
-    // so every term issues kWidePT independent loads (the arithmetic per column is unchanged)
-    double rv[kWidePT];
-#pragma unroll
-    for (int i = 0; i < kWidePT; ++i) {
-        const int s = s0 + threadIdx.x + 256 * i;
-        rv[i] = s < s1 ? kentry(kp, pr, cols[s]) : 0.0;
-    }
-    const int nch = (rank + kChunk - 1) / kChunk;
-    for (int ch = 0; ch < nch; ++ch) {
-        const int l0 = ch * kChunk, l1 = min(rank, l0 + kChunk);
-        for (int q = l0 + threadIdx.x; q < l1; q += 256) {
-            coef[q - l0] = wsr[tab[2 * q] + rp];
-            cofs[q - l0] = tab[2 * q + 1];
-        }
-        __syncthreads();
-        for (int q = l0; q < l1; ++q) {
-            const double c = coef[q - l0];
-            const double *v = wsr + cofs[q - l0];
-#pragma unroll
-            for (int i = 0; i < kWidePT; ++i) {
-                const int s = s0 + threadIdx.x + 256 * i;
-                if (s < s1) rv[i] -= c * v[s];
-            }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < kWidePT; ++i) {
-        const int s = s0 + threadIdx.x + 256 * i;
-        if (s < s1) {
-            Vr[s] = rv[i];
-            vn2 += rv[i] * rv[i];
-            if (!cu[s]) amax_update(am, rv[i], s);
-        }
-    }
-    double dummy = 0.0;
-    block_reduce<256>(red, vn2, dummy, am);
-    if (threadIdx.x == 0) part[(int64_t)blockIdx.y * pstride + blockIdx.x] = WidePart{vn2, am.a, am.idx, 0, am.sv};
+// Values handed from the workgroups of a pass to the one that finishes its block, within one launch:
+// agent-scope accesses go past the caches that the XCDs do not share.
+__device__ __forceinline__ void st_agent(double *p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double ld_agent(const double *p) {
+    return __hip_atomic_load(const_cast<double *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// reduce a wide pass's partials: sum of squares and the first argmax
-__device__ __forceinline__ void wide_reduce(const WidePart *p, int np, double &ss, AMax &am) {
-    __shared__ BlockRed<256> red;
+// every tile's partials (sum of squares, first argmax) of one block
+__device__ __forceinline__ void wide_reduce(const double *part, int t0, int nt, BlockRed<256> &red, double &ss,
+                                            AMax &am) {
     ss = 0.0;
     am = AMax{-1.0, INT_MAX, 0.0};
-    for (int w = threadIdx.x; w < np; w += 256) {
-        ss += p[w].ss;
-        AMax o{p[w].a, p[w].idx, p[w].sv};
+    for (int w = threadIdx.x; w < nt; w += 256) {
+        const double *p = part + 4 * (int64_t)(t0 + w);
+        ss += ld_agent(p);
+        AMax o{ld_agent(p + 1), (int)ld_agent(p + 2), ld_agent(p + 3)};
         amax_merge(am, o);
     }
     double dummy = 0.0;
     block_reduce<256>(red, ss, dummy, am);
 }
 
-// row reduction: the pivot column (first step: a row with a nonzero entry, else the next row)
-__global__ __launch_bounds__(256) void k_wide_row_reduce(const AcaJob *__restrict__ jobs,
-                                                         WideState *__restrict__ state,
-                                                         const WidePart *__restrict__ part, int pstride) {
-    const AcaJob jb = jobs[blockIdx.x];
-    WideState st = state[blockIdx.x];
-    if (st.done) return;
-    const int np = (jb.n + kWideCols - 1) / kWideCols;
-    double vn2;
-    AMax am;
-    wide_reduce(part + (int64_t)blockIdx.x * pstride, np, vn2, am);
-    if (threadIdx.x != 0) return;
+// the pivot column of a row pass (first step: a row with a nonzero entry, else the next row)
+__device__ __forceinline__ void wide_row_end(WideState &st, const AcaJob &jb, double vn2, const AMax &am) {
     if (st.rank == 0) {
         if (am.idx != INT_MAX && am.a > 1e-36) {
             st.cp = am.idx;
@@ -536,102 +306,26 @@ __global__ __launch_bounds__(256) void k_wide_row_reduce(const AcaJob *__restric
             st.rp = st.l;
         }
     } else if (am.idx == INT_MAX) {
-        st.done = 1;  // no unused column left
+        st.closing = 1;  // no unused column left
     } else {
         st.cp = am.idx;
         st.piv = am.sv;
         st.vn2 = vn2;
     }
-    state[blockIdx.x] = st;
 }
 
-// residual column cp -> U slot (divided by the pivot); partial sum of squares, argmax over unused rows != rp
-__global__ __launch_bounds__(256) void k_wide_col(const AcaJob *__restrict__ jobs, const int32_t *__restrict__ idx,
-                                                  const double *__restrict__ wsr, double *__restrict__ ws,
-                                                  const int64_t *__restrict__ tab_all, const uint8_t *__restrict__ flags,
-                                                  const WideState *__restrict__ state, WidePart *__restrict__ part,
-                                                  int pstride, KParams kp) {
-    const AcaJob jb = jobs[blockIdx.y];
-    const WideState st = state[blockIdx.y];
-    const int t0 = blockIdx.x * kWideCols;
-    if (st.done || t0 >= jb.m || (st.rank == 0 && !st.found)) return;
-    const int t1 = min(jb.m, t0 + kWideCols);
-    const int rank = st.rank, rp = st.rp, cp = st.cp;
-    const double piv = st.piv;
-    const int32_t *rows = idx + jb.rows, *cols = idx + jb.cols;
-    const int64_t *tab = tab_all + jb.tab;
-    const uint8_t *ru = flags + jb.wsF;
-    double *Ur = ws + st.off;
-    __shared__ double coef[kChunk];
-    __shared__ int64_t cofs[kChunk];
-    __shared__ BlockRed<256> red;
-    PointI pc = load_point(kp, cols[cp]);
-    AMax an{-1.0, INT_MAX, 0.0};
-    double un2 = 0.0;
-    double cv[kWidePT];  // (as in k_wide_row)
-#pragma unroll
-    for (int i = 0; i < kWidePT; ++i) {
-        const int t = t0 + threadIdx.x + 256 * i;
-        cv[i] = t < t1 ? kentry(kp, pc, rows[t]) : 0.0;
-    }
-    const int nch = (rank + kChunk - 1) / kChunk;
-    for (int ch = 0; ch < nch; ++ch) {
-        const int l0 = ch * kChunk, l1 = min(rank, l0 + kChunk);
-        for (int q = l0 + threadIdx.x; q < l1; q += 256) {
-            coef[q - l0] = wsr[tab[2 * q + 1] + cp];
-            cofs[q - l0] = tab[2 * q];
-        }
-        __syncthreads();
-        for (int q = l0; q < l1; ++q) {
-            const double c = coef[q - l0];
-            const double *v = wsr + cofs[q - l0];
-#pragma unroll
-            for (int i = 0; i < kWidePT; ++i) {
-                const int t = t0 + threadIdx.x + 256 * i;
-                if (t < t1) cv[i] -= c * v[t];
-            }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < kWidePT; ++i) {
-        const int t = t0 + threadIdx.x + 256 * i;
-        if (t < t1) {
-            const double u = cv[i] / piv;
-            Ur[t] = u;
-            un2 += u * u;
-            if (t != rp && !ru[t]) amax_update(an, cv[i], t);
-        }
-    }
-    double dummy = 0.0;
-    block_reduce<256>(red, un2, dummy, an);
-    if (threadIdx.x == 0) part[(int64_t)blockIdx.y * pstride + blockIdx.x] = WidePart{un2, an.a, an.idx, 0, an.sv};
-}
-
-// column reduction and acceptance of the step; the first step also checks the loop condition
-// and reserves the next step (later steps do that after the normS update)
-__global__ __launch_bounds__(256) void k_wide_accept(const AcaJob *__restrict__ jobs, WideState *__restrict__ state,
-                                                     const WidePart *__restrict__ part, int pstride,
-                                                     uint8_t *__restrict__ flags, int32_t *__restrict__ rowpiv,
-                                                     int32_t *__restrict__ colpiv, double *__restrict__ hist_all,
-                                                     int64_t *__restrict__ tab_all, unsigned long long *ws_top,
-                                                     int64_t ws_cap, double tol) {
-    const AcaJob jb = jobs[blockIdx.x];
-    WideState st = state[blockIdx.x];
-    if (st.done || (st.rank == 0 && !st.found)) return;
-    const int np = (jb.m + kWideCols - 1) / kWideCols;
-    double un2;
-    AMax an;
-    wide_reduce(part + (int64_t)blockIdx.x * pstride, np, un2, an);
-    if (threadIdx.x != 0) return;
+// Acceptance of a step after its column pass, and what the next step does.
+__device__ __forceinline__ void wide_accept(WideState &st, const AcaJob &jb, const WideBlk &wb, double un2,
+                                            const AMax &an, uint8_t *flags, int32_t *rowpiv, int32_t *colpiv,
+                                            double *hist, int64_t *tab, unsigned long long *ws_top, int64_t ws_cap,
+                                            double tol) {
     const double un = sqrt(un2), vn = sqrt(st.vn2);
     uint8_t *ru = flags + jb.wsF, *cu = ru + jb.m;
-    double *hist = hist_all + 2 * jb.piv;
+    const int mn = min(jb.m, jb.n);
     const bool fixed = st.kfix > 1 && st.dots_rank >= 0;  // (dots_rank < 0: the fixed phase was judged)
     if (st.rank > 0 && (un < 1e-36 || vn < 1e-36)) {
         st.done = 1;  // the step is dropped
         if (fixed && st.rank >= 2) st.status = 3;
-        state[blockIdx.x] = st;
         return;
     }
     rowpiv[jb.piv + st.rank] = st.rp;
@@ -642,97 +336,236 @@ __global__ __launch_bounds__(256) void k_wide_accept(const AcaJob *__restrict__ 
     st.vn = vn;
     st.next_rp = an.idx;
     ++st.rank;
+    hist[2 * (st.rank - 1)] = un * vn;
+    hist[2 * (st.rank - 1) + 1] = 0.0;
+    st.rp = st.next_rp;
     if (fixed) {
         // fixed phase: no normS update and no stopping test until kfix steps are taken (the stopping
         // rule is applied afterwards to all of them at once, from their Gram products)
-        hist[2 * (st.rank - 1)] = un * vn;
-        hist[2 * (st.rank - 1) + 1] = 0.0;
         st.dots_rank = st.rank;
-        const int mn = min(jb.m, jb.n);
         if (st.rank >= st.kfix || st.rank >= mn || st.next_rp == INT_MAX) {
             st.done = 1;
             st.status = st.rank >= st.kfix && st.rank < mn && st.next_rp != INT_MAX ? 2 : 3;
         } else {
-            st.rp = st.next_rp;
-            wide_reserve(st, jb, tab_all + jb.tab, ws_top, ws_cap);
+            wide_reserve(st, jb, wb.cap, tab, ws_top, ws_cap);
         }
-        state[blockIdx.x] = st;
+    } else if (st.rank == 1) {
+        // the first term enters without a normS update (normS stays 0)
+        st.normS = 0.0;
+        if (!(un * vn > 0.0 && st.rank < mn) || st.next_rp == INT_MAX) st.done = 1;
+        else wide_reserve(st, jb, wb.cap, tab, ws_top, ws_cap);
+    } else if (st.rank >= mn || st.next_rp == INT_MAX) {
+        st.closing = 1;
+    } else if (!wide_take(st, jb, wb.cap, tab, ws_top, ws_cap)) {
+        st.closing = 2;
+    }
+}
+
+// One pass of a pivot step over every block, one workgroup per tile of 512 entries.
+// COL = 0: residual row rp -> V slot of the current step; COL = 1: residual column cp -> U slot (divided
+// by the pivot).  Each workgroup also leaves the sum of squares and the first argmax over unused entries
+// of its tile, and its share of the inner products of the newest accepted term with every term (V columns
+// in the row pass, U columns in the column pass): the residual and the products read the same earlier
+// columns, so reading them once serves both.  The products decide whether the newest term was the last
+// one, so the step taken beside them is a step ahead of the stopping rule: the workgroup that ends the
+// column pass applies the rule first and drops the step where the rule ends the block.  (Products in a
+// pass of their own, and separate launches for the reductions: six launches and two reads per step.)
+// A block that cannot take another step whatever the rule says (every row or column used, no workspace)
+// is closing: its last passes form the products only.
+// The workgroup that arrives last on a block's counter reduces the tiles' partials, in tile order.
+template <int COL>
+__global__ __launch_bounds__(256) void k_wide_pass(const AcaJob *__restrict__ jobs, const WideBlk *__restrict__ blk,
+                                                   const int2 *__restrict__ tiles, const int32_t *__restrict__ idx,
+                                                   const double *wsr, double *ws, int64_t *tab_all, uint8_t *flags,
+                                                   WideState *state, double *part, double *pdot,
+                                                   uint32_t *__restrict__ arrived, int32_t *__restrict__ rowpiv,
+                                                   int32_t *__restrict__ colpiv, double *__restrict__ hist_all,
+                                                   unsigned long long *ws_top, int64_t ws_cap, KParams kp, double tol) {
+    typedef double D2 __attribute__((ext_vector_type(2)));
+    const int2 bt = tiles[blockIdx.x];
+    WideState st = state[bt.x];
+    if (st.done || (COL && st.rank == 0 && !st.found)) return;
+    const AcaJob jb = jobs[bt.x];
+    const WideBlk wb = blk[bt.x];
+    const int len = COL ? jb.m : jb.n;
+    const int nt = COL ? wb.nct : wb.nrt;
+    const int rank = st.rank;
+    const bool resid = !st.closing;
+    const bool dots = rank >= 2 && st.dots_rank != rank;  // the newest term's products are due
+    int64_t *tab = tab_all + jb.tab;
+    __shared__ double wpart[4][kChunk];
+    __shared__ BlockRed<256> red;
+    __shared__ int last;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int s = bt.y * kWideTile + 2 * threadIdx.x;
+    const bool in0 = s < len, in1 = s + 1 < len;
+    const int sl = in0 ? s : 0;  // (threads past the end read the column's first entries and use none of them)
+    const int pr = COL ? st.cp : st.rp;
+    const int32_t *run_i = idx + (COL ? jb.rows : jb.cols);
+    const int j0 = run_i[sl], j1 = run_i[in1 ? s + 1 : sl];
+    double r0 = 0.0, r1 = 0.0;
+    double *out = ws + st.off + (COL ? 0 : (jb.m + 1) & ~1);
+    D2 w = {0.0, 0.0};
+    if (dots && in0) w = *(const D2 *)(wsr + tab[2 * (rank - 1) + (COL ? 0 : 1)] + s);
+    double *pd = pdot + wb.pd + (int64_t)(COL ? wb.nrt + bt.y : bt.y) * wb.cap;
+    // The earlier terms' column offsets and coefficients (this tile's residual row or column at their
+    // pivots): lane q of a wave holds those of term l0 + q, the next 64 terms' are on their way, and each
+    // term's are broadcast from there.  Groups of kWideU columns are loaded two ahead, unconditionally, so
+    // that the waits count exactly the loads in flight; past the last term they read its column again
+    // (at rank 0 the step's own, unwritten one) and are masked.
+    auto term = [&](int l) { return *(const longlong2 *)(tab + 2 * max(0, min(l + lane, rank - 1))); };
+    auto weight = [&](const longlong2 &o, int l) {
+        return resid && l + lane < rank ? wsr[(COL ? o.y : o.x) + pr] : 0.0;
+    };
+    auto lane_of = [&](int64_t v, int l) -> int64_t {
+        const int lo = __builtin_amdgcn_readlane((int)v, l), hi = __builtin_amdgcn_readlane((int)(v >> 32), l);
+        return ((int64_t)hi << 32) | (uint32_t)lo;
+    };
+    D2 A[kWideU], B[kWideU];
+    auto load = [&](D2(&v)[kWideU], const longlong2 &o, int q) {
+#pragma unroll
+        for (int u = 0; u < kWideU; ++u) v[u] = *(const D2 *)(wsr + lane_of(COL ? o.x : o.y, q + u) + sl);
+    };
+    auto use = [&](D2(&v)[kWideU], double cf, int l0, int q) {
+        if (l0 + q + kWideU > rank) {
+#pragma unroll
+            for (int u = 0; u < kWideU; ++u)
+                if (l0 + q + u >= rank) v[u] = (D2)0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < kWideU; ++u) {
+            const double c = __longlong_as_double(lane_of(__double_as_longlong(cf), q + u));
+            r0 -= c * v[u].x;
+            r1 -= c * v[u].y;
+        }
+        if (dots) {
+            typedef double D8 __attribute__((ext_vector_type(kWideU)));
+            D8 p;
+#pragma unroll
+            for (int u = 0; u < kWideU; ++u) p[u] = fma(v[u].y, w.y, v[u].x * w.x);
+            // sums over the wave: three exchanges that halve the values per lane, then three plain ones
+            int ui = 0;
+#pragma unroll
+            for (int k = kWideU, o = 1; k > 1; k >>= 1, o <<= 1) {
+                const bool hi = lane & o;
+#pragma unroll
+                for (int i = 0; i < k / 2; ++i) {
+                    const double snd = hi ? p[i] : p[i + k / 2];
+                    const double keep = hi ? p[i + k / 2] : p[i];
+                    p[i] = keep + (o == 1 ? fold_lane<1>(snd) : o == 2 ? fold_lane<2>(snd) : fold_lane<4>(snd));
+                }
+                ui += hi ? k / 2 : 0;
+            }
+            const double t = sum_halves(p[0] + fold_lane<8>(p[0]));
+            if (lane < kWideU) wpart[wv][((l0 + q) & (kChunk - 1)) + ui] = t;
+        }
+    };
+    longlong2 o0 = term(0), o1 = term(64);
+    double cf0 = weight(o0, 0);
+    load(A, o0, 0);
+    load(B, o0, kWideU);
+    if (resid) {
+        // (the entries' own loads and logarithms pass behind the first groups; a closing block has no row
+        // or column pr)
+        const PointI p = load_point(kp, (idx + (COL ? jb.cols : jb.rows))[pr]);
+        r0 = kentry(kp, p, j0);
+        r1 = kentry(kp, p, j1);
+    }
+    for (int l0 = 0; l0 < rank; l0 += 64) {
+        const double cf1 = weight(o1, l0 + 64);
+        const longlong2 o2 = term(l0 + 128);
+        for (int q = 0; q < 64 && l0 + q < rank; q += 2 * kWideU) {
+            const bool nx = q + 2 * kWideU == 64;
+            const longlong2 on{nx ? o1.x : o0.x, nx ? o1.y : o0.y};
+            const int qn = (q + 2 * kWideU) & 63;
+            use(A, cf0, l0, q);
+            load(A, on, qn);
+            use(B, cf0, l0, q + kWideU);
+            load(B, on, qn + kWideU);
+        }
+        o0 = o1;
+        o1 = o2;
+        cf0 = cf1;
+        if (dots && (l0 + 64 >= rank || ((l0 + 64) & (kChunk - 1)) == 0)) {
+            // the waves' sums of up to kChunk terms
+            const int f0 = l0 / kChunk * kChunk, nq = min(rank - f0, kChunk);
+            __syncthreads();
+            for (int q = threadIdx.x; q < nq; q += 256)
+                st_agent(pd + f0 + q, (wpart[0][q] + wpart[1][q]) + (wpart[2][q] + wpart[3][q]));
+            __syncthreads();
+        }
+    }
+    double ss = 0.0, dummy = 0.0;
+    AMax am{-1.0, INT_MAX, 0.0};
+    if (resid) {
+        const uint8_t *used = flags + jb.wsF + (COL ? 0 : jb.m);
+        double v0 = in0 ? r0 : 0.0, v1 = in1 ? r1 : 0.0;
+        if (in0 && !used[s] && !(COL && s == st.rp)) amax_update(am, v0, s);
+        if (in1 && !used[s + 1] && !(COL && s + 1 == st.rp)) amax_update(am, v1, s + 1);
+        if (COL) {
+            v0 = v0 / st.piv;
+            v1 = in1 ? v1 / st.piv : 0.0;
+        }
+        if (in0) {
+            ss = v0 * v0 + v1 * v1;
+            *(D2 *)(out + s) = D2{v0, v1};  // (the padding entry of an odd column is zero)
+        }
+    }
+    block_reduce<256>(red, ss, dummy, am);
+    if (threadIdx.x == 0) {
+        double *p = part + 4 * (int64_t)((COL ? wb.ct0 : wb.rt0) + bt.y);
+        st_agent(p, ss);
+        st_agent(p + 1, am.a);
+        st_agent(p + 2, (double)am.idx);
+        st_agent(p + 3, am.sv);
+    }
+    // every partial of this workgroup is at the coherence point before its arrival is counted
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x == 0) last = atomicAdd(arrived + bt.x, 1u) == (uint32_t)(nt - 1);
+    __syncthreads();
+    if (!last) return;
+
+    // ---- the block's last workgroup of this pass
+    wide_reduce(part, COL ? wb.ct0 : wb.rt0, nt, red, ss, am);
+    if (!COL) {
+        if (threadIdx.x != 0) return;
+        arrived[bt.x] = 0;
+        if (resid) wide_row_end(st, jb, ss, am);
+        if (st.closing && !dots) st.done = 1;  // nothing left to form
+        state[bt.x] = st;
         return;
     }
-    if (st.rank == 1) {
-        // the first term enters without a normS update (normS stays 0)
-        hist[0] = un * vn;
-        hist[1] = 0.0;
-        st.normS = 0.0;
-        const int mn = min(jb.m, jb.n);
-        if (!(un * vn > tol * st.normS && st.rank < mn) || st.next_rp == INT_MAX) st.done = 1;
-        else {
-            st.rp = st.next_rp;
-            wide_reserve(st, jb, tab_all + jb.tab, ws_top, ws_cap);
-        }
-    }
-    state[blockIdx.x] = st;
-}
-
-// |<U_q, u><V_q, v>| of the newest term (u, v) with every term q <= newest, one workgroup per q
-__global__ __launch_bounds__(256) void k_wide_dots(const AcaJob *__restrict__ jobs, const double *__restrict__ ws,
-                                                   const int64_t *__restrict__ tab_all,
-                                                   const WideState *__restrict__ state, double *__restrict__ dots,
-                                                   int dstride) {
-    const AcaJob jb = jobs[blockIdx.y];
-    const WideState st = state[blockIdx.y];
-    const int q = blockIdx.x;
-    if (st.done || st.rank < 2 || q >= st.rank || st.dots_rank == st.rank) return;
-    const int64_t *tab = tab_all + jb.tab;
-    const double *Uq = ws + tab[2 * q], *Vq = ws + tab[2 * q + 1];
-    const double *Uk = ws + tab[2 * (st.rank - 1)], *Vk = ws + tab[2 * (st.rank - 1) + 1];
-    // four partial sums per thread: four independent load pairs in flight
-    auto dot = [](const double *a, const double *b, int len) {
-        double p0 = 0.0, p1 = 0.0, p2 = 0.0, p3 = 0.0;
-        int t = threadIdx.x;
-        for (; t + 768 < len; t += 1024) {
-            p0 += a[t] * b[t];
-            p1 += a[t + 256] * b[t + 256];
-            p2 += a[t + 512] * b[t + 512];
-            p3 += a[t + 768] * b[t + 768];
-        }
-        for (; t < len; t += 256) p0 += a[t] * b[t];
-        return (p0 + p1) + (p2 + p3);
-    };
-    double du = dot(Uq, Uk, jb.m), dv = dot(Vq, Vk, jb.n);
-    __shared__ BlockRed<256> red;
-    AMax dummy{-1.0, INT_MAX, 0.0};
-    block_reduce<256>(red, du, dv, dummy);
-    if (threadIdx.x == 0) dots[(int64_t)blockIdx.y * dstride + q] = fabs(du * dv);
-}
-
-// normS update of the newest term, loop condition, next step's reservation
-__global__ __launch_bounds__(256) void k_wide_norm(const AcaJob *__restrict__ jobs, WideState *__restrict__ state,
-                                                   const double *__restrict__ dots, int dstride,
-                                                   double *__restrict__ hist_all, int64_t *__restrict__ tab_all,
-                                                   unsigned long long *ws_top, int64_t ws_cap, double tol) {
-    const AcaJob jb = jobs[blockIdx.x];
-    WideState st = state[blockIdx.x];
-    if (st.done || st.rank < 2 || st.dots_rank == st.rank) return;
-    double S = 0.0, dummy = 0.0;
-    for (int q = threadIdx.x; q < st.rank; q += 256) S += dots[(int64_t)blockIdx.x * dstride + q];
-    __shared__ BlockRed<256> red;
-    AMax am{-1.0, INT_MAX, 0.0};
-    block_reduce<256>(red, S, dummy, am);
-    if (threadIdx.x != 0) return;
-    const double uv = st.un * st.vn;
-    st.normS = sqrt(st.normS * st.normS + uv * uv + 2.0 * S);
     double *hist = hist_all + 2 * jb.piv;
-    hist[2 * (st.rank - 1)] = uv;
-    hist[2 * (st.rank - 1) + 1] = st.normS;
-    st.dots_rank = st.rank;
     const int mn = min(jb.m, jb.n);
-    if (!(uv > tol * st.normS && st.rank < mn) || st.next_rp == INT_MAX) st.done = 1;
-    else {
-        st.rp = st.next_rp;
-        wide_reserve(st, jb, tab_all + jb.tab, ws_top, ws_cap);
+    if (dots) {
+        double S = 0.0;
+        for (int q = threadIdx.x; q < rank; q += 256) {
+            double du = 0.0, dv = 0.0;
+            const double *pv = pdot + wb.pd + q, *pu = pv + (int64_t)wb.nrt * wb.cap;
+#pragma unroll 8
+            for (int t = 0; t < wb.nrt; ++t) dv += ld_agent(pv + (int64_t)t * wb.cap);
+#pragma unroll 8
+            for (int t = 0; t < wb.nct; ++t) du += ld_agent(pu + (int64_t)t * wb.cap);
+            S += fabs(du * dv);
+        }
+        AMax none{-1.0, INT_MAX, 0.0};
+        block_reduce<256>(red, S, dummy, none);
+        const double uv = st.un * st.vn;
+        st.normS = sqrt(st.normS * st.normS + uv * uv + 2.0 * S);
+        st.dots_rank = rank;
+        const bool more = uv > tol * st.normS && rank < mn;
+        if (threadIdx.x == 0) hist[2 * (rank - 1) + 1] = st.normS;
+        if (!more || st.closing) {
+            st.done = 1;
+            if (more && st.closing == 2) st.status = 1;  // out of workspace before the rule was met
+        }
     }
-    state[blockIdx.x] = st;
+    if (threadIdx.x != 0) return;
+    arrived[bt.x] = 0;
+    if (!st.done)
+        wide_accept(st, jb, wb, ss, am, flags, rowpiv, colpiv, hist, tab, ws_top, ws_cap, tol);
+    state[bt.x] = st;
 }
 
 __global__ void k_wide_finish(const WideState *__restrict__ state, int nb, int32_t *__restrict__ rank_out,
@@ -806,7 +639,8 @@ __global__ __launch_bounds__(256) void k_wide_gram(const GramJob *__restrict__ g
 }
 
 // decisions of the host on the judged blocks (one thread per block)
-__global__ void k_wide_judge(const AcaJob *__restrict__ jobs, int nb, WideState *__restrict__ state,
+__global__ void k_wide_judge(const AcaJob *__restrict__ jobs, const WideBlk *__restrict__ blk, int nb,
+                             WideState *__restrict__ state,
                              const int32_t *__restrict__ final_rank, const double *__restrict__ normS_in,
                              int64_t *__restrict__ tab_all, unsigned long long *ws_top, int64_t ws_cap) {
     for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < nb; b += gridDim.x * blockDim.x) {
@@ -826,7 +660,7 @@ __global__ void k_wide_judge(const AcaJob *__restrict__ jobs, int nb, WideState 
             st.status = 0;
             st.kfix = 0;
             st.rp = st.next_rp;
-            wide_reserve(st, jobs[b], tab_all + jobs[b].tab, ws_top, ws_cap);
+            wide_reserve(st, jobs[b], blk[b].cap, tab_all + jobs[b].tab, ws_top, ws_cap);
         }
         state[b] = st;
     }
@@ -981,39 +815,6 @@ __global__ void k_cur(const CurJob *__restrict__ jobs, const int32_t *__restrict
 template <typename V>
 __device__ __forceinline__ V ld_nt(const V *p) {
     return __builtin_nontemporal_load((const __attribute__((address_space(1))) V *)p);
-}
-
-// Value of lane (lane ^ O) for a power of two O < 64: quad permutes (DPP) for 1 and 2,
-// ds_swizzle in its bit-mask mode for 4 .. 16, ds_bpermute for 32.  Every lane of the
-// aligned group of 2 O lanes must be active.
-template <int O>
-__device__ __forceinline__ int xor_lane(int v) {
-    if constexpr (O == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false);
-    else if constexpr (O == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false);
-    else if constexpr (O < 32) return __builtin_amdgcn_ds_swizzle(v, 0x1F | (O << 10));
-    else return __builtin_amdgcn_ds_bpermute((int)(((threadIdx.x & 63) ^ O) << 2), v);
-}
-template <int O>
-__device__ __forceinline__ float xor_lane(float v) {
-    return __int_as_float(xor_lane<O>(__float_as_int(v)));
-}
-template <int O>
-__device__ __forceinline__ double xor_lane(double v) {
-    const int64_t b = __double_as_longlong(v);
-    const int lo = xor_lane<O>((int)(uint32_t)b), hi = xor_lane<O>((int)(b >> 32));
-    return __longlong_as_double((int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo));
-}
-// the same with O known only after unrolling
-template <typename T>
-__device__ __forceinline__ T xor_lane_n(T v, int o) {
-    switch (o) {
-    case 1: return xor_lane<1>(v);
-    case 2: return xor_lane<2>(v);
-    case 4: return xor_lane<4>(v);
-    case 8: return xor_lane<8>(v);
-    case 16: return xor_lane<16>(v);
-    default: return xor_lane<32>(v);
-    }
 }
 
 // Raw buffer access (gfx9 resource word 3): a lane whose offset lies at or past the
@@ -2539,15 +2340,6 @@ inline int grid_for(int64_t n, int nt = 256, int cap = 8192) {
 }  // namespace
 
 // ------------------------------------------------------------------ launch wrappers
-void launch_aca(const AcaJob *jobs, int njobs, const int32_t *idx, double *ws, int64_t ws_cap,
-                unsigned long long *ws_top, int64_t *tab, uint8_t *flags, int32_t *rank, int32_t *status,
-                int32_t *rowpiv, int32_t *colpiv, KParams kp, double tol, double *hist, int big, hipStream_t s) {
-    if (njobs <= 0) return;
-    if (big) hipLaunchKernelGGL(k_aca<1024>, dim3(njobs), dim3(1024), 0, s, jobs, idx, ws, ws_cap, ws_top, tab, flags,
-                                rank, status, rowpiv, colpiv, kp, tol, hist);
-    else hipLaunchKernelGGL(k_aca<256>, dim3(njobs), dim3(256), 0, s, jobs, idx, ws, ws_cap, ws_top, tab, flags, rank,
-                            status, rowpiv, colpiv, kp, tol, hist);
-}
 void launch_lr_extract(const LrJob *jobs, int njobs, const double *ws, const int64_t *tab, const int32_t *rowpiv,
                        const int32_t *colpiv, double *out, hipStream_t s) {
     if (njobs > 0)
@@ -2794,55 +2586,31 @@ void launch_scatter_b(const double *v, const int64_t *src, const int32_t *ld, in
 void launch_rank_mlp(const float *feat, int n, const uint16_t *w, float *out, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_rank_mlp, dim3((n + 255) / 256), dim3(256), 0, s, feat, n, w, out);
 }
-void launch_wide_init(const AcaJob *jobs, int nb, int maxmn, WideState *state, uint8_t *flags, int64_t *tab,
+void launch_wide_init(const AcaJob *jobs, const WideBlk *blk, int nb, WideState *state, uint8_t *flags, int64_t *tab,
                       unsigned long long *ws_top, int64_t ws_cap, hipStream_t s) {
-    hipLaunchKernelGGL(k_wide_init, dim3(std::max(1, std::min(1024, (maxmn + 2047) / 2048)), nb), dim3(256), 0, s,
-                       jobs, state, flags, tab, ws_top, ws_cap);
+    hipLaunchKernelGGL(k_wide_init, dim3(nb), dim3(256), 0, s, jobs, blk, state, flags, tab, ws_top, ws_cap);
 }
-void launch_wide_step(const AcaJob *jobs, int nb, int maxm, int maxn, int maxrank, const int32_t *idx, double *ws,
-                      int64_t *tab, uint8_t *flags, WideState *state, WidePart *part, int pstride, double *dots,
-                      int dstride, int32_t *rowpiv, int32_t *colpiv, double *hist, unsigned long long *ws_top,
-                      int64_t ws_cap, KParams kp, double tol, hipStream_t s) {
-    const int gr = std::max(1, (maxn + kWideCols - 1) / kWideCols), gc = std::max(1, (maxm + kWideCols - 1) / kWideCols);
-    hipLaunchKernelGGL(k_wide_row, dim3(gr, nb), dim3(256), 0, s, jobs, idx, ws, ws, tab, flags, state, part, pstride,
-                       kp);
-    hipLaunchKernelGGL(k_wide_row_reduce, dim3(nb), dim3(256), 0, s, jobs, state, part, pstride);
-    hipLaunchKernelGGL(k_wide_col, dim3(gc, nb), dim3(256), 0, s, jobs, idx, ws, ws, tab, flags, state, part, pstride,
-                       kp);
-    hipLaunchKernelGGL(k_wide_accept, dim3(nb), dim3(256), 0, s, jobs, state, part, pstride, flags, rowpiv, colpiv,
-                       hist, tab, ws_top, ws_cap, tol);
-    if (maxrank >= 2) {
-        hipLaunchKernelGGL(k_wide_dots, dim3(std::max(1, maxrank), nb), dim3(256), 0, s, jobs, ws, tab, state, dots,
-                           dstride);
-        hipLaunchKernelGGL(k_wide_norm, dim3(nb), dim3(256), 0, s, jobs, state, dots, dstride, hist, tab, ws_top,
-                           ws_cap, tol);
-    }
+int wide_tile() { return kWideTile; }
+void launch_wide_step(const AcaJob *jobs, const WideArgs &w, const int32_t *idx, double *ws, int64_t *tab,
+                      uint8_t *flags, WideState *state, int32_t *rowpiv, int32_t *colpiv, double *hist,
+                      unsigned long long *ws_top, int64_t ws_cap, KParams kp, double tol, hipStream_t s) {
+    hipLaunchKernelGGL(k_wide_pass<0>, dim3(w.nrow), dim3(256), 0, s, jobs, w.blk, w.tiles, idx, ws, ws, tab, flags,
+                       state, w.part, w.pdot, w.arrived, rowpiv, colpiv, hist, ws_top, ws_cap, kp, tol);
+    hipLaunchKernelGGL(k_wide_pass<1>, dim3(w.ncol), dim3(256), 0, s, jobs, w.blk, w.tiles + w.nrow, idx, ws, ws, tab,
+                       flags, state, w.part, w.pdot, w.arrived, rowpiv, colpiv, hist, ws_top, ws_cap, kp, tol);
 }
 void launch_wide_finish(const WideState *state, int nb, int32_t *rank_out, int32_t *status_out, int32_t *ndone,
                         hipStream_t s) {
     hipLaunchKernelGGL(k_wide_finish, dim3(1), dim3(64), 0, s, state, nb, rank_out, status_out, ndone);
 }
-void launch_wide_fixed_step(const AcaJob *jobs, int nb, int maxm, int maxn, const int32_t *idx, double *ws,
-                            int64_t *tab, uint8_t *flags, WideState *state, WidePart *part, int pstride,
-                            int32_t *rowpiv, int32_t *colpiv, double *hist, unsigned long long *ws_top, int64_t ws_cap,
-                            KParams kp, double tol, hipStream_t s) {
-    const int gr = std::max(1, (maxn + kWideCols - 1) / kWideCols), gc = std::max(1, (maxm + kWideCols - 1) / kWideCols);
-    hipLaunchKernelGGL(k_wide_row, dim3(gr, nb), dim3(256), 0, s, jobs, idx, ws, ws, tab, flags, state, part, pstride,
-                       kp);
-    hipLaunchKernelGGL(k_wide_row_reduce, dim3(nb), dim3(256), 0, s, jobs, state, part, pstride);
-    hipLaunchKernelGGL(k_wide_col, dim3(gc, nb), dim3(256), 0, s, jobs, idx, ws, ws, tab, flags, state, part, pstride,
-                       kp);
-    hipLaunchKernelGGL(k_wide_accept, dim3(nb), dim3(256), 0, s, jobs, state, part, pstride, flags, rowpiv, colpiv,
-                       hist, tab, ws_top, ws_cap, tol);
-}
 void launch_wide_gram(const GramJob *gj, int njobs, const AcaJob *jobs, const WideState *state, const double *ws,
                       const int64_t *tab, double *prod, hipStream_t s) {
     if (njobs > 0) hipLaunchKernelGGL(k_wide_gram, dim3(njobs), dim3(256), 0, s, gj, jobs, state, ws, tab, prod);
 }
-void launch_wide_judge(const AcaJob *jobs, int nb, WideState *state, const int32_t *final_rank, const double *normS_in,
-                       int64_t *tab, unsigned long long *ws_top, int64_t ws_cap, hipStream_t s) {
+void launch_wide_judge(const AcaJob *jobs, const WideBlk *blk, int nb, WideState *state, const int32_t *final_rank,
+                       const double *normS_in, int64_t *tab, unsigned long long *ws_top, int64_t ws_cap, hipStream_t s) {
     if (nb > 0)
-        hipLaunchKernelGGL(k_wide_judge, dim3((nb + 63) / 64), dim3(64), 0, s, jobs, nb, state, final_rank, normS_in,
+        hipLaunchKernelGGL(k_wide_judge, dim3((nb + 63) / 64), dim3(64), 0, s, jobs, blk, nb, state, final_rank, normS_in,
                            tab, ws_top, ws_cap);
 }
 void launch_aca_sample(const AcaJob *jobs, int nb, const int32_t *rank, const int32_t *idx, const double *ws,
