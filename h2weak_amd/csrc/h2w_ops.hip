@@ -943,55 +943,68 @@ void add_item_whole(WorkList &W, int64_t y, int64_t xb, int rows, const std::vec
     }
 }
 
-// A launch of few large items (the transfer passes near the root) leaves most of the
-// GPU idle while a handful of workgroups stream their items: split such items by
-// columns (the pieces accumulate atomically) until the launch has about kMinItems
-// items of at least kMinPiece elements.  Lists with symmetric terms are left alone.
+// A launch of few large items leaves part of the GPU idle while the last of them stream: the transfer
+// passes near the root, the semi-nested factors of the large boxes beside the small ones', and the fused
+// M2L + near-field launch of anything but the largest systems.  Items above twice the launch's mean at
+// about so many items are split by columns (the pieces accumulate atomically): 2048 for transfers and
+// column factors, where an item is one column run, and 8192 for the fused launch, whose items are runs of
+// blocks and accumulate atomically anyway.
+// Measured (fused launch, FP64, unsplit / 2048 / 4096 / 8192 / 16384 items): 3D N = 20011 279 / 166 / 139 /
+// 137 / 141 us, 32^3 grid at 1e-10 472 / 363 / 343 / 323 / 313 us, 2D N = 90000 191 / 195 / 176 / 174 /
+// 178 us; complex 32^3 product 879 / 884 / 736 / 726 / 653 us.  The 16-wide launch stages its item's input
+// rows and likes larger pieces: 328 / 250 / 265 / 275 / 327 us and 565 / 486 / 486 / 514 / 598 us.  The
+// leaf launch of the 2D semi-nested 400 x 400 grid (more than 2048 items, some of 4 MB) 214 -> 137 us.
 constexpr int64_t kMinItems = 2048, kMinPiece = 128 * 64;
+constexpr int64_t kMinItemsFused = 8192, kMinPieceFused = 128 * 128;
 void rebalance(WorkList &W) {
-    if ((int64_t)W.items.size() >= kMinItems) return;
+    const bool fused = W.role == 1;
     int64_t E = 0;
     for (auto &it : W.items)
-        for (int32_t k = it.t0; k < it.t1; ++k) {
-            if (W.terms[k].t >= 0) return;
-            E += (int64_t)it.rows * W.terms[k].cols;
-        }
-    const int64_t target = std::max<int64_t>(E / kMinItems, kMinPiece);
+        for (int32_t k = it.t0; k < it.t1; ++k) E += (int64_t)it.rows * W.terms[k].cols;
+    const int64_t target = std::min(kItemWork, std::max<int64_t>(E / (fused ? kMinItemsFused : kMinItems),
+                                                                 fused ? kMinPieceFused : kMinPiece));
     WorkList out;
     out.role = W.role;
     out.stage = W.stage;
     out.step = W.step;
+    out.items.reserve(W.items.size());
+    out.terms.reserve(W.terms.size());
     for (const GItem &it : W.items) {
         int64_t work = 0;
         for (int32_t k = it.t0; k < it.t1; ++k) work += (int64_t)it.rows * W.terms[k].cols;
         GItem nt = it;
         nt.t0 = (int32_t)out.terms.size();
         if (work <= 2 * target) {
-            for (int32_t k = it.t0; k < it.t1; ++k) out.terms.push_back(W.terms[k]);
+            out.terms.insert(out.terms.end(), W.terms.begin() + it.t0, W.terms.begin() + it.t1);
             nt.t1 = (int32_t)out.terms.size();
             out.items.push_back(nt);
             continue;
         }
-        const int64_t maxc = std::max<int64_t>(1, target / it.rows);
+        // equal pieces of whole 16-column groups; a piece ends early rather than cut a term in two
+        const int64_t np = (work + target - 1) / target;
+        const int64_t maxc = align_up((work / it.rows + np - 1) / np, 16);
         nt.flags |= 1;
         int64_t used = 0;
+        auto close = [&]() {
+            nt.t1 = (int32_t)out.terms.size();
+            if (nt.t1 > nt.t0) out.items.push_back(nt);
+            nt.t0 = nt.t1;
+            used = 0;
+        };
         for (int32_t k = it.t0; k < it.t1; ++k) {
             const GTerm &t = W.terms[k];
+            if (used > 0 && t.cols <= maxc && used + t.cols > maxc + maxc / 4) close();
             for (int64_t c0 = 0; c0 < t.cols;) {
-                const int64_t take = std::min<int64_t>(t.cols - c0, maxc - used);
-                out.terms.push_back(GTerm{t.a + c0 * it.lda, t.x + c0, -1, (int32_t)take, t.ld});
+                const int64_t left = t.cols - c0;
+                const int64_t take = left <= maxc + maxc / 4 - used ? left : maxc - used;
+                out.terms.push_back(
+                    GTerm{t.a + c0 * it.lda, t.x + c0, t.t >= 0 ? t.t + c0 : -1, (int32_t)take, t.ld});
                 used += take;
                 c0 += take;
-                if (used == maxc) {
-                    nt.t1 = (int32_t)out.terms.size();
-                    out.items.push_back(nt);
-                    nt.t0 = nt.t1;
-                    used = 0;
-                }
+                if (used >= maxc) close();
             }
         }
-        nt.t1 = (int32_t)out.terms.size();
-        if (nt.t1 > nt.t0) out.items.push_back(nt);
+        close();
     }
     W = std::move(out);
 }
@@ -1403,7 +1416,7 @@ void build_inner(Handle &h, double irp) {
             IL.push_back(std::move(W));
         }
         for (auto &W : IL)
-            if (W.role == 0) rebalance(W);
+            rebalance(W);
         upload_lists(IL, h.inner, s);
         h.inner_elems = 0;
         for (auto e : h.inner.elems) h.inner_elems += e;
@@ -1889,7 +1902,7 @@ void assemble_operators(Handle &h, double t0) {
     std::vector<GItem> items;
     std::vector<GTerm> terms;
     for (auto &W : WL)
-        if (W.role == 0) rebalance(W);
+        rebalance(W);
     h.launches.clear();
     for (auto &W : WL) {
         if (W.items.empty()) continue;
