@@ -943,6 +943,31 @@ void add_item_whole(WorkList &W, int64_t y, int64_t xb, int rows, const std::vec
     }
 }
 
+// Terms of an item whose blocks and vector segments follow one another become one: a box's blocks with
+// consecutive partner boxes (their segments are in box order), a semi-nested box's pairs.  The kernels walk
+// an item's terms one by one, about 1 us a term and wave from the next term's descriptor to its data, so
+// short ones cost them most of their time: fused launch of the 16^3 grid (leaves of 8 points) 63 -> 22 us,
+// 2D semi-nested 400 x 400 106 -> 101 us, its column factors 111 -> 106 us, 3D semi-nested N = 20000
+// 110 -> 104 us; 16-wide 276 -> 258 us at 3D N = 20011.
+void merge_terms(WorkList &W) {
+    size_t n = 0;
+    for (GItem &it : W.items) {
+        const size_t t0 = n;
+        for (int32_t k = it.t0; k < it.t1; ++k) {
+            const GTerm t = W.terms[k];
+            GTerm *p = n > t0 ? &W.terms[n - 1] : nullptr;
+            const bool sym = t.t >= 0;
+            if (p && (p->t >= 0) == sym && t.a == p->a + (int64_t)p->cols * it.lda && t.x == p->x + p->cols &&
+                (!sym || t.t == p->t + p->cols) && t.ld == p->ld)
+                p->cols += t.cols;
+            else W.terms[n++] = t;
+        }
+        it.t0 = (int32_t)t0;
+        it.t1 = (int32_t)n;
+    }
+    W.terms.resize(n);
+}
+
 // A launch of few large items leaves part of the GPU idle while the last of them stream: the transfer
 // passes near the root, the semi-nested factors of the large boxes beside the small ones', and the fused
 // M2L + near-field launch of anything but the largest systems.  Items above twice the launch's mean at
@@ -957,6 +982,7 @@ void add_item_whole(WorkList &W, int64_t y, int64_t xb, int rows, const std::vec
 constexpr int64_t kMinItems = 2048, kMinPiece = 128 * 64;
 constexpr int64_t kMinItemsFused = 8192, kMinPieceFused = 128 * 128;
 void rebalance(WorkList &W) {
+    merge_terms(W);
     const bool fused = W.role == 1;
     int64_t E = 0;
     for (auto &it : W.items)
@@ -1173,9 +1199,14 @@ void build_inner(Handle &h, double irp) {
         for (size_t q = 0; q < m2l.size(); ++q) {
             const M2LBlk &m = m2l[q];
             const FamLevel &fl = h.fam[m.f][m.j];
-            if (fl.kin[m.b] > 0 && fl.kin[m.p] > 0)
-                m2l_in.push_back({q, take_in(pad_ld(fl.kin[m.b]) * fl.kin[m.p])});
+            // (the blocks of one box one after another, as in the full operator)
+            if (q > 0 && (m2l[q - 1].f != m.f || m2l[q - 1].j != m.j || m2l[q - 1].b != m.b)) in_len = align_up(in_len, 32);
+            if (fl.kin[m.b] > 0 && fl.kin[m.p] > 0) {
+                m2l_in.push_back({q, in_len});
+                in_len += pad_ld(fl.kin[m.b]) * fl.kin[m.p];
+            }
         }
+        in_len = align_up(in_len, 32);
     }
     if (inner_on) h.mat32in.alloc(std::max<int64_t>(in_len, 32));
     if (inner_on && in_len > 0) H2W_HIP(hipMemsetAsync(h.mat32in.p, 0, in_len * 4, s));
@@ -1522,6 +1553,11 @@ void assemble_operators(Handle &h, double t0) {
         mo += align_up(elems, 32);
         return o;
     };
+    auto run = [&](int64_t elems) {  // right behind the block before (columns are multiples of 4 elements)
+        int64_t o = mo;
+        mo += elems;
+        return o;
+    };
     double memory = 0.0;
     for (int f = 0; f < 2; ++f) {
         if (!fam_on[f]) continue;
@@ -1545,15 +1581,18 @@ void assemble_operators(Handle &h, double t0) {
         for (int j = nfam_lo[f]; j <= P.nL; ++j) {
             FamLevel &fl = h.fam[f][j];
             for (int b = 0; b < fl.nb; ++b) {
+                // (in box order, one after another: neighbouring partners then form one run of columns)
                 auto partners = f == 0 ? P.far_of(j, b) : P.vert_of(j, b);
+                std::sort(partners.begin(), partners.end());
                 for (int p : partners) {
                     int64_t e = (int64_t)fl.rank[b] * fl.rank[p];
                     memory += (double)e;  // the reference counts both directions
                     // K(Ir_p, Ir_b) = K(Ir_b, Ir_p)^T entry for entry (the kernel depends on |x - y|
                     // only): one block per unordered pair, the lower-numbered box's
                     if (e == 0 || p < b) continue;
-                    m2l.push_back(M2LBlk{f, j, b, p, take(pad_ld(fl.rank[b]) * fl.rank[p])});
+                    m2l.push_back(M2LBlk{f, j, b, p, run(pad_ld(fl.rank[b]) * fl.rank[p])});
                 }
+                mo = align_up(mo, 32);
             }
         }
     }
@@ -1563,13 +1602,15 @@ void assemble_operators(Handle &h, double t0) {
     const bool count_near = !(P.dim == 1 && h.variant == H2W_SEMI_NESTED);  // 1D findMemory_sn skips it
     for (int b = 0; b < nleaf; ++b) {
         std::vector<int32_t> lst = P.near[b];
-        lst.push_back(b);  // self last (3D/codes/HODLR3Dtree.hpp:2388)
+        lst.push_back(b);
+        std::sort(lst.begin(), lst.end());
         for (int n : lst) {
             int64_t e = P.bcount[P.nL][b] * P.bcount[P.nL][n];
             if (count_near) memory += (double)e;
             if (e == 0 || n < b) continue;  // one block per unordered pair (self blocks kept)
-            nearb.push_back(NearBlk{b, n, take(pad_ld(P.bcount[P.nL][b]) * P.bcount[P.nL][n])});
+            nearb.push_back(NearBlk{b, n, run(pad_ld(P.bcount[P.nL][b]) * P.bcount[P.nL][n])});
         }
+        mo = align_up(mo, 32);
     }
     for (auto &p : h.pairs) {
         int64_t mb = P.bcount[p.level][p.b], nv = P.bcount[p.level][p.v];
@@ -1577,9 +1618,15 @@ void assemble_operators(Handle &h, double t0) {
         else memory += 2.0 * p.rank * p.rank + (double)(mb * p.rank + (int64_t)p.rank * nv);  // L + R + Ac + Ar
         p.ac_off = p.ar_off = -1;
         if (p.rank == 0) continue;
-        p.ac_off = take(pad_ld(mb) * p.rank);
         p.ar_off = take(pad_ld(p.rank) * nv);
     }
+    // (the pairs of one box are consecutive, and so are their intermediate vectors: one run of columns)
+    for (size_t q = 0; q < h.pairs.size(); ++q) {
+        Pair &p = h.pairs[q];
+        if (q > 0 && (h.pairs[q - 1].level != p.level || h.pairs[q - 1].b != p.b)) mo = align_up(mo, 32);
+        if (p.rank > 0) p.ac_off = run(pad_ld(P.bcount[p.level][p.b]) * p.rank);
+    }
+    mo = align_up(mo, 32);
     h.mat_len = std::max<int64_t>(mo, 32);
     h.memory = memory;
     // (complex kernels: pools of (re, im) pairs at the same element offsets)
