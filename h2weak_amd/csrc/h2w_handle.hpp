@@ -164,6 +164,14 @@ struct Launch {
 inline bool per_wave_items(const Launch &L) {
     return L.nitems >= 2048 && L.avg_item_elems > 0 && L.avg_item_elems <= 4096;
 }
+// The same on the single-vector path.  Measured, four waves / one wave per item: 1D N = 250000 leaf up
+// pass (4096 items of 1500 elements on average) 21 / 16 us and fused launch (8000 of 2200) 50 / 40 us, 2D
+// semi-nested 400 x 400 fused launch (of 7500) 101 / 92 us and column factors 106 / 99 us.  Above 8192
+// elements the four waves win: 3D N = 20011 fused (of 10300) 134 / 177 us; so they do with fewer than 2048
+// items, which leave compute units without a wave: 16^3 fused 22 / 48 us.
+inline bool per_wave_gemv(const Launch &L) {
+    return L.nitems >= 2048 && L.avg_item_elems > 0 && L.avg_item_elems <= 8192;
+}
 // narrow slabs for the transposed 16-wide products when the blocks have few rows
 inline int trans_narrow(const Launch &L, bool fp32) { return L.avg_cols <= (fp32 ? 32 : 16); }
 

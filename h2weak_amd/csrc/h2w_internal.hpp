@@ -212,9 +212,9 @@ void launch_copy32(const CopyJob *jobs, int njobs, const float *src, float *dst,
 // operator pool A0, or A1 for items whose flags have bit 1 set; unr in {2, 4, 8}.  Role 1:
 // symmetric terms (t >= 0) also add A^T x_item to vec[t ..] atomically.
 void launch_bgemv64(const GItem *items, int nitems, const GTerm *terms, const double *A0, const double *A1,
-                    double *vec, int role, int unr, hipStream_t s);
+                    double *vec, int role, int unr, bool per_wave, hipStream_t s);
 void launch_bgemv32(const GItem *items, int nitems, const GTerm *terms, const float *A0, const float *A1,
-                    float *vec, int role, int unr, hipStream_t s);
+                    float *vec, int role, int unr, bool per_wave, hipStream_t s);
 void launch_otf32(const GItem *items, int nitems, const GTerm *terms, SlotPoints sp, float *vec, hipStream_t s);
 void launch_otf64(const GItem *items, int nitems, const GTerm *terms, SlotPoints sp, double *vec, hipStream_t s);
 void launch_to_fp32(const double *a, float *b, int64_t n, hipStream_t s);

@@ -2028,10 +2028,11 @@ void run_launch(Handle &h, const Launch &Lh, int precision) {
     const bool in = precision == H2W_FP32_INNER;
     const GItem *items = (in ? h.inner.d_items.p : h.d_items.p) + Lh.item0;
     const GTerm *terms = in ? h.inner.d_terms.p : h.d_terms.p;
-    if (in) launch_bgemv32(items, (int)Lh.nitems, terms, h.mat32.p, h.mat32in.p, h.vec32.p, Lh.role, Lh.unr, s);
+    const bool pw = per_wave_gemv(Lh);
+    if (in) launch_bgemv32(items, (int)Lh.nitems, terms, h.mat32.p, h.mat32in.p, h.vec32.p, Lh.role, Lh.unr, pw, s);
     else if (is32(precision))
-        launch_bgemv32(items, (int)Lh.nitems, terms, h.mat32.p, nullptr, h.vec32.p, Lh.role, Lh.unr32, s);
-    else launch_bgemv64(items, (int)Lh.nitems, terms, h.mat64.p, nullptr, h.vec64.p, Lh.role, Lh.unr, s);
+        launch_bgemv32(items, (int)Lh.nitems, terms, h.mat32.p, nullptr, h.vec32.p, Lh.role, Lh.unr32, pw, s);
+    else launch_bgemv64(items, (int)Lh.nitems, terms, h.mat64.p, nullptr, h.vec64.p, Lh.role, Lh.unr, pw, s);
 }
 
 void zero_outputs(Handle &h, int precision) {

@@ -8,6 +8,7 @@
 
 #include <cfloat>
 #include <climits>
+#include <type_traits>
 
 #include "h2w_internal.hpp"
 
@@ -888,15 +889,20 @@ __device__ __forceinline__ GTerm term_at(const CGTerm *p, int k) {
 // the loads of the next are issued before the current one is multiplied.  Every load
 // is unconditional (lanes out of range address past the buffer's end), so the
 // compiler's waits count exactly the outstanding operations.
-template <typename T, int VEC, int ROLE, int UNR>
-__global__ __launch_bounds__(256) void k_bgemv(const GItem *__restrict__ items, const GTerm *__restrict__ terms,
-                                               const T *__restrict__ A0, const T *__restrict__ A1, T *vec) {
+// WPI waves share an item: 4, whose sums meet in LDS, or 1, four items per workgroup.
+template <typename T, int VEC, int ROLE, int UNR, int WPI>
+__global__ __launch_bounds__(256) void k_bgemv(const GItem *__restrict__ items, int nitems,
+                                               const GTerm *__restrict__ terms, const T *__restrict__ A0,
+                                               const T *__restrict__ A1, T *vec) {
     typedef T V __attribute__((ext_vector_type(VEC)));
-    const GItem it = items[blockIdx.x];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int item = WPI == 4 ? blockIdx.x : 4 * blockIdx.x + wave;
+    if (WPI == 1 && item >= nitems) return;
+    const int wv = WPI == 4 ? wave : 0;
+    const GItem it = items[item];
     const CGTerm *const tms = (const CGTerm *)terms;
     const T *__restrict__ A = (it.flags & 2) ? A1 : A0;
-    const int lane = threadIdx.x & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rows = it.rows;
     // (the fused launch gives a column at least UNR lanes, so that its transposed sums
     // end on UNR distinct lanes; the extra lanes of a short tile are inactive)
@@ -905,7 +911,7 @@ __global__ __launch_bounds__(256) void k_bgemv(const GItem *__restrict__ items, 
     const int cpw = 64 / lpc;
     const int q = lane / lpc, r0 = (lane % lpc) * VEC;
     const bool act = r0 < rows;
-    __shared__ T part[4][kRowTile];
+    __shared__ T part[WPI == 4 ? 4 : 1][kRowTile];
     V acc = (V)0;
     // this tile's own input rows: the x of the transposed products of symmetric terms
     T xb[VEC];
@@ -948,7 +954,7 @@ __global__ __launch_bounds__(256) void k_bgemv(const GItem *__restrict__ items, 
         // their A entries are zero and they are dropped below)
         buf_ld_n<T, UNR>(B.xv, rx, act && B.cb < B.cols ? (uint32_t)(B.cb * sizeof(T)) : kOutOfRange);
         if (has) {
-            c0 += 4 * chunk;
+            c0 += WPI * chunk;
             settle();
         }
         return has;
@@ -1012,6 +1018,17 @@ __global__ __launch_bounds__(256) void k_bgemv(const GItem *__restrict__ items, 
 #pragma unroll
     for (int v = 0; v < VEC; ++v)
         for (int o = lpc; o < 64; o <<= 1) acc[v] += __shfl_xor(acc[v], o, 64);
+    if (WPI == 1) {
+        if (q == 0 && act)
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) {
+                T *y = vec + it.y + r0 + v;
+                if (r0 + v >= rows) continue;
+                if (it.flags & 5) atomicAdd(y, acc[v]);
+                else *y += acc[v];
+            }
+        return;
+    }
     if (q == 0 && act)
 #pragma unroll
         for (int v = 0; v < VEC; ++v)
@@ -2358,34 +2375,40 @@ void launch_cur(const CurJob *jobs, int njobs, const int32_t *idx, const double 
 }
 template <typename T, int ROLE>
 static void launch_bgemv_r(const GItem *items, int nitems, const GTerm *terms, const T *A0, const T *A1, T *vec,
-                           int unr, hipStream_t s) {
+                           int unr, bool per_wave, hipStream_t s) {
     constexpr int VEC = sizeof(T) == 8 ? 2 : 4;
-    if (unr <= 2)
-        hipLaunchKernelGGL((k_bgemv<T, VEC, ROLE, 2>), dim3(nitems), dim3(256), 0, s, items, terms, A0, A1, vec);
-    else if (unr >= 8)
-        hipLaunchKernelGGL((k_bgemv<T, VEC, ROLE, 8>), dim3(nitems), dim3(256), 0, s, items, terms, A0, A1, vec);
-    else
-        hipLaunchKernelGGL((k_bgemv<T, VEC, ROLE, 4>), dim3(nitems), dim3(256), 0, s, items, terms, A0, A1, vec);
+    auto go = [&](auto U) {
+        constexpr int UNR = decltype(U)::value;
+        if (per_wave)
+            hipLaunchKernelGGL((k_bgemv<T, VEC, ROLE, UNR, 1>), dim3((nitems + 3) / 4), dim3(256), 0, s, items, nitems,
+                               terms, A0, A1, vec);
+        else
+            hipLaunchKernelGGL((k_bgemv<T, VEC, ROLE, UNR, 4>), dim3(nitems), dim3(256), 0, s, items, nitems, terms, A0,
+                               A1, vec);
+    };
+    if (unr <= 2) go(std::integral_constant<int, 2>{});
+    else if (unr >= 8) go(std::integral_constant<int, 8>{});
+    else go(std::integral_constant<int, 4>{});
 }
 template <typename T>
 static void launch_bgemv_t(const GItem *items, int nitems, const GTerm *terms, const T *A0, const T *A1, T *vec,
-                           int role, int unr, hipStream_t s) {
+                           int role, int unr, bool per_wave, hipStream_t s) {
     if (nitems <= 0) return;
     if (!A1) A1 = A0;
-    if (role == 1) launch_bgemv_r<T, 1>(items, nitems, terms, A0, A1, vec, unr, s);
-    else if (role == 2) launch_bgemv_r<T, 2>(items, nitems, terms, A0, A1, vec, unr, s);
-    else launch_bgemv_r<T, 0>(items, nitems, terms, A0, A1, vec, unr, s);
+    if (role == 1) launch_bgemv_r<T, 1>(items, nitems, terms, A0, A1, vec, unr, per_wave, s);
+    else if (role == 2) launch_bgemv_r<T, 2>(items, nitems, terms, A0, A1, vec, unr, per_wave, s);
+    else launch_bgemv_r<T, 0>(items, nitems, terms, A0, A1, vec, unr, per_wave, s);
 }
 void launch_copy32(const CopyJob *jobs, int njobs, const float *src, float *dst, hipStream_t s) {
     if (njobs > 0) hipLaunchKernelGGL(k_copy32, dim3(njobs), dim3(256), 0, s, jobs, src, dst);
 }
 void launch_bgemv64(const GItem *items, int nitems, const GTerm *terms, const double *A0, const double *A1,
-                    double *vec, int role, int unr, hipStream_t s) {
-    launch_bgemv_t<double>(items, nitems, terms, A0, A1, vec, role, unr, s);
+                    double *vec, int role, int unr, bool per_wave, hipStream_t s) {
+    launch_bgemv_t<double>(items, nitems, terms, A0, A1, vec, role, unr, per_wave, s);
 }
 void launch_bgemv32(const GItem *items, int nitems, const GTerm *terms, const float *A0, const float *A1,
-                    float *vec, int role, int unr, hipStream_t s) {
-    launch_bgemv_t<float>(items, nitems, terms, A0, A1, vec, role, unr, s);
+                    float *vec, int role, int unr, bool per_wave, hipStream_t s) {
+    launch_bgemv_t<float>(items, nitems, terms, A0, A1, vec, role, unr, per_wave, s);
 }
 template <typename T>
 static void launch_otf_t(const GItem *items, int nitems, const GTerm *terms, Coords<T> C, const SlotPoints &sp, T *vec,
