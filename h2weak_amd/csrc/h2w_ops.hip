@@ -813,7 +813,7 @@ void cur_pairs(Handle &h, AcaPool &pool) {
 }
 
 // The rows of a transfer (columns of a CUR row factor) are independent: sub-jobs of
-// 64 rows (256 columns) spread one large box over many workgroups.
+// 64 rows (columns) spread one large box over many workgroups.
 std::vector<XferJob> split_xfer(const std::vector<XferJob> &in) {
     std::vector<XferJob> out;
     for (const XferJob &J : in)
@@ -830,9 +830,9 @@ std::vector<XferJob> split_xfer(const std::vector<XferJob> &in) {
 std::vector<CurJob> split_cur(const std::vector<CurJob> &in) {
     std::vector<CurJob> out;
     for (const CurJob &J : in)
-        for (int c0 = 0; c0 < J.n; c0 += 256) {
+        for (int c0 = 0; c0 < J.n; c0 += 64) {
             CurJob K = J;
-            K.n = std::min(256, J.n - c0);
+            K.n = std::min(64, J.n - c0);
             K.v = J.v + c0;
             K.a = J.a + (int64_t)c0 * J.lda;
             out.push_back(K);

@@ -738,40 +738,94 @@ __global__ void k_eval(const EvalJob *__restrict__ jobs, const int32_t *__restri
 // is L2P (3D/codes/HODLR3Dtree.hpp:1926-1927); for the vertex-sharing field it
 // is the transpose of M2M_ver = (L R)^{-T} K(Ic, S) (:2110-2133), the same
 // matrix since the kernel is symmetric.  One thread per row of S.
-__global__ void k_xfer(const XferJob *__restrict__ jobs, const int32_t *__restrict__ idx,
-                       const double *__restrict__ lr, double *__restrict__ A, KParams kp) {
+// kSolveB columns are solved together: each earlier column's entry is loaded once
+// for all of them, their sums are independent chains, and the triangle's entries
+// (the same for every row) come by scalar loads of consecutive elements.
+// (One column at a time, a load of E and a dependent subtraction per multiply:
+// 13.1 -> 1.8 ms for the transfers at 3D N = 20011, 42.7 -> 4.9 ms at 32^3, tol 1e-10.)
+constexpr int kSolveB = 8;
+__global__ __launch_bounds__(64) void k_xfer(const XferJob *__restrict__ jobs, const int32_t *__restrict__ idx,
+                                             const double *__restrict__ lr, double *__restrict__ A, KParams kp) {
     const XferJob jb = jobs[blockIdx.x];
     const int m = jb.m, r = jb.r;
     const int64_t lde = jb.lde, ldet = jb.ldet;
     const double *L = lr + jb.lr;
     const double *R = L + (int64_t)r * r;
-    double *E = A + jb.e;
-    double *ET = A + jb.et;
     const int32_t *S = idx + jb.s;
     const int32_t *Ic = idx + jb.ic;
     for (int t = threadIdx.x; t < m; t += blockDim.x) {
-        PointI p = load_point(kp, S[t]);
+        double *E = A + jb.e + t;
+        double *ET = A + jb.et + t * ldet;
+        const PointI p = load_point(kp, S[t]);
+        double s[kSolveB], e[kSolveB];
         // X R = K(S_t, Ic)
-        for (int k = 0; k < r; ++k) {
-            double s = kentry(kp, p, Ic[k]);
-            for (int q = 0; q < k; ++q) s -= E[q * lde + t] * R[(int64_t)k * r + q];
-            E[k * lde + t] = s / R[(int64_t)k * r + k];
+        for (int k0 = 0; k0 < r; k0 += kSolveB) {
+#pragma unroll
+            for (int u = 0; u < kSolveB; ++u) s[u] = kentry(kp, p, Ic[min(k0 + u, r - 1)]);
+            for (int q0 = 0; q0 < k0; q0 += kSolveB) {
+#pragma unroll
+                for (int v = 0; v < kSolveB; ++v) e[v] = E[(q0 + v) * lde];
+#pragma unroll
+                for (int u = 0; u < kSolveB; ++u) {
+                    const double *Rk = R + (int64_t)min(k0 + u, r - 1) * r + q0;
+#pragma unroll
+                    for (int v = 0; v < kSolveB; ++v) s[u] = fma(-e[v], Rk[v], s[u]);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kSolveB; ++u) {
+                const double *Rk = R + (int64_t)min(k0 + u, r - 1) * r + k0;
+                if (k0 + u < r) {
+#pragma unroll
+                    for (int v = 0; v < kSolveB; ++v)
+                        if (v < u) s[u] = fma(-s[v], Rk[v], s[u]);
+                    s[u] = s[u] / Rk[u];
+                    E[(k0 + u) * lde] = s[u];
+                }
+            }
         }
-        // Y L = X
-        for (int k = r - 1; k >= 0; --k) {
-            double s = E[k * lde + t];
-            for (int q = k + 1; q < r; ++q) s -= E[q * lde + t] * L[(int64_t)k * r + q];
-            E[k * lde + t] = s / L[(int64_t)k * r + k];
+        // Y L = X, from the last columns
+        for (int k0 = (r - 1) / kSolveB * kSolveB; k0 >= 0; k0 -= kSolveB) {
+#pragma unroll
+            for (int u = 0; u < kSolveB; ++u) s[u] = E[min(k0 + u, r - 1) * lde];
+            int q0 = k0 + kSolveB;
+            for (; q0 + kSolveB <= r; q0 += kSolveB) {
+#pragma unroll
+                for (int v = 0; v < kSolveB; ++v) e[v] = E[(q0 + v) * lde];
+#pragma unroll
+                for (int u = 0; u < kSolveB; ++u) {
+                    const double *Lk = L + (int64_t)(k0 + u) * r + q0;
+#pragma unroll
+                    for (int v = 0; v < kSolveB; ++v) s[u] = fma(-e[v], Lk[v], s[u]);
+                }
+            }
+            for (; q0 < r; ++q0) {
+                const double eq = E[q0 * lde];
+#pragma unroll
+                for (int u = 0; u < kSolveB; ++u) s[u] = fma(-eq, L[(int64_t)(k0 + u) * r + q0], s[u]);
+            }
+#pragma unroll
+            for (int u = kSolveB - 1; u >= 0; --u) {
+                if (k0 + u < r) {
+                    const double *Lk = L + (int64_t)(k0 + u) * r + k0;
+#pragma unroll
+                    for (int v = 0; v < kSolveB; ++v)
+                        if (v > u && k0 + v < r) s[u] = fma(-s[v], Lk[v], s[u]);
+                    s[u] = s[u] / Lk[u];
+                    E[(k0 + u) * lde] = s[u];
+                    ET[k0 + u] = s[u];
+                }
+            }
         }
-        for (int k = 0; k < r; ++k) ET[t * ldet + k] = E[k * lde + t];
     }
 }
 
 // A = R^{-1} L^{-1} K(Ir, V) (r x n), one thread per column: the semi-nested
 // vertex block's row factor with the two triangular solves of the reference's
-// apply (3D/codes/HODLR3Dtree.hpp:2341-2344) folded in at assembly.
-__global__ void k_cur(const CurJob *__restrict__ jobs, const int32_t *__restrict__ idx,
-                      const double *__restrict__ lr, double *__restrict__ A, KParams kp) {
+// apply (3D/codes/HODLR3Dtree.hpp:2341-2344) folded in at assembly.  kSolveB rows
+// are solved together, as in k_xfer (4.9 -> 0.9 ms at 3D N = 20000, tol 1e-8).
+__global__ __launch_bounds__(64) void k_cur(const CurJob *__restrict__ jobs, const int32_t *__restrict__ idx,
+                                            const double *__restrict__ lr, double *__restrict__ A, KParams kp) {
     const CurJob jb = jobs[blockIdx.x];
     const int r = jb.r, n = jb.n;
     const double *L = lr + jb.lr;
@@ -780,17 +834,45 @@ __global__ void k_cur(const CurJob *__restrict__ jobs, const int32_t *__restrict
     const int32_t *Vv = idx + jb.v;
     for (int t = threadIdx.x; t < n; t += blockDim.x) {
         double *a = A + jb.a + (int64_t)t * jb.lda;
-        PointI p = load_point(kp, Vv[t]);
-        for (int k = 0; k < r; ++k) a[k] = kentry(kp, p, Ir[k]);
-        for (int k = 0; k < r; ++k) {
-            double s = a[k];
-            for (int q = 0; q < k; ++q) s -= L[(int64_t)q * r + k] * a[q];
-            a[k] = s / L[(int64_t)k * r + k];
+        const PointI p = load_point(kp, Vv[t]);
+        double s[kSolveB];
+        for (int k0 = 0; k0 < r; k0 += kSolveB) {
+#pragma unroll
+            for (int u = 0; u < kSolveB; ++u) s[u] = kentry(kp, p, Ir[min(k0 + u, r - 1)]);
+            for (int q = 0; q < k0; ++q) {
+                const double aq = a[q];
+                const double *Lq = L + (int64_t)q * r + k0;
+#pragma unroll
+                for (int u = 0; u < kSolveB; ++u) s[u] = fma(-aq, Lq[min(u, r - 1 - k0)], s[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < kSolveB; ++u)
+                if (k0 + u < r) {
+#pragma unroll
+                    for (int v = 0; v < kSolveB; ++v)
+                        if (v < u) s[u] = fma(-s[v], L[(int64_t)(k0 + v) * r + k0 + u], s[u]);
+                    s[u] = s[u] / L[(int64_t)(k0 + u) * r + k0 + u];
+                    a[k0 + u] = s[u];
+                }
         }
-        for (int k = r - 1; k >= 0; --k) {
-            double s = a[k];
-            for (int q = k + 1; q < r; ++q) s -= R[(int64_t)q * r + k] * a[q];
-            a[k] = s / R[(int64_t)k * r + k];
+        for (int k0 = (r - 1) / kSolveB * kSolveB; k0 >= 0; k0 -= kSolveB) {
+#pragma unroll
+            for (int u = 0; u < kSolveB; ++u) s[u] = a[min(k0 + u, r - 1)];
+            for (int q = k0 + kSolveB; q < r; ++q) {
+                const double aq = a[q];
+                const double *Rq = R + (int64_t)q * r + k0;
+#pragma unroll
+                for (int u = 0; u < kSolveB; ++u) s[u] = fma(-aq, Rq[u], s[u]);
+            }
+#pragma unroll
+            for (int u = kSolveB - 1; u >= 0; --u)
+                if (k0 + u < r) {
+#pragma unroll
+                    for (int v = 0; v < kSolveB; ++v)
+                        if (v > u && k0 + v < r) s[u] = fma(-s[v], R[(int64_t)(k0 + v) * r + k0 + u], s[u]);
+                    s[u] = s[u] / R[(int64_t)(k0 + u) * r + k0 + u];
+                    a[k0 + u] = s[u];
+                }
         }
     }
 }
@@ -2371,7 +2453,7 @@ void launch_xfer(const XferJob *jobs, int njobs, const int32_t *idx, const doubl
 }
 void launch_cur(const CurJob *jobs, int njobs, const int32_t *idx, const double *lr, double *A, KParams kp,
                 hipStream_t s) {
-    if (njobs > 0) hipLaunchKernelGGL(k_cur, dim3(njobs), dim3(256), 0, s, jobs, idx, lr, A, kp);
+    if (njobs > 0) hipLaunchKernelGGL(k_cur, dim3(njobs), dim3(64), 0, s, jobs, idx, lr, A, kp);
 }
 template <typename T, int ROLE>
 static void launch_bgemv_r(const GItem *items, int nitems, const GTerm *terms, const T *A0, const T *A1, T *vec,
