@@ -117,7 +117,7 @@ struct AcaBlock {
     bool has_feat = false;
     int rank = 0;
     std::vector<int32_t> rb, cb;  // local pivot indices
-    std::vector<double> lr;       // L then R, rank x rank column-major each
+    int64_t lr = -1;              // L then R, rank x rank column-major each: offset in the handle's d_lr
     std::vector<double> hist;     // per step: |u||v| and normS after the step
 };
 
@@ -126,7 +126,7 @@ struct FamLevel {
     int nb = 0;
     std::vector<int> rank;
     std::vector<std::vector<int32_t>> Ir, Ic;  // tree-order indices
-    std::vector<std::vector<double>> lr;
+    std::vector<int64_t> lr;                   // L and R of every box: offset in the handle's d_lr
     std::vector<std::vector<double>> hist;     // ACA history (|u||v|, normS) per step
     std::vector<int> kin;                      // rank of the inner (truncated) operator
     std::vector<int64_t> ein_off, eint_off;    // inner transfers in the FP32 pool
@@ -139,7 +139,7 @@ struct Pair {                                  // semi-nested vertex pair (B <- 
     int level, b, v;
     int rank;
     std::vector<int32_t> Ir, Ic;
-    std::vector<double> lr;
+    int64_t lr = -1;                           // L and R: offset in the handle's d_lr
     int64_t ac_off, ar_off, t_off;
 };
 
@@ -286,6 +286,9 @@ struct h2w_handle {
     int64_t vec_len = 0, off_x = 0, off_y = 0;
     std::vector<h2w::FamLevel> fam[2];
     std::vector<h2w::Pair> pairs;
+    // L and R of every skeleton, where the transfers (also the inner operator's, rebuilt at will) and saved
+    // files take them from: offsets in elements, two doubles each with a complex kernel
+    h2w::DevBuf<double> d_lr;
     std::vector<h2w::Launch> launches;
     std::vector<int64_t> launch_elems;  // operator elements each launch streams
     std::vector<h2w::M2LBlk> m2l;

@@ -98,7 +98,8 @@ struct AcaJob {
 
 struct LrJob {     // copy L (unit lower) and R (upper) out of an ACA workspace
     int64_t tab, piv;
-    int32_t m, n, rank, pad;
+    int32_t m, n, rank;
+    int32_t pk;    // offset (terms) of the block's packed pivots and history
     int64_t out;   // offset (doubles): L at out, R at out + rank*rank, both column-major
 };
 
@@ -115,6 +116,7 @@ struct EvalJob {   // A = K(rows, cols), m x n column-major at a, leading dimens
 struct XferJob {   // E = K(S, Ic) (L R)^{-1}, m x r at e (ld lde); E^T (r x m) at et (ld ldet)
     int64_t s, ic, lr, e, et;
     int32_t m, r, lde, ldet;
+    int32_t ldr, pad;  // leading dimension of L and R (R at lr + ldr^2): r, or more for their leading blocks
 };
 
 struct CurJob {    // A = (L R)^{-1} K(Ir, V), r x n column-major at a, leading dimension lda
@@ -203,6 +205,13 @@ void launch_aca_sample(const AcaJob *jobs, int nb, const int32_t *rank, const in
                        const int64_t *tab, KParams kp, int ns, double *err2, double *ref2, hipStream_t s);
 void launch_lr_extract(const LrJob *jobs, int njobs, const double *ws, const int64_t *tab,
                        const int32_t *rowpiv, const int32_t *colpiv, double *out, hipStream_t s);
+// the pivots and step histories of a batch's blocks one after another (at pk, rank entries each)
+void launch_pack_pivots(const LrJob *jobs, int njobs, const int32_t *rowpiv, const int32_t *colpiv, const double *hist,
+                        int32_t *prow, int32_t *pcol, double *phist, hipStream_t s);
+// the coordinates of every slot's point (zeros where pid < 0)
+void launch_slot_points(const int32_t *pid, int64_t n, const double *px, const double *py, const double *pz, double *xd,
+                        double *yd, double *zd, float *x, float *y, float *z, float *xl, float *yl, float *zl,
+                        hipStream_t s);
 void launch_eval(const EvalJob *jobs, int njobs, const int32_t *idx, double *A, KParams kp, hipStream_t s);
 void launch_xfer(const XferJob *jobs, int njobs, const int32_t *idx, const double *lr, double *A, KParams kp,
                  hipStream_t s);

@@ -19,6 +19,7 @@
 #include <thread>
 
 #include <algorithm>
+#include <deque>
 #include <chrono>
 #include <cmath>
 #include <complex>
@@ -179,6 +180,17 @@ struct AcaPool {
     DevBuf<double> wpart, wdot;
     DevBuf<uint32_t> warrived;
     DevBuf<int32_t> wdone;
+    // a batch's jobs, index lists and results, also kept over the assembly's batches
+    DevBuf<uint8_t> flags;
+    DevBuf<int32_t> idx, rank, stat, rp, cp, prow, pcol;
+    DevBuf<double> hist, phist;
+    DevBuf<int64_t> tab;
+    DevBuf<AcaJob> jobs;
+    DevBuf<LrJob> lrj;
+    // L and R of the batches so far, part by part (offsets in elements)
+    std::deque<DevBuf<double>> lr;
+    std::vector<std::pair<int64_t, int64_t>> lr_part;  // first element, elements
+    int64_t lr_len = 0;
 };
 
 // The workspace holds the U and V columns of every block of a batch.  It is sized
@@ -487,13 +499,12 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
     for (size_t b = 0; b < blocks.size(); ++b) need += space_of(b);
     ensure_pool(h, pool, need * esz);
     h.aca_pool_bytes = std::max<int64_t>(h.aca_pool_bytes, pool.cap * 8);
-    DevBuf<uint8_t> flags;
-    DevBuf<int32_t> didx, drank, dstat, drp, dcp;
-    DevBuf<double> dhist;
-    DevBuf<int64_t> dtab;
-    DevBuf<AcaJob> djobs;
-    DevBuf<LrJob> dlr;
-    DevBuf<double> dlrout;
+    DevBuf<uint8_t> &flags = pool.flags;
+    DevBuf<int32_t> &didx = pool.idx, &drank = pool.rank, &dstat = pool.stat, &drp = pool.rp, &dcp = pool.cp;
+    DevBuf<double> &dhist = pool.hist;
+    DevBuf<int64_t> &dtab = pool.tab;
+    DevBuf<AcaJob> &djobs = pool.jobs;
+    DevBuf<LrJob> &dlr = pool.lrj;
     const size_t kBig = 16384;    // complex kernels: m + n above which a block gets a 1024-thread workgroup
     // m + n above which a block with a predicted rank takes a fixed-rank phase (H2W_WIDE_MIN overrides):
     // its judgement costs host work per block, which small blocks do not repay
@@ -574,13 +585,9 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
                          tol);
             }
             H2W_HIP(hipGetLastError());
-            std::vector<int32_t> rk(batch.size()), st(batch.size()), rp(po), cp(po);
-            std::vector<double> hs(2 * po);
-            H2W_HIP(hipMemcpyAsync(hs.data(), dhist.p, 2 * po * 8, hipMemcpyDeviceToHost, s));
+            std::vector<int32_t> rk(batch.size()), st(batch.size());
             H2W_HIP(hipMemcpyAsync(rk.data(), drank.p, rk.size() * 4, hipMemcpyDeviceToHost, s));
             H2W_HIP(hipMemcpyAsync(st.data(), dstat.p, st.size() * 4, hipMemcpyDeviceToHost, s));
-            H2W_HIP(hipMemcpyAsync(rp.data(), drp.p, po * 4, hipMemcpyDeviceToHost, s));
-            H2W_HIP(hipMemcpyAsync(cp.data(), dcp.p, po * 4, hipMemcpyDeviceToHost, s));
             H2W_HIP(hipStreamSynchronize(s));
             if (verbose) {
                 int mr = 0, nov = 0;
@@ -593,7 +600,7 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
             }
             std::vector<LrJob> lj;
             std::vector<size_t> lb;
-            int64_t lo = 0;
+            int64_t lo = 0, pk = 0;
             for (size_t q = 0; q < batch.size(); ++q) {
                 size_t b = batch[q];
                 if (st[q] != 0) {
@@ -616,9 +623,6 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
                     h.rank_pred_under += rk[q] > est0[b];
                     h.rank_pred_abs_log2 += std::fabs((double)plog[b] - std::log2(1.0 + rk[q]));
                 }
-                B.rb.assign(rp.begin() + jobs[q].piv, rp.begin() + jobs[q].piv + rk[q]);
-                B.cb.assign(cp.begin() + jobs[q].piv, cp.begin() + jobs[q].piv + rk[q]);
-                B.hist.assign(hs.begin() + 2 * jobs[q].piv, hs.begin() + 2 * (jobs[q].piv + rk[q]));
                 if (rk[q] > 0) {
                     LrJob J;
                     J.tab = jobs[q].tab;
@@ -626,7 +630,8 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
                     J.m = jobs[q].m;
                     J.n = jobs[q].n;
                     J.rank = rk[q];
-                    J.pad = 0;
+                    J.pk = (int32_t)pk;
+                    pk += rk[q];
                     J.out = lo;
                     lo += 2LL * rk[q] * rk[q];
                     lj.push_back(J);
@@ -634,22 +639,38 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
                 }
             }
             if (!lj.empty()) {
+                if (pk > INT32_MAX) throw Error{H2W_ENOMEM, "too many pivots in one batch"};
                 dlr.upload(lj, s);
-                dlrout.ensure(lo * esz);
+                // L and R stay on the device, where the transfers are made from them
+                pool.lr.emplace_back();
+                DevBuf<double> &part = pool.lr.back();
+                part.alloc(lo * esz);
+                pool.lr_part.push_back({pool.lr_len, lo});
                 if (cx)
                     launch_lr_extract_c(dlr.p, (int)lj.size(), reinterpret_cast<const double2 *>(pool.ws.p), dtab.p,
-                                        drp.p, dcp.p, reinterpret_cast<double2 *>(dlrout.p), s);
-                else launch_lr_extract(dlr.p, (int)lj.size(), pool.ws.p, dtab.p, drp.p, dcp.p, dlrout.p, s);
+                                        drp.p, dcp.p, reinterpret_cast<double2 *>(part.p), s);
+                else launch_lr_extract(dlr.p, (int)lj.size(), pool.ws.p, dtab.p, drp.p, dcp.p, part.p, s);
+                pool.prow.ensure(pk);
+                pool.pcol.ensure(pk);
+                pool.phist.ensure(2 * pk);
+                launch_pack_pivots(dlr.p, (int)lj.size(), drp.p, dcp.p, dhist.p, pool.prow.p, pool.pcol.p, pool.phist.p,
+                                   s);
                 H2W_HIP(hipGetLastError());
-                std::vector<double> hl(lo * esz);
-                H2W_HIP(hipMemcpyAsync(hl.data(), dlrout.p, lo * esz * 8, hipMemcpyDeviceToHost, s));
+                std::vector<int32_t> rp(pk), cp(pk);
+                std::vector<double> hs(2 * pk);
+                H2W_HIP(hipMemcpyAsync(hs.data(), pool.phist.p, 2 * pk * 8, hipMemcpyDeviceToHost, s));
+                H2W_HIP(hipMemcpyAsync(rp.data(), pool.prow.p, pk * 4, hipMemcpyDeviceToHost, s));
+                H2W_HIP(hipMemcpyAsync(cp.data(), pool.pcol.p, pk * 4, hipMemcpyDeviceToHost, s));
                 H2W_HIP(hipStreamSynchronize(s));
                 for (size_t q = 0; q < lj.size(); ++q) {
                     AcaBlock &B = blocks[lb[q]];
-                    // (L then R, r x r each; complex entries as (re, im) pairs)
-                    B.lr.assign(hl.begin() + lj[q].out * esz,
-                                hl.begin() + (lj[q].out + 2LL * lj[q].rank * lj[q].rank) * esz);
+                    const int64_t o = lj[q].pk, r = lj[q].rank;
+                    B.rb.assign(rp.begin() + o, rp.begin() + o + r);
+                    B.cb.assign(cp.begin() + o, cp.begin() + o + r);
+                    B.hist.assign(hs.begin() + 2 * o, hs.begin() + 2 * (o + r));
+                    B.lr = pool.lr_len + lj[q].out;
                 }
+                pool.lr_len += lo;
             }
         }
         todo.swap(rerun);
@@ -700,7 +721,7 @@ void far_nca(Handle &h, AcaPool &pool) {
         fl.rank.resize(fl.nb);
         fl.Ir.resize(fl.nb);
         fl.Ic.resize(fl.nb);
-        fl.lr.resize(fl.nb);
+        fl.lr.assign(fl.nb, -1);
         fl.hist.resize(fl.nb);
         for (int b = 0; b < fl.nb; ++b) {
             AcaBlock &B = blocks[b];
@@ -710,7 +731,7 @@ void far_nca(Handle &h, AcaPool &pool) {
                 fl.Ir[b].push_back(B.rows[B.rb[q]]);
                 fl.Ic[b].push_back(B.cols[B.cb[q]]);
             }
-            fl.lr[b] = std::move(B.lr);
+            fl.lr[b] = B.lr;
         }
         if (std::getenv("H2W_VERBOSE")) std::fprintf(stderr, "[h2w]  far level %d done\n", j);
     }
@@ -750,7 +771,7 @@ void vertex_nca(Handle &h, AcaPool &pool) {
         fl.rank.resize(fl.nb);
         fl.Ir.resize(fl.nb);
         fl.Ic.resize(fl.nb);
-        fl.lr.resize(fl.nb);
+        fl.lr.assign(fl.nb, -1);
         fl.hist.resize(fl.nb);
         for (int b = 0; b < fl.nb; ++b) {
             AcaBlock &B = blocks[b];
@@ -760,7 +781,7 @@ void vertex_nca(Handle &h, AcaPool &pool) {
                 fl.Ir[b].push_back(B.rows[B.rb[q]]);
                 fl.Ic[b].push_back(B.cols[B.cb[q]]);
             }
-            fl.lr[b] = std::move(B.lr);
+            fl.lr[b] = B.lr;
         }
         if (std::getenv("H2W_VERBOSE")) std::fprintf(stderr, "[h2w]  vertex level %d done\n", j);
     }
@@ -808,7 +829,7 @@ void cur_pairs(Handle &h, AcaPool &pool) {
             p.Ir.push_back(B.rows[B.rb[k]]);
             p.Ic.push_back(B.cols[B.cb[k]]);
         }
-        p.lr = std::move(B.lr);
+        p.lr = B.lr;
     }
 }
 
@@ -1213,20 +1234,13 @@ void build_inner(Handle &h, double irp) {
     if (inner_on && in_len > 0) {
         std::vector<int32_t> idx;
         std::vector<XferJob> xj;
-        std::vector<double> lr;
         for (int f = 0; f < 2; ++f) {
             if (!fam_on[f]) continue;
             for (int j = nfam_lo[f]; j <= P.nL; ++j) {
                 FamLevel &fl = h.fam[f][j];
                 for (int b = 0; b < fl.nb; ++b) {
                     if (fl.ein_off[b] < 0) continue;
-                    const int k = fl.kin[b], r = fl.rank[b];
-                    // leading k x k blocks of L and R
-                    const int64_t lro = (int64_t)lr.size();
-                    for (int part = 0; part < 2; ++part)
-                        for (int cc = 0; cc < k; ++cc)
-                            for (int rr = 0; rr < k; ++rr)
-                                lr.push_back(fl.lr[b][(size_t)part * r * r + (size_t)cc * r + rr]);
+                    const int k = fl.kin[b];
                     const int64_t icq = (int64_t)idx.size();
                     idx.insert(idx.end(), fl.Ic[b].begin(), fl.Ic[b].begin() + k);
                     int64_t m = 0;
@@ -1242,7 +1256,9 @@ void build_inner(Handle &h, double irp) {
                         J.s = (int64_t)idx.size();
                         idx.insert(idx.end(), S, S + ms);
                         J.ic = icq;
-                        J.lr = lro;
+                        J.lr = fl.lr[b];  // (the leading k x k blocks of L and R)
+                        J.ldr = fl.rank[b];
+                        J.pad = 0;
                         J.e = fl.ein_off[b] + row;
                         J.et = fl.eint_off[b] + row * ldet;
                         J.lde = lde;
@@ -1265,15 +1281,14 @@ void build_inner(Handle &h, double irp) {
             }
         }
         DevBuf<int32_t> didx;
-        DevBuf<double> dlr, tmp;
+        DevBuf<double> tmp;
         DevBuf<XferJob> dxj;
         didx.upload(idx, s);
-        dlr.upload(lr, s);
         xj = split_xfer(xj);
         dxj.upload(xj, s);
         tmp.alloc(in_len);
         H2W_HIP(hipMemsetAsync(tmp.p, 0, in_len * 8, s));
-        launch_xfer(dxj.p, (int)xj.size(), didx.p, dlr.p, tmp.p, h.kp, s);
+        launch_xfer(dxj.p, (int)xj.size(), didx.p, h.d_lr.p, tmp.p, h.kp, s);
         H2W_HIP(hipGetLastError());
         launch_to_fp32(tmp.p, h.mat32in.p, in_len, s);
         H2W_HIP(hipGetLastError());
@@ -1494,6 +1509,12 @@ void assemble(Handle &h) {
             cur_pairs(h, pool);
         }
         phase("vertex NCA / CUR");
+        const int64_t es = h.cplx ? 2 : 1;
+        h.d_lr.alloc(pool.lr_len * es);
+        for (size_t q = 0; q < pool.lr.size(); ++q)
+            H2W_HIP(hipMemcpyAsync(h.d_lr.p + pool.lr_part[q].first * es, pool.lr[q].p, pool.lr_part[q].second * es * 8,
+                                   hipMemcpyDeviceToDevice, h.stream));
+        H2W_HIP(hipStreamSynchronize(h.stream));
     }
     assemble_operators(h, t0);
 }
@@ -1648,31 +1669,12 @@ void assemble_operators(Handle &h, double t0) {
                     for (int k = 0; k < fl.rank[b]; ++k) pid[fl.o_off[b] + k] = pid[fl.u_off[b] + k] = fl.Ir[b][k];
             }
         }
-        std::vector<float> fx(h.vec_len, 0.f), fy(h.vec_len, 0.f), fz(h.vec_len, 0.f);
-        std::vector<float> lx(h.vec_len, 0.f), ly(h.vec_len, 0.f), lz(h.vec_len, 0.f);
-        std::vector<double> dx(h.vec_len, 0.0), dy(h.vec_len, 0.0), dz(h.vec_len, 0.0);
-        for (int64_t v = 0; v < h.vec_len; ++v) {
-            if (pid[v] < 0) continue;
-            dx[v] = P.px[pid[v]];
-            dy[v] = P.py[pid[v]];
-            dz[v] = P.pz[pid[v]];
-            fx[v] = (float)dx[v];
-            fy[v] = (float)dy[v];
-            fz[v] = (float)dz[v];
-            lx[v] = (float)(dx[v] - (double)fx[v]);
-            ly[v] = (float)(dy[v] - (double)fy[v]);
-            lz[v] = (float)(dz[v] - (double)fz[v]);
-        }
         h.spid.upload(pid, s);
-        h.sx32.upload(fx, s);
-        h.sy32.upload(fy, s);
-        h.sz32.upload(fz, s);
-        h.sxl.upload(lx, s);
-        h.syl.upload(ly, s);
-        h.szl.upload(lz, s);
-        h.sx64.upload(dx, s);
-        h.sy64.upload(dy, s);
-        h.sz64.upload(dz, s);
+        for (DevBuf<float> *v : {&h.sx32, &h.sy32, &h.sz32, &h.sxl, &h.syl, &h.szl}) v->ensure(h.vec_len);
+        for (DevBuf<double> *v : {&h.sx64, &h.sy64, &h.sz64}) v->ensure(h.vec_len);
+        launch_slot_points(h.spid.p, h.vec_len, h.d_px.p, h.d_py.p, h.d_pz.p, h.sx64.p, h.sy64.p, h.sz64.p, h.sx32.p,
+                           h.sy32.p, h.sz32.p, h.sxl.p, h.syl.p, h.szl.p, s);
+        H2W_HIP(hipGetLastError());
         H2W_HIP(hipStreamSynchronize(s));
         h.sp.x = h.sx32.p;
         h.sp.y = h.sy32.p;
@@ -1694,7 +1696,6 @@ void assemble_operators(Handle &h, double t0) {
         // transfers
         std::vector<int32_t> idx;
         std::vector<XferJob> xj;
-        std::vector<double> lr;
         for (int f = 0; f < 2; ++f) {
             if (!fam_on[f]) continue;
             for (int j = nfam_lo[f]; j <= P.nL; ++j) {
@@ -1708,8 +1709,9 @@ void assemble_operators(Handle &h, double t0) {
                     idx.insert(idx.end(), fl.S[b].begin(), fl.S[b].end());
                     J.ic = (int64_t)idx.size();
                     idx.insert(idx.end(), fl.Ic[b].begin(), fl.Ic[b].end());
-                    J.lr = (int64_t)lr.size() / esz;
-                    lr.insert(lr.end(), fl.lr[b].begin(), fl.lr[b].end());
+                    J.lr = fl.lr[b];
+                    J.ldr = J.r;
+                    J.pad = 0;
                     J.e = fl.e_off[b];
                     J.et = fl.et_off[b];
                     J.lde = (int32_t)pad_ld(J.m);
@@ -1730,31 +1732,28 @@ void assemble_operators(Handle &h, double t0) {
             J.v = (int64_t)idx.size();
             auto vr = range_list(P.bstart[p.level][p.v], J.n);
             idx.insert(idx.end(), vr.begin(), vr.end());
-            J.lr = (int64_t)lr.size() / esz;
-            lr.insert(lr.end(), p.lr.begin(), p.lr.end());
+            J.lr = p.lr;
             J.a = p.ar_off;
             J.lda = (int32_t)pad_ld(J.r);
             J.pad = 0;
             cj.push_back(J);
         }
         DevBuf<int32_t> didx;
-        DevBuf<double> dlr;
         DevBuf<XferJob> dxj;
         DevBuf<CurJob> dcj;
         didx.upload(idx, s);
-        dlr.upload(lr, s);
         xj = split_xfer(xj);
         dxj.upload(xj, s);
         cj = split_cur(cj);
         dcj.upload(cj, s);
         if (h.cplx) {
-            launch_xfer_c(dxj.p, (int)xj.size(), didx.p, reinterpret_cast<const double2 *>(dlr.p),
+            launch_xfer_c(dxj.p, (int)xj.size(), didx.p, reinterpret_cast<const double2 *>(h.d_lr.p),
                           reinterpret_cast<double2 *>(h.mat64.p), h.kpc, s);
-            launch_cur_c(dcj.p, (int)cj.size(), didx.p, reinterpret_cast<const double2 *>(dlr.p),
+            launch_cur_c(dcj.p, (int)cj.size(), didx.p, reinterpret_cast<const double2 *>(h.d_lr.p),
                          reinterpret_cast<double2 *>(h.mat64.p), h.kpc, s);
         } else {
-            launch_xfer(dxj.p, (int)xj.size(), didx.p, dlr.p, h.mat64.p, h.kp, s);
-            launch_cur(dcj.p, (int)cj.size(), didx.p, dlr.p, h.mat64.p, h.kp, s);
+            launch_xfer(dxj.p, (int)xj.size(), didx.p, h.d_lr.p, h.mat64.p, h.kp, s);
+            launch_cur(dcj.p, (int)cj.size(), didx.p, h.d_lr.p, h.mat64.p, h.kp, s);
         }
         H2W_HIP(hipGetLastError());
         H2W_HIP(hipStreamSynchronize(s));

@@ -721,6 +721,38 @@ __global__ void k_lr_extract(const LrJob *__restrict__ jobs, const double *__res
     }
 }
 
+__global__ void k_pack_pivots(const LrJob *__restrict__ jobs, const int32_t *__restrict__ rowpiv,
+                              const int32_t *__restrict__ colpiv, const double *__restrict__ hist,
+                              int32_t *__restrict__ prow, int32_t *__restrict__ pcol, double *__restrict__ phist) {
+    const LrJob jb = jobs[blockIdx.x];
+    for (int k = threadIdx.x; k < jb.rank; k += blockDim.x) {
+        prow[jb.pk + k] = rowpiv[jb.piv + k];
+        pcol[jb.pk + k] = colpiv[jb.piv + k];
+        phist[2 * ((int64_t)jb.pk + k)] = hist[2 * (jb.piv + k)];
+        phist[2 * ((int64_t)jb.pk + k) + 1] = hist[2 * (jb.piv + k) + 1];
+    }
+}
+
+__global__ void k_slot_points(const int32_t *__restrict__ pid, int64_t n, const double *__restrict__ px,
+                              const double *__restrict__ py, const double *__restrict__ pz, double *__restrict__ xd,
+                              double *__restrict__ yd, double *__restrict__ zd, float *__restrict__ x,
+                              float *__restrict__ y, float *__restrict__ z, float *__restrict__ xl,
+                              float *__restrict__ yl, float *__restrict__ zl) {
+    const int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (v >= n) return;
+    const int32_t i = pid[v];
+    const double a = i < 0 ? 0.0 : px[i], b = i < 0 ? 0.0 : py[i], c = i < 0 ? 0.0 : pz[i];
+    xd[v] = a;
+    yd[v] = b;
+    zd[v] = c;
+    x[v] = (float)a;
+    y[v] = (float)b;
+    z[v] = (float)c;
+    xl[v] = (float)(a - (double)(float)a);
+    yl[v] = (float)(b - (double)(float)b);
+    zl[v] = (float)(c - (double)(float)c);
+}
+
 // A = K(rows, cols), column-major (getMatrix, 3D/codes/kernel.hpp:58-71)
 __global__ void k_eval(const EvalJob *__restrict__ jobs, const int32_t *__restrict__ idx, double *__restrict__ A,
                        KParams kp) {
@@ -748,9 +780,10 @@ __global__ __launch_bounds__(64) void k_xfer(const XferJob *__restrict__ jobs, c
                                              const double *__restrict__ lr, double *__restrict__ A, KParams kp) {
     const XferJob jb = jobs[blockIdx.x];
     const int m = jb.m, r = jb.r;
+    const int64_t ldr = jb.ldr;
     const int64_t lde = jb.lde, ldet = jb.ldet;
     const double *L = lr + jb.lr;
-    const double *R = L + (int64_t)r * r;
+    const double *R = L + ldr * ldr;
     const int32_t *S = idx + jb.s;
     const int32_t *Ic = idx + jb.ic;
     for (int t = threadIdx.x; t < m; t += blockDim.x) {
@@ -767,14 +800,14 @@ __global__ __launch_bounds__(64) void k_xfer(const XferJob *__restrict__ jobs, c
                 for (int v = 0; v < kSolveB; ++v) e[v] = E[(q0 + v) * lde];
 #pragma unroll
                 for (int u = 0; u < kSolveB; ++u) {
-                    const double *Rk = R + (int64_t)min(k0 + u, r - 1) * r + q0;
+                    const double *Rk = R + min(k0 + u, r - 1) * ldr + q0;
 #pragma unroll
                     for (int v = 0; v < kSolveB; ++v) s[u] = fma(-e[v], Rk[v], s[u]);
                 }
             }
 #pragma unroll
             for (int u = 0; u < kSolveB; ++u) {
-                const double *Rk = R + (int64_t)min(k0 + u, r - 1) * r + k0;
+                const double *Rk = R + min(k0 + u, r - 1) * ldr + k0;
                 if (k0 + u < r) {
 #pragma unroll
                     for (int v = 0; v < kSolveB; ++v)
@@ -794,7 +827,7 @@ __global__ __launch_bounds__(64) void k_xfer(const XferJob *__restrict__ jobs, c
                 for (int v = 0; v < kSolveB; ++v) e[v] = E[(q0 + v) * lde];
 #pragma unroll
                 for (int u = 0; u < kSolveB; ++u) {
-                    const double *Lk = L + (int64_t)(k0 + u) * r + q0;
+                    const double *Lk = L + (k0 + u) * ldr + q0;
 #pragma unroll
                     for (int v = 0; v < kSolveB; ++v) s[u] = fma(-e[v], Lk[v], s[u]);
                 }
@@ -802,12 +835,12 @@ __global__ __launch_bounds__(64) void k_xfer(const XferJob *__restrict__ jobs, c
             for (; q0 < r; ++q0) {
                 const double eq = E[q0 * lde];
 #pragma unroll
-                for (int u = 0; u < kSolveB; ++u) s[u] = fma(-eq, L[(int64_t)(k0 + u) * r + q0], s[u]);
+                for (int u = 0; u < kSolveB; ++u) s[u] = fma(-eq, L[(k0 + u) * ldr + q0], s[u]);
             }
 #pragma unroll
             for (int u = kSolveB - 1; u >= 0; --u) {
                 if (k0 + u < r) {
-                    const double *Lk = L + (int64_t)(k0 + u) * r + k0;
+                    const double *Lk = L + (k0 + u) * ldr + k0;
 #pragma unroll
                     for (int v = 0; v < kSolveB; ++v)
                         if (v > u && k0 + v < r) s[u] = fma(-s[v], Lk[v], s[u]);
@@ -2443,6 +2476,18 @@ void launch_lr_extract(const LrJob *jobs, int njobs, const double *ws, const int
                        const int32_t *colpiv, double *out, hipStream_t s) {
     if (njobs > 0)
         hipLaunchKernelGGL(k_lr_extract, dim3(njobs), dim3(256), 0, s, jobs, ws, tab, rowpiv, colpiv, out);
+}
+void launch_pack_pivots(const LrJob *jobs, int njobs, const int32_t *rowpiv, const int32_t *colpiv, const double *hist,
+                        int32_t *prow, int32_t *pcol, double *phist, hipStream_t s) {
+    if (njobs > 0)
+        hipLaunchKernelGGL(k_pack_pivots, dim3(njobs), dim3(64), 0, s, jobs, rowpiv, colpiv, hist, prow, pcol, phist);
+}
+void launch_slot_points(const int32_t *pid, int64_t n, const double *px, const double *py, const double *pz, double *xd,
+                        double *yd, double *zd, float *x, float *y, float *z, float *xl, float *yl, float *zl,
+                        hipStream_t s) {
+    if (n > 0)
+        hipLaunchKernelGGL(k_slot_points, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, pid, n, px, py, pz, xd, yd,
+                           zd, x, y, z, xl, yl, zl);
 }
 void launch_eval(const EvalJob *jobs, int njobs, const int32_t *idx, double *A, KParams kp, hipStream_t s) {
     if (njobs > 0) hipLaunchKernelGGL(k_eval, dim3(njobs), dim3(256), 0, s, jobs, idx, A, kp);

@@ -116,6 +116,12 @@ int h2w_save(const h2w_handle *h, const char *path) {
         if (!fp) throw Error{H2W_EINVAL, std::string("cannot open ") + path};
         h2w::Writer w{fp.get()};
         const h2w::Plan &P = h->plan;
+        std::vector<double> lr(h->d_lr.n);  // L and R of every skeleton
+        H2W_HIP(hipSetDevice(h->opts.device));
+        if (!lr.empty()) H2W_HIP(hipMemcpy(lr.data(), h->d_lr.p, lr.size() * 8, hipMemcpyDeviceToHost));
+        auto put_lr = [&](int64_t off, int64_t r) {
+            if (r > 0) w.raw(lr.data() + off, (size_t)(2 * r * r) * sizeof(double));
+        };
         w.raw(h2w::kMagic, 8);
         const int32_t hdr[8] = {h->dim, h->variant, h->choice, h->tol_pow, h->n_max, P.nL, h->opts.compat, 0};
         w.raw(hdr, sizeof(hdr));
@@ -139,7 +145,7 @@ int h2w_save(const h2w_handle *h, const char *path) {
                     w.put<int32_t>(r);
                     w.vec(fl->Ir[b], r);
                     w.vec(fl->Ic[b], r);
-                    w.vec(fl->lr[b], (size_t)2 * r * r);
+                    put_lr(fl->lr[b], r);
                     w.put<int32_t>((int32_t)fl->hist[b].size());
                     w.vec(fl->hist[b], fl->hist[b].size());
                 }
@@ -150,7 +156,7 @@ int h2w_save(const h2w_handle *h, const char *path) {
             w.raw(v, sizeof(v));
             w.vec(p.Ir, p.rank);
             w.vec(p.Ic, p.rank);
-            w.vec(p.lr, (size_t)2 * p.rank * p.rank);
+            put_lr(p.lr, p.rank);
         }
         const uint64_t hash = w.hash;
         w.put<uint64_t>(hash);
@@ -206,6 +212,14 @@ int h2w_load(const char *path, const h2w_opts *opts, h2w_handle **out) {
                 if (i < 0 || i >= N) return false;
             return true;
         };
+        // L and R of a skeleton: their offset in what goes to the device
+        std::vector<double> lr, one;
+        auto get_lr = [&](int64_t rk) {
+            const int64_t o = (int64_t)lr.size();
+            r.vec(one, 2 * rk * rk, 2 * rk * rk);
+            lr.insert(lr.end(), one.begin(), one.end());
+            return o;
+        };
         // levels each family's skeletons exist on (far: 2..nL, vertex: 1..nL; see the assembly)
         const bool fam_used[2] = {dim >= 2 && variant != H2W_NON_NESTED, variant == H2W_NESTED};
         const int fam_lo[2] = {2, 1};
@@ -220,7 +234,7 @@ int h2w_load(const char *path, const h2w_opts *opts, h2w_handle **out) {
                 fl.rank.resize(nb);
                 fl.Ir.resize(nb);
                 fl.Ic.resize(nb);
-                fl.lr.resize(nb);
+                fl.lr.assign(nb, -1);
                 fl.hist.resize(nb);
                 for (int b = 0; b < nb; ++b) {
                     const int32_t rk = r.get<int32_t>();
@@ -228,7 +242,7 @@ int h2w_load(const char *path, const h2w_opts *opts, h2w_handle **out) {
                     fl.rank[b] = rk;
                     r.vec(fl.Ir[b], rk, N);
                     r.vec(fl.Ic[b], rk, N);
-                    r.vec(fl.lr[b], (int64_t)2 * rk * rk, (int64_t)2 * rk * rk);
+                    fl.lr[b] = get_lr(rk);
                     const int32_t nh = r.get<int32_t>();
                     r.vec(fl.hist[b], nh, (int64_t)2 * N);
                     if (!pivots_ok(fl.Ir[b]) || !pivots_ok(fl.Ic[b]))
@@ -266,7 +280,7 @@ int h2w_load(const char *path, const h2w_opts *opts, h2w_handle **out) {
             p.rank = v[3];
             r.vec(p.Ir, p.rank, N);
             r.vec(p.Ic, p.rank, N);
-            r.vec(p.lr, (int64_t)2 * p.rank * p.rank, (int64_t)2 * p.rank * p.rank);
+            p.lr = get_lr(p.rank);
             if (!pivots_ok(p.Ir) || !pivots_ok(p.Ic)) throw Error{H2W_EINVAL, "corrupt operator file (pair pivot)"};
         }
         const uint64_t want = r.hash;
@@ -281,6 +295,8 @@ int h2w_load(const char *path, const h2w_opts *opts, h2w_handle **out) {
             return H2W_OK;
         }
         h2w::attach_device(*h);
+        h->d_lr.upload(lr, h->stream);
+        H2W_HIP(hipStreamSynchronize(h->stream));
         h2w::rebuild_operators(*h);
         h->assembly_seconds = h2w::now_s() - t0;
         *out = h;
