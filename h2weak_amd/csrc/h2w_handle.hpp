@@ -133,6 +133,7 @@ struct FamLevel {
     std::vector<std::vector<int32_t>> S;       // transfer row set (leaf: box points; else children's Ir)
     std::vector<int64_t> o_off, u_off;         // vec pool
     std::vector<int64_t> e_off, et_off;        // mat pool
+    std::vector<int64_t> c_off, ct_off;        // mat pool: composite transfers (level_groups)
 };
 
 struct Pair {                                  // semi-nested vertex pair (B <- V) at a level

@@ -119,6 +119,11 @@ struct XferJob {   // E = K(S, Ic) (L R)^{-1}, m x r at e (ld lde); E^T (r x m) 
     int32_t ldr, pad;  // leading dimension of L and R (R at lr + ldr^2): r, or more for their leading blocks
 };
 
+struct ComposeJob {  // D = A B (m x k times k x n), or D = A (m x n) when k = 0; DT = D^T where dt >= 0
+    int64_t a, b, d, dt;
+    int32_t m, k, n, lda, ldb, ldd, ldt, pad;
+};
+
 struct CurJob {    // A = (L R)^{-1} K(Ir, V), r x n column-major at a, leading dimension lda
     int64_t ir, v, lr, a;
     int32_t r, n, lda, pad;
@@ -217,6 +222,8 @@ void launch_xfer(const XferJob *jobs, int njobs, const int32_t *idx, const doubl
                  hipStream_t s);
 void launch_cur(const CurJob *jobs, int njobs, const int32_t *idx, const double *lr, double *A, KParams kp,
                 hipStream_t s);
+// lo: low parts of the blocks at offsets lo0 and up
+void launch_compose(const ComposeJob *jobs, int njobs, double *A, double *lo, int64_t lo0, hipStream_t s);
 void launch_copy32(const CopyJob *jobs, int njobs, const float *src, float *dst, hipStream_t s);
 // operator pool A0, or A1 for items whose flags have bit 1 set; unr in {2, 4, 8}.  Role 1:
 // symmetric terms (t >= 0) also add A^T x_item to vec[t ..] atomically.

@@ -1519,6 +1519,52 @@ void assemble(Handle &h) {
     assemble_operators(h, t0);
 }
 
+// The transfer passes near the root are launches of a few hundred kilobytes, one after another, 3 to 4 us
+// each whatever they hold (10 of the 12 levels of a 1D system with N = 250000).  Levels B .. T-1 can be one
+// launch each way: their skeletons go straight to those of their descendants at level T and back, by the
+// products of the transfers between them.  Such blocks hold a full row of blocks each, so that every level
+// of the group has as many bytes as the widest; a group grows while the launches it saves outweigh the bytes
+// it adds, and while no block is so large that the launch would cut it into pieces that accumulate
+// atomically (a box's outgoing vector stays one sum in one order).  Returns the groups from the leaves up as
+// (T, B), B = T - 1 for a level by itself (real kernels; the inner operator keeps its own chain).
+// Measured, products without / with: 1D N = 250000 214 / 173 us (FP32 177 / 132), 1D N = 2048 62 / 48 us.
+constexpr double kLaunchUs = 3.0, kBytesPerUs = 4.0e6;
+std::vector<std::pair<int, int>> level_groups(const Handle &h, const int (&lo)[2], const bool (&on)[2]) {
+    const Plan &P = h.plan;
+    std::vector<std::pair<int, int>> G;
+    for (int T = P.nL; T > 1;) {
+        int best = T - 1;
+        double gain = 0.0, extra = 0.0;  // elements, each way
+        int levels = 0;
+        for (int j = T - 1; j >= 1 && !h.cplx; --j) {
+            bool any = false, fits = true;
+            for (int f = 0; f < 2; ++f) {
+                if (!on[f] || j < lo[f]) continue;
+                const FamLevel &fl = h.fam[f][j], &ft = h.fam[f][T];
+                const int64_t nd = (int64_t)1 << (P.dim * (T - j));
+                for (int b = 0; b < fl.nb; ++b) {
+                    if (fl.rank[b] == 0) continue;
+                    any = true;
+                    int64_t R = 0;
+                    for (int64_t c = b * nd; c < (b + 1) * nd; ++c) R += ft.rank[c];
+                    fits = fits && std::min<int64_t>(fl.rank[b], kRowTile) * R <= 2 * kMinPiece;
+                    extra += (double)fl.rank[b] * (double)(R - (int64_t)fl.S[b].size());
+                }
+            }
+            if (j < T - 1 && !fits) break;
+            levels += any;
+            const double g = 2.0 * (levels - 1) * kLaunchUs - 2.0 * 8.0 * extra / kBytesPerUs;
+            if (g > gain) {
+                gain = g;
+                best = j;
+            }
+        }
+        G.push_back({T, best});
+        T = best;
+    }
+    return G;
+}
+
 // Everything after the skeletons: pools, transfer / M2L / near-field / CUR blocks,
 // the FP32 shadow, work lists and the inner operator.  Reads h.fam (ranks, pivots,
 // L and R, ACA histories, row sets S) and h.pairs only, so it also rebuilds an
@@ -1595,6 +1641,38 @@ void assemble_operators(Handle &h, double t0) {
             }
         }
     }
+    // composite transfers of the groups of several levels: per box c at T the blocks of all its ancestors of
+    // the group side by side (down), per box above T - 1 its descendants' blocks transposed (up; at T - 1
+    // that is the transfer itself)
+    const auto groups = level_groups(h, nfam_lo, fam_on);
+    auto ancestor = [&](int c, int T, int j) { return c >> (P.dim * (T - j)); };
+    auto first_at = [&](int b, int j, int T) { return (int)((int64_t)b << (P.dim * (T - j))); };
+    auto rank_at = [&](int f, int b, int j, int T) {
+        int64_t R = 0;
+        for (int c = first_at(b, j, T); c < first_at(b + 1, j, T); ++c) R += h.fam[f][T].rank[c];
+        return R;
+    };
+    const int64_t comp0 = mo;
+    for (auto [T, B] : groups)
+        for (int f = 0; f < 2 && B < T - 1; ++f) {
+            if (!fam_on[f]) continue;
+            FamLevel &ft = h.fam[f][T];
+            ft.c_off.assign(ft.nb, -1);
+            for (int c = 0; c < ft.nb; ++c) {
+                int64_t n = 0;
+                for (int j = T - 1; j >= std::max(B, nfam_lo[f]); --j) n += h.fam[f][j].rank[ancestor(c, T, j)];
+                if (ft.rank[c] > 0 && n > 0) ft.c_off[c] = take(pad_ld(ft.rank[c]) * n);
+            }
+            for (int j = T - 2; j >= std::max(B, nfam_lo[f]); --j) {
+                FamLevel &fl = h.fam[f][j];
+                fl.ct_off.assign(fl.nb, -1);
+                for (int b = 0; b < fl.nb; ++b) {
+                    const int64_t R = rank_at(f, b, j, T);
+                    if (fl.rank[b] > 0 && R > 0) fl.ct_off[b] = take(pad_ld(fl.rank[b]) * R);
+                }
+            }
+        }
+    const int64_t comp_len = mo - comp0;
     auto &m2l = h.m2l;
     m2l.clear();
     for (int f = 0; f < 2; ++f) {
@@ -1758,6 +1836,54 @@ void assemble_operators(Handle &h, double t0) {
         H2W_HIP(hipGetLastError());
         H2W_HIP(hipStreamSynchronize(s));
     }
+    // composite transfers, level by level away from T (block (c, a) from block (c, a's child))
+    DevBuf<double> comp_lo;
+    comp_lo.alloc(comp_len);
+    for (auto [T, B] : groups)
+        for (int j = T - 1; j >= B && B < T - 1; --j) {
+            std::vector<ComposeJob> jobs;
+            for (int f = 0; f < 2; ++f) {
+                if (!fam_on[f] || j < nfam_lo[f]) continue;
+                const FamLevel &fl = h.fam[f][j], &ft = h.fam[f][T];
+                for (int c = 0; c < ft.nb; ++c) {
+                    const int a = ancestor(c, T, j);
+                    if (ft.c_off[c] < 0 || fl.rank[a] == 0) continue;
+                    int64_t row = 0, col = 0;  // of the child's rows in a's transfer, of the block in c's run
+                    const int ch = ancestor(c, T, j + 1);
+                    for (int q = a * P.nchild; q < ch; ++q) row += h.fam[f][j + 1].rank[q];
+                    for (int i = T - 1; i > j; --i) col += h.fam[f][i].rank[ancestor(c, T, i)];
+                    const int kc = h.fam[f][j + 1].rank[ch];
+                    if (kc == 0) continue;
+                    ComposeJob J;
+                    J.m = ft.rank[c];
+                    J.n = fl.rank[a];
+                    J.ldd = (int32_t)pad_ld(J.m);
+                    J.d = ft.c_off[c] + col * J.ldd;
+                    J.dt = -1;
+                    J.ldt = (int32_t)pad_ld(J.n);
+                    J.pad = 0;
+                    J.lda = J.ldb = (int32_t)pad_ld((int64_t)fl.S[a].size());
+                    if (j == T - 1) {
+                        J.k = 0;
+                        J.a = fl.e_off[a] + row;
+                        J.b = 0;
+                    } else {
+                        J.k = kc;
+                        J.lda = J.ldd;
+                        J.a = J.d - (int64_t)kc * J.ldd;  // (c, ch), the block before
+                        J.b = fl.e_off[a] + row;
+                        J.dt = fl.ct_off[a] + (ft.o_off[c] - ft.o_off[first_at(a, j, T)]) * J.ldt;
+                    }
+                    jobs.push_back(J);
+                }
+            }
+            DevBuf<ComposeJob> dj;
+            dj.upload(jobs, s);
+            launch_compose(dj.p, (int)jobs.size(), h.mat64.p, comp_lo.p, comp0, s);
+            H2W_HIP(hipGetLastError());
+            H2W_HIP(hipStreamSynchronize(s));
+        }
+    comp_lo.release();
     phase("transfer operators");
     {
         // plain entry blocks: M2L, near field, semi-nested column factors
@@ -1835,14 +1961,23 @@ void assemble_operators(Handle &h, double t0) {
                          false, (int)pad_ld(p.rank));
         WL.push_back(std::move(W));
     }
-    // up, levels nL-1 .. 1
-    for (int j = P.nL - 1; j >= 1; --j) {
+    // up, levels nL-1 .. 1 (the levels of a group in one launch)
+    for (auto [T, B] : groups) {
         WorkList W;
-        W.step = P.nL - j;
+        W.step = P.nL - (T - 1);
         for (int f = 0; f < 2; ++f) {
-            if (!fam_on[f] || j < nfam_lo[f]) continue;
-            for (int b = 0; b < P.nboxes[j]; ++b)
-                fam_up_item(W, f, j, b, h.fam[f][j + 1].o_off[b * P.nchild]);
+            if (!fam_on[f]) continue;
+            for (int b = 0; T - 1 >= nfam_lo[f] && b < P.nboxes[T - 1]; ++b)
+                fam_up_item(W, f, T - 1, b, h.fam[f][T].o_off[b * P.nchild]);
+            for (int j = T - 2; j >= std::max(B, nfam_lo[f]); --j) {
+                const FamLevel &fl = h.fam[f][j];
+                for (int b = 0; b < fl.nb; ++b)
+                    if (fl.ct_off[b] >= 0)
+                        add_item(W, fl.o_off[b], fl.rank[b],
+                                 {TermSpec{fl.ct_off[b], h.fam[f][T].o_off[first_at(b, j, T)],
+                                           (int32_t)rank_at(f, b, j, T)}},
+                                 false, (int)pad_ld(fl.rank[b]));
+            }
         }
         WL.push_back(std::move(W));
     }
@@ -1897,19 +2032,36 @@ void assemble_operators(Handle &h, double t0) {
         upload_lists(tl, h.trans, s);
         upload_lists(ol, h.otf, s);
     }
-    // down, levels 1 .. nL-1
-    for (int j = 1; j <= P.nL - 1; ++j) {
+    // down, levels 1 .. nL-1 (from the levels of a group in one launch)
+    for (auto g = groups.rbegin(); g != groups.rend(); ++g) {
+        const auto [T, B] = *g;
         WorkList W;
         W.stage = 2;
-        W.step = P.nL - j;
+        W.step = P.nL - (T - 1);
         for (int f = 0; f < 2; ++f) {
-            if (!fam_on[f] || j < nfam_lo[f]) continue;
-            FamLevel &fl = h.fam[f][j];
-            for (int b = 0; b < fl.nb; ++b) {
-                if (fl.e_off[b] < 0) continue;
-                int64_t m = (int64_t)fl.S[b].size();
-                add_item(W, h.fam[f][j + 1].u_off[b * P.nchild], (int)m,
-                         {TermSpec{fl.e_off[b], fl.u_off[b], (int32_t)fl.rank[b]}}, false, (int)pad_ld(m));
+            if (!fam_on[f] || T - 1 < nfam_lo[f]) continue;
+            const FamLevel &fl = h.fam[f][T - 1], &ft = h.fam[f][T];
+            if (B == T - 1) {
+                for (int b = 0; b < fl.nb; ++b) {
+                    if (fl.e_off[b] < 0) continue;
+                    int64_t m = (int64_t)fl.S[b].size();
+                    add_item(W, ft.u_off[b * P.nchild], (int)m,
+                             {TermSpec{fl.e_off[b], fl.u_off[b], (int32_t)fl.rank[b]}}, false, (int)pad_ld(m));
+                }
+                continue;
+            }
+            for (int c = 0; c < ft.nb; ++c) {
+                if (ft.c_off[c] < 0) continue;
+                const int ld = (int)pad_ld(ft.rank[c]);
+                std::vector<TermSpec> t;
+                int64_t col = 0;
+                for (int j = T - 1; j >= std::max(B, nfam_lo[f]); --j) {
+                    const FamLevel &fa = h.fam[f][j];
+                    const int a = ancestor(c, T, j);
+                    if (fa.rank[a] > 0) t.push_back(TermSpec{ft.c_off[c] + col * ld, fa.u_off[a], (int32_t)fa.rank[a]});
+                    col += fa.rank[a];
+                }
+                add_item(W, ft.u_off[c], ft.rank[c], t, false, ld);
             }
         }
         WL.push_back(std::move(W));
