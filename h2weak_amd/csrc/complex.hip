@@ -11,6 +11,7 @@
 
 #include <cfloat>
 #include <climits>
+#include <algorithm>
 
 #include "h2w_internal.hpp"
 
@@ -543,6 +544,15 @@ __global__ __launch_bounds__(256) void k_cgemv(const GItem *__restrict__ items, 
 }
 
 // ------------------------------------------------------------------ vectors
+// pool input from x and zeroed outputs (the real path's k_begin)
+__global__ __launch_bounds__(256) void k_cbegin(const double2 *x, const int32_t *perm, double2 *px, int64_t N,
+                                                double2 *py, int64_t len) {
+    const int64_t step = (int64_t)gridDim.x * 256;
+    for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < max(N, len); i += step) {
+        if (i < N) px[i] = x[perm ? perm[i] : i];
+        if (i < len) py[i] = cmk(0.0, 0.0);
+    }
+}
 __global__ void k_cfill(double2 *a, int64_t n) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         a[i] = cmk(0.0, 0.0);
@@ -682,6 +692,12 @@ void launch_cur_c(const CurJob *jobs, int njobs, const int32_t *idx, const doubl
 }
 void launch_cgemv(const GItem *items, int nitems, const GTerm *terms, const double2 *A, double2 *vec, hipStream_t s) {
     if (nitems > 0) hipLaunchKernelGGL(k_cgemv, dim3(nitems), dim3(256), 0, s, items, terms, A, vec);
+}
+void launch_cbegin(const double2 *x, const int32_t *perm, double2 *px, int64_t N, double2 *py, int64_t len,
+                   hipStream_t s) {
+    const int64_t n = std::max(N, len);
+    hipLaunchKernelGGL(k_cbegin, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 2048)), dim3(256), 0, s, x, perm, px,
+                       N, py, len);
 }
 void launch_cfill(double2 *a, int64_t n, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_cfill, dim3(cgrid(n)), dim3(256), 0, s, a, n);

@@ -241,11 +241,14 @@ int64_t stream_chunk_bytes();
 void launch_stream_read(const void *p, int64_t bytes, uint32_t *out, int grid, hipStream_t s);
 void launch_fill(double *a, int64_t n, double v, hipStream_t s);
 void launch_fill32(float *a, int64_t n, float v, hipStream_t s);
+// start of a product: px[t] = x[perm ? perm[t] : t] for t < N, py[0 .. len) = 0
+void launch_begin64(const double *x, const int32_t *perm, double *px, int64_t N, double *py, int64_t len, hipStream_t s);
+void launch_begin32(const double *x, const int32_t *perm, float *px, int64_t N, float *py, int64_t len, hipStream_t s);
+void launch_cbegin(const double2 *x, const int32_t *perm, double2 *px, int64_t N, double2 *py, int64_t len,
+                   hipStream_t s);
 // tree-order gather/scatter with optional precision change, nrhs vectors of leading dimension ld
 void launch_permute_in(const double *x, int64_t ldx, double *xt, int64_t ldt, const int32_t *perm, int64_t N,
                        int nrhs, hipStream_t s);
-void launch_permute_in32(const double *x, int64_t ldx, float *xt, int64_t ldt, const int32_t *perm, int64_t N,
-                         int nrhs, hipStream_t s);
 void launch_permute_out(const double *yt, int64_t ldt, double *y, int64_t ldy, const int32_t *perm, int64_t N,
                         int nrhs, hipStream_t s);
 void launch_permute_out32(const float *yt, int64_t ldt, double *y, int64_t ldy, const int32_t *perm, int64_t N,

@@ -2201,17 +2201,28 @@ const std::vector<Launch> &launches_for(Handle &h, int precision) {
 }
 
 void run_launches_eager(Handle &h, int precision) {
-    const auto &L = launches_for(h, precision);
-    zero_outputs(h, precision);
-    for (auto &Lh : L) run_launch(h, Lh, precision);
+    for (auto &Lh : launches_for(h, precision)) run_launch(h, Lh, precision);
     H2W_HIP(hipGetLastError());
 }
 
 // The launch sequence of a matvec is fixed per handle and precision (pool pointers and work
 // lists do not change after assembly), so it is captured once into a HIP graph and replayed.
-// Every node is a kernel (the output zeroing included).
+// Every node is a kernel.  The outputs are zeroed before it (with the input, in one kernel, or
+// by zero_outputs).
+// A replay costs the host about 6 us more than its first kernel alone, each plain launch 4.7 us, which pass
+// while the GPU works on the launches before it: the graph is for sequences that run faster than the host
+// can launch them.  (Plain launches against replays, whole products: 1D N = 2048, 5 launches 37 / 45 us, its
+// inner operator's 11 launches 81 / 64 us; 1D N = 250000, 11 launches 169 / 174 us; 3D N = 20011 220 / 224 us.)
+bool replay_pays(Handle &h, int precision) {
+    const auto &L = launches_for(h, precision);
+    const auto &e = precision == H2W_FP32_INNER ? h.inner.elems : h.launch_elems;
+    const double bytes = h.cplx ? 16.0 : is32(precision) ? 4.0 : 8.0;
+    double gpu = 6.0;
+    for (size_t q = 0; q < L.size(); ++q) gpu += std::max(3.5, (double)e[q] * bytes / 5.0e6);
+    return 4.7 * (double)L.size() > gpu;
+}
 void run_launches(Handle &h, int precision) {
-    if (!h.use_graph) {
+    if (!h.use_graph || !replay_pays(h, precision)) {
         run_launches_eager(h, precision);
         return;
     }
@@ -2262,8 +2273,7 @@ void matvec_dev(Handle &h, const double *x, double *y, int precision, bool tree)
         double2 *pool = reinterpret_cast<double2 *>(h.vec64.p);
         const double2 *xc = reinterpret_cast<const double2 *>(x);
         double2 *yc = reinterpret_cast<double2 *>(y);
-        if (tree) H2W_HIP(hipMemcpyAsync(pool + h.off_x, xc, N * 16, hipMemcpyDeviceToDevice, s));
-        else launch_cpermute_in(xc, pool + h.off_x, h.d_perm.p, N, s);
+        launch_cbegin(xc, tree ? nullptr : h.d_perm.p, pool + h.off_x, N, pool + h.off_y, h.vec_len - h.off_y, s);
         run_launches(h, precision);
         if (tree) H2W_HIP(hipMemcpyAsync(yc, pool + h.off_y, N * 16, hipMemcpyDeviceToDevice, s));
         else launch_cpermute_out(pool + h.off_y, yc, h.d_perm.p, N, s);
@@ -2272,14 +2282,14 @@ void matvec_dev(Handle &h, const double *x, double *y, int precision, bool tree)
     }
     if (is32(precision)) {
         if (!h.mat32.p) throw Error{H2W_ESTATE, "FP32 matvec requested but the FP32 shadow was not built"};
-        if (tree) launch_to_fp32(x, h.vec32.p + h.off_x, N, s);
-        else launch_permute_in32(x, N, h.vec32.p + h.off_x, N, h.d_perm.p, N, 1, s);
+        launch_begin32(x, tree ? nullptr : h.d_perm.p, h.vec32.p + h.off_x, N, h.vec32.p + h.off_y, h.vec_len - h.off_y,
+                       s);
         run_launches(h, precision);
         if (tree) launch_to_fp64(h.vec32.p + h.off_y, y, N, s);
         else launch_permute_out32(h.vec32.p + h.off_y, N, y, N, h.d_perm.p, N, 1, s);
     } else {
-        if (tree) H2W_HIP(hipMemcpyAsync(h.vec64.p + h.off_x, x, N * 8, hipMemcpyDeviceToDevice, s));
-        else launch_permute_in(x, N, h.vec64.p + h.off_x, N, h.d_perm.p, N, 1, s);
+        launch_begin64(x, tree ? nullptr : h.d_perm.p, h.vec64.p + h.off_x, N, h.vec64.p + h.off_y, h.vec_len - h.off_y,
+                       s);
         run_launches(h, precision);
         if (tree) H2W_HIP(hipMemcpyAsync(y, h.vec64.p + h.off_y, N * 8, hipMemcpyDeviceToDevice, s));
         else launch_permute_out(h.vec64.p + h.off_y, N, y, N, h.d_perm.p, N, 1, s);
@@ -2971,7 +2981,10 @@ double time_matvec(Handle &h, int precision, int nrep) {
     tune_inputs(h, precision);
     run_launches(h, precision);
     H2W_HIP(hipEventRecord(ev.a, h.stream));
-    for (int r = 0; r < nrep; ++r) run_launches(h, precision);
+    for (int r = 0; r < nrep; ++r) {
+        zero_outputs(h, precision);
+        run_launches(h, precision);
+    }
     H2W_HIP(hipEventRecord(ev.b, h.stream));
     return ev.ms(h.stream) / nrep;
 }
@@ -3752,11 +3765,15 @@ int h2w_bench_matvec(h2w_handle *h, int nrep, int precision, h2w_bench *out) {
     std::vector<h2w::Event> ev(nl + 2);
     std::vector<double> acc(nl + 1, 0.0);
     // warm-up
+    h2w::zero_outputs(*h, precision);
     h2w::run_launches(*h, precision);
     H2W_HIP(hipStreamSynchronize(s));
     h2w::Event t0, t1;
     H2W_HIP(hipEventRecord(t0, s));
-    for (int r = 0; r < nrep; ++r) h2w::run_launches(*h, precision);
+    for (int r = 0; r < nrep; ++r) {
+        h2w::zero_outputs(*h, precision);
+        h2w::run_launches(*h, precision);
+    }
     H2W_HIP(hipEventRecord(t1, s));
     out->ms_per_matvec = h2w::elapsed_ms(t0, t1) / nrep;
     // per-launch durations: fill + each bgemv launch

@@ -2089,6 +2089,17 @@ __global__ void k_permute_in(const double *x, int64_t ldx, T *xt, int64_t ldt, c
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < N; t += (int64_t)gridDim.x * blockDim.x)
         xt[r * ldt + t] = (T)x[r * ldx + perm[t]];
 }
+// What comes before the launches of a product, in one pass: the pool's input from x (tree order, or input
+// order through perm) and zeros in everything the product accumulates into.
+template <typename T>
+__global__ __launch_bounds__(256) void k_begin(const double *x, const int32_t *perm, T *px, int64_t N, T *py,
+                                               int64_t len) {
+    const int64_t step = (int64_t)gridDim.x * 256;
+    for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < max(N, len); i += step) {
+        if (i < N) px[i] = (T)x[perm ? perm[i] : i];
+        if (i < len) py[i] = T(0);
+    }
+}
 template <typename T>
 __global__ void k_permute_out(const T *yt, int64_t ldt, double *y, int64_t ldy, const int32_t *perm, int64_t N) {
     const int r = blockIdx.y;
@@ -2607,14 +2618,17 @@ void launch_fill(double *a, int64_t n, double v, hipStream_t s) {
 void launch_fill32(float *a, int64_t n, float v, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_fill<float>, dim3(grid_for(n)), dim3(256), 0, s, a, n, v);
 }
+void launch_begin64(const double *x, const int32_t *perm, double *px, int64_t N, double *py, int64_t len, hipStream_t s) {
+    hipLaunchKernelGGL(k_begin<double>, dim3(grid_for(std::max(N, len), 256, 2048)), dim3(256), 0, s, x, perm, px, N, py,
+                       len);
+}
+void launch_begin32(const double *x, const int32_t *perm, float *px, int64_t N, float *py, int64_t len, hipStream_t s) {
+    hipLaunchKernelGGL(k_begin<float>, dim3(grid_for(std::max(N, len), 256, 2048)), dim3(256), 0, s, x, perm, px, N, py,
+                       len);
+}
 void launch_permute_in(const double *x, int64_t ldx, double *xt, int64_t ldt, const int32_t *perm, int64_t N,
                        int nrhs, hipStream_t s) {
     hipLaunchKernelGGL(k_permute_in<double>, dim3(grid_for(N, 256, 2048), nrhs), dim3(256), 0, s, x, ldx, xt, ldt,
-                       perm, N);
-}
-void launch_permute_in32(const double *x, int64_t ldx, float *xt, int64_t ldt, const int32_t *perm, int64_t N,
-                         int nrhs, hipStream_t s) {
-    hipLaunchKernelGGL(k_permute_in<float>, dim3(grid_for(N, 256, 2048), nrhs), dim3(256), 0, s, x, ldx, xt, ldt,
                        perm, N);
 }
 void launch_permute_out(const double *yt, int64_t ldt, double *y, int64_t ldy, const int32_t *perm, int64_t N,
