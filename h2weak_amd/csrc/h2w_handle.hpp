@@ -322,6 +322,9 @@ struct h2w_handle {
     int defl_serial = 0;                // incremented whenever the space is rebuilt or dropped
     int gv_defl = -1;                   // serial of the space whose U, C sit in g_U / g_V's first columns
     h2w::PinBuf g_pin;                // GMRES read-backs (Hessenberg columns)
+    h2w::DevBuf<uint32_t> g_cnt;      // arrival counter of the Arnoldi passes
+    h2w::PinBuf g_flag;               // sequence number of the last pass whose results are in g_pin
+    uint64_t g_seq = 0;
     int64_t g_Vcols = 0;
     // kNR-wide lockstep GMRES (interleaved N x kNR vectors)
     h2w::LockBufs mbuf;

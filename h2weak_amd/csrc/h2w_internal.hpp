@@ -241,9 +241,12 @@ int64_t stream_chunk_bytes();
 void launch_stream_read(const void *p, int64_t bytes, uint32_t *out, int grid, hipStream_t s);
 void launch_fill(double *a, int64_t n, double v, hipStream_t s);
 void launch_fill32(float *a, int64_t n, float v, hipStream_t s);
-// start of a product: px[t] = x[perm ? perm[t] : t] for t < N, py[0 .. len) = 0
-void launch_begin64(const double *x, const int32_t *perm, double *px, int64_t N, double *py, int64_t len, hipStream_t s);
-void launch_begin32(const double *x, const int32_t *perm, float *px, int64_t N, float *py, int64_t len, hipStream_t s);
+// start of a product: px[t] = scale x[perm ? perm[t] : t] for t < N (scale / sqrt(*norm2) with norm2 given), also to
+// copy[t] if given; py[0 .. len) = 0
+void launch_begin64(const double *x, double scale, const double *norm2, double *copy, const int32_t *perm, double *px,
+                    int64_t N, double *py, int64_t len, hipStream_t s);
+void launch_begin32(const double *x, double scale, const double *norm2, double *copy, const int32_t *perm, float *px,
+                    int64_t N, float *py, int64_t len, hipStream_t s);
 void launch_cbegin(const double2 *x, const int32_t *perm, double2 *px, int64_t N, double2 *py, int64_t len,
                    hipStream_t s);
 // tree-order gather/scatter with optional precision change, nrhs vectors of leading dimension ld
@@ -256,10 +259,27 @@ void launch_permute_out32(const float *yt, int64_t ldt, double *y, int64_t ldy, 
 void launch_dense_rows(const int32_t *rows, int64_t nrows, const double *xt, double *y, int64_t N, KParams kp,
                        hipStream_t s);
 // BLAS-1 for the Arnoldi process (all FP64)
-void launch_mdot(const double *V, int64_t ldv, int k, const double *w, int64_t n, double *partial, int nblk,
-                 hipStream_t s);
-void launch_mdot_reduce(const double *partial, int nblk, int k, double *out, hipStream_t s);
-void launch_mgemv_sub(const double *V, int64_t ldv, int k, const double *h, double *w, int64_t n, hipStream_t s);
+struct CgsArgs {          // one pass (k_cgs)
+    const double *V;
+    int64_t ldv;
+    const float *src32 = nullptr;  // w's values, if they are the FP32 product's
+    double *w;
+    int64_t n;
+    int s0 = 0, ns = 0;   // columns subtracted, with the coefficients sub
+    const double *sub = nullptr;
+    int d0 = 0, nd = 0;   // columns dotted into out, or (norm) out[0] = w . w
+    int norm = 0;
+    double *partial;      // cgs_blocks(n) x max(nd, 1)
+    uint32_t *arrived;    // zero between launches
+    double *out;
+    const double *all_h = nullptr;  // host[0 .. nhost) = all_h, host[nhost ..) = out (host non-null: always one launch)
+    int nhost = 0;
+    double *host = nullptr;
+    uint64_t *flag = nullptr;      // (page-locked, with host) receives seq after host is written
+    uint64_t seq = 0;
+};
+int cgs_blocks(int64_t n);
+void launch_cgs(const CgsArgs &a, hipStream_t s);
 void launch_axpby(double a, const double *x, double b, double *y, int64_t n, hipStream_t s);
 void launch_scal(double a, double *y, int64_t n, hipStream_t s);  // y *= a
 void launch_vec_update(const double *V, int64_t ldv, int k, const double *c, double *x, int64_t n, hipStream_t s);
@@ -322,7 +342,6 @@ void launch_bdot16_reduce(const double *partial, int nblk, int k, const int32_t 
 void launch_bgemv16(const double *V, int64_t ldv, int k, const double *h, int S, double sign, double *w, int64_t n,
                     const int32_t *seg, hipStream_t s);
 void launch_bscale16(const double *src, const double *sc, double *dst, int64_t n, const int32_t *seg, hipStream_t s);
-int mdot_blocks(int64_t n);
 
 // complex kernels (complex.hip): operator and vector pools of double2 (re, im), element offsets as
 // in the real path

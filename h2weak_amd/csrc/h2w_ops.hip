@@ -19,6 +19,7 @@
 #include <thread>
 
 #include <algorithm>
+#include <atomic>
 #include <deque>
 #include <chrono>
 #include <cmath>
@@ -2263,6 +2264,16 @@ void drop_graphs(Handle &h) {
     for (int p = 0; p < 5; ++p) drop_graph(h, p);
 }
 
+// pool input (scale x, or x / sqrt(*norm2); tree order, kept at copy too) and zeroed outputs of a product
+// (real kernels)
+void begin_product(Handle &h, const double *x, double scale, const double *norm2, double *copy, int precision) {
+    const int64_t len = h.vec_len - h.off_y;
+    if (is32(precision))
+        launch_begin32(x, scale, norm2, copy, nullptr, h.vec32.p + h.off_x, h.N, h.vec32.p + h.off_y, len, h.stream);
+    else
+        launch_begin64(x, scale, norm2, copy, nullptr, h.vec64.p + h.off_x, h.N, h.vec64.p + h.off_y, len, h.stream);
+}
+
 // device-pointer matvec on one vector; tree-ordered in/out when tree == true
 void matvec_dev(Handle &h, const double *x, double *y, int precision, bool tree) {
     hipStream_t s = h.stream;
@@ -2282,13 +2293,13 @@ void matvec_dev(Handle &h, const double *x, double *y, int precision, bool tree)
     }
     if (is32(precision)) {
         if (!h.mat32.p) throw Error{H2W_ESTATE, "FP32 matvec requested but the FP32 shadow was not built"};
-        launch_begin32(x, tree ? nullptr : h.d_perm.p, h.vec32.p + h.off_x, N, h.vec32.p + h.off_y, h.vec_len - h.off_y,
+        launch_begin32(x, 1.0, nullptr, nullptr, tree ? nullptr : h.d_perm.p, h.vec32.p + h.off_x, N, h.vec32.p + h.off_y, h.vec_len - h.off_y,
                        s);
         run_launches(h, precision);
         if (tree) launch_to_fp64(h.vec32.p + h.off_y, y, N, s);
         else launch_permute_out32(h.vec32.p + h.off_y, N, y, N, h.d_perm.p, N, 1, s);
     } else {
-        launch_begin64(x, tree ? nullptr : h.d_perm.p, h.vec64.p + h.off_x, N, h.vec64.p + h.off_y, h.vec_len - h.off_y,
+        launch_begin64(x, 1.0, nullptr, nullptr, tree ? nullptr : h.d_perm.p, h.vec64.p + h.off_x, N, h.vec64.p + h.off_y, h.vec_len - h.off_y,
                        s);
         run_launches(h, precision);
         if (tree) H2W_HIP(hipMemcpyAsync(y, h.vec64.p + h.off_y, N * 8, hipMemcpyDeviceToDevice, s));
@@ -2340,30 +2351,65 @@ void ensure_V(Handle &h, int64_t cols) {
     h.g_Vcols = nc;
 }
 
-double dev_norm(Handle &h, const double *v) {
-    int nb = mdot_blocks(h.N);
-    h.g_part.ensure((size_t)nb * 4);
-    h.g_h.ensure(8);
-    launch_mdot(v, h.N, 1, v, h.N, h.g_part.p, nb, h.stream);
-    launch_mdot_reduce(h.g_part.p, nb, 1, h.g_h.p, h.stream);
-    double r = 0.0;
-    H2W_HIP(hipMemcpyAsync(&r, h.g_h.p, 8, hipMemcpyDeviceToHost, h.stream));
-    H2W_HIP(hipStreamSynchronize(h.stream));
-    return std::sqrt(r);
+// work arrays of the Arnoldi passes for up to k columns
+CgsArgs cgs_args(Handle &h, double *w, int64_t k) {
+    if (!h.g_cnt.p) {
+        h.g_cnt.alloc(1);
+        H2W_HIP(hipMemsetAsync(h.g_cnt.p, 0, 4, h.stream));
+    }
+    h.g_part.ensure((size_t)cgs_blocks(h.N) * std::max<int64_t>(k, 1));
+    CgsArgs a;
+    a.V = nullptr;
+    a.ldv = a.n = h.N;
+    a.w = w;
+    a.partial = h.g_part.p;
+    a.arrived = h.g_cnt.p;
+    a.out = nullptr;
+    return a;
 }
 
+// A pass whose results go to the host, and the wait for them: a poll of the flag that the pass writes last,
+// in page-locked memory, with a look at the stream now and then (an error there, or a stream that ended
+// without the flag, ends the wait).
+void launch_cgs_host(Handle &h, CgsArgs &a) {
+    if (!h.g_flag.p) {
+        h.g_flag.ensure(1);
+        std::memset(h.g_flag.p, 0, sizeof(uint64_t));
+    }
+    a.flag = reinterpret_cast<uint64_t *>(h.g_flag.p);
+    a.seq = ++h.g_seq;
+    launch_cgs(a, h.stream);
+    H2W_HIP(hipGetLastError());
+}
+void wait_cgs_host(Handle &h) {
+    const volatile uint64_t *f = reinterpret_cast<const volatile uint64_t *>(h.g_flag.p);
+    for (int64_t spin = 1; *f < h.g_seq; ++spin) {
+        if (spin % 16384 != 0) continue;
+        const hipError_t e = hipStreamQuery(h.stream);
+        if (e == hipErrorNotReady) continue;
+        H2W_HIP(e);
+        if (*f < h.g_seq) throw Error{H2W_EHIP, "an Arnoldi pass ended without its results"};
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+}
+
+// a . b (b == nullptr: a . a), read back through page-locked memory; neither is written
 double dev_dot(Handle &h, const double *a, const double *b) {
-    int nb = mdot_blocks(h.N);
-    h.g_part.ensure((size_t)nb * 4);
+    CgsArgs c = cgs_args(h, const_cast<double *>(a), 1);
     h.g_h.ensure(8);
-    launch_mdot(a, h.N, 1, b, h.N, h.g_part.p, nb, h.stream);
-    launch_mdot_reduce(h.g_part.p, nb, 1, h.g_h.p, h.stream);
-    double r = 0.0;
-    H2W_HIP(hipMemcpyAsync(&r, h.g_h.p, 8, hipMemcpyDeviceToHost, h.stream));
-    H2W_HIP(hipStreamSynchronize(h.stream));
-    return r;
+    c.V = b;
+    c.nd = b ? 1 : 0;
+    c.norm = !b;
+    c.out = h.g_h.p;
+    c.host = h.g_pin.ensure(8);
+    c.all_h = h.g_h.p;
+    c.nhost = 1;  // (out follows at host[1])
+    launch_cgs_host(h, c);
+    wait_cgs_host(h);
+    return h.g_pin.p[1];
 }
 
+double dev_norm(Handle &h, const double *v) { return std::sqrt(dev_dot(h, v, nullptr)); }
 
 // Solves A x = b (tree order, device).  x_zero: x0 = 0 and no initial matvec.
 // normb_in > 0 overrides ||b|| in the stopping test.
@@ -2374,7 +2420,7 @@ GmresOut gmres_core(Handle &h, const double *b, double *x, int max_iter, double 
     GmresOut out;
     h.g_w.ensure(N);
     h.g_b.ensure(N);  // residual of this solve
-    double *w = h.g_w.p, *r = h.g_b.p;
+    double *r = h.g_b.p;
     double normb = normb_in > 0 ? normb_in : dev_norm(h, b);
     // recycled space (x starts at zero): x = U C^T r, r -= C C^T r, and every Arnoldi vector is
     // orthogonalised against C as well (its coefficients B = C^T A v_j enter the update of x)
@@ -2382,24 +2428,38 @@ GmresOut gmres_core(Handle &h, const double *b, double *x, int max_iter, double 
     const bool once = kc > 0 && rc->invariant;
     if (!once) h.gv_defl = -1;  // (its basis overwrites the first columns of g_V)
     const int m = max_iter;
-    const int nb = mdot_blocks(N);
-    h.g_part.ensure((size_t)nb * (kc + m + 2));
+    CgsArgs A = cgs_args(h, r, kc + m + 2);
     h.g_h.ensure((size_t)2 * (kc + m + 2) + 2);
+    double *hh = h.g_pin.ensure(2 * (kc + m + 2) + 8);
     if (x_zero) {
         H2W_HIP(hipMemcpyAsync(r, b, N * 8, hipMemcpyDeviceToDevice, s));
     } else {
-        matvec_dev(h, x, w, prec, true);
+        matvec_dev(h, x, h.g_w.p, prec, true);
         out.matvecs++;
         H2W_HIP(hipMemcpyAsync(r, b, N * 8, hipMemcpyDeviceToDevice, s));
-        launch_axpby(-1.0, w, 1.0, r, N, s);
+        launch_axpby(-1.0, h.g_w.p, 1.0, r, N, s);
     }
+    double beta;
     if (kc > 0) {
-        launch_mdot(h.g_V.p, N, kc, r, N, h.g_part.p, nb, s);
-        launch_mdot_reduce(h.g_part.p, nb, kc, h.g_h.p, s);
-        launch_mgemv_sub(h.g_V.p, N, kc, h.g_h.p, r, N, s);
+        A.V = h.g_V.p;
+        A.nd = kc;
+        A.out = h.g_h.p;
+        launch_cgs(A, s);  // C^T r
         launch_vec_update(h.g_U.p, N, kc, h.g_h.p, x, N, s);
+        CgsArgs B = A;
+        B.ns = kc;
+        B.sub = h.g_h.p;
+        B.norm = 1;
+        B.out = h.g_h.p + kc;
+        B.all_h = h.g_h.p;
+        B.nhost = 1;
+        B.host = hh;
+        launch_cgs_host(h, B);  // r -= C C^T r, and its norm
+        wait_cgs_host(h);
+        beta = std::sqrt(hh[1]);
+    } else {
+        beta = dev_norm(h, r);
     }
-    double beta = dev_norm(h, r);
     if (normb == 0.0) normb = 1;
     out.resid = beta / normb;
     if (out.resid <= tol) {
@@ -2411,28 +2471,60 @@ GmresOut gmres_core(Handle &h, const double *b, double *x, int max_iter, double 
     std::vector<double> sv(m + 1, 0.0), cs(m + 1, 0.0), sn(m + 1, 0.0);
     auto Hh = [&](int i, int j) -> double & { return H[j][i]; };
     ensure_V(h, kc + std::min<int64_t>(m + 1, 32));
-    launch_axpby(1.0 / beta, r, 0.0, h.g_V.p + (int64_t)kc * N, N, s);
     sv[0] = beta;
-    double *hh = h.g_pin.ensure(2 * (kc + m + 2) + 2);
+    const double *next = r;  // v_i = next scale
+    double scale = 1.0 / beta;
+    // The product of step i + 1 needs the norm of step i's vector only, which the device has: it is queued
+    // before the host has read step i's coefficients, unless the residual, shrinking as it did in the step
+    // before, would reach the tolerance (a product too many costs more than the idle time it hides).
+    bool ahead = false;
+    double res1 = out.resid, res2 = 0.0;  // residuals of the last two steps
     for (int i = 0; i < m; ++i) {
-        ensure_V(h, kc + i + 2);
+        ensure_V(h, kc + i + 3);
         double *C = h.g_V.p, *V = h.g_V.p + (int64_t)kc * N;
-        matvec_dev(h, V + (int64_t)i * N, w, prec, true);
+        // w = A v_i: left in the pool (FP64) or taken from there by the first pass (FP32)
+        const bool f32 = is32(prec);
+        if (!ahead) {
+            begin_product(h, next, scale, nullptr, V + (int64_t)i * N, prec);
+            run_launches(h, prec);
+        }
         out.matvecs++;
+        double *w = f32 ? h.g_w.p : h.vec64.p + h.off_y;
         const int k = kc + i + 1;  // vectors orthogonalised against: C, v_0 .. v_i (contiguous)
-        launch_mdot(C, N, k, w, N, h.g_part.p, nb, s);
-        launch_mdot_reduce(h.g_part.p, nb, k, h.g_h.p, s);
-        launch_mgemv_sub(C, N, k, h.g_h.p, w, N, s);
         // second pass: against C as well, or (a deflation space) against v_0 .. v_i only
         const int k0 = once ? kc : 0;
-        if (once) launch_fill(h.g_h.p + k, kc, 0.0, s);
-        launch_mdot(C + (int64_t)k0 * N, N, k - k0, w, N, h.g_part.p, nb, s);
-        launch_mdot_reduce(h.g_part.p, nb, k - k0, h.g_h.p + k + k0, s);
-        launch_mgemv_sub(C + (int64_t)k0 * N, N, k - k0, h.g_h.p + k + k0, w, N, s);
-        launch_mdot(w, N, 1, w, N, h.g_part.p, nb, s);
-        launch_mdot_reduce(h.g_part.p, nb, 1, h.g_h.p + 2 * k, s);
-        H2W_HIP(hipMemcpyAsync(hh, h.g_h.p, (2 * k + 1) * 8, hipMemcpyDeviceToHost, s));
-        H2W_HIP(hipStreamSynchronize(s));
+        A.V = C;
+        A.w = w;
+        A.src32 = f32 ? h.vec32.p + h.off_y : nullptr;
+        A.nd = k;
+        A.out = h.g_h.p;
+        launch_cgs(A, s);  // h = V^T w
+        CgsArgs B = A;
+        B.src32 = nullptr;
+        B.ns = k;
+        B.sub = h.g_h.p;
+        B.d0 = k0;
+        B.nd = k - k0;
+        B.out = h.g_h.p + k + k0;
+        if (f32) B.w = w;
+        launch_cgs(B, s);  // w -= V h, second dots
+        B.s0 = k0;
+        B.ns = k - k0;
+        B.sub = h.g_h.p + k + k0;
+        B.norm = 1;
+        B.out = h.g_h.p + 2 * k;
+        B.all_h = h.g_h.p;
+        B.nhost = 2 * k;
+        B.host = hh;
+        launch_cgs_host(h, B);  // w -= V h, norm; all of it to the host
+        const double guess = res2 > res1 ? res1 * (res1 / res2) : res1;
+        ahead = i + 1 < m && !(guess < tol);
+        if (ahead) {
+            begin_product(h, w, 1.0, h.g_h.p + 2 * k, V + (int64_t)(i + 1) * N, prec);
+            run_launches(h, prec);
+        }
+        wait_cgs_host(h);
+        for (int q = 0; q < k0; ++q) hh[k + q] = 0.0;
         if (kc > 0) {
             Bc.emplace_back(kc);
             for (int q = 0; q < kc; ++q) Bc.back()[q] = hh[q] + hh[k + q];
@@ -2445,16 +2537,21 @@ GmresOut gmres_core(Handle &h, const double *b, double *x, int max_iter, double 
         // (the reference's gap, 1D/codes/gmres.hpp:153-154, divides by it); the next basis
         // vector is left zero, the rotation below leaves s_{i+1} = 0 and the solve ends here
         const bool breakdown = !(Hh(i + 1, i) > 0.0);
-        if (breakdown) launch_fill(V + (int64_t)(i + 1) * N, N, 0.0, s);
-        else launch_axpby(1.0 / Hh(i + 1, i), w, 0.0, V + (int64_t)(i + 1) * N, N, s);
+        next = w;
+        scale = breakdown ? 0.0 : 1.0 / Hh(i + 1, i);
         for (int q = 0; q < i; ++q) app_rot(Hh(q, i), Hh(q + 1, i), cs[q], sn[q]);
         gen_rot(Hh(i, i), Hh(i + 1, i), cs[i], sn[i]);
         app_rot(Hh(i, i), Hh(i + 1, i), cs[i], sn[i]);
         app_rot(sv[i], sv[i + 1], cs[i], sn[i]);
         out.resid = std::fabs(sv[i + 1]) / normb;
         out.iters = i + 1;
+        res2 = res1;
+        res1 = out.resid;
         bool done = out.resid < tol || i == m - 1 || breakdown;
         if (done) {
+            // (the next basis vector, for a space kept from this solve)
+            if (keep_h && breakdown) launch_fill(V + (int64_t)(i + 1) * N, N, 0.0, s);
+            else if (keep_h && !ahead) launch_axpby(scale, w, 0.0, V + (int64_t)(i + 1) * N, N, s);
             std::vector<double> y(sv.begin(), sv.begin() + i + 1);
             for (int q = i; q >= 0; q--) {
                 y[q] /= Hh(q, q);

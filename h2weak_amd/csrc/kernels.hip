@@ -2089,14 +2089,20 @@ __global__ void k_permute_in(const double *x, int64_t ldx, T *xt, int64_t ldt, c
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < N; t += (int64_t)gridDim.x * blockDim.x)
         xt[r * ldt + t] = (T)x[r * ldx + perm[t]];
 }
-// What comes before the launches of a product, in one pass: the pool's input from x (tree order, or input
-// order through perm) and zeros in everything the product accumulates into.
+// What comes before the launches of a product, in one pass: the pool's input from scale x (tree order, or
+// input order through perm; scale / sqrt(*norm2) where a norm is given), a copy of it where the caller keeps
+// one, and zeros in everything the product accumulates into.  x may lie in py (an entry is read before it is zeroed, by the same thread).
 template <typename T>
-__global__ __launch_bounds__(256) void k_begin(const double *x, const int32_t *perm, T *px, int64_t N, T *py,
-                                               int64_t len) {
+__global__ __launch_bounds__(256) void k_begin(const double *x, double scale, const double *norm2, double *copy,
+                                               const int32_t *perm, T *px, int64_t N, T *py, int64_t len) {
+    if (norm2) scale /= sqrt(*norm2);
     const int64_t step = (int64_t)gridDim.x * 256;
     for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < max(N, len); i += step) {
-        if (i < N) px[i] = (T)x[perm ? perm[i] : i];
+        if (i < N) {
+            const double v = scale * x[perm ? perm[i] : i];
+            if (copy) copy[i] = v;
+            px[i] = (T)v;
+        }
         if (i < len) py[i] = T(0);
     }
 }
@@ -2144,35 +2150,7 @@ __global__ __launch_bounds__(256) void k_dense_rows(const int32_t *__restrict__ 
 }
 
 // ------------------------------------------------------------------ BLAS-1 for Arnoldi (FP64)
-constexpr int kDotThreads = 256;
-
-// partial[l * nblk + b] = sum over block b's rows of V_l . w
-__global__ __launch_bounds__(kDotThreads) void k_mdot(const double *__restrict__ V, int64_t ldv,
-                                                      const double *__restrict__ w, int64_t n,
-                                                      double *__restrict__ partial) {
-    const int b = blockIdx.x, l = blockIdx.y, nblk = gridDim.x;
-    const double *v = V + (int64_t)l * ldv;
-    double acc = 0.0;
-    for (int64_t i = (int64_t)b * kDotThreads + threadIdx.x; i < n; i += (int64_t)nblk * kDotThreads)
-        acc = fma(v[i], w[i], acc);
-    acc = wave_sum(acc);
-    __shared__ double sh[kDotThreads / 64];
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int q = 0; q < kDotThreads / 64; ++q) s += sh[q];
-        partial[(int64_t)l * nblk + b] = s;
-    }
-}
-__global__ void k_mdot_reduce(const double *__restrict__ partial, int nblk, double *__restrict__ out) {
-    const int l = blockIdx.x;
-    double acc = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += 64) acc += partial[(int64_t)l * nblk + b];
-    acc = wave_sum(acc);
-    if (threadIdx.x == 0) out[l] = acc;
-}
-// w -= V h  (sign = -1) or x += V c (sign = +1)
+// x += sign V c
 __global__ void k_mgemv(const double *__restrict__ V, int64_t ldv, int k, const double *__restrict__ h,
                         double *__restrict__ w, int64_t n, double sign) {
     __shared__ double hs[1024];
@@ -2189,6 +2167,143 @@ __global__ void k_mgemv(const double *__restrict__ V, int64_t ldv, int k, const 
         }
         if (i < n) w[i] += sign * acc;
     }
+}
+// One pass of the Arnoldi process over a vector w of n rows, 256 R rows per workgroup, rows in registers:
+//   w = src                      (the product's FP32 output, when src is given)
+//   w -= sum_l V_l sub[l]        for the ns columns from s0 on
+//   out[l] = V_l . w             for the nd columns from d0 on, or out[0] = w . w when norm is set
+// A Gram-Schmidt step (dots, subtraction with the second dots, second subtraction with the norm) is three
+// such launches; the workgroup that arrives last sums the others' dots, in workgroup order, and copies
+// nhost numbers from all_h, then out, to page-locked host memory, then seq to flag, which the host polls.
+// (Dots, their reduction and each subtraction as launches of their own, and a copy to the host, were eight
+// launches of 4 to 5 us and 30 us of idle GPU while the host waited, rotated and launched.)
+constexpr int kCgsCols = 128;  // columns whose coefficients, or sums, are in LDS at a time
+template <int R, typename S>
+__global__ __launch_bounds__(256) void k_cgs(const double *__restrict__ V, int64_t ldv, const S *src, double *w,
+                                             int64_t n, int s0, int ns, const double *__restrict__ sub, int d0, int nd,
+                                             int norm, double *partial, uint32_t *arrived, double *out, int last_sums,
+                                             const double *all_h, int nhost, double *host, uint64_t *flag,
+                                             uint64_t seq) {
+    __shared__ double hs[256];
+    __shared__ double wpart[4][kCgsCols];
+    __shared__ int last;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, tid = threadIdx.x;
+    const int64_t i0 = blockIdx.x * (int64_t)(256 * R) + tid;
+    double x[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int64_t i = i0 + 256 * r;
+        x[r] = i < n ? (src ? (double)src[i] : w[i]) : 0.0;
+    }
+    for (int l0 = 0; l0 < ns; l0 += kCgsCols) {
+        const int nl = min(ns - l0, kCgsCols);
+        __syncthreads();
+        for (int l = tid; l < nl; l += 256) hs[l] = sub[l0 + l];
+        __syncthreads();
+        const double *v = V + (int64_t)(s0 + l0) * ldv;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int64_t i = i0 + 256 * r;
+            if (i >= n) continue;
+            double a = 0.0;
+#pragma unroll 8
+            for (int l = 0; l < nl; ++l) a = fma(v[(int64_t)l * ldv + i], hs[l], a);
+            x[r] -= a;
+        }
+    }
+    if (src || ns > 0)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int64_t i = i0 + 256 * r;
+            if (i < n) w[i] = x[r];
+        }
+    const int nt = norm ? 1 : nd;
+    if (norm) {
+        double a = 0.0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) a = fma(x[r], x[r], a);
+        a = wave_sum(a);
+        if (lane == 0) wpart[wv][0] = a;
+        __syncthreads();
+        if (tid == 0)
+            st_agent(partial + blockIdx.x, (wpart[0][0] + wpart[1][0]) + (wpart[2][0] + wpart[3][0]));
+    }
+    for (int l0 = 0; l0 < nd && !norm; l0 += kCgsCols) {
+        const int nl = min(nd - l0, kCgsCols);
+        const double *v = V + (int64_t)(d0 + l0) * ldv;
+        for (int l = 0; l < nl; l += 8) {
+            typedef double D8 __attribute__((ext_vector_type(8)));
+            D8 p = (D8)0.0;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int64_t i = i0 + 256 * r;
+                const int64_t ii = i < n ? i : 0;  // (x is zero there)
+#pragma unroll
+                for (int u = 0; u < 8; ++u) p[u] = fma(v[(int64_t)min(l + u, nl - 1) * ldv + ii], x[r], p[u]);
+            }
+            int ui = 0;
+#pragma unroll
+            for (int k = 8, o = 1; k > 1; k >>= 1, o <<= 1) {
+                const bool hi = lane & o;
+#pragma unroll
+                for (int q = 0; q < k / 2; ++q) {
+                    const double snd = hi ? p[q] : p[q + k / 2];
+                    const double keep = hi ? p[q + k / 2] : p[q];
+                    p[q] = keep + (o == 1 ? fold_lane<1>(snd) : o == 2 ? fold_lane<2>(snd) : fold_lane<4>(snd));
+                }
+                ui += hi ? k / 2 : 0;
+            }
+            const double t = sum_halves(p[0] + fold_lane<8>(p[0]));
+            if (lane < 8 && l + ui < nl) wpart[wv][l + ui] = t;
+        }
+        __syncthreads();
+        for (int l = tid; l < nl; l += 256)
+            st_agent(partial + (int64_t)blockIdx.x * nd + l0 + l,
+                     (wpart[0][l] + wpart[1][l]) + (wpart[2][l] + wpart[3][l]));
+        __syncthreads();
+    }
+    if (!last_sums) return;
+    __builtin_amdgcn_s_waitcnt(0);  // (the partials are at the coherence point before the arrival is counted)
+    __syncthreads();
+    if (tid == 0) last = atomicAdd(arrived, 1u) == gridDim.x - 1;
+    __syncthreads();
+    if (!last) return;
+    if (tid == 0) *arrived = 0;
+    // K threads side by side on the columns, 256 / K shares of the workgroups each
+    int K = 1;
+    while (K < nt && K < 256) K <<= 1;
+    const int share = tid / K, nsh = 256 / K;
+    for (int l0 = 0; l0 < nt; l0 += K) {
+        const int l = l0 + tid % K;
+        double a = 0.0;
+        if (l < nt)
+#pragma unroll 8
+            for (int b = share; b < (int)gridDim.x; b += nsh) a += ld_agent(partial + (int64_t)b * nt + l);
+        __syncthreads();
+        hs[tid] = a;
+        __syncthreads();
+        if (tid < K && l < nt) {
+            double t = 0.0;
+            for (int q = 0; q < nsh; ++q) t += hs[q * K + tid];
+            out[l] = t;
+            if (host) __hip_atomic_store(host + nhost + l, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+    if (!host) return;
+    for (int q = tid; q < nhost; q += 256)
+        __hip_atomic_store(host + q, all_h[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (tid == 0) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// the sums of many workgroups' dots of many columns, one wave per column
+__global__ __launch_bounds__(64) void k_cgs_sums(const double *__restrict__ partial, int nblk, int nd,
+                                                 double *__restrict__ out) {
+    const int l = blockIdx.x;
+    double a = 0.0;
+    for (int b = threadIdx.x; b < nblk; b += 64) a += partial[(int64_t)b * nd + l];
+    a = wave_sum(a);
+    if (threadIdx.x == 0) out[l] = a;
 }
 __global__ void k_axpby(double a, const double *__restrict__ x, double b, double *__restrict__ y, int64_t n) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
@@ -2618,13 +2733,15 @@ void launch_fill(double *a, int64_t n, double v, hipStream_t s) {
 void launch_fill32(float *a, int64_t n, float v, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_fill<float>, dim3(grid_for(n)), dim3(256), 0, s, a, n, v);
 }
-void launch_begin64(const double *x, const int32_t *perm, double *px, int64_t N, double *py, int64_t len, hipStream_t s) {
-    hipLaunchKernelGGL(k_begin<double>, dim3(grid_for(std::max(N, len), 256, 2048)), dim3(256), 0, s, x, perm, px, N, py,
-                       len);
+void launch_begin64(const double *x, double scale, const double *norm2, double *copy, const int32_t *perm, double *px,
+                    int64_t N, double *py, int64_t len, hipStream_t s) {
+    hipLaunchKernelGGL(k_begin<double>, dim3(grid_for(std::max(N, len), 256, 2048)), dim3(256), 0, s, x, scale, norm2, copy,
+                       perm, px, N, py, len);
 }
-void launch_begin32(const double *x, const int32_t *perm, float *px, int64_t N, float *py, int64_t len, hipStream_t s) {
-    hipLaunchKernelGGL(k_begin<float>, dim3(grid_for(std::max(N, len), 256, 2048)), dim3(256), 0, s, x, perm, px, N, py,
-                       len);
+void launch_begin32(const double *x, double scale, const double *norm2, double *copy, const int32_t *perm, float *px,
+                    int64_t N, float *py, int64_t len, hipStream_t s) {
+    hipLaunchKernelGGL(k_begin<float>, dim3(grid_for(std::max(N, len), 256, 2048)), dim3(256), 0, s, x, scale, norm2, copy,
+                       perm, px, N, py, len);
 }
 void launch_permute_in(const double *x, int64_t ldx, double *xt, int64_t ldt, const int32_t *perm, int64_t N,
                        int nrhs, hipStream_t s) {
@@ -2647,21 +2764,29 @@ void launch_dense_rows(const int32_t *rows, int64_t nrows, const double *xt, dou
         hipLaunchKernelGGL(k_dense_rows, dim3((unsigned)((nrows + 63) / 64)), dim3(256), 0, s, rows, nrows, xt, y, N,
                            kp);
 }
-int mdot_blocks(int64_t n) {
-    int64_t b = (n + kDotThreads * 8 - 1) / (kDotThreads * 8);
-    if (b < 1) b = 1;
-    if (b > 512) b = 512;
-    return (int)b;
-}
-void launch_mdot(const double *V, int64_t ldv, int k, const double *w, int64_t n, double *partial, int nblk,
-                 hipStream_t s) {
-    if (k > 0) hipLaunchKernelGGL(k_mdot, dim3(nblk, k), dim3(kDotThreads), 0, s, V, ldv, w, n, partial);
-}
-void launch_mdot_reduce(const double *partial, int nblk, int k, double *out, hipStream_t s) {
-    if (k > 0) hipLaunchKernelGGL(k_mdot_reduce, dim3(k), dim3(64), 0, s, partial, nblk, out);
-}
-void launch_mgemv_sub(const double *V, int64_t ldv, int k, const double *h, double *w, int64_t n, hipStream_t s) {
-    if (k > 0) hipLaunchKernelGGL(k_mgemv, dim3(grid_for(n, 256, 4096)), dim3(256), 0, s, V, ldv, k, h, w, n, -1.0);
+// rows per thread: up to 256 workgroups, whose dots one workgroup still sums in a few microseconds
+static int cgs_rows(int64_t n) { return n <= 131072 ? 2 : n <= 262144 ? 4 : 8; }
+int cgs_blocks(int64_t n) { return (int)((n + 256 * cgs_rows(n) - 1) / (256 * cgs_rows(n))); }
+void launch_cgs(const CgsArgs &a, hipStream_t s) {
+    const int nb = cgs_blocks(a.n), nt = a.norm ? 1 : a.nd;
+    if (nt <= 0) return;
+    // the last workgroup's share: nb nt numbers from one compute unit, 2 us up to about 16384 of them
+    const int last = a.norm || a.host || (int64_t)nb * nt <= 16384;
+    auto go = [&](auto R, const auto *src) {
+        hipLaunchKernelGGL((k_cgs<decltype(R)::value, std::decay_t<decltype(*src)>>), dim3(nb), dim3(256), 0, s, a.V,
+                           a.ldv, src, a.w, a.n, a.s0, a.ns, a.sub, a.d0, a.nd, a.norm, a.partial, a.arrived, a.out,
+                           last, a.all_h, a.nhost, a.host, a.flag, a.seq);
+    };
+    auto rows = [&](const auto *src) {
+        switch (cgs_rows(a.n)) {
+        case 2: go(std::integral_constant<int, 2>{}, src); break;
+        case 4: go(std::integral_constant<int, 4>{}, src); break;
+        default: go(std::integral_constant<int, 8>{}, src);
+        }
+    };
+    if (a.src32) rows(a.src32);
+    else rows((const double *)nullptr);
+    if (!last) hipLaunchKernelGGL(k_cgs_sums, dim3(nt), dim3(64), 0, s, a.partial, nb, nt, a.out);
 }
 void launch_vec_update(const double *V, int64_t ldv, int k, const double *c, double *x, int64_t n, hipStream_t s) {
     if (k > 0) hipLaunchKernelGGL(k_mgemv, dim3(grid_for(n, 256, 4096)), dim3(256), 0, s, V, ldv, k, c, x, n, 1.0);
