@@ -14,6 +14,7 @@
 #include <algorithm>
 
 #include "h2w_internal.hpp"
+#include "h2w_device.hpp"
 
 namespace h2w {
 
@@ -462,84 +463,160 @@ __global__ void k_cur_c(const CurJob *__restrict__ jobs, const int32_t *__restri
 // ------------------------------------------------------------------ complex batched GEMV
 // The real path's work lists over complex pools: item rows y (+)= sum_t A_t x_t; symmetric
 // terms (t >= 0) also add A_t^T x_item to vec[t ..] (plain transpose, atomics per real part).
-// One workgroup per item; lane = row (rows > 64: two passes), 16-byte loads of whole complex
-// entries.  Wave wv takes groups of kCU consecutive columns (wv, wv + 4, ...), all kCU columns'
-// loads issued before they are used.  The transposed sums of a group are reduced together: a
-// butterfly halves the kCU values per exchange (lane bit o keeps one half, sends the other), so
-// log2(64) exchanges serve kCU columns and lanes 0 .. kCU-1 end with one column sum each.  Role 2
-// items and atomic items (flags bit 0 or 2) add their rows atomically.
-__device__ __forceinline__ void catomic_add(double2 *p, double2 v) {
-    double *d = reinterpret_cast<double *>(p);
-    atomicAdd(d, v.x);
-    atomicAdd(d + 1, v.y);
-}
-__device__ __forceinline__ double2 cshfl_xor(double2 v, int o) {
-    return cmk(__shfl_xor(v.x, o, 64), __shfl_xor(v.y, o, 64));
-}
-constexpr int kCU = 8;  // columns in flight per wave
-__global__ __launch_bounds__(256) void k_cgemv(const GItem *__restrict__ items, const GTerm *__restrict__ terms,
-                                               const double2 *__restrict__ A, double2 *__restrict__ vec) {
-    const GItem it = items[blockIdx.x];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    __shared__ double2 part[4][kRowTile];
-    __shared__ double2 xb[kRowTile];
+// A column is covered by lpc lanes, the power of two at or above half the item's rows; a lane holds
+// rows r and lpc + r of kCU consecutive columns, so that every load instruction reads whole runs of
+// 16-byte entries and one read of x serves two of them.  As in the real kernel (k_bgemv) a wave-uniform
+// cursor walks (term, columns) iterations, two in flight, every load unconditional (lanes out of range
+// address past the buffer's end, which is set per iteration: a dense block may pass 4 GiB).
+// The transposed sums of a group are 2 kCU real numbers per lane: a butterfly halves them per exchange
+// (lane bit o keeps one half, sends the other), after which lane l < 2 kCU of every column group finishes
+// one number.  WPI waves share an item: 4, whose sums meet in LDS, or 1, four items per workgroup.  Role
+// 2 items and atomic items (flags bit 0 or 2) add their rows atomically.
+// Bound by the read of A.  Measured against a lane per row with the loads under branches and one iteration
+// in flight (the same lists): 3D Helmholtz 32^3 at 1e-8, 2.4 GB, 674 -> 488 us (4.9 TB/s); 3D semi-nested
+// N = 20000 670 (uncut lists) -> 259 us; 2D Hankel 300 x 300 371 -> 294 us.  Two columns per lane instead of
+// four: 508 us on the first, 77 against 72 us on 16^3.
+typedef double D2 __attribute__((ext_vector_type(2)));
+constexpr int kCU = 4;  // columns per lane and iteration
+// role 1 (fused) has transposed products; the others only name the launch in profiles
+template <int ROLE, int WPI>
+__global__ __launch_bounds__(256) void k_cgemv(const GItem *__restrict__ items, int nitems,
+                                               const GTerm *__restrict__ terms, const double2 *__restrict__ A,
+                                               double2 *vec) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int item = WPI == 4 ? blockIdx.x : 4 * blockIdx.x + wave;
+    if (WPI == 1 && item >= nitems) return;
+    const int wv = WPI == 4 ? wave : 0;
+    const GItem it = items[item];
+    const CGTerm *const tms = (const CGTerm *)terms;
     const int rows = it.rows;
-    // (zero beyond the item's rows: the transposed sums then need no row test)
-    for (int r = threadIdx.x; r < kRowTile; r += 256) xb[r] = r < rows ? vec[it.xb + r] : cmk(0.0, 0.0);
-    __syncthreads();
-    const bool two = rows > 64;
-    const bool in0 = lane < rows, in1 = two && 64 + lane < rows;
-    const double2 xb0 = xb[lane], xb1 = xb[64 + lane];
-    double2 acc0 = cmk(0.0, 0.0), acc1 = cmk(0.0, 0.0);
-    for (int tt = it.t0; tt < it.t1; ++tt) {
-        const GTerm tm = terms[tt];
-        const double2 *Ab = A + tm.a + it.row0;
-        for (int c0 = kCU * wv; c0 < tm.cols; c0 += 4 * kCU) {
-            double2 v0[kCU], v1[kCU], xv[kCU];
-#pragma unroll
-            for (int u = 0; u < kCU; ++u) {
-                const int c = c0 + u;
-                const bool ok = c < tm.cols;
-                xv[u] = ok ? vec[tm.x + c] : cmk(0.0, 0.0);
-                const double2 *col = Ab + (int64_t)(ok ? c : c0) * it.lda;
-                v0[u] = ok && in0 ? col[lane] : cmk(0.0, 0.0);
-                v1[u] = ok && in1 ? col[64 + lane] : cmk(0.0, 0.0);
-            }
-#pragma unroll
-            for (int u = 0; u < kCU; ++u) {
-                acc0 = cadd(acc0, cmul(v0[u], xv[u]));
-                if (two) acc1 = cadd(acc1, cmul(v1[u], xv[u]));
-            }
-            if (tm.t >= 0) {
-                double2 d[kCU];
-#pragma unroll
-                for (int u = 0; u < kCU; ++u) d[u] = cadd(cmul(v0[u], xb0), cmul(v1[u], xb1));
-                int ui = 0;
-#pragma unroll
-                for (int k = kCU, o = 1; k > 1; k >>= 1, o <<= 1) {
-                    const bool hi = lane & o;
-#pragma unroll
-                    for (int i = 0; i < k / 2; ++i) {
-                        const double2 snd = hi ? d[i] : d[i + k / 2];
-                        const double2 keep = hi ? d[i + k / 2] : d[i];
-                        d[i] = cadd(keep, cshfl_xor(snd, o));
-                    }
-                    ui += hi ? k / 2 : 0;
-                }
-#pragma unroll
-                for (int o = kCU; o < 64; o <<= 1) d[0] = cadd(d[0], cshfl_xor(d[0], o));
-                if (lane < kCU && c0 + ui < tm.cols) catomic_add(vec + tm.t + c0 + ui, d[0]);
-            }
-        }
+    __shared__ double2 part[WPI == 4 ? 4 : 1][kRowTile];
+    int lpc = ROLE == 1 ? 2 * kCU : 1;  // (distinct lanes for the transposed sums)
+    // (an iteration's columns stay within a buffer's 32-bit offsets, however tall the block)
+    while (2 * lpc < rows || (lpc < 64 && (64 / lpc) * kCU * it.lda * (int64_t)sizeof(D2) > INT_MAX)) lpc <<= 1;
+    const int cpw = 64 / lpc;
+    const int q = lane / lpc, r0 = lane % lpc, r1 = lpc + r0;
+    const bool in0 = r0 < rows, in1 = r1 < rows;
+    D2 acc0 = (D2)0.0, acc1 = (D2)0.0, xb0 = (D2)0.0, xb1 = (D2)0.0;
+    if (ROLE == 1) {
+        const __amdgpu_buffer_rsrc_t rb = buf_rsrc(vec + it.xb, (uint32_t)(rows * sizeof(D2)));
+        xb0 = buf_ld16<D2>(rb, in0 ? (uint32_t)(r0 * sizeof(D2)) : kOutOfRange);
+        xb1 = buf_ld16<D2>(rb, in1 ? (uint32_t)(r1 * sizeof(D2)) : kOutOfRange);
     }
-    part[wv][lane] = acc0;
-    part[wv][64 + lane] = acc1;
-    __syncthreads();
-    for (int r = threadIdx.x; r < rows; r += 256) {
-        const double2 sum = cadd(cadd(part[0][r], part[1][r]), cadd(part[2][r], part[3][r]));
+    const int64_t lda = it.lda;
+    const int chunk = cpw * kCU;
+    const uint32_t roff0 = (uint32_t)((it.row0 + r0) * sizeof(D2)), roff1 = (uint32_t)((it.row0 + r1) * sizeof(D2));
+    struct Iter {
+        D2 a0[kCU], a1[kCU], x[kCU];
+        int left;   // columns from this lane's first one to the term's end
+        int64_t t;  // transposed outputs of the lane's first column, -1: none
+    };
+    int tt = it.t0, c0 = wv * chunk;
+    auto settle = [&]() {
+        while (tt < it.t1 && c0 >= tms[tt].cols) {
+            ++tt;
+            c0 = wv * chunk;
+        }
+    };
+    auto load = [&](Iter &B) -> bool {
+        const bool has = tt < it.t1;
+        const GTerm tm = term_at(tms, has ? tt : it.t1 - 1);
+        const int b = has ? c0 : 0, n = has ? min(chunk, tm.cols - c0) : 0;
+        B.left = n - q * kCU;
+        B.t = has && tm.t >= 0 ? tm.t + b + q * kCU : -1;
+        const __amdgpu_buffer_rsrc_t ra = buf_rsrc(A + tm.a + b * lda, (uint32_t)(n * lda * sizeof(D2)));
+        const __amdgpu_buffer_rsrc_t rx = buf_rsrc(vec + tm.x + b, (uint32_t)(n * sizeof(D2)));
+#pragma unroll
+        for (int u = 0; u < kCU; ++u) {
+            const uint32_t o = (uint32_t)((q * kCU + u) * lda * sizeof(D2));
+            const bool ok = u < B.left;
+            B.a0[u] = buf_ld16_nt<D2>(ra, ok && in0 ? o + roff0 : kOutOfRange);
+            B.a1[u] = buf_ld16_nt<D2>(ra, ok && in1 ? o + roff1 : kOutOfRange);
+        }
+#pragma unroll
+        for (int u = 0; u < kCU; ++u)  // (past the resource's end: zeros)
+            B.x[u] = buf_ld16<D2>(rx, (uint32_t)((q * kCU + u) * sizeof(D2)));
+        if (has) {
+            c0 += WPI * chunk;
+            settle();
+        }
+        return has;
+    };
+    auto cfma = [](D2 a, D2 b, D2 c) {
+        c.x = fma(a.x, b.x, fma(-a.y, b.y, c.x));
+        c.y = fma(a.x, b.y, fma(a.y, b.x, c.y));
+        return c;
+    };
+    auto compute = [&](const Iter &B) {
+#pragma unroll
+        for (int u = 0; u < kCU; ++u) {
+            acc0 = cfma(B.a0[u], B.x[u], acc0);
+            acc1 = cfma(B.a1[u], B.x[u], acc1);
+        }
+        if (ROLE == 1) {
+            typedef double DU __attribute__((ext_vector_type(2 * kCU)));
+            DU d;
+#pragma unroll
+            for (int u = 0; u < kCU; ++u) {
+                const D2 s = cfma(B.a1[u], xb1, cfma(B.a0[u], xb0, (D2)0.0));
+                d[2 * u] = s.x;
+                d[2 * u + 1] = s.y;
+            }
+            int ui = 0;
+#pragma unroll
+            for (int k = 2 * kCU, o = 1; k > 1; k >>= 1, o <<= 1) {
+                const bool hi = lane & o;
+#pragma unroll
+                for (int i = 0; i < k / 2; ++i) {
+                    const double snd = hi ? d[i] : d[i + k / 2];
+                    const double keep = hi ? d[i + k / 2] : d[i];
+                    d[i] = keep + xor_lane_n(snd, o);
+                }
+                ui += hi ? k / 2 : 0;
+            }
+#pragma unroll
+            for (int o = 2 * kCU; o < 64; o <<= 1)
+                if (o < lpc) d[0] += xor_lane_n(d[0], o);
+            if (r0 < 2 * kCU && ui < 2 * B.left && B.t >= 0)
+                atomicAdd(reinterpret_cast<double *>(vec + B.t) + ui, d[0]);
+        }
+    };
+    // (an iteration loaded past the last one reads nothing and adds nothing)
+    Iter B0, B1;
+    settle();
+    bool h0 = load(B0);
+    load(B1);
+    while (h0) {
+        compute(B0);
+        h0 = load(B0);
+        compute(B1);
+        load(B1);
+    }
+    for (int o = lpc; o < 64; o <<= 1) {
+        acc0.x += __shfl_xor(acc0.x, o, 64);
+        acc0.y += __shfl_xor(acc0.y, o, 64);
+        acc1.x += __shfl_xor(acc1.x, o, 64);
+        acc1.y += __shfl_xor(acc1.y, o, 64);
+    }
+    auto add = [&](int r, double2 v) {
         double2 *y = vec + it.y + r;
-        if (it.flags & 5) catomic_add(y, sum);
-        else *y = cadd(*y, sum);
+        if (it.flags & 5) {
+            atomicAdd(&y->x, v.x);
+            atomicAdd(&y->y, v.y);
+        } else *y = cadd(*y, v);
+    };
+    if (WPI == 1) {
+        if (q == 0 && in0) add(r0, cmk(acc0.x, acc0.y));
+        if (q == 0 && in1) add(r1, cmk(acc1.x, acc1.y));
+        return;
+    }
+    if (q == 0 && in0) part[wave][r0] = cmk(acc0.x, acc0.y);
+    if (q == 0 && in1) part[wave][r1] = cmk(acc1.x, acc1.y);
+    __syncthreads();
+    if (threadIdx.x < rows) {
+        const int r = threadIdx.x;
+        add(r, cadd(cadd(part[0][r], part[1][r]), cadd(part[2][r], part[3][r])));
     }
 }
 
@@ -690,8 +767,20 @@ void launch_cur_c(const CurJob *jobs, int njobs, const int32_t *idx, const doubl
                   hipStream_t s) {
     if (njobs > 0) hipLaunchKernelGGL(k_cur_c, dim3(njobs), dim3(64), 0, s, jobs, idx, lr, A, kp);
 }
-void launch_cgemv(const GItem *items, int nitems, const GTerm *terms, const double2 *A, double2 *vec, hipStream_t s) {
-    if (nitems > 0) hipLaunchKernelGGL(k_cgemv, dim3(nitems), dim3(256), 0, s, items, terms, A, vec);
+void launch_cgemv(const GItem *items, int nitems, const GTerm *terms, const double2 *A, double2 *vec, int role,
+                  bool per_wave, hipStream_t s) {
+    if (nitems <= 0) return;
+    auto go = [&](auto R) {
+        if (per_wave)
+            hipLaunchKernelGGL((k_cgemv<decltype(R)::value, 1>), dim3((nitems + 3) / 4), dim3(256), 0, s, items, nitems,
+                               terms, A, vec);
+        else
+            hipLaunchKernelGGL((k_cgemv<decltype(R)::value, 4>), dim3(nitems), dim3(256), 0, s, items, nitems, terms, A,
+                               vec);
+    };
+    if (role == 1) go(std::integral_constant<int, 1>{});
+    else if (role == 2) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, 0>{});
 }
 void launch_cbegin(const double2 *x, const int32_t *perm, double2 *px, int64_t N, double2 *py, int64_t len,
                    hipStream_t s) {

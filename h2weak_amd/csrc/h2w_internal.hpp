@@ -355,7 +355,8 @@ void launch_xfer_c(const XferJob *jobs, int njobs, const int32_t *idx, const dou
                    hipStream_t s);
 void launch_cur_c(const CurJob *jobs, int njobs, const int32_t *idx, const double2 *lr, double2 *A, KParamsC kp,
                   hipStream_t s);
-void launch_cgemv(const GItem *items, int nitems, const GTerm *terms, const double2 *A, double2 *vec, hipStream_t s);
+void launch_cgemv(const GItem *items, int nitems, const GTerm *terms, const double2 *A, double2 *vec, int role,
+                  bool per_wave, hipStream_t s);
 void launch_cfill(double2 *a, int64_t n, hipStream_t s);
 void launch_cpermute_in(const double2 *x, double2 *xt, const int32_t *perm, int64_t N, hipStream_t s);
 void launch_cpermute_out(const double2 *yt, double2 *y, const int32_t *perm, int64_t N, hipStream_t s);

@@ -2164,7 +2164,7 @@ void run_launch(Handle &h, const Launch &Lh, int precision) {
     hipStream_t s = h.stream;
     if (h.cplx) {  // complex operators: FP64 only, every role through the complex GEMV
         launch_cgemv(h.d_items.p + Lh.item0, (int)Lh.nitems, h.d_terms.p, reinterpret_cast<const double2 *>(h.mat64.p),
-                     reinterpret_cast<double2 *>(h.vec64.p), s);
+                     reinterpret_cast<double2 *>(h.vec64.p), Lh.role, per_wave_gemv(Lh), s);
         return;
     }
     const bool otf = (precision == H2W_FP32_OTF || precision == H2W_FP64_OTF) && Lh.role == 1;
