@@ -120,7 +120,11 @@ void merge_lists(Batch &B, int which) {
                 items.push_back(it);
             }
         }
-        Lm.nitems = (int64_t)items.size() - Lm.item0;
+        if (Lm.role == 1 && B.sym16) {
+            const int64_t end = (int64_t)items.size();
+            if (wide_items(items, Lm.item0, terms) > 0) items.erase(items.begin() + Lm.item0, items.begin() + end);
+        }
+        Lm.nitems = Lm.nitemsm = (int64_t)items.size() - Lm.item0;
         Lm.nterms = (int64_t)terms.size() - Lm.term0;
         int64_t sc = 0;
         for (int64_t t = Lm.term0; t < (int64_t)terms.size(); ++t) sc += terms[t].cols;

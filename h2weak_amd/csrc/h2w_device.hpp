@@ -8,6 +8,11 @@
 #include "h2w_internal.hpp"
 
 namespace h2w {
+// the buffer atomics' intrinsics (they have no clang builtin)
+__device__ double buf_fadd64(double v, __amdgpu_buffer_rsrc_t r, int voff, int soff, int aux) __asm(
+    "llvm.amdgcn.raw.ptr.buffer.atomic.fadd.f64");
+__device__ float buf_fadd32(float v, __amdgpu_buffer_rsrc_t r, int voff, int soff, int aux) __asm(
+    "llvm.amdgcn.raw.ptr.buffer.atomic.fadd.f32");
 namespace {
 
 // Value of lane (lane ^ O) for a power of two O < 64: quad permutes (DPP) for 1 and 2,
@@ -98,6 +103,13 @@ __device__ __forceinline__ V buf_ld16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
 template <typename V>
 __device__ __forceinline__ V buf_ld16_nt(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 2));
+}
+// Atomic addition without a result; lanes out of range add nothing.
+__device__ __forceinline__ void buf_atomic_add(__amdgpu_buffer_rsrc_t r, uint32_t off, double v) {
+    (void)buf_fadd64(v, r, (int)off, 0, 0);
+}
+__device__ __forceinline__ void buf_atomic_add(__amdgpu_buffer_rsrc_t r, uint32_t off, float v) {
+    (void)buf_fadd32(v, r, (int)off, 0, 0);
 }
 // one 4-, 8- or 16-byte vector, streamed (not kept in the caches)
 template <typename V>

@@ -151,6 +151,7 @@ struct Pair {                                  // semi-nested vertex pair (B <- 
 // at the leaves.
 struct Launch {
     int64_t item0, nitems, term0, nterms;
+    int64_t item0m = 0, nitemsm = 0;  // the 16-wide path's items (wide_items)
     int role;      // 0 transfer pass, 1 M2L + near field, 2 semi-nested column factors,
                    // 3 transposed products of the symmetric blocks (16-wide lists)
     int stage = 0, step = 0;
@@ -158,12 +159,13 @@ struct Launch {
     int unr32 = 4; // the same for the stored FP32 copy
     int avg_cols = 0;  // mean inner size of the terms (picks the transposed 16-wide kernel's slabs)
     int64_t avg_item_elems = 0;  // mean operator elements per item
+    void set_wide(std::vector<GItem> &items, const std::vector<GTerm> &terms);
 };
 // one item per wave on the 16-wide path: launches of enough items that are small on average
 // (the transfer passes at the leaves of small systems), where a workgroup's set-up and the
 // reduction across its waves would outweigh the item
 inline bool per_wave_items(const Launch &L) {
-    return L.nitems >= 2048 && L.avg_item_elems > 0 && L.avg_item_elems <= 4096;
+    return L.nitemsm >= 2048 && L.avg_item_elems > 0 && L.avg_item_elems <= 4096;
 }
 // The same on the single-vector path.  Measured, four waves / one wave per item: 1D N = 250000 leaf up
 // pass (4096 items of 1500 elements on average) 21 / 16 us and fused launch (8000 of 2200) 50 / 40 us, 2D
@@ -173,6 +175,7 @@ inline bool per_wave_items(const Launch &L) {
 inline bool per_wave_gemv(const Launch &L) {
     return L.nitems >= 2048 && L.avg_item_elems > 0 && L.avg_item_elems <= 8192;
 }
+int64_t wide_items(std::vector<GItem> &items, int64_t item0, const std::vector<GTerm> &terms);
 // narrow slabs for the transposed 16-wide products when the blocks have few rows
 inline int trans_narrow(const Launch &L, bool fp32) { return L.avg_cols <= (fp32 ? 32 : 16); }
 

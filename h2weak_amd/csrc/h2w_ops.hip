@@ -998,8 +998,8 @@ void merge_terms(WorkList &W) {
 // blocks and accumulate atomically anyway.
 // Measured (fused launch, FP64, unsplit / 2048 / 4096 / 8192 / 16384 items): 3D N = 20011 279 / 166 / 139 /
 // 137 / 141 us, 32^3 grid at 1e-10 472 / 363 / 343 / 323 / 313 us, 2D N = 90000 191 / 195 / 176 / 174 /
-// 178 us; complex 32^3 product 879 / 884 / 736 / 726 / 653 us.  The 16-wide launch stages its item's input
-// rows and likes larger pieces: 328 / 250 / 265 / 275 / 327 us and 565 / 486 / 486 / 514 / 598 us.  The
+// 178 us; complex 32^3 product 879 / 884 / 736 / 726 / 653 us.  The 16-wide launch likes larger
+// pieces (wide_items).  The
 // leaf launch of the 2D semi-nested 400 x 400 grid (more than 2048 items, some of 4 MB) 214 -> 137 us.
 constexpr int64_t kMinItems = 2048, kMinPiece = 128 * 64;
 constexpr int64_t kMinItemsFused = 8192, kMinPieceFused = 128 * 128;
@@ -1121,6 +1121,52 @@ int inner_rank(const std::vector<double> &hist, int rank, double tau) {
     return rank;
 }
 
+}  // namespace
+
+// The 16-wide path's items of a fused launch, appended to items, whose entries from item0 on are the
+// single-vector path's: consecutive pieces of one row tile (their terms follow one another) are put together again,
+// up to a 2048th of the launch's elements.  A workgroup of the 16-wide kernel reads 16 input rows per item row,
+// and sums and adds as many at the end: about 5 us an item beside its data.
+// Measured (fused launch, FP64, uncombined pieces / 4096 / 2048 / 1024): 32^3 grid at 1e-10 492 / 452 / 448 / 458
+// us, 3D N = 20011 231 / 229 / 204 / 202 us, 2D N = 90000 317 / 297 / 292 / 304 us.  (The transfers' pieces stay:
+// 2D semi-nested 400 x 400 207 us of them, 2048 / 1024 / 512: 207 / 215 / 248 us.)
+// Returns the number of items appended; 0 where nothing combines.
+int64_t wide_items(std::vector<GItem> &items, int64_t item0, const std::vector<GTerm> &terms) {
+    const int64_t end = (int64_t)items.size();
+    auto work = [&](const GItem &it) {
+        int64_t w = 0;
+        for (int32_t k = it.t0; k < it.t1; ++k) w += (int64_t)it.rows * terms[k].cols;
+        return w;
+    };
+    int64_t E = 0, sum = 0;
+    for (int64_t q = item0; q < end; ++q) E += work(items[q]);
+    const int64_t most = E / 2048 + E / 8192;
+    for (int64_t q = item0; q < end; ++q) {
+        const GItem it = items[q];
+        const int64_t w = work(it);
+        GItem &l = items.back();
+        if (q > item0 && l.y == it.y && l.xb == it.xb && l.rows == it.rows && l.lda == it.lda && l.row0 == it.row0 &&
+            l.flags == it.flags && l.t1 == it.t0 && sum + w <= most) {
+            l.t1 = it.t1;
+            sum += w;
+        } else {
+            items.push_back(it);
+            sum = w;
+        }
+    }
+    const int64_t n = (int64_t)items.size() - end;
+    if (n < end - item0) return n;
+    items.resize(end);
+    return 0;
+}
+void Launch::set_wide(std::vector<GItem> &items, const std::vector<GTerm> &terms) {
+    const int64_t n = (int64_t)items.size();
+    nitemsm = role == 1 ? wide_items(items, item0, terms) : 0;
+    item0m = nitemsm ? n : item0;
+    if (!nitemsm) nitemsm = nitems;
+}
+
+namespace {
 void upload_lists(std::vector<WorkList> &WL, LaunchSet &LS, hipStream_t s) {
     std::vector<GItem> items;
     std::vector<GTerm> terms;
@@ -1147,6 +1193,7 @@ void upload_lists(std::vector<WorkList> &WL, LaunchSet &LS, hipStream_t s) {
         }
         terms.insert(terms.end(), W.terms.begin(), W.terms.end());
         Lh.avg_item_elems = e / Lh.nitems;
+        Lh.set_wide(items, terms);
         LS.launches.push_back(Lh);
         LS.elems.push_back(e);
     }
@@ -2119,6 +2166,7 @@ void assemble_operators(Handle &h, double t0) {
             items.push_back(it);
         }
         terms.insert(terms.end(), W.terms.begin(), W.terms.end());
+        Lh.set_wide(items, terms);
         h.launches.push_back(Lh);
     }
     h.d_items.upload(items, s);

@@ -1254,250 +1254,221 @@ __global__ __launch_bounds__(256) void k_bgemm(const GItem *__restrict__ items, 
 }
 
 // Direct and transposed products of the stored blocks in one read, kNR right-hand sides
-// (the fused M2L + near-field launch of the multi-vector pass).  One item (box b, rows <= 128)
-// per workgroup.  The item's terms K(b, p) are cut into 16-column groups (never across a term);
-// wave wv takes groups wv, wv + 4, ... and walks each group's row groups of RG = 16 VEC rows as
-// slabs, the next slab in flight while one is multiplied.  A slab is loaded in the direct
-// product's layout (lane (m, q): VEC consecutive rows of column 4 j + q, j < 4: 16-byte loads,
-// 256-byte runs per column) and multiplied at once into the item's rows (as k_bgemm: A(m, q) =
-// K(VEC m + e, 4 j + q),
-// B(q, m) = X_p(4 j + q, m)).  For a symmetric term (t >= 0) the wave also writes the slab to one
-// of its two LDS buffers; one slab later it reads it back with a column per lane % 16 and a row
-// per lane / 16, the A operand of K^T: with B(q, m) = X_b(4 s + q, m) from the item's input rows
-// (staged in LDS once) it accumulates the 16 x kNR block Y_p(c0 .. c0 + 15, :) += K(rows, c0 ..)^T
-// X_b over the row groups, and adds it to the partner's output with atomics when the group ends.
-// (Reading a slab one step after writing it overlaps the LDS round trip with the next slab's
-// direct products.)  The item's own rows are added atomically too (other items' transposes land
-// in them).  Each stored element is read once per pass, where k_bgemm + k_bgemm_tl read it twice.
+// (the fused M2L + near-field launch of the multi-vector pass).  One item (box b, rows <= 128) per
+// workgroup, its rows in passes of up to RG NG (RG = 16 VEC).  The item's terms K(b, p) are cut into
+// 16-column groups (never across a term); wave wv takes groups wv, wv + 4, ...  A group is NG slabs of
+// RG rows x 16 columns, loaded in the direct product's layout (lane (m, q): VEC consecutive rows of column
+// 4 j + q, j < 4: 16-byte loads, 256-byte runs per column; the next group in flight) and multiplied into
+// the pass's rows (as k_bgemm: A(m, q) = K(VEC m + e, 4 j + q), B(q, m) = X_p(4 j + q, m)).  For a
+// symmetric term (t >= 0) the wave also writes the slabs to its LDS buffers and reads them back with a
+// column per lane % 16 and a row per lane / 16, the A operand of K^T: with B(q, m) = X_b(4 s + q, m), held in
+// registers, it forms the 16 x kNR block Y_p(c0 .. c0 + 15, :) += K(rows, c0 ..)^T X_b and adds it to the
+// partner's output with atomics.  MFMAs over columns past the term or rows past the pass are left out, four at
+// a time.  The item's own rows are added atomically too (other items' transposes land in them).  Each
+// stored element is read once per pass, where k_bgemm + k_bgemm_tl read it twice.
+// The terms of an item (64 of them at a time) sit one per lane, and a group's term is found by a ballot over
+// the running group counts: a cursor over descriptors in memory waited on two or three dependent scalar
+// loads a group, and those waits cover the LDS counter too.
 // FP64: 64 MFMA flops per stored element (direct and transposed, 16 right-hand sides) against
 // 8 bytes, so the launch needs both HBM and the FP64 matrix cores (78.6 TFLOP/s) at once;
 // launch bounds cap it at 256 registers a lane (two waves per SIMD).
-template <typename T, int VEC>
-__device__ __forceinline__ void bgemm_sym_item(const GItem it, const GTerm *__restrict__ terms,
-                                               const T *__restrict__ A0, const T *__restrict__ A1,
-                                               const T *const *__restrict__ tab, T *vec, T *smem) {
+// Measured against slabs of 128-row items from a scalar cursor, with the atomics before the next loads (the same
+// lists), FP64 / FP32: 32^3 grid at 1e-10 (1.9 GB) 517 / 277 -> 492 / 255 us, 3D N = 20011 258 / 148 -> 231 /
+// 129, 2D N = 90000 328 / 195 -> 317 / 162; with the lists of wide_items 448 / 232, 204 / 113, 292 / 143.
+// Without loads from HBM it takes 440 us on the first, without the partner's atomics 350, with the direct
+// products only 155 (MFMA time 105 each way): the matrix pipe and the atomics share the bound.
+template <typename T, int VEC, int NG>
+__device__ __forceinline__ void bgemm_sym_rows(const GItem &it, int h0, int rows, const GTerm *__restrict__ terms,
+                                               const T *__restrict__ A, T *vec, T *smem) {
     typedef typename Mfma16<T>::v4 V4;
-    constexpr int RG = 16 * VEC;           // rows of a slab
-    constexpr int NG = kRowTile / RG;      // row groups of a full item
-    constexpr int NA = NG * VEC;           // direct accumulators
-    constexpr int NS = RG / 4;             // MFMA k-steps of a slab's transposed product
-    constexpr int kPipe = 2;               // slabs in the load rotation (3 measured no faster)
-    constexpr int LDR = RG + VEC;          // LDS column of a slab, padded by 16 bytes
-    constexpr int XS = kRowTile * kNR;     // staged input rows
-    constexpr int SLB = 16 * LDR;          // one slab buffer
     typedef T VL __attribute__((ext_vector_type(VEC)));
-    T *const xs = smem;                    // [kRowTile][kNR]
-    const T *__restrict__ A = tab ? tab[2 * (it.flags >> 8) + ((it.flags >> 1) & 1)] : ((it.flags & 2) ? A1 : A0);
-    const CGTerm *const tms = (const CGTerm *)terms;
+    constexpr int RG = 16 * VEC;         // rows of a slab
+    constexpr int NS = RG / 4;           // MFMA k-steps of a slab's transposed product
+    constexpr int LDR = RG + VEC;        // LDS column of a slab, padded by 16 bytes
+    constexpr int SLB = 16 * LDR;        // one slab buffer
+    constexpr uint32_t kNoRow = 0x80000000u;  // past any group's size, also with its column offsets added
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    T *const slab0 = smem + XS + 2 * wv * SLB;  // this wave's two buffers, [16][LDR] each
-    const int rows = it.rows;
-    const int ng = (rows + RG - 1) / RG;
     const int m = lane & 15, q = lane >> 4;
     const int64_t lda = it.lda;
-    // the item's input rows X_b (zero beyond rows, up to the last row group)
-    for (int e = threadIdx.x; e < ng * RG * kNR; e += 256) {
-        const int r = e / kNR;
-        xs[e] = r < rows ? vec[(it.xb + r) * kNR + (e % kNR)] : T(0);
-    }
-    __syncthreads();
-    V4 acc[NA];
+    T *const mine = smem + wv * NG * SLB;  // this wave's buffers, [NG][16][LDR]
+    // lane (q, m), element v of the transposed product is column q + 4 v of the group: whole 256- or 512-byte
+    // runs per atomic instruction (the FP32 MFMA's row 4 q + v takes its A rows in that order)
+    const int tc = sizeof(T) == 8 ? m : (m >> 2) + 4 * (m & 3);
+    // X_b(RG g + 4 s + q, m) (zero beyond the rows)
+    T xb[NG * NS];
+    const __amdgpu_buffer_rsrc_t rb = buf_rsrc(vec + (it.xb + h0) * kNR, (uint32_t)(rows * kNR * sizeof(T)));
 #pragma unroll
-    for (int a = 0; a < NA; ++a) acc[a] = (V4)0;
-    V4 acct[2] = {(V4)0, (V4)0};  // (two chains of the transposed MFMAs)
-    // this lane's rows of every row group (out of range: past the end of any resource)
-    uint32_t roff[NG];
+    for (int s = 0; s < NG * NS; ++s) xb[s] = buf_ld<T>(rb, (uint32_t)(((4 * s + q) * kNR + m) * sizeof(T)));
+    V4 acc[NG * VEC];
+#pragma unroll
+    for (int a = 0; a < NG * VEC; ++a) acc[a] = (V4)0;
+    uint32_t off[NG][4];
 #pragma unroll
     for (int g = 0; g < NG; ++g)
-        roff[g] = (g < ng && RG * g + VEC * m < rows) ? (uint32_t)((it.row0 + VEC * m + RG * g) * sizeof(T)) : kOutOfRange;
-    // cursor: term tt, 16-column group cg of that term, row group rg
-    int tt = it.t0, cg = wv, rg = 0;
-    auto settle = [&]() {
-        while (tt < it.t1) {
-            const int ngr = (tms[tt].cols + 15) >> 4;
-            if (cg < ngr) break;
-            cg -= ngr;
-            ++tt;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            off[g][j] = RG * g + VEC * m < rows
+                            ? (uint32_t)(((4 * j + q) * lda + it.row0 + h0 + RG * g + VEC * m) * sizeof(T))
+                            : kNoRow;
+    const uint32_t xoff = (uint32_t)((q * kNR + m) * sizeof(T));
+    // the window: terms w0 .. w0 + 63, lane k holding term w0 + k and the groups up to its end
+    int w0 = it.t0, ends = 0, total = 0, cols = 0;
+    int64_t ta = 0, tx = 0, tp = 0;
+    auto window = [&]() {
+        const bool in = w0 + lane < it.t1;
+        const GTerm t = terms[in ? w0 + lane : it.t0];
+        ta = t.a;
+        tx = t.x;
+        tp = t.t;
+        cols = in ? t.cols : 0;
+        // (wait for them here: a wait left to the loop would be for every load in flight)
+        asm volatile("" : "+v"(ta), "+v"(tx), "+v"(tp), "+v"(cols));
+        ends = (cols + 15) >> 4;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl_up(ends, o, 64);
+            ends += lane >= o ? u : 0;
         }
+        total = __builtin_amdgcn_readlane(ends, 63);
     };
-    struct Slab {
-        VL av[4];
+    window();
+    int G = wv;  // next group of this wave, counted in the window
+    auto lane64 = [](int64_t v, int k) {
+        const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, k), hi = __builtin_amdgcn_readlane((int)(v >> 32), k);
+        return (int64_t)(((uint64_t)hi << 32) | lo);
+    };
+    struct Group {
+        VL av[NG][4];
         T bx[4];
         int64_t t;
-        int cols, c0, g;
-        bool has;
+        int left;  // columns of the term from the group's first one, 0: no group
     };
-    auto load = [&](Slab &S) {
-        S.has = tt < it.t1;
-        const GTerm tm = term_at(tms, S.has ? tt : it.t1 - 1);
-        S.t = tm.t;
-        S.cols = tm.cols;
-        S.c0 = 16 * cg;
-        S.g = rg;
-        const __amdgpu_buffer_rsrc_t ra = buf_rsrc(A + tm.a, (uint32_t)((int64_t)tm.cols * lda * sizeof(T)));
-        const __amdgpu_buffer_rsrc_t rx = buf_rsrc(vec + tm.x * kNR, (uint32_t)((int64_t)tm.cols * kNR * sizeof(T)));
-        uint32_t ro = kOutOfRange;
-#pragma unroll
-        for (int g = 0; g < NG; ++g) ro = g == rg ? roff[g] : ro;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int c = S.c0 + 4 * j + q;
-            const bool ok = S.has && c < tm.cols;
-            // (the group's X_p rows only with its first row group; later slabs keep them)
-            S.bx[j] = buf_ld<T>(rx, opaque_off(ok && rg == 0 ? (uint32_t)((c * kNR + m) * sizeof(T)) : kOutOfRange));
-            S.av[j] = buf_ldv_nt<VL>(
-                ra, opaque_off(ok && ro != kOutOfRange ? (uint32_t)(c * lda * sizeof(T)) + ro : kOutOfRange));
+    auto load = [&](Group &S) {
+        while (G >= total && w0 + 64 < it.t1) {
+            G -= total;
+            w0 += 64;
+            window();
         }
-        if (S.has) {
-            if (++rg == ng) {
-                rg = 0;
-                cg += 4;
-                settle();
-            }
-        }
+        const bool has = G < total;
+        const int k = has ? (int)__builtin_ctzll(__ballot(ends > G)) : 0;
+        const int nc = __builtin_amdgcn_readlane(cols, k);
+        const int c0 = has ? 16 * (G - __builtin_amdgcn_readlane(ends, k) + ((nc + 15) >> 4)) : 0;
+        const int64_t t = lane64(tp, k);
+        S.left = has ? nc - c0 : 0;
+        S.t = t >= 0 ? t + c0 : -1;
+        const int n = min(S.left, 16);
+        const __amdgpu_buffer_rsrc_t ra = buf_rsrc(A + lane64(ta, k) + c0 * lda, (uint32_t)(n * lda * sizeof(T)));
+        const __amdgpu_buffer_rsrc_t rx = buf_rsrc(vec + (lane64(tx, k) + c0) * kNR, (uint32_t)(n * kNR * sizeof(T)));
+        const uint32_t xo = opaque_off(xoff);  // (row steps fold into the loads: hoisted, each would be a register)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) S.bx[j] = buf_ld<T>(rx, xo + (uint32_t)(4 * j * kNR * sizeof(T)));
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) S.av[g][j] = buf_ldv_nt<VL>(ra, off[g][j]);
+        G += 4;
     };
     auto wave_sync = [] {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
-    // the slab waiting in LDS for its transposed product
-    bool pend = false;
-    int64_t pt = 0;
-    int pcols = 0, pc0 = 0, pg = 0, pbuf = 0, cur = 0;
-    T bxc[4] = {T(0), T(0), T(0), T(0)};
-    auto compute = [&](const Slab &S) {
-        // read back the pending slab (its LDS round trip overlaps the direct products below)
-        T ta[NS], tb[NS];
-        if (pend) {
-            const T *sl = slab0 + pbuf * SLB;
-            const T *xr = xs + (RG * pg) * kNR;
+    auto put = [&](const Group &S, int g) {
+        T *sl = mine + g * SLB;
 #pragma unroll
-            for (int st = 0; st < NS; ++st) {
-                ta[st] = sl[m * LDR + 4 * st + q];
-                tb[st] = xr[(4 * st + q) * kNR + m];
-            }
-        }
-        if (S.has) {
-            if (S.g == 0) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) bxc[j] = S.bx[j];
-            }
-            // direct: rows of row group S.g
-#pragma unroll
-            for (int g = 0; g < NG; ++g)
-                if (g == S.g)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-#pragma unroll
-                        for (int e = 0; e < VEC; ++e)
-                            acc[g * VEC + e] = Mfma16<T>::op(S.av[j][e], bxc[j], acc[g * VEC + e]);
-        }
-        if (pend) {
-#pragma unroll
-            for (int st = 0; st < NS; ++st) acct[st & 1] = Mfma16<T>::op(ta[st], tb[st], acct[st & 1]);
-            if (pg == ng - 1) {
-                T *yp = vec + pt * kNR + m;
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int c = pc0 + Mfma16<T>::row(q, v);
-                    if (c < pcols) atomicAdd(yp + (int64_t)c * kNR, acct[0][v] + acct[1][v]);
-                }
-                acct[0] = acct[1] = (V4)0;
-            }
-        }
-        pend = S.has && S.t >= 0;
-        if (pend) {
-            // (the buffer written here was last read two slabs ago, and those reads are complete)
-            T *sl = slab0 + cur * SLB;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) *(VL *)&sl[(4 * j + q) * LDR + VEC * m] = S.av[j];
-            pt = S.t;
-            pcols = S.cols;
-            pc0 = S.c0;
-            pg = S.g;
-            pbuf = cur;
-            cur ^= 1;
-        }
-        wave_sync();
+        for (int j = 0; j < 4; ++j) *(VL *)&sl[(4 * j + q) * LDR + VEC * m] = S.av[g][j];
     };
-    settle();
-    // kPipe slabs rotate: while one is multiplied the next kPipe - 1 are in flight (a slab
-    // loaded past the last one has has = false and adds nothing)
-    Slab S[kPipe];
+    auto direct = [&](const Group &S, int g) {
 #pragma unroll
-    for (int i = 0; i < kPipe; ++i) load(S[i]);
-    while (S[0].has) {
+        for (int j = 0; j < 4; ++j)
+            if (4 * j < S.left)
 #pragma unroll
-        for (int i = 0; i < kPipe; ++i) {
-            compute(S[i]);
-            load(S[i]);
+                for (int e = 0; e < VEC; ++e) acc[g * VEC + e] = Mfma16<T>::op(S.av[g][j][e], S.bx[j], acc[g * VEC + e]);
+    };
+    // the transposed product of a group, added to the partner's output after the next loads are issued: loads
+    // and atomics share a counter that retires in order, and a wait for loads behind atomics is one for both
+    struct Out {
+        V4 y;
+        int64_t t;
+        int left;
+    };
+    auto compute = [&](const Group &S) {
+        Out o{(V4)0, S.t, S.t >= 0 ? S.left : 0};
+        if (S.t >= 0) {
+            V4 y[2] = {(V4)0, (V4)0};  // (two chains of the transposed MFMAs)
+#pragma unroll
+            for (int g = 0; g < NG; ++g) put(S, g);
+            wave_sync();
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                T tr[NS];
+#pragma unroll
+                for (int s = 0; s < NS; ++s) tr[s] = mine[g * SLB + tc * LDR + 4 * s + q];
+                direct(S, g);  // (the LDS round trip overlaps the direct products)
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+                    if (RG * g + 4 * s < rows) y[s & 1] = Mfma16<T>::op(tr[s], xb[g * NS + s], y[s & 1]);
+            }
+            wave_sync();  // (the next group's slabs overwrite these)
+            o.y = y[0] + y[1];
+        } else {
+#pragma unroll
+            for (int g = 0; g < NG; ++g) direct(S, g);
         }
+        return o;
+    };
+    auto flush = [&](const Out &o) {
+        const __amdgpu_buffer_rsrc_t ry =
+            buf_rsrc(vec + (o.left > 0 ? o.t : 0) * kNR, (uint32_t)(min(o.left, 16) * kNR * sizeof(T)));
+        const uint32_t xo = opaque_off(xoff);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) buf_atomic_add(ry, xo + (uint32_t)(4 * v * kNR * sizeof(T)), o.y[v]);
+    };
+    // two groups rotate (one loaded past the last reads nothing and adds nothing)
+    Group S0, S1;
+    load(S0);
+    load(S1);
+    while (S0.left > 0) {
+        const Out o0 = compute(S0);
+        load(S0);
+        flush(o0);
+        const Out o1 = compute(S1);
+        load(S1);
+        flush(o1);
     }
-    if (pend) compute(S[0]);  // (S[0].has is false: the last pending transposed product only)
-    // the four waves' direct products: 3 and 2 into 1 and 0, then 1 into 0 (LDS reused)
-    T(*red)[kRowTile][kNR] = (T(*)[kRowTile][kNR])smem;
-    auto row_of = [&](int g, int e, int v) { return RG * g + VEC * Mfma16<T>::row(q, v) + e; };
-    auto put = [&](int slot) {
+    // the four waves' direct products, summed through LDS (each wave's rows lie in its own buffers)
+    wave_sync();
 #pragma unroll
-        for (int g = 0; g < NG; ++g)
-            if (g < ng)
+    for (int g = 0; g < NG; ++g)
 #pragma unroll
-                for (int e = 0; e < VEC; ++e)
+        for (int e = 0; e < VEC; ++e)
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) red[slot][row_of(g, e, v)][m] = acc[g * VEC + e][v];
-    };
-    auto add = [&](int slot) {
-#pragma unroll
-        for (int g = 0; g < NG; ++g)
-            if (g < ng)
-#pragma unroll
-                for (int e = 0; e < VEC; ++e)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) acc[g * VEC + e][v] += red[slot][row_of(g, e, v)][m];
-    };
-    __syncthreads();  // (xs and the slabs are no longer read)
-    if (wv >= 2) put(wv - 2);
+            for (int v = 0; v < 4; ++v) mine[(RG * g + VEC * Mfma16<T>::row(q, v) + e) * kNR + m] = acc[g * VEC + e][v];
     __syncthreads();
-    if (wv < 2) add(wv);
-    __syncthreads();
-    if (wv == 1) put(0);
-    __syncthreads();
-    if (wv == 0) {
-        T *y = vec + it.y * kNR + m;
-#pragma unroll
-        for (int g = 0; g < NG; ++g)
-            if (g < ng)
-#pragma unroll
-                for (int e = 0; e < VEC; ++e)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const int r = row_of(g, e, v);
-                        if (r < rows) atomicAdd(y + (int64_t)r * kNR, acc[g * VEC + e][v] + red[0][r][m]);
-                    }
-    }
+    T *y = vec + (it.y + h0) * kNR;
+    for (int e = threadIdx.x; e < rows * kNR; e += 256)
+        atomicAdd(y + e, (smem[e] + smem[NG * SLB + e]) + (smem[2 * NG * SLB + e] + smem[3 * NG * SLB + e]));
 }
-template <typename T, int VEC>
-constexpr int sym_smem() {
-    constexpr int RG = 16 * VEC, SLB = 16 * (RG + VEC), XS = kRowTile * kNR, RED = 2 * kRowTile * kNR;
-    return XS + 8 * SLB > RED ? XS + 8 * SLB : RED;
-}
-// One item per workgroup.  An item that fits in one narrower row group (16 VEC rows: 8- or 4-byte
-// loads per lane) runs in it: a box of 20 rows takes one 32-row group where a 64-row group would
-// leave two thirds of every MFMA on zero rows.  Taller items keep the 16-byte loads (measured: more
-// row groups of narrower loads are slower even when they pad less).
+// A pass's rows: as many as two slabs of 16-byte loads hold (64 in FP64, 128 in FP32), the last rows of an item
+// in the narrowest slab that holds them (a box of 20 rows takes one 32-row slab, one of 10 a 16-row slab of
+// 8- or 4-byte loads).
 template <typename T>
 __global__ __launch_bounds__(256, 2) void k_bgemm_sym(const GItem *__restrict__ items, const GTerm *__restrict__ terms,
                                                       const T *__restrict__ A0, const T *__restrict__ A1,
                                                       const T *const *__restrict__ tab, T *vec) {
     constexpr int VMAX = 16 / sizeof(T);
-    __shared__ __attribute__((aligned(16))) T smem[sym_smem<T, VMAX>()];
+    __shared__ __attribute__((aligned(16))) T smem[4 * 2 * 16 * (16 * VMAX + VMAX)];
     const GItem it = items[blockIdx.x];
-    const int best = it.rows <= 16 ? 1 : it.rows <= 32 ? 2 : VMAX;
-    if (best == VMAX) bgemm_sym_item<T, VMAX>(it, terms, A0, A1, tab, vec, smem);
-    else if (best == 1) bgemm_sym_item<T, 1>(it, terms, A0, A1, tab, vec, smem);
-    else if constexpr (VMAX == 4) bgemm_sym_item<T, 2>(it, terms, A0, A1, tab, vec, smem);
+    const T *__restrict__ A = tab ? tab[2 * (it.flags >> 8) + ((it.flags >> 1) & 1)] : ((it.flags & 2) ? A1 : A0);
+    for (int h0 = 0; h0 < it.rows; h0 += 32 * VMAX) {
+        const int left = min(it.rows - h0, 32 * VMAX);
+        if (h0 > 0) __syncthreads();  // (the sums of the pass before are still read)
+        if (left > 16 * VMAX) bgemm_sym_rows<T, VMAX, 2>(it, h0, left, terms, A, vec, smem);
+        else if (left <= 16) bgemm_sym_rows<T, 1, 1>(it, h0, left, terms, A, vec, smem);
+        else if (VMAX == 4 && left <= 32) bgemm_sym_rows<T, 2, 1>(it, h0, left, terms, A, vec, smem);
+        else bgemm_sym_rows<T, VMAX, 1>(it, h0, left, terms, A, vec, smem);
+    }
 }
 
 // Transposed products of the symmetric blocks on the 16-wide path:

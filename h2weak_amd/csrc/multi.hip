@@ -47,22 +47,22 @@ void run_launch_m(Handle &h, const Launch &Lh, int precision, bool trans) {
     } else if (Lh.role == 1 && h.sym16) {
         // direct and transposed products in one read of every block
         if (precision == H2W_FP32_INNER)
-            launch_bgemm_sym32(h.inner.d_items.p + Lh.item0, (int)Lh.nitems, h.inner.d_terms.p, h.mat32.p,
+            launch_bgemm_sym32(h.inner.d_items.p + Lh.item0m, (int)Lh.nitemsm, h.inner.d_terms.p, h.mat32.p,
                                h.mat32in.p, nullptr, h.vec32m.p, s);
         else if (precision == H2W_FP32)
-            launch_bgemm_sym32(h.d_items.p + Lh.item0, (int)Lh.nitems, h.d_terms.p, h.mat32.p, nullptr, nullptr,
+            launch_bgemm_sym32(h.d_items.p + Lh.item0m, (int)Lh.nitemsm, h.d_terms.p, h.mat32.p, nullptr, nullptr,
                                h.vec32m.p, s);
         else
-            launch_bgemm_sym64(h.d_items.p + Lh.item0, (int)Lh.nitems, h.d_terms.p, h.mat64.p, nullptr, nullptr,
+            launch_bgemm_sym64(h.d_items.p + Lh.item0m, (int)Lh.nitemsm, h.d_terms.p, h.mat64.p, nullptr, nullptr,
                                h.vec64m.p, s);
     } else if (precision == H2W_FP32_INNER) {
-        launch_bgemm32(h.inner.d_items.p + Lh.item0, (int)Lh.nitems, h.inner.d_terms.p, h.mat32.p, h.mat32in.p,
+        launch_bgemm32(h.inner.d_items.p + Lh.item0m, (int)Lh.nitemsm, h.inner.d_terms.p, h.mat32.p, h.mat32in.p,
                        h.vec32m.p, Lh.role, per_wave_items(Lh), s);
     } else if (precision == H2W_FP32) {
-        launch_bgemm32(h.d_items.p + Lh.item0, (int)Lh.nitems, h.d_terms.p, h.mat32.p, nullptr, h.vec32m.p, Lh.role,
+        launch_bgemm32(h.d_items.p + Lh.item0m, (int)Lh.nitemsm, h.d_terms.p, h.mat32.p, nullptr, h.vec32m.p, Lh.role,
                        per_wave_items(Lh), s);
     } else {
-        launch_bgemm64(h.d_items.p + Lh.item0, (int)Lh.nitems, h.d_terms.p, h.mat64.p, nullptr, h.vec64m.p, Lh.role,
+        launch_bgemm64(h.d_items.p + Lh.item0m, (int)Lh.nitemsm, h.d_terms.p, h.mat64.p, nullptr, h.vec64m.p, Lh.role,
                        per_wave_items(Lh), s);
     }
 }
