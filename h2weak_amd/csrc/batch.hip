@@ -120,9 +120,10 @@ void merge_lists(Batch &B, int which) {
                 items.push_back(it);
             }
         }
-        if (Lm.role == 1 && B.sym16) {
+        if (Lm.role != 3) {
             const int64_t end = (int64_t)items.size();
-            if (wide_items(items, Lm.item0, terms) > 0) items.erase(items.begin() + Lm.item0, items.begin() + end);
+            if (wide_items(items, Lm.item0, terms, Lm.role) > 0)
+                items.erase(items.begin() + Lm.item0, items.begin() + end);
         }
         Lm.nitems = Lm.nitemsm = (int64_t)items.size() - Lm.item0;
         Lm.nterms = (int64_t)terms.size() - Lm.term0;

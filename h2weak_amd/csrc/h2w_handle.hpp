@@ -175,7 +175,7 @@ inline bool per_wave_items(const Launch &L) {
 inline bool per_wave_gemv(const Launch &L) {
     return L.nitems >= 2048 && L.avg_item_elems > 0 && L.avg_item_elems <= 8192;
 }
-int64_t wide_items(std::vector<GItem> &items, int64_t item0, const std::vector<GTerm> &terms);
+int64_t wide_items(std::vector<GItem> &items, int64_t item0, const std::vector<GTerm> &terms, int role);
 // narrow slabs for the transposed 16-wide products when the blocks have few rows
 inline int trans_narrow(const Launch &L, bool fp32) { return L.avg_cols <= (fp32 ? 32 : 16); }
 

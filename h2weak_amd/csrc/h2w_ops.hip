@@ -1123,15 +1123,18 @@ int inner_rank(const std::vector<double> &hist, int rank, double tau) {
 
 }  // namespace
 
-// The 16-wide path's items of a fused launch, appended to items, whose entries from item0 on are the
-// single-vector path's: consecutive pieces of one row tile (their terms follow one another) are put together again,
-// up to a 2048th of the launch's elements.  A workgroup of the 16-wide kernel reads 16 input rows per item row,
-// and sums and adds as many at the end: about 5 us an item beside its data.
-// Measured (fused launch, FP64, uncombined pieces / 4096 / 2048 / 1024): 32^3 grid at 1e-10 492 / 452 / 448 / 458
-// us, 3D N = 20011 231 / 229 / 204 / 202 us, 2D N = 90000 317 / 297 / 292 / 304 us.  (The transfers' pieces stay:
-// 2D semi-nested 400 x 400 207 us of them, 2048 / 1024 / 512: 207 / 215 / 248 us.)
+// The 16-wide path's items of a launch, appended to items, whose entries from item0 on are the single-vector
+// path's: consecutive pieces of one row tile (their terms follow one another) are put together again.  A workgroup
+// of the 16-wide kernels reads 16 input rows per item row, and sums and adds as many at the end: about 5 us an item
+// beside its data.  Fused launches (role 1) up to a 2048th of the launch's elements, the others up to 256 columns,
+// four 16-column groups per wave.  Measured, FP64, uncombined first:
+//   fused, 4096 / 2048 / 1024 items: 32^3 grid at 1e-10 492, 452 / 448 / 458 us, 3D N = 20011 231, 229 / 204 / 202,
+//     2D N = 90000 317, 297 / 292 / 304;
+//   transfers of a product, 128 / 256 / 512 columns: 32^3 188, 168 / 161 / 154 us, 3D N = 20011 114, 106 / 102 / 101,
+//     2D N = 90000 369, 352 / 348 / 352, 2D semi-nested 400 x 400 156, 156 / 157 / 158, 16^3 55, 55 / 56 / 59.
+//     (By elements instead, a 512th of the launch: the semi-nested one, a few tall boxes among many, 172.)
 // Returns the number of items appended; 0 where nothing combines.
-int64_t wide_items(std::vector<GItem> &items, int64_t item0, const std::vector<GTerm> &terms) {
+int64_t wide_items(std::vector<GItem> &items, int64_t item0, const std::vector<GTerm> &terms, int role) {
     const int64_t end = (int64_t)items.size();
     auto work = [&](const GItem &it) {
         int64_t w = 0;
@@ -1140,10 +1143,11 @@ int64_t wide_items(std::vector<GItem> &items, int64_t item0, const std::vector<G
     };
     int64_t E = 0, sum = 0;
     for (int64_t q = item0; q < end; ++q) E += work(items[q]);
-    const int64_t most = E / 2048 + E / 8192;
+    const int64_t share = E / 2048 + E / 8192;
     for (int64_t q = item0; q < end; ++q) {
         const GItem it = items[q];
         const int64_t w = work(it);
+        const int64_t most = role == 1 ? share : 256 * (int64_t)it.rows;
         GItem &l = items.back();
         if (q > item0 && l.y == it.y && l.xb == it.xb && l.rows == it.rows && l.lda == it.lda && l.row0 == it.row0 &&
             l.flags == it.flags && l.t1 == it.t0 && sum + w <= most) {
@@ -1161,7 +1165,7 @@ int64_t wide_items(std::vector<GItem> &items, int64_t item0, const std::vector<G
 }
 void Launch::set_wide(std::vector<GItem> &items, const std::vector<GTerm> &terms) {
     const int64_t n = (int64_t)items.size();
-    nitemsm = role == 1 ? wide_items(items, item0, terms) : 0;
+    nitemsm = wide_items(items, item0, terms, role);
     item0m = nitemsm ? n : item0;
     if (!nitemsm) nitemsm = nitems;
 }

@@ -1071,10 +1071,7 @@ __global__ __launch_bounds__(256) void k_bgemv(const GItem *__restrict__ items, 
 // column -- is the B operand of all of them.  An MFMA's D(row(q, v), m) then
 // belongs to item row  group * 16 VEC + VEC row(q, v) + u, where row(q, v) =
 // 4q + v (FP32) or q + 4v (FP64) are the two instructions' result layouts,
-// checked on gfx950.  An item's columns, term after term, form 4-column chunks;
-// the four waves take every fourth chunk (a scalar cursor walks the terms), four
-// chunks in flight per wave whatever the terms' widths, and their partial
-// products are summed through LDS by wave 0.
+// checked on gfx950.
 template <typename T>
 struct Mfma16;
 template <>
@@ -1094,201 +1091,28 @@ struct Mfma16<double> {
     static __device__ __forceinline__ int row(int q, int v) { return q + 4 * v; }
 };
 
-// One item with VEC rows per lane load, NG load groups (rows <= 16 VEC NG) and UNR
-// 4-column chunks per iteration, two iterations in flight (the next one's loads are
-// issued before the current one is multiplied).  Loads are raw buffer loads whose
-// out-of-range lanes read zeros, so no branch guards them and the waits before the
-// MFMAs count only the current iteration's loads.  WPI waves share the item: 4 (the
-// waves take every fourth chunk and sum their products through red, the workgroup's
-// LDS reduction buffer) or 1 (the wave takes every chunk and writes its rows itself;
-// red is unused and no barrier is reached).
-template <typename T, int VEC, int NG, int UNR, int WPI>
-__device__ __forceinline__ void bgemm_item(const GItem &it, const GTerm *__restrict__ terms, const T *__restrict__ A,
-                                           T *vec, T (*red)[kRowTile][kNR]) {
-    typedef typename Mfma16<T>::v4 V4;
-    typedef T VL __attribute__((ext_vector_type(VEC)));
-    constexpr int RG = 16 * VEC;  // rows of one load group
-    constexpr int NA = NG * VEC;  // accumulators
-    const CGTerm *const tms = (const CGTerm *)terms;
-    const int lane = threadIdx.x & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int rows = it.rows;
-    const int ng = (rows + RG - 1) / RG;
-    const int m = lane & 15, q = lane >> 4;
-    V4 acc[NA];
-#pragma unroll
-    for (int a = 0; a < NA; ++a) acc[a] = (V4)0;
-    const int64_t lda = it.lda;
-    // The item's columns, term after term, in 4-column chunks; wave wv takes chunks
-    // wv, wv + 4, ... through a cursor (term tt, chunk ck of that term).
-    int tt = it.t0, ck = WPI == 4 ? wv : 0;
-    auto settle = [&]() {
-        while (tt < it.t1) {
-            const int nk = (tms[tt].cols + 3) >> 2;
-            if (ck < nk) break;
-            ck -= nk;
-            ++tt;
-        }
-    };
-    struct Iter {
-        VL av[UNR][NG];
-        T bx[UNR];
-        bool has;
-    };
-    // this lane's rows of every load group (out of range: past the end of any resource)
-    uint32_t roff[NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g)
-        roff[g] = (g < ng && RG * g + VEC * m < rows) ? (uint32_t)((it.row0 + VEC * m + RG * g) * sizeof(T)) : kOutOfRange;
-    auto load = [&](Iter &B) -> bool {
-        B.has = tt < it.t1;
-#pragma unroll
-        for (int u = 0; u < UNR; ++u) {
-            const bool has = tt < it.t1;
-            const GTerm tm = term_at(tms, has ? tt : it.t1 - 1);
-            const int c = 4 * ck + q;
-            const bool ok = has && c < tm.cols;
-            const __amdgpu_buffer_rsrc_t ra = buf_rsrc(A + tm.a, (uint32_t)((int64_t)tm.cols * lda * sizeof(T)));
-            const __amdgpu_buffer_rsrc_t rx = buf_rsrc(vec + tm.x * kNR, (uint32_t)((int64_t)tm.cols * kNR * sizeof(T)));
-            B.bx[u] = buf_ld<T>(rx, opaque_off(ok ? (uint32_t)((c * kNR + m) * sizeof(T)) : kOutOfRange));
-            const uint32_t coff = ok ? (uint32_t)(c * lda * sizeof(T)) : kOutOfRange;
-#pragma unroll
-            for (int g = 0; g < NG; ++g)
-                B.av[u][g] =
-                    buf_ld16_nt<VL>(ra, opaque_off(ok && roff[g] != kOutOfRange ? coff + roff[g] : kOutOfRange));
-            if (has) {
-                ck += WPI;
-                settle();
-            }
-        }
-        return B.has;
-    };
-    auto compute = [&](const Iter &B) {
-#pragma unroll
-        for (int u = 0; u < UNR; ++u)
-#pragma unroll
-            for (int g = 0; g < NG; ++g)
-                if (g < ng)
-#pragma unroll
-                    for (int e = 0; e < VEC; ++e)
-                        acc[g * VEC + e] = Mfma16<T>::op(B.av[u][g][e], B.bx[u], acc[g * VEC + e]);
-    };
-    settle();
-    // (a buffer loaded past the last chunk holds zeros: multiplying it adds nothing, so
-    // both halves run unconditionally and the loop has a single path for the waits)
-    Iter B0, B1;
-    bool h0 = load(B0);
-    load(B1);
-    while (h0) {
-        compute(B0);
-        h0 = load(B0);
-        compute(B1);
-        load(B1);
-    }
-    // item row held by accumulator (g, e), result element v of this lane
-    auto row_of = [&](int g, int e, int v) { return RG * g + VEC * Mfma16<T>::row(q, v) + e; };
-    // sum the four waves' partial products: 3 and 2 into 1 and 0, then 1 into 0
-    auto put = [&](int slot) {
-#pragma unroll
-        for (int g = 0; g < NG; ++g)
-            if (g < ng)
-#pragma unroll
-                for (int e = 0; e < VEC; ++e)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) red[slot][row_of(g, e, v)][m] = acc[g * VEC + e][v];
-    };
-    auto add = [&](int slot) {
-#pragma unroll
-        for (int g = 0; g < NG; ++g)
-            if (g < ng)
-#pragma unroll
-                for (int e = 0; e < VEC; ++e)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) acc[g * VEC + e][v] += red[slot][row_of(g, e, v)][m];
-    };
-    if constexpr (WPI == 4) {
-        if (wv >= 2) put(wv - 2);
-        __syncthreads();
-        if (wv < 2) add(wv);
-        __syncthreads();
-        if (wv == 1) put(0);
-        __syncthreads();
-        if (wv == 0) add(0);
-    }
-    if (WPI == 1 || wv == 0) {
-        T *y = vec + it.y * kNR + m;
-#pragma unroll
-        for (int g = 0; g < NG; ++g)
-            if (g < ng)
-#pragma unroll
-                for (int e = 0; e < VEC; ++e)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const int r = row_of(g, e, v);
-                        if (r < rows) {
-                            if (it.flags & 1) atomicAdd(y + (int64_t)r * kNR, acc[g * VEC + e][v]);
-                            else y[(int64_t)r * kNR] += acc[g * VEC + e][v];
-                        }
-                    }
-    }
-}
-
-// WPI 4: one item per workgroup; WPI 1: one item per wave (launches of many small items:
-// no cross-wave reduction, four items in flight per workgroup), nitems bounds the last one.
-template <typename T, int ROLE, int WPI>
-__global__ __launch_bounds__(256) void k_bgemm(const GItem *__restrict__ items, int nitems,
-                                               const GTerm *__restrict__ terms, const T *__restrict__ A0,
-                                               const T *__restrict__ A1, const T *const *__restrict__ tab, T *vec) {
-    const int idx = WPI == 4 ? (int)blockIdx.x : 4 * (int)blockIdx.x + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (idx >= nitems) return;  // (WPI 1 only: whole waves, and no barrier follows)
-    const GItem it = items[idx];
-    // batched systems: pool pair of system flags >> 8 from the table
-    const T *__restrict__ A = tab ? tab[2 * (it.flags >> 8) + ((it.flags >> 1) & 1)] : ((it.flags & 2) ? A1 : A0);
-    constexpr int VEC = 16 / sizeof(T);
-    if constexpr (WPI == 4) {
-        __shared__ T red[2][kRowTile][kNR];
-        bgemm_item<T, VEC, kRowTile / (16 * VEC), 2, 4>(it, terms, A, vec, red);
-    } else {
-        bgemm_item<T, VEC, kRowTile / (16 * VEC), 2, 1>(it, terms, A, vec, nullptr);
-    }
-}
-
-// Direct and transposed products of the stored blocks in one read, kNR right-hand sides
-// (the fused M2L + near-field launch of the multi-vector pass).  One item (box b, rows <= 128) per
-// workgroup, its rows in passes of up to RG NG (RG = 16 VEC).  The item's terms K(b, p) are cut into
-// 16-column groups (never across a term); wave wv takes groups wv, wv + 4, ...  A group is NG slabs of
-// RG rows x 16 columns, loaded in the direct product's layout (lane (m, q): VEC consecutive rows of column
-// 4 j + q, j < 4: 16-byte loads, 256-byte runs per column; the next group in flight) and multiplied into
-// the pass's rows (as k_bgemm: A(m, q) = K(VEC m + e, 4 j + q), B(q, m) = X_p(4 j + q, m)).  For a
-// symmetric term (t >= 0) the wave also writes the slabs to its LDS buffers and reads them back with a
-// column per lane % 16 and a row per lane / 16, the A operand of K^T: with B(q, m) = X_b(4 s + q, m), held in
-// registers, it forms the 16 x kNR block Y_p(c0 .. c0 + 15, :) += K(rows, c0 ..)^T X_b and adds it to the
-// partner's output with atomics.  MFMAs over columns past the term or rows past the pass are left out, four at
-// a time.  The item's own rows are added atomically too (other items' transposes land in them).  Each
-// stored element is read once per pass, where k_bgemm + k_bgemm_tl read it twice.
-// The terms of an item (64 of them at a time) sit one per lane, and a group's term is found by a ballot over
-// the running group counts: a cursor over descriptors in memory waited on two or three dependent scalar
-// loads a group, and those waits cover the LDS counter too.
-// FP64: 64 MFMA flops per stored element (direct and transposed, 16 right-hand sides) against
-// 8 bytes, so the launch needs both HBM and the FP64 matrix cores (78.6 TFLOP/s) at once;
-// launch bounds cap it at 256 registers a lane (two waves per SIMD).
-// Measured against slabs of 128-row items from a scalar cursor, with the atomics before the next loads (the same
-// lists), FP64 / FP32: 32^3 grid at 1e-10 (1.9 GB) 517 / 277 -> 492 / 255 us, 3D N = 20011 258 / 148 -> 231 /
-// 129, 2D N = 90000 328 / 195 -> 317 / 162; with the lists of wide_items 448 / 232, 204 / 113, 292 / 143.
-// Without loads from HBM it takes 440 us on the first, without the partner's atomics 350, with the direct
-// products only 155 (MFMA time 105 each way): the matrix pipe and the atomics share the bound.
-template <typename T, int VEC, int NG>
-__device__ __forceinline__ void bgemm_sym_rows(const GItem &it, int h0, int rows, const GTerm *__restrict__ terms,
-                                               const T *__restrict__ A, T *vec, T *smem) {
+// One pass over an item's terms for `rows` of its rows, from h0 on: NG slabs of RG = 16 VEC rows.  The terms are cut
+// into 16-column groups (never across a term); of WPI waves each takes every WPI-th group, the next group's loads
+// in flight while one is multiplied (raw buffer loads: out-of-range lanes read zeros, no branch guards them).
+// The terms of an item (64 of them at a time) sit one per lane, and a group's term is found by a ballot over the
+// running group counts: a cursor over descriptors in memory waited on two or three dependent scalar loads a
+// group, and those waits cover the LDS counter too.  MFMAs over columns past the term or rows past the pass are
+// left out, four at a time.  SYM: the transposed products of symmetric terms as well (below).
+// Transfers of a 16-wide product against 128-row items by 4-column chunks from a scalar cursor (FP64, the same
+// lists, then those of wide_items): 32^3 grid at 1e-10 193 -> 187 -> 161 us, 3D N = 20011 148 -> 114 -> 102, 2D
+// N = 90000 422 -> 370 -> 348, 2D semi-nested 400 x 400 207 -> 156, 16^3 77 -> 55, 1D N = 65536 147 -> 110.
+template <typename T, int VEC, int NG, bool SYM, int WPI>
+__device__ __forceinline__ void bgemm_rows(const GItem &it, int h0, int rows, const GTerm *__restrict__ terms,
+                                           const T *__restrict__ A, T *vec, T *smem) {
     typedef typename Mfma16<T>::v4 V4;
     typedef T VL __attribute__((ext_vector_type(VEC)));
     constexpr int RG = 16 * VEC;         // rows of a slab
     constexpr int NS = RG / 4;           // MFMA k-steps of a slab's transposed product
     constexpr int LDR = RG + VEC;        // LDS column of a slab, padded by 16 bytes
-    constexpr int SLB = 16 * LDR;        // one slab buffer
+    constexpr int SLB = SYM ? 16 * LDR : 16 * RG;  // one slab buffer (or its rows' sums)
     constexpr uint32_t kNoRow = 0x80000000u;  // past any group's size, also with its column offsets added
     const int lane = threadIdx.x & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wv = WPI == 4 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
     const int m = lane & 15, q = lane >> 4;
     const int64_t lda = it.lda;
     T *const mine = smem + wv * NG * SLB;  // this wave's buffers, [NG][16][LDR]
@@ -1296,10 +1120,10 @@ __device__ __forceinline__ void bgemm_sym_rows(const GItem &it, int h0, int rows
     // runs per atomic instruction (the FP32 MFMA's row 4 q + v takes its A rows in that order)
     const int tc = sizeof(T) == 8 ? m : (m >> 2) + 4 * (m & 3);
     // X_b(RG g + 4 s + q, m) (zero beyond the rows)
-    T xb[NG * NS];
+    T xb[SYM ? NG * NS : 1];
     const __amdgpu_buffer_rsrc_t rb = buf_rsrc(vec + (it.xb + h0) * kNR, (uint32_t)(rows * kNR * sizeof(T)));
 #pragma unroll
-    for (int s = 0; s < NG * NS; ++s) xb[s] = buf_ld<T>(rb, (uint32_t)(((4 * s + q) * kNR + m) * sizeof(T)));
+    for (int s = 0; s < (SYM ? NG * NS : 0); ++s) xb[s] = buf_ld<T>(rb, (uint32_t)(((4 * s + q) * kNR + m) * sizeof(T)));
     V4 acc[NG * VEC];
 #pragma unroll
     for (int a = 0; a < NG * VEC; ++a) acc[a] = (V4)0;
@@ -1356,7 +1180,7 @@ __device__ __forceinline__ void bgemm_sym_rows(const GItem &it, int h0, int rows
         const int c0 = has ? 16 * (G - __builtin_amdgcn_readlane(ends, k) + ((nc + 15) >> 4)) : 0;
         const int64_t t = lane64(tp, k);
         S.left = has ? nc - c0 : 0;
-        S.t = t >= 0 ? t + c0 : -1;
+        S.t = SYM && t >= 0 ? t + c0 : -1;
         const int n = min(S.left, 16);
         const __amdgpu_buffer_rsrc_t ra = buf_rsrc(A + lane64(ta, k) + c0 * lda, (uint32_t)(n * lda * sizeof(T)));
         const __amdgpu_buffer_rsrc_t rx = buf_rsrc(vec + (lane64(tx, k) + c0) * kNR, (uint32_t)(n * kNR * sizeof(T)));
@@ -1367,7 +1191,7 @@ __device__ __forceinline__ void bgemm_sym_rows(const GItem &it, int h0, int rows
         for (int g = 0; g < NG; ++g)
 #pragma unroll
             for (int j = 0; j < 4; ++j) S.av[g][j] = buf_ldv_nt<VL>(ra, off[g][j]);
-        G += 4;
+        G += WPI;
     };
     auto wave_sync = [] {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1395,7 +1219,7 @@ __device__ __forceinline__ void bgemm_sym_rows(const GItem &it, int h0, int rows
     };
     auto compute = [&](const Group &S) {
         Out o{(V4)0, S.t, S.t >= 0 ? S.left : 0};
-        if (S.t >= 0) {
+        if (SYM && S.t >= 0) {
             V4 y[2] = {(V4)0, (V4)0};  // (two chains of the transposed MFMAs)
 #pragma unroll
             for (int g = 0; g < NG; ++g) put(S, g);
@@ -1419,6 +1243,7 @@ __device__ __forceinline__ void bgemm_sym_rows(const GItem &it, int h0, int rows
         return o;
     };
     auto flush = [&](const Out &o) {
+        if (!SYM) return;
         const __amdgpu_buffer_rsrc_t ry =
             buf_rsrc(vec + (o.left > 0 ? o.t : 0) * kNR, (uint32_t)(min(o.left, 16) * kNR * sizeof(T)));
         const uint32_t xo = opaque_off(xoff);
@@ -1437,22 +1262,99 @@ __device__ __forceinline__ void bgemm_sym_rows(const GItem &it, int h0, int rows
         load(S1);
         flush(o1);
     }
-    // the four waves' direct products, summed through LDS (each wave's rows lie in its own buffers)
-    wave_sync();
-#pragma unroll
-    for (int g = 0; g < NG; ++g)
-#pragma unroll
-        for (int e = 0; e < VEC; ++e)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) mine[(RG * g + VEC * Mfma16<T>::row(q, v) + e) * kNR + m] = acc[g * VEC + e][v];
-    __syncthreads();
+    auto row_of = [&](int g, int e, int v) { return RG * g + VEC * Mfma16<T>::row(q, v) + e; };
     T *y = vec + (it.y + h0) * kNR;
-    for (int e = threadIdx.x; e < rows * kNR; e += 256)
-        atomicAdd(y + e, (smem[e] + smem[NG * SLB + e]) + (smem[2 * NG * SLB + e] + smem[3 * NG * SLB + e]));
+    const bool atomic = SYM || (it.flags & 1);
+    if constexpr (WPI == 1) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+            for (int e = 0; e < VEC; ++e)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int r = row_of(g, e, v);
+                    if (r >= rows) continue;
+                    if (atomic) atomicAdd(y + r * kNR + m, acc[g * VEC + e][v]);
+                    else y[r * kNR + m] += acc[g * VEC + e][v];
+                }
+    } else {
+        // the four waves' direct products, summed through LDS (each wave's rows lie in its own buffers)
+        wave_sync();
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+            for (int e = 0; e < VEC; ++e)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) mine[row_of(g, e, v) * kNR + m] = acc[g * VEC + e][v];
+        __syncthreads();
+        for (int e = threadIdx.x; e < rows * kNR; e += 256) {
+            const T sum = (smem[e] + smem[NG * SLB + e]) + (smem[2 * NG * SLB + e] + smem[3 * NG * SLB + e]);
+            if (atomic) atomicAdd(y + e, sum);
+            else y[e] += sum;
+        }
+    }
 }
 // A pass's rows: as many as two slabs of 16-byte loads hold (64 in FP64, 128 in FP32), the last rows of an item
 // in the narrowest slab that holds them (a box of 20 rows takes one 32-row slab, one of 10 a 16-row slab of
 // 8- or 4-byte loads).
+template <typename T>
+constexpr int kPassRows = 2 * 16 * (16 / sizeof(T));
+template <typename T, bool SYM, int WPI>
+__device__ __forceinline__ void bgemm_pass(const GItem &it, int h0, const GTerm *__restrict__ terms,
+                                           const T *__restrict__ A, T *vec, T *smem) {
+    constexpr int VMAX = 16 / sizeof(T);
+    const int left = min(it.rows - h0, kPassRows<T>);
+    if (left > 16 * VMAX) bgemm_rows<T, VMAX, 2, SYM, WPI>(it, h0, left, terms, A, vec, smem);
+    else if (left <= 16) bgemm_rows<T, 1, 1, SYM, WPI>(it, h0, left, terms, A, vec, smem);
+    else if (VMAX == 4 && left <= 32) bgemm_rows<T, 2, 1, SYM, WPI>(it, h0, left, terms, A, vec, smem);
+    else bgemm_rows<T, VMAX, 1, SYM, WPI>(it, h0, left, terms, A, vec, smem);
+}
+
+// WPI 4: one item per workgroup; WPI 1: one item per wave (launches of many small items: no cross-wave
+// reduction, four items in flight per workgroup), nitems bounds the last one.  blockIdx.y: the pass.
+template <typename T, int ROLE, int WPI>
+__global__ __launch_bounds__(256) void k_bgemm(const GItem *__restrict__ items, int nitems,
+                                               const GTerm *__restrict__ terms, const T *__restrict__ A0,
+                                               const T *__restrict__ A1, const T *const *__restrict__ tab, T *vec) {
+    const int idx = WPI == 4 ? (int)blockIdx.x : 4 * (int)blockIdx.x + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (idx >= nitems) return;  // (WPI 1 only: whole waves, and no barrier follows)
+    const GItem it = items[idx];
+    const int h0 = blockIdx.y * kPassRows<T>;
+    if (h0 >= it.rows) return;
+    // batched systems: pool pair of system flags >> 8 from the table
+    const T *__restrict__ A = tab ? tab[2 * (it.flags >> 8) + ((it.flags >> 1) & 1)] : ((it.flags & 2) ? A1 : A0);
+    if constexpr (WPI == 4) {
+        __shared__ __attribute__((aligned(16))) T smem[4 * kPassRows<T> * kNR];
+        bgemm_pass<T, false, 4>(it, h0, terms, A, vec, smem);
+    } else {
+        bgemm_pass<T, false, 1>(it, h0, terms, A, vec, nullptr);
+    }
+}
+
+// Direct and transposed products of the stored blocks in one read, kNR right-hand sides
+// (the fused M2L + near-field launch of the multi-vector pass).  One item (box b, rows <= 128) per
+// workgroup, its rows in passes of up to RG NG (RG = 16 VEC).  The item's terms K(b, p) are cut into
+// 16-column groups (never across a term); wave wv takes groups wv, wv + 4, ...  A group is NG slabs of
+// RG rows x 16 columns, loaded in the direct product's layout (lane (m, q): VEC consecutive rows of column
+// 4 j + q, j < 4: 16-byte loads, 256-byte runs per column; the next group in flight) and multiplied into
+// the pass's rows (as k_bgemm: A(m, q) = K(VEC m + e, 4 j + q), B(q, m) = X_p(4 j + q, m)).  For a
+// symmetric term (t >= 0) the wave also writes the slabs to its LDS buffers and reads them back with a
+// column per lane % 16 and a row per lane / 16, the A operand of K^T: with B(q, m) = X_b(4 s + q, m), held in
+// registers, it forms the 16 x kNR block Y_p(c0 .. c0 + 15, :) += K(rows, c0 ..)^T X_b and adds it to the
+// partner's output with atomics.  MFMAs over columns past the term or rows past the pass are left out, four at
+// a time.  The item's own rows are added atomically too (other items' transposes land in them).  Each
+// stored element is read once per pass, where k_bgemm + k_bgemm_tl read it twice.
+// The terms of an item (64 of them at a time) sit one per lane, and a group's term is found by a ballot over
+// the running group counts: a cursor over descriptors in memory waited on two or three dependent scalar
+// loads a group, and those waits cover the LDS counter too.
+// FP64: 64 MFMA flops per stored element (direct and transposed, 16 right-hand sides) against
+// 8 bytes, so the launch needs both HBM and the FP64 matrix cores (78.6 TFLOP/s) at once;
+// launch bounds cap it at 256 registers a lane (two waves per SIMD).
+// Measured against slabs of 128-row items from a scalar cursor, with the atomics before the next loads (the same
+// lists), FP64 / FP32: 32^3 grid at 1e-10 (1.9 GB) 517 / 277 -> 492 / 255 us, 3D N = 20011 258 / 148 -> 231 /
+// 129, 2D N = 90000 328 / 195 -> 317 / 162; with the lists of wide_items 448 / 232, 204 / 113, 292 / 143.
+// Without loads from HBM it takes 440 us on the first, without the partner's atomics 350, with the direct
+// products only 155 (MFMA time 105 each way): the matrix pipe and the atomics share the bound.
 template <typename T>
 __global__ __launch_bounds__(256, 2) void k_bgemm_sym(const GItem *__restrict__ items, const GTerm *__restrict__ terms,
                                                       const T *__restrict__ A0, const T *__restrict__ A1,
@@ -1461,13 +1363,9 @@ __global__ __launch_bounds__(256, 2) void k_bgemm_sym(const GItem *__restrict__ 
     __shared__ __attribute__((aligned(16))) T smem[4 * 2 * 16 * (16 * VMAX + VMAX)];
     const GItem it = items[blockIdx.x];
     const T *__restrict__ A = tab ? tab[2 * (it.flags >> 8) + ((it.flags >> 1) & 1)] : ((it.flags & 2) ? A1 : A0);
-    for (int h0 = 0; h0 < it.rows; h0 += 32 * VMAX) {
-        const int left = min(it.rows - h0, 32 * VMAX);
+    for (int h0 = 0; h0 < it.rows; h0 += kPassRows<T>) {
         if (h0 > 0) __syncthreads();  // (the sums of the pass before are still read)
-        if (left > 16 * VMAX) bgemm_sym_rows<T, VMAX, 2>(it, h0, left, terms, A, vec, smem);
-        else if (left <= 16) bgemm_sym_rows<T, 1, 1>(it, h0, left, terms, A, vec, smem);
-        else if (VMAX == 4 && left <= 32) bgemm_sym_rows<T, 2, 1>(it, h0, left, terms, A, vec, smem);
-        else bgemm_sym_rows<T, VMAX, 1>(it, h0, left, terms, A, vec, smem);
+        bgemm_pass<T, true, 4>(it, h0, terms, A, vec, smem);
     }
 }
 
@@ -2646,11 +2544,12 @@ void launch_scal(double a, double *y, int64_t n, hipStream_t s) {
 template <typename T, int ROLE>
 static void launch_bgemm_r(const GItem *items, int nitems, const GTerm *terms, const T *A0, const T *A1,
                            const T *const *tab, T *vec, bool per_wave, hipStream_t s) {
+    constexpr int np = kRowTile / kPassRows<T>;
     if (per_wave)
-        hipLaunchKernelGGL((k_bgemm<T, ROLE, 1>), dim3((nitems + 3) / 4), dim3(256), 0, s, items, nitems, terms, A0, A1,
+        hipLaunchKernelGGL((k_bgemm<T, ROLE, 1>), dim3((nitems + 3) / 4, np), dim3(256), 0, s, items, nitems, terms, A0, A1,
                            tab, vec);
     else
-        hipLaunchKernelGGL((k_bgemm<T, ROLE, 4>), dim3(nitems), dim3(256), 0, s, items, nitems, terms, A0, A1, tab,
+        hipLaunchKernelGGL((k_bgemm<T, ROLE, 4>), dim3(nitems, np), dim3(256), 0, s, items, nitems, terms, A0, A1, tab,
                            vec);
 }
 template <typename T>
