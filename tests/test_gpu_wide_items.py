@@ -52,3 +52,15 @@ def test_batch_agrees():
     Y = h2w.Batch(G).matvec(X)
     for g, x, y in zip(G, X, Y):
         _agree(y, g, x, h2w.FP64, 1e-12)
+
+
+def test_host_columns_with_gaps():
+    g = _system(CASES[4])
+    N, nrhs, ld = g.N, 19, g.N + 7
+    X = np.full((nrhs, ld), np.nan)
+    X[:, :N] = np.random.default_rng(6).normal(size=(nrhs, N))
+    Y = np.full((nrhs, ld), -1.0)
+    rc = h2w.lib().h2w_matvec_ex(g._h, h2w._ptr(X), h2w._ptr(Y), nrhs, ld, h2w.FP64, h2w.ORDER_INPUT, h2w.HOST)
+    assert rc == h2w.H2W_OK
+    _agree(Y[:, :N], g, np.ascontiguousarray(X[:, :N]), h2w.FP64, 1e-12)
+    assert np.all(Y[:, N:] == -1.0)
