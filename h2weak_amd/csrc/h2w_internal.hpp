@@ -223,7 +223,8 @@ void launch_xfer(const XferJob *jobs, int njobs, const int32_t *idx, const doubl
 void launch_cur(const CurJob *jobs, int njobs, const int32_t *idx, const double *lr, double *A, KParams kp,
                 hipStream_t s);
 // lo: low parts of the blocks at offsets lo0 and up
-void launch_compose(const ComposeJob *jobs, int njobs, double *A, double *lo, int64_t lo0, hipStream_t s);
+void launch_compose(const ComposeJob *jobs, int njobs, double *A, double *lo, int64_t lo0, unsigned long long *most,
+                    hipStream_t s);
 void launch_copy32(const CopyJob *jobs, int njobs, const float *src, float *dst, hipStream_t s);
 // operator pool A0, or A1 for items whose flags have bit 1 set; unr in {2, 4, 8}.  Role 1:
 // symmetric terms (t >= 0) also add A^T x_item to vec[t ..] atomically.

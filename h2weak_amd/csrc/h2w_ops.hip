@@ -1572,15 +1572,22 @@ void assemble(Handle &h) {
 }
 
 // The transfer passes near the root are launches of a few hundred kilobytes, one after another, 3 to 4 us
-// each whatever they hold (10 of the 12 levels of a 1D system with N = 250000).  Levels B .. T-1 can be one
+// each whatever they hold (all of a 1D system with N = 2048).  Levels B .. T-1 can be one
 // launch each way: their skeletons go straight to those of their descendants at level T and back, by the
 // products of the transfers between them.  Such blocks hold a full row of blocks each, so that every level
 // of the group has as many bytes as the widest; a group grows while the launches it saves outweigh the bytes
 // it adds, and while no block is so large that the launch would cut it into pieces that accumulate
 // atomically (a box's outgoing vector stays one sum in one order).  Returns the groups from the leaves up as
 // (T, B), B = T - 1 for a level by itself (real kernels; the inner operator keeps its own chain).
-// Measured, products without / with: 1D N = 250000 214 / 173 us (FP32 177 / 132), 1D N = 2048 62 / 48 us.
+// Measured, products without / with: 1D N = 2048 62 / 48 us.
 constexpr double kLaunchUs = 3.0, kBytesPerUs = 4.0e6;
+// A group ends before the first level whose composites have entries above this.  Rounding in a chain of transfers
+// perturbs the skeleton charges between two levels, and the next transfer reproduces the far field of whatever
+// charges it is given; rounding in a composite of large entries of both signs is not so absorbed.  At 512 it stays at
+// 1e-13.  (1D, uniform points, N = 70003 at 1e-12, entries to 2e4: the product of a random vector 1.9e-13 from the
+// dense one by the chain, 6.4e-13 with composites, and the residual of a solve from x0 = 1 3e-7 / 1e-5; N = 2048,
+// entries to 330: 1.1e-13 both.)
+constexpr double kComposeMost = 512.0;
 std::vector<std::pair<int, int>> level_groups(const Handle &h, const int (&lo)[2], const bool (&on)[2]) {
     const Plan &P = h.plan;
     std::vector<std::pair<int, int>> G;
@@ -1696,7 +1703,7 @@ void assemble_operators(Handle &h, double t0) {
     // composite transfers of the groups of several levels: per box c at T the blocks of all its ancestors of
     // the group side by side (down), per box above T - 1 its descendants' blocks transposed (up; at T - 1
     // that is the transfer itself)
-    const auto groups = level_groups(h, nfam_lo, fam_on);
+    auto groups = level_groups(h, nfam_lo, fam_on);
     auto ancestor = [&](int c, int T, int j) { return c >> (P.dim * (T - j)); };
     auto first_at = [&](int b, int j, int T) { return (int)((int64_t)b << (P.dim * (T - j))); };
     auto rank_at = [&](int f, int b, int j, int T) {
@@ -1891,7 +1898,11 @@ void assemble_operators(Handle &h, double t0) {
     // composite transfers, level by level away from T (block (c, a) from block (c, a's child))
     DevBuf<double> comp_lo;
     comp_lo.alloc(comp_len);
-    for (auto [T, B] : groups)
+    DevBuf<unsigned long long> comp_most;
+    comp_most.alloc(1);
+    std::vector<std::pair<int, int>> kept;
+    for (auto [T, B] : groups) {
+        int low = T - 1;  // the group's levels from here on are kept
         for (int j = T - 1; j >= B && B < T - 1; --j) {
             std::vector<ComposeJob> jobs;
             for (int f = 0; f < 2; ++f) {
@@ -1931,10 +1942,19 @@ void assemble_operators(Handle &h, double t0) {
             }
             DevBuf<ComposeJob> dj;
             dj.upload(jobs, s);
-            launch_compose(dj.p, (int)jobs.size(), h.mat64.p, comp_lo.p, comp0, s);
+            H2W_HIP(hipMemsetAsync(comp_most.p, 0, 8, s));
+            launch_compose(dj.p, (int)jobs.size(), h.mat64.p, comp_lo.p, comp0, comp_most.p, s);
             H2W_HIP(hipGetLastError());
+            double most;
+            H2W_HIP(hipMemcpyAsync(&most, comp_most.p, 8, hipMemcpyDeviceToHost, s));
             H2W_HIP(hipStreamSynchronize(s));
+            if (j < T - 1 && most > kComposeMost) break;
+            low = j;
         }
+        kept.push_back({T, low});
+        for (int q = low; q > B; --q) kept.push_back({q, q - 1});
+    }
+    groups = std::move(kept);
     comp_lo.release();
     phase("transfer operators");
     {
@@ -2265,7 +2285,7 @@ void run_launches_eager(Handle &h, int precision) {
 // A replay costs the host about 6 us more than its first kernel alone, each plain launch 4.7 us, which pass
 // while the GPU works on the launches before it: the graph is for sequences that run faster than the host
 // can launch them.  (Plain launches against replays, whole products: 1D N = 2048, 5 launches 37 / 45 us, its
-// inner operator's 11 launches 81 / 64 us; 1D N = 250000, 11 launches 169 / 174 us; 3D N = 20011 220 / 224 us.)
+// inner operator's 11 launches 81 / 64 us; 3D N = 20011 220 / 224 us.)
 bool replay_pays(Handle &h, int precision) {
     const auto &L = launches_for(h, precision);
     const auto &e = precision == H2W_FP32_INNER ? h.inner.elems : h.launch_elems;

@@ -862,9 +862,11 @@ __global__ __launch_bounds__(64) void k_cur(const CurJob *__restrict__ jobs, con
 // above one whose products cancel, so the products are carried as unevaluated pairs (lo: the low parts of the
 // blocks from offset lo0 on) and rounded once: with plain products the operator of a 1D system with
 // N = 250000 was four times further from the dense one (1.2e-12 for 3.3e-13).
+// most receives the largest entry, by which the caller decides whether the products are used.
 __global__ __launch_bounds__(256) void k_compose(const ComposeJob *__restrict__ jobs, double *A, double *lo,
-                                                 int64_t lo0) {
+                                                 int64_t lo0, unsigned long long *most) {
     const ComposeJob jb = jobs[blockIdx.x];
+    double mc = 0.0;
     for (int e = threadIdx.x; e < jb.m * jb.n; e += 256) {
         const int i = e % jb.m, j = e / jb.m;
         double v = jb.k == 0 ? A[jb.a + (int64_t)j * jb.lda + i] : 0.0, r = 0.0;
@@ -880,7 +882,11 @@ __global__ __launch_bounds__(256) void k_compose(const ComposeJob *__restrict__ 
         A[jb.d + (int64_t)j * jb.ldd + i] = h;
         lo[jb.d - lo0 + (int64_t)j * jb.ldd + i] = (v - h) + r;
         if (jb.dt >= 0) A[jb.dt + (int64_t)i * jb.ldt + j] = h;
+        mc = fmax(mc, fabs(h));
     }
+    // the largest entry (the bits of doubles that are not negative are in their order)
+    for (int o = 32; o > 0; o >>= 1) mc = fmax(mc, __shfl_xor(mc, o, 64));
+    if ((threadIdx.x & 63) == 0) atomicMax(most, (unsigned long long)__double_as_longlong(mc));
 }
 
 // ------------------------------------------------------------------ batched skinny GEMV
@@ -2420,8 +2426,9 @@ static void launch_bgemv_t(const GItem *items, int nitems, const GTerm *terms, c
     else if (role == 2) launch_bgemv_r<T, 2>(items, nitems, terms, A0, A1, vec, unr, per_wave, s);
     else launch_bgemv_r<T, 0>(items, nitems, terms, A0, A1, vec, unr, per_wave, s);
 }
-void launch_compose(const ComposeJob *jobs, int njobs, double *A, double *lo, int64_t lo0, hipStream_t s) {
-    if (njobs > 0) hipLaunchKernelGGL(k_compose, dim3(njobs), dim3(256), 0, s, jobs, A, lo, lo0);
+void launch_compose(const ComposeJob *jobs, int njobs, double *A, double *lo, int64_t lo0, unsigned long long *most,
+                    hipStream_t s) {
+    if (njobs > 0) hipLaunchKernelGGL(k_compose, dim3(njobs), dim3(256), 0, s, jobs, A, lo, lo0, most);
 }
 void launch_copy32(const CopyJob *jobs, int njobs, const float *src, float *dst, hipStream_t s) {
     if (njobs > 0) hipLaunchKernelGGL(k_copy32, dim3(njobs), dim3(256), 0, s, jobs, src, dst);
