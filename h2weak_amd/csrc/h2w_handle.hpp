@@ -235,7 +235,7 @@ inline void app_rot(double &dx, double &dy, double cs, double sn) {
 
 // device work buffers of a lockstep solve
 struct LockBufs {
-    DevBuf<double> V, w, r, d, b, part, h, sc;
+    DevBuf<double> V, w, r, d, b, part, h, sc, mask;
     DevBuf<double> spart, sh;  // shared-space dot products: per-block partials, reduced (2 passes)
     PinBuf pin;  // read-backs of the Hessenberg columns
     int64_t Vcols = 0;

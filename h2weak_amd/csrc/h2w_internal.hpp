@@ -342,7 +342,10 @@ void launch_bdot16_reduce(const double *partial, int nblk, int k, const int32_t 
                           hipStream_t s);
 void launch_bgemv16(const double *V, int64_t ldv, int k, const double *h, int S, double sign, double *w, int64_t n,
                     const int32_t *seg, hipStream_t s);
-void launch_bscale16(const double *src, const double *sc, double *dst, int64_t n, const int32_t *seg, hipStream_t s);
+void launch_bsub_dot16(const double *V, int64_t ldv, int k, const double *h, int S, double *w, int nd, const int2 *blk,
+                       int nblk, const int32_t *seg, double *partial, hipStream_t s);
+void launch_bscale16(const double *src, const double *sc, const double *norm2, double *dst, int64_t n,
+                     const int32_t *seg, hipStream_t s);
 
 // complex kernels (complex.hip): operator and vector pools of double2 (re, im), element offsets as
 // in the real path

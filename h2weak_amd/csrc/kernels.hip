@@ -2135,6 +2135,62 @@ __global__ __launch_bounds__(256) void k_bgemv16(const double *__restrict__ V, i
         w[e] += sign * acc;
     }
 }
+// A subtraction and the dot products that follow it in the Arnoldi process, in one pass over a block's slots:
+// w(t, r) -= sum_{l < k} V_l(t, r) h(l, s, r), then partial as k_bdot16's for the nd columns of V, or of w with
+// itself (nd = 0).  A thread's entries share one column, so its products need no exchange until the end, and it
+// reads back only entries of w that it wrote.  Bound by the reads of V: 14 columns of 55000 slots take 33 us, as the
+// subtraction and the dots in two launches do (17 each); without dots, for the norm, 20 us.  (The entries of 24
+// columns kept in registers between the two: two waves per SIMD, 2% slower solves.)
+__global__ __launch_bounds__(256) void k_bsub_dot16(const double *__restrict__ V, int64_t ldv, int k,
+                                                    const double *__restrict__ h, int S, double *w, int nd,
+                                                    const int2 *__restrict__ blk, const int32_t *__restrict__ seg,
+                                                    double *__restrict__ partial) {
+    const int b = blockIdx.x, nblk = gridDim.x;
+    const int2 rg = blk[b];
+    const int r = threadIdx.x & 15, wv = threadIdx.x >> 6;
+    const int64_t e0 = (int64_t)rg.x * kNR + threadIdx.x, e1 = (int64_t)rg.y * kNR;
+    const int64_t col = (seg ? (int64_t)seg[rg.x] * kNR : 0) + r;
+    for (int64_t e = e0; e < e1; e += 1024) {
+        double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+        for (int l = 0; l < k; ++l) {
+            const double c = h[(int64_t)l * S * kNR + col];
+            const double *v = V + (int64_t)l * ldv;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) acc[u] = fma(v[min(e + 256 * u, e1 - 1)], c, acc[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (e + 256 * u < e1) w[e + 256 * u] -= acc[u];
+    }
+    constexpr int kG = 4, kL = 16;  // columns at a time, columns per round of LDS
+    __shared__ double sh[4][kL][kNR];
+    const int nt = nd > 0 ? nd : 1;
+    for (int j0 = 0; j0 < nt; j0 += kL) {
+        for (int j1 = j0; j1 < min(j0 + kL, nt); j1 += kG) {
+            double acc[kG] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+            for (int64_t e = e0; e < e1; e += 256) {
+                const double x = w[e];
+#pragma unroll
+                for (int u = 0; u < kG; ++u)
+                    acc[u] = fma(nd > 0 ? V[(int64_t)min(j1 + u, nd - 1) * ldv + e] : x, x, acc[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < kG; ++u) {
+                acc[u] += __shfl_xor(acc[u], 16, 64);
+                acc[u] += __shfl_xor(acc[u], 32, 64);
+                if ((threadIdx.x & 63) < 16) sh[wv][j1 - j0 + u][r] = acc[u];
+            }
+        }
+        __syncthreads();
+        for (int q = threadIdx.x; q < min(kL, nt - j0) * kNR; q += 256) {
+            const int j = q / kNR, c = q % kNR;
+            partial[((int64_t)(j0 + j) * nblk + b) * kNR + c] = sh[0][j][c] + sh[1][j][c] + sh[2][j][c] + sh[3][j][c];
+        }
+        __syncthreads();
+    }
+}
 // A space shared by every column of a one-system lockstep vector (the deflation space): k vectors
 // of n slots, stored row-major (Cs[t * k + q]), so that the k values of a slot are contiguous.
 // Both products with it are tall-skinny GEMMs and run on the FP64 matrix cores (16x16x4 MFMA:
@@ -2273,11 +2329,15 @@ __global__ void k_to_rowmajor(const double *__restrict__ src, int64_t n, int k, 
         dst[e] = src[(e % k) * n + e / k];
 }
 
-// dst(t, r) = sc(seg(t), r) * src(t, r)
-__global__ void k_bscale16(const double *__restrict__ src, const double *__restrict__ sc, double *dst, int64_t n,
-                           const int32_t *__restrict__ seg) {
-    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n * kNR; e += (int64_t)gridDim.x * blockDim.x)
-        dst[e] = sc[(seg ? (int64_t)seg[e / kNR] * kNR : 0) + (e % kNR)] * src[e];
+// dst(t, r) = sc(seg(t), r) * src(t, r), or with norm2 that over sqrt(norm2(seg(t), r)), zero where either is zero
+__global__ void k_bscale16(const double *__restrict__ src, const double *__restrict__ sc,
+                           const double *__restrict__ norm2, double *dst, int64_t n, const int32_t *__restrict__ seg) {
+    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n * kNR; e += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t c = (seg ? (int64_t)seg[e / kNR] * kNR : 0) + (e % kNR);
+        double f = sc[c];
+        if (norm2) f = f != 0.0 && norm2[c] > 0.0 ? f / sqrt(norm2[c]) : 0.0;
+        dst[e] = f * src[e];
+    }
 }
 
 
@@ -2628,8 +2688,13 @@ void launch_supd16(const double *Cs, int k, const double *h, int S, double sign,
 void launch_to_rowmajor(const double *src, int64_t n, int k, double *dst, hipStream_t s) {
     if (k > 0) hipLaunchKernelGGL(k_to_rowmajor, dim3(grid_for(n * k, 256, 4096)), dim3(256), 0, s, src, n, k, dst);
 }
-void launch_bscale16(const double *src, const double *sc, double *dst, int64_t n, const int32_t *seg, hipStream_t s) {
-    hipLaunchKernelGGL(k_bscale16, dim3(grid_for(n * kNR)), dim3(256), 0, s, src, sc, dst, n, seg);
+void launch_bsub_dot16(const double *V, int64_t ldv, int k, const double *h, int S, double *w, int nd, const int2 *blk,
+                       int nblk, const int32_t *seg, double *partial, hipStream_t s) {
+    hipLaunchKernelGGL(k_bsub_dot16, dim3(nblk), dim3(256), 0, s, V, ldv, k, h, S, w, nd, blk, seg, partial);
+}
+void launch_bscale16(const double *src, const double *sc, const double *norm2, double *dst, int64_t n,
+                     const int32_t *seg, hipStream_t s) {
+    hipLaunchKernelGGL(k_bscale16, dim3(grid_for(n * kNR)), dim3(256), 0, s, src, sc, norm2, dst, n, seg);
 }
 void launch_map_in64(const double *X, const int32_t *map, int64_t n, double *pool, hipStream_t s) {
     hipLaunchKernelGGL(k_map_in<double>, dim3(grid_for(n * kNR)), dim3(256), 0, s, X, map, n, pool);

@@ -175,7 +175,7 @@ void lscale(Lockstep &L, const std::vector<double> &sc, const double *src, doubl
     LockBufs &B = *L.buf;
     B.sc.ensure(sc.size());
     H2W_HIP(hipMemcpyAsync(B.sc.p, sc.data(), sc.size() * 8, hipMemcpyHostToDevice, L.s));
-    launch_bscale16(src, B.sc.p, dst, L.n, L.seg, L.s);
+    launch_bscale16(src, B.sc.p, nullptr, dst, L.n, L.seg, L.s);
 }
 
 void ensure_V(Lockstep &L, int64_t cols) {
@@ -287,31 +287,54 @@ LockOut lock_gmres(Lockstep &L, const double *b, double *x, const std::vector<ch
     lscale(L, tmp, r, B.V.p + (int64_t)kc * len);
     double *hh = B.pin.ensure((size_t)(2 * (kc + m + 2) + 2) * C + (size_t)2 * ks * C);
     int last = 0;
+    // The next step's vectors need the norms only, which the device has: they are scaled there (by mask, 0 for
+    // columns that stopped in an earlier step) and their product is queued before the host has read this step's
+    // coefficients, unless every running column, its residual shrinking as in the step before, would reach its
+    // tolerance.  (Read, rotated, scaled from the host first: 65 us of idle GPU per step.)
+    bool ahead = false, fresh = false;
+    std::vector<double> mask(C), res2(C, 0.0);
+    Event read;
+    B.mask.ensure(C);
     for (int i = 0; i < m && nrun > 0; ++i) {
         ensure_V(L, kc + i + 2);
         double *Cb = B.V.p, *V = B.V.p + (int64_t)kc * len;
-        L.matvec(V + (int64_t)i * len, w, prec);
+        if (!ahead) L.matvec(V + (int64_t)i * len, w, prec);
         out.matvecs++;
         const int k = kc + i + 1;  // vectors orthogonalised against: C, v_0 .. v_i (contiguous)
         // classical Gram-Schmidt twice; the shared space's dot products come from the same w
-        for (int pass = 0; pass < 2; ++pass) {
-            launch_bdot16(Cb, len, k, w, L.blk, L.nblk, B.part.p, s);
-            launch_bdot16_reduce(B.part.p, L.nblk, k, L.sblk, L.S, B.h.p + (size_t)pass * k * C, s);
-            if (ks > 0 && pass == 0) {
-                // (the shared space spans approximate eigenvectors: one pass against it, as the
-                // single-vector solve does)
-                launch_sdot16(L.dC, ks, w, L.blk, L.nblk, B.spart.p, s);
-                launch_bdot16_reduce(B.spart.p, L.nblk, ks, L.sblk, L.S, B.sh.p, s);
-                launch_supd16(L.dC, ks, B.sh.p, L.S, -1.0, w, L.n, L.seg, s);
-            }
-            launch_bgemv16(Cb, len, k, B.h.p + (size_t)pass * k * C, L.S, -1.0, w, L.n, L.seg, s);
+        double *h1 = B.h.p, *h2 = h1 + (size_t)k * C, *nn = h2 + (size_t)k * C;
+        launch_bdot16(Cb, len, k, w, L.blk, L.nblk, B.part.p, s);
+        launch_bdot16_reduce(B.part.p, L.nblk, k, L.sblk, L.S, h1, s);
+        if (ks > 0) {
+            // (the shared space spans approximate eigenvectors: one pass against it, as the
+            // single-vector solve does)
+            launch_sdot16(L.dC, ks, w, L.blk, L.nblk, B.spart.p, s);
+            launch_bdot16_reduce(B.spart.p, L.nblk, ks, L.sblk, L.S, B.sh.p, s);
+            launch_supd16(L.dC, ks, B.sh.p, L.S, -1.0, w, L.n, L.seg, s);
         }
-        launch_bdot16(w, 0, 1, w, L.blk, L.nblk, B.part.p, s);
-        launch_bdot16_reduce(B.part.p, L.nblk, 1, L.sblk, L.S, B.h.p + (size_t)2 * k * C, s);
+        launch_bsub_dot16(Cb, len, k, h1, L.S, w, k, L.blk, L.nblk, L.seg, B.part.p, s);
+        launch_bdot16_reduce(B.part.p, L.nblk, k, L.sblk, L.S, h2, s);
+        launch_bsub_dot16(Cb, len, k, h2, L.S, w, 0, L.blk, L.nblk, L.seg, B.part.p, s);
+        launch_bdot16_reduce(B.part.p, L.nblk, 1, L.sblk, L.S, nn, s);
         H2W_HIP(hipMemcpyAsync(hh, B.h.p, (size_t)(2 * k + 1) * C * 8, hipMemcpyDeviceToHost, s));
         double *shh = hh + (size_t)(2 * k + 1) * C;
         if (ks > 0) H2W_HIP(hipMemcpyAsync(shh, B.sh.p, (size_t)ks * C * 8, hipMemcpyDeviceToHost, s));
-        H2W_HIP(hipStreamSynchronize(s));
+        H2W_HIP(hipEventRecord(read, s));
+        ahead = false;
+        for (int c = 0; c < C && i + 1 < m; ++c) {
+            const double r1 = out.resid[c], guess = res2[c] > r1 ? r1 * (r1 / res2[c]) : r1;
+            ahead = ahead || (run[c] && !(guess < tol[c]));
+        }
+        if (ahead) {
+            if (!fresh) {
+                for (int c = 0; c < C; ++c) mask[c] = run[c];
+                H2W_HIP(hipMemcpyAsync(B.mask.p, mask.data(), (size_t)C * 8, hipMemcpyHostToDevice, s));
+                fresh = true;
+            }
+            launch_bscale16(w, B.mask.p, nn, V + (int64_t)(i + 1) * len, L.n, L.seg, s);
+            L.matvec(V + (int64_t)(i + 1) * len, w, prec);
+        }
+        H2W_HIP(hipEventSynchronize(read));
         last = i;
         H.emplace_back((size_t)(i + 2) * C, 0.0);
         Y.resize((size_t)(i + 1) * C, 0.0);
@@ -334,6 +357,7 @@ LockOut lock_gmres(Lockstep &L, const double *b, double *x, const std::vector<ch
             gen_rot(Hh(c, i, i), Hh(c, i + 1, i), csc[i], snc[i]);
             app_rot(Hh(c, i, i), Hh(c, i + 1, i), csc[i], snc[i]);
             app_rot(svc[i], svc[i + 1], csc[i], snc[i]);
+            res2[c] = out.resid[c];
             out.resid[c] = std::fabs(svc[i + 1]) / normb[c];
             out.iters[c] = i + 1;
             if (out.resid[c] < tol[c] || i == m - 1 || tmp[c] == 0.0) {
@@ -345,11 +369,12 @@ LockOut lock_gmres(Lockstep &L, const double *b, double *x, const std::vector<ch
                 for (int q = 0; q <= i; ++q) Y[(size_t)q * C + c] = y[q];
                 out.conv[c] = out.resid[c] < tol[c];
                 run[c] = 0;
+                fresh = false;
                 if (!hkeep) tmp[c] = 0.0;  // (kept: the column's last basis vector enters C)
                 --nrun;
             }
         }
-        if (nrun > 0 || hkeep) lscale(L, tmp, w, V + (int64_t)(i + 1) * len);
+        if (!ahead && (nrun > 0 || hkeep)) lscale(L, tmp, w, V + (int64_t)(i + 1) * len);
     }
     // x += V Y over the basis vectors the columns used, - U (B Y) with a recycled space
     H2W_HIP(hipMemcpyAsync(B.h.p, Y.data(), (size_t)(last + 1) * C * 8, hipMemcpyHostToDevice, s));
