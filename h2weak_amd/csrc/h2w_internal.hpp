@@ -123,6 +123,7 @@ struct ComposeJob {  // D = A B (m x k times k x n), or D = A (m x n) when k = 0
     int64_t a, b, d, dt;
     int32_t m, k, n, lda, ldb, ldd, ldt, pad;
 };
+static_assert(sizeof(ComposeJob) % 8 == 0, "uploaded behind 8-byte words");
 
 struct CurJob {    // A = (L R)^{-1} K(Ir, V), r x n column-major at a, leading dimension lda
     int64_t ir, v, lr, a;
@@ -183,6 +184,9 @@ struct WideArgs {  // device arrays of one run of the wide cross
     uint32_t *arrived;    // one counter per block, zero between launches
 };
 int wide_tile();          // entries of one tile
+void launch_aca_small(const AcaJob *jobs, int njobs, const int32_t *idx, double *ws, int64_t ws_cap,
+                      unsigned long long *ws_top, int64_t *tab, uint8_t *flags, int32_t *rank, int32_t *status,
+                      int32_t *rowpiv, int32_t *colpiv, KParams kp, double tol, double *hist, hipStream_t s);
 void launch_wide_init(const AcaJob *jobs, const WideBlk *blk, int nb, WideState *state, uint8_t *flags, int64_t *tab,
                       unsigned long long *ws_top, int64_t ws_cap, hipStream_t s);
 // one pivot step of every block (in a block's fixed-rank phase, AcaJob.pad = kfix > 1 steps, without the

@@ -19,6 +19,7 @@
 #include <thread>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <deque>
 #include <chrono>
@@ -175,12 +176,7 @@ struct AcaPool {
     DevBuf<unsigned long long> top;
     int64_t cap = 0;  // doubles
     // the wide cross: tiles, states and partials of a batch, kept over the batches of an assembly
-    DevBuf<WideState> wstate;
-    DevBuf<WideBlk> wblk;
-    DevBuf<int2> wtiles;
-    DevBuf<double> wpart, wdot;
-    DevBuf<uint32_t> warrived;
-    DevBuf<int32_t> wdone;
+    DevBuf<uint8_t> wide;  // a batch's tables and partials of the passes (run_wide), one allocation
     // a batch's jobs, index lists and results, also kept over the assembly's batches
     DevBuf<uint8_t> flags;
     DevBuf<int32_t> idx, rank, stat, rp, cp, prow, pcol;
@@ -303,20 +299,30 @@ void run_wide(Handle &h, const std::vector<AcaJob> &jobs, const std::vector<int>
     const int nrow = (int)rt.size(), ncol = (int)ct.size();
     for (WideBlk &W : wb) W.ct0 += nrow;
     rt.insert(rt.end(), ct.begin(), ct.end());
-    pool.wblk.upload(wb, s);
-    pool.wtiles.upload(rt, s);
-    pool.wstate.ensure(nb);
-    pool.wpart.ensure(std::max<size_t>(4 * rt.size(), 1));
-    pool.wdot.ensure(std::max<int64_t>(pd, 1));
-    pool.wdone.ensure(1);
-    pool.warrived.ensure(nb);
-    H2W_HIP(hipMemsetAsync(pool.warrived.p, 0, nb * sizeof(uint32_t), s));
-    const WideArgs W{pool.wblk.p, pool.wtiles.p, nrow, ncol, pool.wpart.p, pool.wdot.p, pool.warrived.p};
-    DevBuf<WideState> &st = pool.wstate;
-    launch_wide_init(djobs, pool.wblk.p, nb, st.p, dflags, dtab, pool.top.p, pool.cap, s);
+    size_t wlen = 0;
+    auto part = [&](size_t bytes) {
+        const size_t o = wlen;
+        wlen += (bytes + 255) / 256 * 256;
+        return o;
+    };
+    const size_t o_blk = part(nb * sizeof(WideBlk)), o_tiles = part(rt.size() * sizeof(int2)),
+                 o_state = part(nb * sizeof(WideState)), o_part = part(rt.size() * 32), o_dot = part(pd * 8),
+                 o_done = part(4), o_arr = part(nb * 4);
+    pool.wide.ensure(std::max<size_t>(wlen, 256));
+    WideBlk *dblk = reinterpret_cast<WideBlk *>(pool.wide.p + o_blk);
+    int2 *dtiles = reinterpret_cast<int2 *>(pool.wide.p + o_tiles);
+    WideState *dst = reinterpret_cast<WideState *>(pool.wide.p + o_state);
+    int32_t *ddone = reinterpret_cast<int32_t *>(pool.wide.p + o_done);
+    uint32_t *darr = reinterpret_cast<uint32_t *>(pool.wide.p + o_arr);
+    H2W_HIP(hipMemcpyAsync(dblk, wb.data(), nb * sizeof(WideBlk), hipMemcpyHostToDevice, s));
+    if (!rt.empty()) H2W_HIP(hipMemcpyAsync(dtiles, rt.data(), rt.size() * sizeof(int2), hipMemcpyHostToDevice, s));
+    H2W_HIP(hipMemsetAsync(darr, 0, nb * sizeof(uint32_t), s));
+    const WideArgs W{dblk, dtiles, nrow, ncol, reinterpret_cast<double *>(pool.wide.p + o_part),
+                     reinterpret_cast<double *>(pool.wide.p + o_dot), darr};
+    launch_wide_init(djobs, dblk, nb, dst, dflags, dtab, pool.top.p, pool.cap, s);
     auto step = [&]() {
         if (nrow > 0 && ncol > 0)
-            launch_wide_step(djobs, W, didx, pool.ws.p, dtab, dflags, st.p, drp, dcp, dhist, pool.top.p, pool.cap, h.kp,
+            launch_wide_step(djobs, W, didx, pool.ws.p, dtab, dflags, dst, drp, dcp, dhist, pool.top.p, pool.cap, h.kp,
                              tol, s);
     };
     // (the step after the last accepted one is taken beside its inner products)
@@ -330,7 +336,7 @@ void run_wide(Handle &h, const std::vector<AcaJob> &jobs, const std::vector<int>
         while (true) {
             for (int64_t c = 0; c < todo; ++c, ++steps) step();
             H2W_HIP(hipGetLastError());
-            H2W_HIP(hipMemcpyAsync(hs.data(), st.p, (size_t)nb * sizeof(WideState), hipMemcpyDeviceToHost, s));
+            H2W_HIP(hipMemcpyAsync(hs.data(), dst, (size_t)nb * sizeof(WideState), hipMemcpyDeviceToHost, s));
             H2W_HIP(hipStreamSynchronize(s));
             int running = 0;
             for (auto &w : hs) running += !w.done;
@@ -358,7 +364,7 @@ void run_wide(Handle &h, const std::vector<AcaJob> &jobs, const std::vector<int>
             DevBuf<double> dprod;
             dgj.upload(gj, s);
             dprod.alloc(std::max<int64_t>(plen, 1));
-            launch_wide_gram(dgj.p, (int)gj.size(), djobs, st.p, pool.ws.p, dtab, dprod.p, s);
+            launch_wide_gram(dgj.p, (int)gj.size(), djobs, dst, pool.ws.p, dtab, dprod.p, s);
             H2W_HIP(hipGetLastError());
             std::vector<double> prod(plen);
             H2W_HIP(hipMemcpyAsync(prod.data(), dprod.p, plen * 8, hipMemcpyDeviceToHost, s));
@@ -406,16 +412,18 @@ void run_wide(Handle &h, const std::vector<AcaJob> &jobs, const std::vector<int>
             DevBuf<double> dnrm;
             dfin.upload(fin, s);
             dnrm.upload(nrm, s);
-            launch_wide_judge(djobs, pool.wblk.p, nb, st.p, dfin.p, dnrm.p, dtab, pool.top.p, pool.cap, s);
+            launch_wide_judge(djobs, dblk, nb, dst, dfin.p, dnrm.p, dtab, pool.top.p, pool.cap, s);
             H2W_HIP(hipGetLastError());
             H2W_HIP(hipStreamSynchronize(s));
         }
     }
     while (true) {
-        launch_wide_finish(st.p, nb, drank, dstat, pool.wdone.p, s);
+        if (steps == 0)
+            for (int c = 0; c < 16; ++c, ++steps) step();
+        launch_wide_finish(dst, nb, drank, dstat, ddone, s);
         H2W_HIP(hipGetLastError());
         int nd = 0;
-        H2W_HIP(hipMemcpyAsync(&nd, pool.wdone.p, 4, hipMemcpyDeviceToHost, s));
+        H2W_HIP(hipMemcpyAsync(&nd, ddone, 4, hipMemcpyDeviceToHost, s));
         H2W_HIP(hipStreamSynchronize(s));
         if (nd == nb) break;
         if (steps > limit) throw Error{H2W_EHIP, "wide cross did not finish within its step bound"};
@@ -511,6 +519,13 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
     // its judgement costs host work per block, which small blocks do not repay
     const size_t kHuge = cx ? SIZE_MAX
                             : std::getenv("H2W_WIDE_MIN") ? (size_t)std::atoll(std::getenv("H2W_WIDE_MIN")) : 8192;
+    // m + n up to which a batch's blocks take every step in one launch, a workgroup each (k_aca_small): a step there
+    // is shorter than two launches, while a workgroup alone is slower on longer rows (blocks of m + n above 8192
+    // for a fixed-rank phase never are).  Assemblies, all in tiles / to 256 / 512 / 1024 / 2048: 1D N = 1584 at 1e-12
+    // 6.4 / 5.4 / 5.1 / 4.9 / 5.4 ms, 1D N = 8000 11.4 / 10.7 / 10.0 / 9.9 / 9.9, 2D N = 1600 8.6 / 7.4 / 7.2 / 7.0 /
+    // 7.0, 2D N = 4000 14.0 / 13.8 / 13.7 / 14.0 / 19.6, 3D N = 2000 9.4 / 9.1 / 8.2 / 10.1 / 10.8.  (1D ranks are 20
+    // to 40, so that longer rows are still cheap to a workgroup alone.)
+    const size_t kSmall = h.plan.dim == 1 ? 1024 : 512;
     while (!todo.empty()) {
         std::vector<size_t> rerun;
         size_t pos = 0;
@@ -559,6 +574,9 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
                 J.piv = po;
                 po += J.tcap;
             }
+            bool small = !cx;
+            for (size_t q = 0; q < batch.size() && small; ++q)
+                small = mn_of(batch[q]) <= std::min(kSmall, kHuge) && jobs[q].pad <= 1;
             flags.ensure(std::max<int64_t>(fo, 1));
             dtab.ensure(std::max<int64_t>(to, 1));
             didx.upload(idx, s);
@@ -579,6 +597,9 @@ void run_aca(Handle &h, std::vector<AcaBlock> &blocks, int rank_hint, AcaPool &p
                 if (batch.size() > nbig)
                     launch_aca_c(djobs.p + nbig, (int)(batch.size() - nbig), didx.p, wsc, pool.cap / 2, pool.top.p,
                                  dtab.p, flags.p, drank.p + nbig, dstat.p + nbig, drp.p, dcp.p, h.kpc, tol, dhist.p, 0, s);
+            } else if (small) {
+                launch_aca_small(djobs.p, (int)batch.size(), didx.p, pool.ws.p, pool.cap, pool.top.p, dtab.p, flags.p,
+                                 drank.p, dstat.p, drp.p, dcp.p, h.kp, tol, dhist.p, s);
             } else {
                 std::vector<int> best(batch.size());
                 for (size_t q = 0; q < batch.size(); ++q) best[q] = est[batch[q]];
@@ -1131,7 +1152,7 @@ int inner_rank(const std::vector<double> &hist, int rank, double tau) {
 //   fused, 4096 / 2048 / 1024 items: 32^3 grid at 1e-10 492, 452 / 448 / 458 us, 3D N = 20011 231, 229 / 204 / 202,
 //     2D N = 90000 317, 297 / 292 / 304;
 //   transfers of a product, 128 / 256 / 512 columns: 32^3 188, 168 / 161 / 154 us, 3D N = 20011 114, 106 / 102 / 101,
-//     2D N = 90000 369, 352 / 348 / 352, 2D semi-nested 400 x 400 156, 156 / 157 / 158, 16^3 55, 55 / 56 / 59.
+//     2D N = 90000 369, 352 / 348 / 352, 2D semi-nested N = 40000 156, 156 / 157 / 158, 16^3 55, 55 / 56 / 59.
 //     (By elements instead, a 512th of the launch: the semi-nested one, a few tall boxes among many, 172.)
 // Returns the number of items appended; 0 where nothing combines.
 int64_t wide_items(std::vector<GItem> &items, int64_t item0, const std::vector<GTerm> &terms, int role) {
@@ -1896,15 +1917,11 @@ void assemble_operators(Handle &h, double t0) {
         H2W_HIP(hipStreamSynchronize(s));
     }
     // composite transfers, level by level away from T (block (c, a) from block (c, a's child))
-    DevBuf<double> comp_lo;
-    comp_lo.alloc(comp_len);
-    DevBuf<unsigned long long> comp_most;
-    comp_most.alloc(1);
-    std::vector<std::pair<int, int>> kept;
-    for (auto [T, B] : groups) {
-        int low = T - 1;  // the group's levels from here on are kept
+    std::vector<ComposeJob> jobs;
+    std::vector<std::array<int64_t, 3>> comp_runs;  // level, its jobs
+    for (auto [T, B] : groups)
         for (int j = T - 1; j >= B && B < T - 1; --j) {
-            std::vector<ComposeJob> jobs;
+            const int64_t job0 = (int64_t)jobs.size();
             for (int f = 0; f < 2; ++f) {
                 if (!fam_on[f] || j < nfam_lo[f]) continue;
                 const FamLevel &fl = h.fam[f][j], &ft = h.fam[f][T];
@@ -1940,22 +1957,32 @@ void assemble_operators(Handle &h, double t0) {
                     jobs.push_back(J);
                 }
             }
-            DevBuf<ComposeJob> dj;
-            dj.upload(jobs, s);
-            H2W_HIP(hipMemsetAsync(comp_most.p, 0, 8, s));
-            launch_compose(dj.p, (int)jobs.size(), h.mat64.p, comp_lo.p, comp0, comp_most.p, s);
-            H2W_HIP(hipGetLastError());
-            double most;
-            H2W_HIP(hipMemcpyAsync(&most, comp_most.p, 8, hipMemcpyDeviceToHost, s));
-            H2W_HIP(hipStreamSynchronize(s));
-            if (j < T - 1 && most > kComposeMost) break;
-            low = j;
+            comp_runs.push_back({j, job0, (int64_t)jobs.size()});
         }
-        kept.push_back({T, low});
-        for (int q = low; q > B; --q) kept.push_back({q, q - 1});
+    if (!jobs.empty()) {
+        // one scratch allocation: the blocks' low parts, the largest entry of each level, the jobs
+        const int64_t nj = (int64_t)(jobs.size() * sizeof(ComposeJob) / 8);
+        DevBuf<double> scratch;
+        scratch.alloc(comp_len + P.nL + 1 + nj);
+        unsigned long long *comp_most = reinterpret_cast<unsigned long long *>(scratch.p + comp_len);
+        ComposeJob *dj = reinterpret_cast<ComposeJob *>(comp_most + P.nL + 1);
+        H2W_HIP(hipMemcpyAsync(dj, jobs.data(), (size_t)nj * 8, hipMemcpyHostToDevice, s));
+        H2W_HIP(hipMemsetAsync(comp_most, 0, (P.nL + 1) * 8, s));
+        for (auto &r : comp_runs)
+            launch_compose(dj + r[1], (int)(r[2] - r[1]), h.mat64.p, scratch.p, comp0, comp_most + r[0], s);
+        H2W_HIP(hipGetLastError());
+        std::vector<double> most(P.nL + 1);
+        H2W_HIP(hipMemcpyAsync(most.data(), comp_most, (P.nL + 1) * 8, hipMemcpyDeviceToHost, s));
+        H2W_HIP(hipStreamSynchronize(s));
+        std::vector<std::pair<int, int>> kept;
+        for (auto [T, B] : groups) {
+            int low = T - 1;  // the group's levels from here on are kept
+            while (low > B && most[low - 1] <= kComposeMost) --low;
+            kept.push_back({T, low});
+            for (int q = low; q > B; --q) kept.push_back({q, q - 1});
+        }
+        groups = std::move(kept);
     }
-    groups = std::move(kept);
-    comp_lo.release();
     phase("transfer operators");
     {
         // plain entry blocks: M2L, near field, semi-nested column factors

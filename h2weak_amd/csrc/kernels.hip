@@ -159,15 +159,242 @@ __device__ __forceinline__ void block_reduce(BlockRed<NT> &sh, double &s0, doubl
 // ones near the leaves, so only all blocks together fill the chip at every level.
 // (One workgroup per block, with only the blocks of m + n > 8192 spread: the vertex
 // level of 64 blocks of m + n up to 8192 took 208 ms at N = 20011, now 13 ms for its
-// 272 steps; assemblies 572 -> 180 ms there, 32^3 grid at tol 1e-10 2440 -> 560 ms.
-// With a workgroup per block kept below m + n = 512, 2048, 8192: 194, 280, 478 ms at
-// N = 20011; 2D N = 40000 95, 102, 136 ms; 1D N = 65536 57, 63, 80 ms against 60 ms
-// with every block spread: the one-workgroup form is gone.)
+// 272 steps; assemblies 572 -> 180 ms there, 32^3 grid at tol 1e-10 2440 -> 560 ms.)
+// Batches of small blocks only keep that form (k_aca_small).
 // U and V columns live in a workspace pool shared by the batch: each step reserves
 // a column pair with an atomic bump; the column offsets go to the job's table.
 // Per-block state lives in WideState; a finished block (converged, exhausted, or out
 // of workspace: status 1, re-run by the host) is skipped by every later launch.
 constexpr int kChunk = 512;
+
+__device__ __forceinline__ bool aca_reserve(int64_t *tab, int k, int m, int n, int tcap,
+                                            unsigned long long *ws_top, int64_t ws_cap, int64_t *sh_off) {
+    if (threadIdx.x == 0) {
+        int64_t off = -1;
+        if (k < tcap) {
+            unsigned long long o = atomicAdd(ws_top, (unsigned long long)(m + n));
+            if ((int64_t)o + m + n <= ws_cap) off = (int64_t)o;
+        }
+        *sh_off = off;
+        if (off >= 0) {
+            tab[2 * k] = off;
+            tab[2 * k + 1] = off + m;
+        }
+    }
+    __syncthreads();
+    return *sh_off >= 0;
+}
+
+// The same cross with one workgroup per block and every step in one launch, for batches of small blocks (the driver's
+// rule): their steps of two launches are latency, 17 us of launch, state and first loads a step against 10 us here.
+__global__ __launch_bounds__(256) void k_aca_small(const AcaJob *__restrict__ jobs, const int32_t *__restrict__ idx,
+                                            double *__restrict__ ws, int64_t ws_cap, unsigned long long *ws_top,
+                                            int64_t *__restrict__ tab_all, uint8_t *__restrict__ flags,
+                                            int32_t *__restrict__ rank_out, int32_t *__restrict__ status_out,
+                                            int32_t *__restrict__ rowpiv, int32_t *__restrict__ colpiv, KParams kp,
+                                            double tol, double *__restrict__ hist_all) {
+    constexpr int NT = 256;
+    const AcaJob jb = jobs[blockIdx.x];
+    const int m = jb.m, n = jb.n, tcap = jb.tcap;
+    double *hist = hist_all + 2 * jb.piv;  // per accepted step: |u||v|, normS after the step
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    constexpr int NW = NT / 64;
+    const int32_t *rows = idx + jb.rows;
+    const int32_t *cols = idx + jb.cols;
+    int64_t *tab = tab_all + jb.tab;
+    uint8_t *ru = flags + jb.wsF;
+    uint8_t *cu = ru + m;
+    int32_t *rp_out = rowpiv + jb.piv;
+    int32_t *cp_out = colpiv + jb.piv;
+    __shared__ double coef[kChunk];
+    __shared__ int64_t cofs[kChunk];
+    __shared__ BlockRed<NT> red;
+    __shared__ double dacc[NW];
+    __shared__ int64_t sh_off;
+
+    if (m == 0 || n == 0 || tcap == 0) {
+        if (tid == 0) {
+            rank_out[blockIdx.x] = 0;
+            status_out[blockIdx.x] = 0;
+        }
+        return;
+    }
+    for (int i = tid; i < m; i += NT) ru[i] = 0;
+    for (int s = tid; s < n; s += NT) cu[s] = 0;
+    const int mn = min(m, n);
+    if (!aca_reserve(tab, 0, m, n, tcap, ws_top, ws_cap, &sh_off)) {
+        if (tid == 0) {
+            rank_out[blockIdx.x] = 0;
+            status_out[blockIdx.x] = 1;
+        }
+        return;
+    }
+    double *U0 = ws + sh_off;
+    double *V0 = U0 + m;
+
+    // ---- first row with a nonzero entry
+    int l = 0, cp = -1;
+    double piv = 0.0;
+    for (l = 0; l < m; ++l) {
+        PointI pr = load_point(kp, rows[l]);
+        AMax am{-1.0, INT_MAX, 0.0};
+        for (int s = tid; s < n; s += NT) {
+            double v = kentry(kp, pr, cols[s]);
+            V0[s] = v;
+            amax_update(am, v, s);
+        }
+        double d0 = 0.0, d1 = 0.0;
+        block_reduce<NT>(red, d0, d1, am);
+        if (am.idx != INT_MAX && am.a > 1e-36) {
+            cp = am.idx;
+            piv = am.sv;
+            break;
+        }
+    }
+    if (l == m) {
+        if (tid == 0) {
+            rank_out[blockIdx.x] = 0;
+            status_out[blockIdx.x] = 0;
+        }
+        return;
+    }
+    int rp = l;
+    // ---- first column
+    double un2 = 0.0, vn2 = 0.0;
+    AMax an{-1.0, INT_MAX, 0.0};
+    {
+        PointI pc = load_point(kp, cols[cp]);
+        for (int t = tid; t < m; t += NT) {
+            double c = kentry(kp, pc, rows[t]);  // A(rows[t], cols[cp]) (symmetric entry)
+            double u = c / piv;
+            U0[t] = u;
+            un2 += u * u;
+            if (t != rp) amax_update(an, c, t);
+        }
+        for (int s = tid; s < n; s += NT) vn2 += V0[s] * V0[s];
+    }
+    block_reduce<NT>(red, un2, vn2, an);
+    if (tid == 0) {
+        rp_out[0] = rp;
+        cp_out[0] = cp;
+        ru[rp] = 1;
+        cu[cp] = 1;
+    }
+    int rank = 1;
+    int status = 0;
+    double normS = 0.0;
+    double un = sqrt(un2), vn = sqrt(vn2);
+    int next_rp = an.idx;
+    if (tid == 0) {
+        hist[0] = un * vn;
+        hist[1] = 0.0;
+    }
+    __syncthreads();
+
+    while (un * vn > tol * normS && rank < mn) {
+        rp = next_rp;
+        if (rp == INT_MAX) break;
+        if (!aca_reserve(tab, rank, m, n, tcap, ws_top, ws_cap, &sh_off)) {
+            status = 1;
+            break;
+        }
+        double *Ur = ws + sh_off;
+        double *Vr = Ur + m;
+        const int nch = (rank + kChunk - 1) / kChunk;
+        // ---- residual row -> V column `rank`
+        PointI pr = load_point(kp, rows[rp]);
+        AMax am{-1.0, INT_MAX, 0.0};
+        vn2 = 0.0;
+        for (int ch = 0; ch < nch; ++ch) {
+            const int l0 = ch * kChunk, l1 = min(rank, l0 + kChunk);
+            for (int q = l0 + tid; q < l1; q += NT) {
+                coef[q - l0] = ws[tab[2 * q] + rp];
+                cofs[q - l0] = tab[2 * q + 1];
+            }
+            __syncthreads();
+            for (int s = tid; s < n; s += NT) {
+                double r = ch == 0 ? kentry(kp, pr, cols[s]) : Vr[s];
+                for (int q = l0; q < l1; ++q) r -= coef[q - l0] * ws[cofs[q - l0] + s];
+                Vr[s] = r;
+                if (ch == nch - 1) {
+                    vn2 += r * r;
+                    if (!cu[s]) amax_update(am, r, s);
+                }
+            }
+            __syncthreads();
+        }
+        double dummy = 0.0;
+        block_reduce<NT>(red, vn2, dummy, am);
+        if (am.idx == INT_MAX) break;
+        cp = am.idx;
+        piv = am.sv;
+        // ---- residual column -> U column `rank`
+        PointI pc = load_point(kp, cols[cp]);
+        an = AMax{-1.0, INT_MAX, 0.0};
+        un2 = 0.0;
+        for (int ch = 0; ch < nch; ++ch) {
+            const int l0 = ch * kChunk, l1 = min(rank, l0 + kChunk);
+            for (int q = l0 + tid; q < l1; q += NT) {
+                coef[q - l0] = ws[tab[2 * q + 1] + cp];
+                cofs[q - l0] = tab[2 * q];
+            }
+            __syncthreads();
+            for (int t = tid; t < m; t += NT) {
+                double c = ch == 0 ? kentry(kp, pc, rows[t]) : Ur[t];
+                for (int q = l0; q < l1; ++q) c -= coef[q - l0] * ws[cofs[q - l0] + t];
+                if (ch == nch - 1) {
+                    double u = c / piv;
+                    Ur[t] = u;
+                    un2 += u * u;
+                    if (t != rp && !ru[t]) amax_update(an, c, t);
+                } else {
+                    Ur[t] = c;
+                }
+            }
+            __syncthreads();
+        }
+        block_reduce<NT>(red, un2, dummy, an);
+        un = sqrt(un2);
+        vn = sqrt(vn2);
+        if (un < 1e-36 || vn < 1e-36) break;
+        if (tid == 0) {
+            rp_out[rank] = rp;
+            cp_out[rank] = cp;
+            ru[rp] = 1;
+            cu[cp] = 1;
+        }
+        ++rank;
+        next_rp = an.idx;
+        // ---- normS update: dots of the new term with every term
+        double acc = 0.0;
+        for (int q = wv; q < rank; q += NW) {
+            const double *Uq = ws + tab[2 * q];
+            const double *Vq = ws + tab[2 * q + 1];
+            double du = 0.0, dv = 0.0;
+            for (int t = lane; t < m; t += 64) du += Uq[t] * Ur[t];
+            for (int s = lane; s < n; s += 64) dv += Vq[s] * Vr[s];
+            du = wave_sum(du);
+            dv = wave_sum(dv);
+            acc += fabs(du * dv);
+        }
+        if (lane == 0) dacc[wv] = acc;
+        __syncthreads();
+        double S = 0.0;
+        for (int q = 0; q < NW; ++q) S += dacc[q];
+        double uv = un * vn;
+        normS = sqrt(normS * normS + uv * uv + 2.0 * S);
+        if (tid == 0) {
+            hist[2 * (rank - 1)] = uv;
+            hist[2 * (rank - 1) + 1] = normS;
+        }
+        __syncthreads();
+    }
+    if (tid == 0) {
+        rank_out[blockIdx.x] = rank;
+        status_out[blockIdx.x] = status;
+    }
+}
+
 
 // A tile of the wide passes: 256 threads x 2 consecutive entries (one 16-byte load per earlier term),
 // kWideU terms in flight twice over: 64 KB of loads outstanding per workgroup.  Large levels are bound by
@@ -1106,7 +1333,7 @@ struct Mfma16<double> {
 // left out, four at a time.  SYM: the transposed products of symmetric terms as well (below).
 // Transfers of a 16-wide product against 128-row items by 4-column chunks from a scalar cursor (FP64, the same
 // lists, then those of wide_items): 32^3 grid at 1e-10 193 -> 187 -> 161 us, 3D N = 20011 148 -> 114 -> 102, 2D
-// N = 90000 422 -> 370 -> 348, 2D semi-nested 400 x 400 207 -> 156, 16^3 77 -> 55, 1D N = 65536 147 -> 110.
+// N = 90000 422 -> 370 -> 348, 2D semi-nested N = 40000 207 -> 156, 16^3 77 -> 55, 1D N = 65536 147 -> 110.
 template <typename T, int VEC, int NG, bool SYM, int WPI>
 __device__ __forceinline__ void bgemm_rows(const GItem &it, int h0, int rows, const GTerm *__restrict__ terms,
                                            const T *__restrict__ A, T *vec, T *smem) {
@@ -2718,6 +2945,13 @@ void launch_scatter_b(const double *v, const int64_t *src, const int32_t *ld, in
 }
 void launch_rank_mlp(const float *feat, int n, const uint16_t *w, float *out, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_rank_mlp, dim3((n + 255) / 256), dim3(256), 0, s, feat, n, w, out);
+}
+void launch_aca_small(const AcaJob *jobs, int njobs, const int32_t *idx, double *ws, int64_t ws_cap,
+                      unsigned long long *ws_top, int64_t *tab, uint8_t *flags, int32_t *rank, int32_t *status,
+                      int32_t *rowpiv, int32_t *colpiv, KParams kp, double tol, double *hist, hipStream_t s) {
+    if (njobs > 0)
+        hipLaunchKernelGGL(k_aca_small, dim3(njobs), dim3(256), 0, s, jobs, idx, ws, ws_cap, ws_top, tab, flags, rank,
+                           status, rowpiv, colpiv, kp, tol, hist);
 }
 void launch_wide_init(const AcaJob *jobs, const WideBlk *blk, int nb, WideState *state, uint8_t *flags, int64_t *tab,
                       unsigned long long *ws_top, int64_t ws_cap, hipStream_t s) {
