@@ -1967,7 +1967,9 @@ void assemble_operators(Handle &h, double t0) {
         unsigned long long *comp_most = reinterpret_cast<unsigned long long *>(scratch.p + comp_len);
         ComposeJob *dj = reinterpret_cast<ComposeJob *>(comp_most + P.nL + 1);
         H2W_HIP(hipMemcpyAsync(dj, jobs.data(), (size_t)nj * 8, hipMemcpyHostToDevice, s));
-        H2W_HIP(hipMemsetAsync(comp_most, 0, (P.nL + 1) * 8, s));
+        // (a block across a box without a skeleton is never formed, but is a factor of the next level's: zero, low
+        // part included)
+        H2W_HIP(hipMemsetAsync(scratch.p, 0, (comp_len + P.nL + 1) * 8, s));
         for (auto &r : comp_runs)
             launch_compose(dj + r[1], (int)(r[2] - r[1]), h.mat64.p, scratch.p, comp0, comp_most + r[0], s);
         H2W_HIP(hipGetLastError());

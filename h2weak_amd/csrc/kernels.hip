@@ -1089,7 +1089,8 @@ __global__ __launch_bounds__(64) void k_cur(const CurJob *__restrict__ jobs, con
 // above one whose products cancel, so the products are carried as unevaluated pairs (lo: the low parts of the
 // blocks from offset lo0 on) and rounded once: with plain products the operator of a 1D system with
 // N = 250000 was four times further from the dense one (1.2e-12 for 3.3e-13).
-// most receives the largest entry, by which the caller decides whether the products are used.
+// most receives the largest entry (infinity for one that is not finite), by which the caller decides whether the
+// products are used.
 __global__ __launch_bounds__(256) void k_compose(const ComposeJob *__restrict__ jobs, double *A, double *lo,
                                                  int64_t lo0, unsigned long long *most) {
     const ComposeJob jb = jobs[blockIdx.x];
@@ -1109,7 +1110,7 @@ __global__ __launch_bounds__(256) void k_compose(const ComposeJob *__restrict__ 
         A[jb.d + (int64_t)j * jb.ldd + i] = h;
         lo[jb.d - lo0 + (int64_t)j * jb.ldd + i] = (v - h) + r;
         if (jb.dt >= 0) A[jb.dt + (int64_t)i * jb.ldt + j] = h;
-        mc = fmax(mc, fabs(h));
+        mc = fabs(h) <= DBL_MAX ? fmax(mc, fabs(h)) : HUGE_VAL;
     }
     // the largest entry (the bits of doubles that are not negative are in their order)
     for (int o = 32; o > 0; o >>= 1) mc = fmax(mc, __shfl_xor(mc, o, 64));
