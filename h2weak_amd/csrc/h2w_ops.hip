@@ -3584,6 +3584,12 @@ int h2w_matvec_ex(h2w_handle *h, const double *x, double *y, int nrhs, int64_t l
             if (ldd == ldv) H2W_HIP(hipMemcpyAsync(d, v, ((nc - 1) * ldv + N) * 8, k, h->stream));
             else H2W_HIP(hipMemcpy2DAsync(d, ldd * 8, v, ldv * 8, N * 8, nc, k, h->stream));
         };
+        // (outputs over the inputs of a later pass: those are read from a copy made before the first)
+        std::vector<double> own;
+        if (where == H2W_HOST && nrhs > h2w::kNR && y > x && y < x + (nrhs - 1) * ld + N) {
+            own.assign(x, x + (nrhs - 1) * ld + N);
+            x = own.data();
+        }
         for (int c0 = 0; c0 < nrhs; c0 += h2w::kNR) {
             const int nc = std::min(h2w::kNR, nrhs - c0);
             const double *xs = x + c0 * ld;
