@@ -100,6 +100,13 @@ void derive_S(Handle &h, int f, int lo) {
     }
 }
 
+// this thread's calls on streams that are not captured, beside captures under way, for the object's lifetime
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { H2W_HIP(hipThreadExchangeStreamCaptureMode(&mode)); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 }  // namespace
 }  // namespace h2w
 
@@ -118,7 +125,13 @@ int h2w_save(const h2w_handle *h, const char *path) {
         const h2w::Plan &P = h->plan;
         std::vector<double> lr(h->d_lr.n);  // L and R of every skeleton
         H2W_HIP(hipSetDevice(h->opts.device));
-        if (!lr.empty()) H2W_HIP(hipMemcpy(lr.data(), h->d_lr.p, lr.size() * 8, hipMemcpyDeviceToHost));
+        if (!lr.empty()) {
+            // The caller, or another thread, may be capturing a graph: the copy and its wait concern the handle's
+            // own stream only, and must not end that capture.
+            h2w::RelaxedCapture relaxed;
+            H2W_HIP(hipMemcpyAsync(lr.data(), h->d_lr.p, lr.size() * 8, hipMemcpyDeviceToHost, h->stream));
+            H2W_HIP(hipStreamSynchronize(h->stream));
+        }
         auto put_lr = [&](int64_t off, int64_t r) {
             if (r > 0) w.raw(lr.data() + off, (size_t)(2 * r * r) * sizeof(double));
         };
