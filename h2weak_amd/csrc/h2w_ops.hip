@@ -2529,7 +2529,7 @@ GmresOut gmres_core(Handle &h, const double *b, double *x, int max_iter, double 
     const bool once = kc > 0 && rc->invariant;
     if (!once) h.gv_defl = -1;  // (its basis overwrites the first columns of g_V)
     const int m = max_iter;
-    CgsArgs A = cgs_args(h, r, kc + m + 2);
+    CgsArgs A = cgs_args(h, r, kc + std::min<int64_t>(m + 1, 32));  // (grows with the basis)
     h.g_h.ensure((size_t)2 * (kc + m + 2) + 2);
     double *hh = h.g_pin.ensure(2 * (kc + m + 2) + 8);
     if (x_zero) {
@@ -2582,6 +2582,7 @@ GmresOut gmres_core(Handle &h, const double *b, double *x, int max_iter, double 
     double res1 = out.resid, res2 = 0.0;  // residuals of the last two steps
     for (int i = 0; i < m; ++i) {
         ensure_V(h, kc + i + 3);
+        A.partial = cgs_args(h, r, h.g_Vcols).partial;
         double *C = h.g_V.p, *V = h.g_V.p + (int64_t)kc * N;
         // w = A v_i: left in the pool (FP64) or taken from there by the first pass (FP32)
         const bool f32 = is32(prec);
