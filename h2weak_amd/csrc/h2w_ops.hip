@@ -3598,8 +3598,8 @@ int h2w_matvec_ex(h2w_handle *h, const double *x, double *y, int nrhs, int64_t l
             int64_t lds = ld;
             if (where == H2W_HOST) {
                 lds = N;
-                h->d_stage_in.ensure((size_t)N * h2w::kNR);
-                h->d_stage_out.ensure((size_t)N * h2w::kNR);
+                h->d_stage_in.ensure((size_t)N * nc);
+                h->d_stage_out.ensure((size_t)N * nc);
                 copy_columns(h->d_stage_in.p, N, xs, ld, nc, hipMemcpyHostToDevice);
                 xs = h->d_stage_in.p;
                 ys = h->d_stage_out.p;
