@@ -319,18 +319,19 @@ LockOut lock_gmres(Lockstep &L, const double *b, double *x, const std::vector<ch
         H2W_HIP(hipMemcpyAsync(hh, B.h.p, (size_t)(2 * k + 1) * C * 8, hipMemcpyDeviceToHost, s));
         double *shh = hh + (size_t)(2 * k + 1) * C;
         if (ks > 0) H2W_HIP(hipMemcpyAsync(shh, B.sh.p, (size_t)ks * C * 8, hipMemcpyDeviceToHost, s));
-        H2W_HIP(hipEventRecord(read, s));
         ahead = false;
         for (int c = 0; c < C && i + 1 < m; ++c) {
             const double r1 = out.resid[c], guess = res2[c] > r1 ? r1 * (r1 / res2[c]) : r1;
             ahead = ahead || (run[c] && !(guess < tol[c]));
         }
+        if (ahead && !fresh) {
+            // (before the event below, whose wait lets a later step write mask again)
+            for (int c = 0; c < C; ++c) mask[c] = run[c];
+            H2W_HIP(hipMemcpyAsync(B.mask.p, mask.data(), (size_t)C * 8, hipMemcpyHostToDevice, s));
+            fresh = true;
+        }
+        H2W_HIP(hipEventRecord(read, s));
         if (ahead) {
-            if (!fresh) {
-                for (int c = 0; c < C; ++c) mask[c] = run[c];
-                H2W_HIP(hipMemcpyAsync(B.mask.p, mask.data(), (size_t)C * 8, hipMemcpyHostToDevice, s));
-                fresh = true;
-            }
             launch_bscale16(w, B.mask.p, nn, V + (int64_t)(i + 1) * len, L.n, L.seg, s);
             L.matvec(V + (int64_t)(i + 1) * len, w, prec);
         }
