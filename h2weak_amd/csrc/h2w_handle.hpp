@@ -96,6 +96,10 @@ struct DevBuf {
     void ensure(size_t cnt) {
         if (cnt > n) alloc(cnt);
     }
+    void swap(DevBuf &o) {
+        std::swap(p, o.p);
+        std::swap(n, o.n);
+    }
     void upload(const std::vector<T> &v, hipStream_t s) {
         ensure(v.size());
         if (!v.empty()) H2W_HIP(hipMemcpyAsync(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, s));

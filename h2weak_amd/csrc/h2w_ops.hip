@@ -1549,7 +1549,7 @@ void build_inner(Handle &h, double irp) {
 
 // ------------------------------------------------------------------ assembly
 
-void assemble_operators(Handle &h, double t0);
+void assemble_operators(Handle &h, double t0, DevBuf<double> &scratch);
 
 void assemble(Handle &h) {
     drop_graphs(h);
@@ -1571,6 +1571,7 @@ void assemble(Handle &h) {
         }
     };
     const Plan &P = h.plan;
+    DevBuf<double> scratch;  // the crosses' workspace, reused
     {
         AcaPool pool;
         if (P.dim >= 2 && h.variant != H2W_NON_NESTED) far_nca(h, pool);
@@ -1588,8 +1589,9 @@ void assemble(Handle &h) {
             H2W_HIP(hipMemcpyAsync(h.d_lr.p + pool.lr_part[q].first * es, pool.lr[q].p, pool.lr_part[q].second * es * 8,
                                    hipMemcpyDeviceToDevice, h.stream));
         H2W_HIP(hipStreamSynchronize(h.stream));
+        scratch.swap(pool.ws);
     }
-    assemble_operators(h, t0);
+    assemble_operators(h, t0, scratch);
 }
 
 // The transfer passes near the root are launches of a few hundred kilobytes, one after another, 3 to 4 us
@@ -1648,8 +1650,8 @@ std::vector<std::pair<int, int>> level_groups(const Handle &h, const int (&lo)[2
 // Everything after the skeletons: pools, transfer / M2L / near-field / CUR blocks,
 // the FP32 shadow, work lists and the inner operator.  Reads h.fam (ranks, pivots,
 // L and R, ACA histories, row sets S) and h.pairs only, so it also rebuilds an
-// operator from saved skeletons.
-void assemble_operators(Handle &h, double t0) {
+// operator from saved skeletons.  scratch: device memory to use, replaced if too small, released when done with.
+void assemble_operators(Handle &h, double t0, DevBuf<double> &scratch) {
     const bool verbose = std::getenv("H2W_VERBOSE") != nullptr;
     auto phase = [&](const char *what) {
         if (verbose) {
@@ -1721,6 +1723,47 @@ void assemble_operators(Handle &h, double t0) {
             }
         }
     }
+    const int64_t xfer_len = mo;
+    // the transfers of every level into a pool
+    auto form_transfers = [&](double *A) {
+        std::vector<int32_t> idx;
+        std::vector<XferJob> xj;
+        for (int f = 0; f < 2; ++f) {
+            if (!fam_on[f]) continue;
+            for (int j = nfam_lo[f]; j <= P.nL; ++j) {
+                FamLevel &fl = h.fam[f][j];
+                for (int b = 0; b < fl.nb; ++b) {
+                    if (fl.e_off[b] < 0) continue;
+                    XferJob J;
+                    J.m = (int32_t)fl.S[b].size();
+                    J.r = fl.rank[b];
+                    J.s = (int64_t)idx.size();
+                    idx.insert(idx.end(), fl.S[b].begin(), fl.S[b].end());
+                    J.ic = (int64_t)idx.size();
+                    idx.insert(idx.end(), fl.Ic[b].begin(), fl.Ic[b].end());
+                    J.lr = fl.lr[b];
+                    J.ldr = J.r;
+                    J.pad = 0;
+                    J.e = fl.e_off[b];
+                    J.et = fl.et_off[b];
+                    J.lde = (int32_t)pad_ld(J.m);
+                    J.ldet = (int32_t)pad_ld(J.r);
+                    xj.push_back(J);
+                }
+            }
+        }
+        DevBuf<int32_t> didx;
+        DevBuf<XferJob> dxj;
+        didx.upload(idx, s);
+        xj = split_xfer(xj);
+        dxj.upload(xj, s);
+        if (h.cplx)
+            launch_xfer_c(dxj.p, (int)xj.size(), didx.p, reinterpret_cast<const double2 *>(h.d_lr.p),
+                          reinterpret_cast<double2 *>(A), h.kpc, s);
+        else launch_xfer(dxj.p, (int)xj.size(), didx.p, h.d_lr.p, A, h.kp, s);
+        H2W_HIP(hipGetLastError());
+        H2W_HIP(hipStreamSynchronize(s));
+    };
     // composite transfers of the groups of several levels: per box c at T the blocks of all its ancestors of
     // the group side by side (down), per box above T - 1 its descendants' blocks transposed (up; at T - 1
     // that is the transfer itself)
@@ -1732,27 +1775,118 @@ void assemble_operators(Handle &h, double t0) {
         for (int c = first_at(b, j, T); c < first_at(b + 1, j, T); ++c) R += h.fam[f][T].rank[c];
         return R;
     };
-    const int64_t comp0 = mo;
-    for (auto [T, B] : groups)
-        for (int f = 0; f < 2 && B < T - 1; ++f) {
-            if (!fam_on[f]) continue;
-            FamLevel &ft = h.fam[f][T];
-            ft.c_off.assign(ft.nb, -1);
-            for (int c = 0; c < ft.nb; ++c) {
-                int64_t n = 0;
-                for (int j = T - 1; j >= std::max(B, nfam_lo[f]); --j) n += h.fam[f][j].rank[ancestor(c, T, j)];
-                if (ft.rank[c] > 0 && n > 0) ft.c_off[c] = take(pad_ld(ft.rank[c]) * n);
-            }
-            for (int j = T - 2; j >= std::max(B, nfam_lo[f]); --j) {
-                FamLevel &fl = h.fam[f][j];
-                fl.ct_off.assign(fl.nb, -1);
-                for (int b = 0; b < fl.nb; ++b) {
-                    const int64_t R = rank_at(f, b, j, T);
-                    if (fl.rank[b] > 0 && R > 0) fl.ct_off[b] = take(pad_ld(fl.rank[b]) * R);
+    // room for the groups' blocks from xfer_len on; returns its length
+    auto place_composites = [&]() {
+        mo = xfer_len;
+        for (auto [T, B] : groups)
+            for (int f = 0; f < 2 && B < T - 1; ++f) {
+                if (!fam_on[f]) continue;
+                FamLevel &ft = h.fam[f][T];
+                ft.c_off.assign(ft.nb, -1);
+                for (int c = 0; c < ft.nb; ++c) {
+                    int64_t n = 0;
+                    for (int j = T - 1; j >= std::max(B, nfam_lo[f]); --j) n += h.fam[f][j].rank[ancestor(c, T, j)];
+                    if (ft.rank[c] > 0 && n > 0) ft.c_off[c] = take(pad_ld(ft.rank[c]) * n);
+                }
+                for (int j = T - 2; j >= std::max(B, nfam_lo[f]); --j) {
+                    FamLevel &fl = h.fam[f][j];
+                    fl.ct_off.assign(fl.nb, -1);
+                    for (int b = 0; b < fl.nb; ++b) {
+                        const int64_t R = rank_at(f, b, j, T);
+                        if (fl.rank[b] > 0 && R > 0) fl.ct_off[b] = take(pad_ld(fl.rank[b]) * R);
+                    }
                 }
             }
+        return mo - xfer_len;
+    };
+    // the placed blocks (len elements) from the transfers in A, level by level away from T (block (c, a) from block
+    // (c, a's child)), with scratch from `at` on; returns the largest entry of every level
+    auto form_composites = [&](double *A, int64_t len, int64_t at) {
+        std::vector<ComposeJob> jobs;
+        std::vector<std::array<int64_t, 3>> runs;  // level, its jobs
+        for (auto [T, B] : groups)
+            for (int j = T - 1; j >= B && B < T - 1; --j) {
+                const int64_t job0 = (int64_t)jobs.size();
+                for (int f = 0; f < 2; ++f) {
+                    if (!fam_on[f] || j < nfam_lo[f]) continue;
+                    const FamLevel &fl = h.fam[f][j], &ft = h.fam[f][T];
+                    for (int c = 0; c < ft.nb; ++c) {
+                        const int a = ancestor(c, T, j);
+                        if (ft.c_off[c] < 0 || fl.rank[a] == 0) continue;
+                        int64_t row = 0, col = 0;  // of the child's rows in a's transfer, of the block in c's run
+                        const int ch = ancestor(c, T, j + 1);
+                        for (int q = a * P.nchild; q < ch; ++q) row += h.fam[f][j + 1].rank[q];
+                        for (int i = T - 1; i > j; --i) col += h.fam[f][i].rank[ancestor(c, T, i)];
+                        const int kc = h.fam[f][j + 1].rank[ch];
+                        if (kc == 0) continue;
+                        ComposeJob J;
+                        J.m = ft.rank[c];
+                        J.n = fl.rank[a];
+                        J.ldd = (int32_t)pad_ld(J.m);
+                        J.d = ft.c_off[c] + col * J.ldd;
+                        J.dt = -1;
+                        J.ldt = (int32_t)pad_ld(J.n);
+                        J.pad = 0;
+                        J.lda = J.ldb = (int32_t)pad_ld((int64_t)fl.S[a].size());
+                        if (j == T - 1) {
+                            J.k = 0;
+                            J.a = fl.e_off[a] + row;
+                            J.b = 0;
+                        } else {
+                            J.k = kc;
+                            J.lda = J.ldd;
+                            J.a = J.d - (int64_t)kc * J.ldd;  // (c, ch), the block before
+                            J.b = fl.e_off[a] + row;
+                            J.dt = fl.ct_off[a] + (ft.o_off[c] - ft.o_off[first_at(a, j, T)]) * J.ldt;
+                        }
+                        jobs.push_back(J);
+                    }
+                }
+                runs.push_back({j, job0, (int64_t)jobs.size()});
+            }
+        // the blocks' low parts, the largest entry of each level, the jobs
+        const int64_t nj = (int64_t)(jobs.size() * sizeof(ComposeJob) / 8);
+        double *lo = scratch.p + at;
+        unsigned long long *dmost = reinterpret_cast<unsigned long long *>(lo + len);
+        ComposeJob *dj = reinterpret_cast<ComposeJob *>(dmost + P.nL + 1);
+        if (nj > 0) H2W_HIP(hipMemcpyAsync(dj, jobs.data(), (size_t)nj * 8, hipMemcpyHostToDevice, s));
+        // (a block across a box without a skeleton is never formed, but is a factor of the next level's: zero, low
+        // part included)
+        H2W_HIP(hipMemsetAsync(lo, 0, (len + P.nL + 1) * 8, s));
+        for (auto &r : runs)
+            launch_compose(dj + r[1], (int)(r[2] - r[1]), A, lo, xfer_len, dmost + r[0], s);
+        H2W_HIP(hipGetLastError());
+        std::vector<double> most(P.nL + 1);
+        H2W_HIP(hipMemcpyAsync(most.data(), dmost, (P.nL + 1) * 8, hipMemcpyDeviceToHost, s));
+        H2W_HIP(hipStreamSynchronize(s));
+        return most;
+    };
+    // Composites are formed in scratch first: the pool holds the groups' levels that are kept only (kComposeMost).
+    int64_t comp_len = place_composites(), formed = 0;
+    bool reform = false;
+    if (comp_len > 0) {
+        formed = mo;
+        int64_t njobs = 0;
+        for (auto [T, B] : groups)
+            for (int f = 0; f < 2; ++f) njobs += B < T - 1 && fam_on[f] ? (int64_t)(T - B) * h.fam[f][T].nb : 0;
+        scratch.ensure(formed + comp_len + P.nL + 1 + njobs * (int64_t)(sizeof(ComposeJob) / 8));
+        H2W_HIP(hipMemsetAsync(scratch.p, 0, formed * 8, s));
+        form_transfers(scratch.p);
+        const auto most = form_composites(scratch.p, comp_len, formed);
+        std::vector<std::pair<int, int>> kept;
+        for (auto [T, B] : groups) {
+            int low = T - 1;  // the group's levels from here on are kept
+            while (low > B && most[low - 1] <= kComposeMost) --low;
+            kept.push_back({T, low});
+            for (int q = low; q > B; --q) kept.push_back({q, q - 1});
         }
-    const int64_t comp_len = mo - comp0;
+        reform = kept != groups;
+        groups = std::move(kept);
+        if (reform) {
+            comp_len = place_composites();
+            formed = xfer_len;
+        }
+    } else scratch.release();
     auto &m2l = h.m2l;
     m2l.clear();
     for (int f = 0; f < 2; ++f) {
@@ -1850,35 +1984,18 @@ void assemble_operators(Handle &h, double t0) {
     }
 
     // ---- evaluate operators on the device
-    {
-        // transfers
-        std::vector<int32_t> idx;
-        std::vector<XferJob> xj;
-        for (int f = 0; f < 2; ++f) {
-            if (!fam_on[f]) continue;
-            for (int j = nfam_lo[f]; j <= P.nL; ++j) {
-                FamLevel &fl = h.fam[f][j];
-                for (int b = 0; b < fl.nb; ++b) {
-                    if (fl.e_off[b] < 0) continue;
-                    XferJob J;
-                    J.m = (int32_t)fl.S[b].size();
-                    J.r = fl.rank[b];
-                    J.s = (int64_t)idx.size();
-                    idx.insert(idx.end(), fl.S[b].begin(), fl.S[b].end());
-                    J.ic = (int64_t)idx.size();
-                    idx.insert(idx.end(), fl.Ic[b].begin(), fl.Ic[b].end());
-                    J.lr = fl.lr[b];
-                    J.ldr = J.r;
-                    J.pad = 0;
-                    J.e = fl.e_off[b];
-                    J.et = fl.et_off[b];
-                    J.lde = (int32_t)pad_ld(J.m);
-                    J.ldet = (int32_t)pad_ld(J.r);
-                    xj.push_back(J);
-                }
-            }
-        }
+    if (formed > 0) {
+        // (transfers, and composites if all are kept, as they are; else those that are, at their new places)
+        H2W_HIP(hipMemcpyAsync(h.mat64.p, scratch.p, formed * 8, hipMemcpyDeviceToDevice, s));
+        if (reform && comp_len > 0) form_composites(h.mat64.p, comp_len, 0);
+        H2W_HIP(hipStreamSynchronize(s));
+        scratch.release();
+    } else {
+        form_transfers(h.mat64.p);
+    }
+    if (!h.pairs.empty()) {
         // semi-nested row factors
+        std::vector<int32_t> idx;
         std::vector<CurJob> cj;
         for (auto &p : h.pairs) {
             if (p.rank == 0) continue;
@@ -1897,93 +2014,16 @@ void assemble_operators(Handle &h, double t0) {
             cj.push_back(J);
         }
         DevBuf<int32_t> didx;
-        DevBuf<XferJob> dxj;
         DevBuf<CurJob> dcj;
         didx.upload(idx, s);
-        xj = split_xfer(xj);
-        dxj.upload(xj, s);
         cj = split_cur(cj);
         dcj.upload(cj, s);
-        if (h.cplx) {
-            launch_xfer_c(dxj.p, (int)xj.size(), didx.p, reinterpret_cast<const double2 *>(h.d_lr.p),
-                          reinterpret_cast<double2 *>(h.mat64.p), h.kpc, s);
+        if (h.cplx)
             launch_cur_c(dcj.p, (int)cj.size(), didx.p, reinterpret_cast<const double2 *>(h.d_lr.p),
                          reinterpret_cast<double2 *>(h.mat64.p), h.kpc, s);
-        } else {
-            launch_xfer(dxj.p, (int)xj.size(), didx.p, h.d_lr.p, h.mat64.p, h.kp, s);
-            launch_cur(dcj.p, (int)cj.size(), didx.p, h.d_lr.p, h.mat64.p, h.kp, s);
-        }
+        else launch_cur(dcj.p, (int)cj.size(), didx.p, h.d_lr.p, h.mat64.p, h.kp, s);
         H2W_HIP(hipGetLastError());
         H2W_HIP(hipStreamSynchronize(s));
-    }
-    // composite transfers, level by level away from T (block (c, a) from block (c, a's child))
-    std::vector<ComposeJob> jobs;
-    std::vector<std::array<int64_t, 3>> comp_runs;  // level, its jobs
-    for (auto [T, B] : groups)
-        for (int j = T - 1; j >= B && B < T - 1; --j) {
-            const int64_t job0 = (int64_t)jobs.size();
-            for (int f = 0; f < 2; ++f) {
-                if (!fam_on[f] || j < nfam_lo[f]) continue;
-                const FamLevel &fl = h.fam[f][j], &ft = h.fam[f][T];
-                for (int c = 0; c < ft.nb; ++c) {
-                    const int a = ancestor(c, T, j);
-                    if (ft.c_off[c] < 0 || fl.rank[a] == 0) continue;
-                    int64_t row = 0, col = 0;  // of the child's rows in a's transfer, of the block in c's run
-                    const int ch = ancestor(c, T, j + 1);
-                    for (int q = a * P.nchild; q < ch; ++q) row += h.fam[f][j + 1].rank[q];
-                    for (int i = T - 1; i > j; --i) col += h.fam[f][i].rank[ancestor(c, T, i)];
-                    const int kc = h.fam[f][j + 1].rank[ch];
-                    if (kc == 0) continue;
-                    ComposeJob J;
-                    J.m = ft.rank[c];
-                    J.n = fl.rank[a];
-                    J.ldd = (int32_t)pad_ld(J.m);
-                    J.d = ft.c_off[c] + col * J.ldd;
-                    J.dt = -1;
-                    J.ldt = (int32_t)pad_ld(J.n);
-                    J.pad = 0;
-                    J.lda = J.ldb = (int32_t)pad_ld((int64_t)fl.S[a].size());
-                    if (j == T - 1) {
-                        J.k = 0;
-                        J.a = fl.e_off[a] + row;
-                        J.b = 0;
-                    } else {
-                        J.k = kc;
-                        J.lda = J.ldd;
-                        J.a = J.d - (int64_t)kc * J.ldd;  // (c, ch), the block before
-                        J.b = fl.e_off[a] + row;
-                        J.dt = fl.ct_off[a] + (ft.o_off[c] - ft.o_off[first_at(a, j, T)]) * J.ldt;
-                    }
-                    jobs.push_back(J);
-                }
-            }
-            comp_runs.push_back({j, job0, (int64_t)jobs.size()});
-        }
-    if (!jobs.empty()) {
-        // one scratch allocation: the blocks' low parts, the largest entry of each level, the jobs
-        const int64_t nj = (int64_t)(jobs.size() * sizeof(ComposeJob) / 8);
-        DevBuf<double> scratch;
-        scratch.alloc(comp_len + P.nL + 1 + nj);
-        unsigned long long *comp_most = reinterpret_cast<unsigned long long *>(scratch.p + comp_len);
-        ComposeJob *dj = reinterpret_cast<ComposeJob *>(comp_most + P.nL + 1);
-        H2W_HIP(hipMemcpyAsync(dj, jobs.data(), (size_t)nj * 8, hipMemcpyHostToDevice, s));
-        // (a block across a box without a skeleton is never formed, but is a factor of the next level's: zero, low
-        // part included)
-        H2W_HIP(hipMemsetAsync(scratch.p, 0, (comp_len + P.nL + 1) * 8, s));
-        for (auto &r : comp_runs)
-            launch_compose(dj + r[1], (int)(r[2] - r[1]), h.mat64.p, scratch.p, comp0, comp_most + r[0], s);
-        H2W_HIP(hipGetLastError());
-        std::vector<double> most(P.nL + 1);
-        H2W_HIP(hipMemcpyAsync(most.data(), comp_most, (P.nL + 1) * 8, hipMemcpyDeviceToHost, s));
-        H2W_HIP(hipStreamSynchronize(s));
-        std::vector<std::pair<int, int>> kept;
-        for (auto [T, B] : groups) {
-            int low = T - 1;  // the group's levels from here on are kept
-            while (low > B && most[low - 1] <= kComposeMost) --low;
-            kept.push_back({T, low});
-            for (int q = low; q > B; --q) kept.push_back({q, q - 1});
-        }
-        groups = std::move(kept);
     }
     phase("transfer operators");
     {
@@ -2253,7 +2293,8 @@ void assemble_operators(Handle &h, double t0) {
 // operator phase of the assembly from skeletons already in the handle (loading a saved operator)
 void rebuild_operators(Handle &h) {
     drop_graphs(h);
-    assemble_operators(h, now_s());
+    DevBuf<double> scratch;
+    assemble_operators(h, now_s(), scratch);
 }
 
 bool is32(int precision) { return precision == H2W_FP32 || precision == H2W_FP32_OTF || precision == H2W_FP32_INNER; }
