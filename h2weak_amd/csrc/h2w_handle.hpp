@@ -294,8 +294,8 @@ struct h2w_handle {
     int64_t vec_len = 0, off_x = 0, off_y = 0;
     std::vector<h2w::FamLevel> fam[2];
     std::vector<h2w::Pair> pairs;
-    // L and R of every skeleton, where the transfers (also the inner operator's, rebuilt at will) and saved
-    // files take them from: offsets in elements, two doubles each with a complex kernel
+    // L and R of every skeleton while the operators are built from them: offsets in elements, two doubles each with a
+    // complex kernel.  (Later users form them from the pivots again: LrForm.)
     h2w::DevBuf<double> d_lr;
     std::vector<h2w::Launch> launches;
     std::vector<int64_t> launch_elems;  // operator elements each launch streams
@@ -343,6 +343,17 @@ struct h2w_handle {
 namespace h2w {
 
 using Handle = h2w_handle;
+
+// L and R of skeletons (or of their leading k pivots) formed from the pivots: add() returns the offset of L, R follows
+// at k^2, both k x k; out holds them after run().
+struct LrForm {
+    std::vector<LrFormJob> jobs;
+    std::vector<int32_t> idx;
+    int64_t len = 0;
+    DevBuf<double> out;
+    int64_t add(const std::vector<int32_t> &Ir, const std::vector<int32_t> &Ic, int k);
+    void run(const Handle &h);
+};
 
 // assembly from skeletons already in h.fam / h.pairs (h2w_ops.hip)
 void rebuild_operators(Handle &h);

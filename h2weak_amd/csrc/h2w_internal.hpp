@@ -108,6 +108,11 @@ struct LrJob {     // copy L (unit lower) and R (upper) out of an ACA workspace
 // the FP64 pool and its FP32 shadow.
 inline int64_t pad_ld(int64_t rows) { return (rows + 3) / 4 * 4; }
 
+struct LrFormJob { // L and R (k x k each, column-major, at out) of the cross with pivots idx[ir ..], idx[ic ..]
+    int64_t ir, ic, out;
+    int32_t k, pad;
+};
+
 struct EvalJob {   // A = K(rows, cols), m x n column-major at a, leading dimension lda
     int64_t rows, cols, a;
     int32_t m, n, lda, pad;
@@ -214,6 +219,7 @@ void launch_aca_sample(const AcaJob *jobs, int nb, const int32_t *rank, const in
                        const int64_t *tab, KParams kp, int ns, double *err2, double *ref2, hipStream_t s);
 void launch_lr_extract(const LrJob *jobs, int njobs, const double *ws, const int64_t *tab,
                        const int32_t *rowpiv, const int32_t *colpiv, double *out, hipStream_t s);
+void launch_lr_form(const LrFormJob *jobs, int njobs, const int32_t *idx, double *out, KParams kp, hipStream_t s);
 // the pivots and step histories of a batch's blocks one after another (at pk, rank entries each)
 void launch_pack_pivots(const LrJob *jobs, int njobs, const int32_t *rowpiv, const int32_t *colpiv, const double *hist,
                         int32_t *prow, int32_t *pcol, double *phist, hipStream_t s);

@@ -1307,6 +1307,7 @@ void build_inner(Handle &h, double irp) {
     if (inner_on && in_len > 0) {
         std::vector<int32_t> idx;
         std::vector<XferJob> xj;
+        LrForm lr;  // (unless the assembly's are still there)
         for (int f = 0; f < 2; ++f) {
             if (!fam_on[f]) continue;
             for (int j = nfam_lo[f]; j <= P.nL; ++j) {
@@ -1314,6 +1315,7 @@ void build_inner(Handle &h, double irp) {
                 for (int b = 0; b < fl.nb; ++b) {
                     if (fl.ein_off[b] < 0) continue;
                     const int k = fl.kin[b];
+                    const int64_t lro = h.d_lr.p ? fl.lr[b] : lr.add(fl.Ir[b], fl.Ic[b], k);
                     const int64_t icq = (int64_t)idx.size();
                     idx.insert(idx.end(), fl.Ic[b].begin(), fl.Ic[b].begin() + k);
                     int64_t m = 0;
@@ -1329,8 +1331,8 @@ void build_inner(Handle &h, double irp) {
                         J.s = (int64_t)idx.size();
                         idx.insert(idx.end(), S, S + ms);
                         J.ic = icq;
-                        J.lr = fl.lr[b];  // (the leading k x k blocks of L and R)
-                        J.ldr = fl.rank[b];
+                        J.lr = lro;  // (the leading k x k blocks of L and R)
+                        J.ldr = h.d_lr.p ? fl.rank[b] : k;
                         J.pad = 0;
                         J.e = fl.ein_off[b] + row;
                         J.et = fl.eint_off[b] + row * ldet;
@@ -1361,7 +1363,8 @@ void build_inner(Handle &h, double irp) {
         dxj.upload(xj, s);
         tmp.alloc(in_len);
         H2W_HIP(hipMemsetAsync(tmp.p, 0, in_len * 8, s));
-        launch_xfer(dxj.p, (int)xj.size(), didx.p, h.d_lr.p, tmp.p, h.kp, s);
+        lr.run(h);
+        launch_xfer(dxj.p, (int)xj.size(), didx.p, h.d_lr.p ? h.d_lr.p : lr.out.p, tmp.p, h.kp, s);
         H2W_HIP(hipGetLastError());
         launch_to_fp32(tmp.p, h.mat32in.p, in_len, s);
         H2W_HIP(hipGetLastError());
@@ -2278,6 +2281,7 @@ void assemble_operators(Handle &h, double t0, DevBuf<double> &scratch) {
     h.stored_elems = se;
     build_inner(h, (double)h.opts.ir_tol_pow);
     H2W_HIP(hipStreamSynchronize(s));
+    h.d_lr.release();
     phase("work lists");
     if (verbose)
         std::fprintf(stderr, "[h2w] memory %.0f elements (%.3f GB fp64), pool %.3f GB, %zu launches, %zu items\n",
@@ -2289,6 +2293,31 @@ void assemble_operators(Handle &h, double t0, DevBuf<double> &scratch) {
 // ------------------------------------------------------------------ matvec
 // y_tree = A x_tree inside the vector pool (x already at off_x)
 }  // namespace
+
+int64_t LrForm::add(const std::vector<int32_t> &Ir, const std::vector<int32_t> &Ic, int k) {
+    LrFormJob J;
+    J.ir = (int64_t)idx.size();
+    idx.insert(idx.end(), Ir.begin(), Ir.begin() + k);
+    J.ic = (int64_t)idx.size();
+    idx.insert(idx.end(), Ic.begin(), Ic.begin() + k);
+    J.out = len;
+    J.k = k;
+    J.pad = 0;
+    len += 2LL * k * k;
+    jobs.push_back(J);
+    return J.out;
+}
+void LrForm::run(const Handle &h) {
+    if (jobs.empty()) return;
+    DevBuf<LrFormJob> dj;
+    DevBuf<int32_t> di;
+    dj.upload(jobs, h.stream);
+    di.upload(idx, h.stream);
+    out.ensure(len);
+    launch_lr_form(dj.p, (int)jobs.size(), di.p, out.p, h.kp, h.stream);
+    H2W_HIP(hipGetLastError());
+    H2W_HIP(hipStreamSynchronize(h.stream));
+}
 
 // operator phase of the assembly from skeletons already in the handle (loading a saved operator)
 void rebuild_operators(Handle &h) {

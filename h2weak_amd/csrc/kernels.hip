@@ -895,6 +895,39 @@ __global__ void k_lr_extract(const LrJob *__restrict__ jobs, const double *__res
     }
 }
 
+// L and R again from a skeleton's pivots, for an operator that no longer holds them: elimination of the pivot block in
+// pivot order.  Every entry takes the products of the earlier terms in rank order, multiplied and subtracted separately,
+// as the cross's residual rows and columns do, so the factors are the cross's to the last bit.
+__global__ __launch_bounds__(1024) void k_lr_form(const LrFormJob *__restrict__ jobs, const int32_t *__restrict__ idx,
+                                                  double *__restrict__ out, KParams kp) {
+    const LrFormJob jb = jobs[blockIdx.x];
+    const int k = jb.k;
+    double *L = out + jb.out;
+    double *R = L + (int64_t)k * k;
+    for (int e = threadIdx.x; e < k * k; e += 1024) {
+        const int i = e % k, j = e / k;
+        R[e] = kentry2(kp, idx[jb.ir + i], idx[jb.ic + j]);
+        L[e] = i == j ? 1.0 : 0.0;
+    }
+    const int ti = threadIdx.x & 63, tj = threadIdx.x >> 6;
+    for (int q = 0; q < k - 1; ++q) {
+        __syncthreads();
+        double *l = L + (int64_t)q * k;
+        const double piv = R[(int64_t)q * k + q];
+        for (int i = q + 1 + threadIdx.x; i < k; i += 1024) l[i] = R[(int64_t)q * k + i] / piv;
+        __syncthreads();
+        for (int j = q + 1 + tj; j < k; j += 16) {
+            double *c = R + (int64_t)j * k;
+            const double v = c[q];
+#pragma unroll 4
+            for (int i = q + 1 + ti; i < k; i += 64) c[i] -= l[i] * v;
+        }
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < k * k; e += 1024)
+        if (e % k > e / k) R[e] = 0.0;
+}
+
 __global__ void k_pack_pivots(const LrJob *__restrict__ jobs, const int32_t *__restrict__ rowpiv,
                               const int32_t *__restrict__ colpiv, const double *__restrict__ hist,
                               int32_t *__restrict__ prow, int32_t *__restrict__ pcol, double *__restrict__ phist) {
@@ -2664,6 +2697,9 @@ void launch_lr_extract(const LrJob *jobs, int njobs, const double *ws, const int
                        const int32_t *colpiv, double *out, hipStream_t s) {
     if (njobs > 0)
         hipLaunchKernelGGL(k_lr_extract, dim3(njobs), dim3(256), 0, s, jobs, ws, tab, rowpiv, colpiv, out);
+}
+void launch_lr_form(const LrFormJob *jobs, int njobs, const int32_t *idx, double *out, KParams kp, hipStream_t s) {
+    if (njobs > 0) hipLaunchKernelGGL(k_lr_form, dim3(njobs), dim3(1024), 0, s, jobs, idx, out, kp);
 }
 void launch_pack_pivots(const LrJob *jobs, int njobs, const int32_t *rowpiv, const int32_t *colpiv, const double *hist,
                         int32_t *prow, int32_t *pcol, double *phist, hipStream_t s) {

@@ -123,17 +123,22 @@ int h2w_save(const h2w_handle *h, const char *path) {
         if (!fp) throw Error{H2W_EINVAL, std::string("cannot open ") + path};
         h2w::Writer w{fp.get()};
         const h2w::Plan &P = h->plan;
-        std::vector<double> lr(h->d_lr.n);  // L and R of every skeleton
         H2W_HIP(hipSetDevice(h->opts.device));
-        if (!lr.empty()) {
-            // The caller, or another thread, may be capturing a graph: the copy and its wait concern the handle's
-            // own stream only, and must not end that capture.
-            h2w::RelaxedCapture relaxed;
-            H2W_HIP(hipMemcpyAsync(lr.data(), h->d_lr.p, lr.size() * 8, hipMemcpyDeviceToHost, h->stream));
+        // The caller, or another thread, may be capturing a graph: what follows concerns the handle's own stream only,
+        // and must not end that capture.
+        h2w::RelaxedCapture relaxed;
+        std::vector<double> lr;
+        auto fetch = [&](h2w::LrForm &form) {  // L and R of a level's skeletons
+            lr.resize(form.len);
+            if (lr.empty()) return;
+            form.run(*h);
+            H2W_HIP(hipMemcpyAsync(lr.data(), form.out.p, lr.size() * 8, hipMemcpyDeviceToHost, h->stream));
             H2W_HIP(hipStreamSynchronize(h->stream));
-        }
-        auto put_lr = [&](int64_t off, int64_t r) {
-            if (r > 0) w.raw(lr.data() + off, (size_t)(2 * r * r) * sizeof(double));
+        };
+        int64_t at = 0;
+        auto put_lr = [&](int64_t r) {
+            w.raw(lr.data() + at, (size_t)(2 * r * r) * sizeof(double));
+            at += 2 * r * r;
         };
         w.raw(h2w::kMagic, 8);
         const int32_t hdr[8] = {h->dim, h->variant, h->choice, h->tol_pow, h->n_max, P.nL, h->opts.compat, 0};
@@ -153,23 +158,33 @@ int h2w_save(const h2w_handle *h, const char *path) {
                 const h2w::FamLevel *fl = have ? &h->fam[f][j] : nullptr;
                 const int32_t nb = fl ? (int32_t)fl->rank.size() : 0;
                 w.put<int32_t>(nb);
+                h2w::LrForm form;
+                for (int b = 0; b < nb; ++b)
+                    if (fl->rank[b] > 0) form.add(fl->Ir[b], fl->Ic[b], fl->rank[b]);
+                fetch(form);
+                at = 0;
                 for (int b = 0; b < nb; ++b) {
                     const int32_t r = fl->rank[b];
                     w.put<int32_t>(r);
                     w.vec(fl->Ir[b], r);
                     w.vec(fl->Ic[b], r);
-                    put_lr(fl->lr[b], r);
+                    put_lr(r);
                     w.put<int32_t>((int32_t)fl->hist[b].size());
                     w.vec(fl->hist[b], fl->hist[b].size());
                 }
             }
         w.put<int64_t>((int64_t)h->pairs.size());
+        h2w::LrForm form;
+        for (const auto &p : h->pairs)
+            if (p.rank > 0) form.add(p.Ir, p.Ic, p.rank);
+        fetch(form);
+        at = 0;
         for (const auto &p : h->pairs) {
             const int32_t v[4] = {p.level, p.b, p.v, p.rank};
             w.raw(v, sizeof(v));
             w.vec(p.Ir, p.rank);
             w.vec(p.Ic, p.rank);
-            put_lr(p.lr, p.rank);
+            put_lr(p.rank);
         }
         const uint64_t hash = w.hash;
         w.put<uint64_t>(hash);
