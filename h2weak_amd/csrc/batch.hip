@@ -131,7 +131,7 @@ void merge_lists(Batch &B, int which) {
         for (int64_t t = Lm.term0; t < (int64_t)terms.size(); ++t) sc += terms[t].cols;
         Lm.avg_cols = Lm.nterms ? (int)(sc / Lm.nterms) : 0;
         if (Lm.nitems == 0) continue;
-        Lm.avg_item_elems = e / Lm.nitems;
+        Lm.avg_item_elems = Lm.avg_item_elemsm = e / Lm.nitems;
         M.launches.push_back(Lm);
         M.elems.push_back(e);
     }

@@ -163,13 +163,16 @@ struct Launch {
     int unr32 = 4; // the same for the stored FP32 copy
     int avg_cols = 0;  // mean inner size of the terms (picks the transposed 16-wide kernel's slabs)
     int64_t avg_item_elems = 0;  // mean operator elements per item
+    int64_t avg_item_elemsm = 0; // and per item of the 16-wide path
     void set_wide(std::vector<GItem> &items, const std::vector<GTerm> &terms);
 };
 // one item per wave on the 16-wide path: launches of enough items that are small on average
 // (the transfer passes at the leaves of small systems), where a workgroup's set-up and the
-// reduction across its waves would outweigh the item
+// reduction across its waves would outweigh the item.  Measured, four waves / one wave per item (FP64): 2D N = 60000
+// leaf up pass (5730 items of 2480 elements) 44 / 25 us, 1D N = 250000 leaves (4096 of 1390) 36 / 27 and 50 / 33 us;
+// above the limit 2D semi-nested column factors (2505 of 5220) 43 / 38 us, 2D N = 90000 leaves (2048 of 7563) 52 / 49.
 inline bool per_wave_items(const Launch &L) {
-    return L.nitemsm >= 2048 && L.avg_item_elems > 0 && L.avg_item_elems <= 4096;
+    return L.nitemsm >= 2048 && L.avg_item_elemsm > 0 && L.avg_item_elemsm <= 4096;
 }
 // The same on the single-vector path.  Measured, four waves / one wave per item: 1D N = 250000 leaf up
 // pass (4096 items of 1500 elements on average) 21 / 16 us and fused launch (8000 of 2200) 50 / 40 us, 2D

@@ -1189,6 +1189,10 @@ void Launch::set_wide(std::vector<GItem> &items, const std::vector<GTerm> &terms
     nitemsm = wide_items(items, item0, terms, role);
     item0m = nitemsm ? n : item0;
     if (!nitemsm) nitemsm = nitems;
+    int64_t e = 0;
+    for (int64_t q = item0; q < item0 + nitems; ++q)
+        for (int32_t k = items[q].t0; k < items[q].t1; ++k) e += (int64_t)items[q].rows * terms[k].cols;
+    avg_item_elemsm = e / nitemsm;
 }
 
 namespace {
