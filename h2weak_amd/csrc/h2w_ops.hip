@@ -1196,7 +1196,8 @@ void Launch::set_wide(std::vector<GItem> &items, const std::vector<GTerm> &terms
 }
 
 namespace {
-void upload_lists(std::vector<WorkList> &WL, LaunchSet &LS, hipStream_t s) {
+// wide: the 16-wide path dispatches these lists by items of its own
+void upload_lists(std::vector<WorkList> &WL, LaunchSet &LS, bool wide, hipStream_t s) {
     std::vector<GItem> items;
     std::vector<GTerm> terms;
     LS.launches.clear();
@@ -1222,7 +1223,7 @@ void upload_lists(std::vector<WorkList> &WL, LaunchSet &LS, hipStream_t s) {
         }
         terms.insert(terms.end(), W.terms.begin(), W.terms.end());
         Lh.avg_item_elems = e / Lh.nitems;
-        Lh.set_wide(items, terms);
+        if (wide) Lh.set_wide(items, terms);
         LS.launches.push_back(Lh);
         LS.elems.push_back(e);
     }
@@ -1485,7 +1486,7 @@ void build_inner(Handle &h, double irp) {
             SL.trans.step = 1;
             std::vector<WorkList> tl;
             tl.push_back(std::move(SL.trans));
-            upload_lists(tl, h.inner_trans, s);
+            upload_lists(tl, h.inner_trans, false, s);
         }
         for (int j = 1; j <= P.nL - 1; ++j) {
             WorkList W;
@@ -1543,7 +1544,7 @@ void build_inner(Handle &h, double irp) {
         }
         for (auto &W : IL)
             rebalance(W);
-        upload_lists(IL, h.inner, s);
+        upload_lists(IL, h.inner, true, s);
         h.inner_elems = 0;
         for (auto e : h.inner.elems) h.inner_elems += e;
     } else {
@@ -2177,8 +2178,8 @@ void assemble_operators(Handle &h, double t0, DevBuf<double> &scratch) {
         std::vector<WorkList> tl, ol;
         tl.push_back(std::move(SL.trans));
         ol.push_back(std::move(SL.otf));
-        upload_lists(tl, h.trans, s);
-        upload_lists(ol, h.otf, s);
+        upload_lists(tl, h.trans, false, s);
+        upload_lists(ol, h.otf, false, s);
     }
     // down, levels 1 .. nL-1 (from the levels of a group in one launch)
     for (auto g = groups.rbegin(); g != groups.rend(); ++g) {
