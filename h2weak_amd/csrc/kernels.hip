@@ -444,7 +444,11 @@ __global__ __launch_bounds__(256) void k_wide_init(const AcaJob *__restrict__ jo
 }
 
 // Values handed from the workgroups of a pass to the one that finishes its block, within one launch:
-// agent-scope accesses go past the caches that the XCDs do not share.
+// agent-scope accesses go past the caches that the XCDs do not share, every wave waits for its stores (s_waitcnt 0)
+// before the barrier behind which the arrival is counted, and the last workgroup reads behind its own count.  That
+// order is gfx950's; the memory model's form of it (release and acquire at agent scope on the count) also writes back
+// whatever the XCD's L2 holds dirty, the residual rows and columns among it: assembly of 20011 3D points 76.6 -> 93.1
+// ms, of 40000 2D points 34.3 -> 36.8.
 __device__ __forceinline__ void st_agent(double *p, double v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
