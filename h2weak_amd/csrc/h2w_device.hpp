@@ -8,11 +8,9 @@
 #include "h2w_internal.hpp"
 
 namespace h2w {
-// the buffer atomics' intrinsics (they have no clang builtin)
+// the FP64 buffer atomic's intrinsic (no clang builtin; a compiler that did not know it would fail at the link)
 __device__ double buf_fadd64(double v, __amdgpu_buffer_rsrc_t r, int voff, int soff, int aux) __asm(
     "llvm.amdgcn.raw.ptr.buffer.atomic.fadd.f64");
-__device__ float buf_fadd32(float v, __amdgpu_buffer_rsrc_t r, int voff, int soff, int aux) __asm(
-    "llvm.amdgcn.raw.ptr.buffer.atomic.fadd.f32");
 namespace {
 
 // Value of lane (lane ^ O) for a power of two O < 64: quad permutes (DPP) for 1 and 2,
@@ -109,7 +107,7 @@ __device__ __forceinline__ void buf_atomic_add(__amdgpu_buffer_rsrc_t r, uint32_
     (void)buf_fadd64(v, r, (int)off, 0, 0);
 }
 __device__ __forceinline__ void buf_atomic_add(__amdgpu_buffer_rsrc_t r, uint32_t off, float v) {
-    (void)buf_fadd32(v, r, (int)off, 0, 0);
+    (void)__builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(v, r, (int)off, 0, 0);
 }
 // one 4-, 8- or 16-byte vector, streamed (not kept in the caches)
 template <typename V>
