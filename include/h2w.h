@@ -81,7 +81,10 @@ typedef struct {
                                 of the top vertex level and of the semi-nested pairs to a shared
                                 workspace batch; a block that outgrows the batch's pool is re-run,
                                 so results do not depend on it                                   */
-    int64_t workspace_bytes; /* ACA workspace budget in bytes (0 = automatic)                    */
+    int64_t workspace_bytes; /* budget in bytes of the ACA workspace, the columns U and V of a batch of
+                                blocks (0 = automatic).  Beside it an assembly holds, until it ends, the
+                                batch's index lists, tables and partial sums (about a hundredth of it)
+                                and the factors L and R of the skeletons (2 rank^2 numbers each)   */
     int plan_only;           /* 1: build the tree and lists only, touch no device (assembly and
                                 products then return H2W_ESTATE); for host-side inspection        */
     int ir_tol_pow;          /* tolerance exponent of the refinement's truncated inner operator
@@ -123,7 +126,10 @@ typedef struct {
     int iterations;          /* Arnoldi steps (FP64 mode) / total inner steps (FP32-IR mode),
                                 counted like the reference's `max_iter` output                   */
     int outer_iterations;    /* refinement steps (FP32-IR mode), 0 for FP64 mode                 */
-    int matvecs_fp64, matvecs_fp32;
+    int matvecs_fp64, matvecs_fp32; /* products whose results the solve used.  The next Arnoldi step's product is
+                                queued before this step's residual is known; where that residual meets
+                                the tolerance against expectation, one product per Arnoldi process runs
+                                on the device beside these                                       */
     double resid;            /* final |s_{i+1}|/||b|| (FP64) or true ||b - A x||/||b|| (IR)      */
     double seconds;          /* wall time, first residual matvec to convergence                  */
     int converged;
