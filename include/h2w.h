@@ -83,8 +83,9 @@ typedef struct {
                                 so results do not depend on it                                   */
     int64_t workspace_bytes; /* budget in bytes of the ACA workspace, the columns U and V of a batch of
                                 blocks (0 = automatic).  Beside it an assembly holds, until it ends, the
-                                batch's index lists, tables and partial sums (about a hundredth of it)
-                                and the factors L and R of the skeletons (2 rank^2 numbers each)   */
+                                batch's index lists, tables and partial sums (up to a tenth of it) and
+                                the factors L and R of the skeletons (2 rank^2 numbers each, at its
+                                end twice)                                                        */
     int plan_only;           /* 1: build the tree and lists only, touch no device (assembly and
                                 products then return H2W_ESTATE); for host-side inspection        */
     int ir_tol_pow;          /* tolerance exponent of the refinement's truncated inner operator
