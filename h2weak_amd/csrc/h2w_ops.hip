@@ -1772,129 +1772,6 @@ void assemble_operators(Handle &h, double t0, DevBuf<double> &scratch) {
         H2W_HIP(hipGetLastError());
         H2W_HIP(hipStreamSynchronize(s));
     };
-    // composite transfers of the groups of several levels: per box c at T the blocks of all its ancestors of
-    // the group side by side (down), per box above T - 1 its descendants' blocks transposed (up; at T - 1
-    // that is the transfer itself)
-    auto groups = level_groups(h, nfam_lo, fam_on);
-    auto ancestor = [&](int c, int T, int j) { return c >> (P.dim * (T - j)); };
-    auto first_at = [&](int b, int j, int T) { return (int)((int64_t)b << (P.dim * (T - j))); };
-    auto rank_at = [&](int f, int b, int j, int T) {
-        int64_t R = 0;
-        for (int c = first_at(b, j, T); c < first_at(b + 1, j, T); ++c) R += h.fam[f][T].rank[c];
-        return R;
-    };
-    // room for the groups' blocks from xfer_len on; returns its length
-    auto place_composites = [&]() {
-        mo = xfer_len;
-        for (auto [T, B] : groups)
-            for (int f = 0; f < 2 && B < T - 1; ++f) {
-                if (!fam_on[f]) continue;
-                FamLevel &ft = h.fam[f][T];
-                ft.c_off.assign(ft.nb, -1);
-                for (int c = 0; c < ft.nb; ++c) {
-                    int64_t n = 0;
-                    for (int j = T - 1; j >= std::max(B, nfam_lo[f]); --j) n += h.fam[f][j].rank[ancestor(c, T, j)];
-                    if (ft.rank[c] > 0 && n > 0) ft.c_off[c] = take(pad_ld(ft.rank[c]) * n);
-                }
-                for (int j = T - 2; j >= std::max(B, nfam_lo[f]); --j) {
-                    FamLevel &fl = h.fam[f][j];
-                    fl.ct_off.assign(fl.nb, -1);
-                    for (int b = 0; b < fl.nb; ++b) {
-                        const int64_t R = rank_at(f, b, j, T);
-                        if (fl.rank[b] > 0 && R > 0) fl.ct_off[b] = take(pad_ld(fl.rank[b]) * R);
-                    }
-                }
-            }
-        return mo - xfer_len;
-    };
-    // the placed blocks (len elements) from the transfers in A, level by level away from T (block (c, a) from block
-    // (c, a's child)), with scratch from `at` on; returns the largest entry of every level
-    auto form_composites = [&](double *A, int64_t len, int64_t at) {
-        std::vector<ComposeJob> jobs;
-        std::vector<std::array<int64_t, 3>> runs;  // level, its jobs
-        for (auto [T, B] : groups)
-            for (int j = T - 1; j >= B && B < T - 1; --j) {
-                const int64_t job0 = (int64_t)jobs.size();
-                for (int f = 0; f < 2; ++f) {
-                    if (!fam_on[f] || j < nfam_lo[f]) continue;
-                    const FamLevel &fl = h.fam[f][j], &ft = h.fam[f][T];
-                    for (int c = 0; c < ft.nb; ++c) {
-                        const int a = ancestor(c, T, j);
-                        if (ft.c_off[c] < 0 || fl.rank[a] == 0) continue;
-                        int64_t row = 0, col = 0;  // of the child's rows in a's transfer, of the block in c's run
-                        const int ch = ancestor(c, T, j + 1);
-                        for (int q = a * P.nchild; q < ch; ++q) row += h.fam[f][j + 1].rank[q];
-                        for (int i = T - 1; i > j; --i) col += h.fam[f][i].rank[ancestor(c, T, i)];
-                        const int kc = h.fam[f][j + 1].rank[ch];
-                        if (kc == 0) continue;
-                        ComposeJob J;
-                        J.m = ft.rank[c];
-                        J.n = fl.rank[a];
-                        J.ldd = (int32_t)pad_ld(J.m);
-                        J.d = ft.c_off[c] + col * J.ldd;
-                        J.dt = -1;
-                        J.ldt = (int32_t)pad_ld(J.n);
-                        J.pad = 0;
-                        J.lda = J.ldb = (int32_t)pad_ld((int64_t)fl.S[a].size());
-                        if (j == T - 1) {
-                            J.k = 0;
-                            J.a = fl.e_off[a] + row;
-                            J.b = 0;
-                        } else {
-                            J.k = kc;
-                            J.lda = J.ldd;
-                            J.a = J.d - (int64_t)kc * J.ldd;  // (c, ch), the block before
-                            J.b = fl.e_off[a] + row;
-                            J.dt = fl.ct_off[a] + (ft.o_off[c] - ft.o_off[first_at(a, j, T)]) * J.ldt;
-                        }
-                        jobs.push_back(J);
-                    }
-                }
-                runs.push_back({j, job0, (int64_t)jobs.size()});
-            }
-        // the blocks' low parts, the largest entry of each level, the jobs
-        const int64_t nj = (int64_t)(jobs.size() * sizeof(ComposeJob) / 8);
-        double *lo = scratch.p + at;
-        unsigned long long *dmost = reinterpret_cast<unsigned long long *>(lo + len);
-        ComposeJob *dj = reinterpret_cast<ComposeJob *>(dmost + P.nL + 1);
-        if (nj > 0) H2W_HIP(hipMemcpyAsync(dj, jobs.data(), (size_t)nj * 8, hipMemcpyHostToDevice, s));
-        // (a block across a box without a skeleton is never formed, but is a factor of the next level's: zero, low
-        // part included)
-        H2W_HIP(hipMemsetAsync(lo, 0, (len + P.nL + 1) * 8, s));
-        for (auto &r : runs)
-            launch_compose(dj + r[1], (int)(r[2] - r[1]), A, lo, xfer_len, dmost + r[0], s);
-        H2W_HIP(hipGetLastError());
-        std::vector<double> most(P.nL + 1);
-        H2W_HIP(hipMemcpyAsync(most.data(), dmost, (P.nL + 1) * 8, hipMemcpyDeviceToHost, s));
-        H2W_HIP(hipStreamSynchronize(s));
-        return most;
-    };
-    // Composites are formed in scratch first: the pool holds the groups' levels that are kept only (kComposeMost).
-    int64_t comp_len = place_composites(), formed = 0;
-    bool reform = false;
-    if (comp_len > 0) {
-        formed = mo;
-        int64_t njobs = 0;
-        for (auto [T, B] : groups)
-            for (int f = 0; f < 2; ++f) njobs += B < T - 1 && fam_on[f] ? (int64_t)(T - B) * h.fam[f][T].nb : 0;
-        scratch.ensure(formed + comp_len + P.nL + 1 + njobs * (int64_t)(sizeof(ComposeJob) / 8));
-        H2W_HIP(hipMemsetAsync(scratch.p, 0, formed * 8, s));
-        form_transfers(scratch.p);
-        const auto most = form_composites(scratch.p, comp_len, formed);
-        std::vector<std::pair<int, int>> kept;
-        for (auto [T, B] : groups) {
-            int low = T - 1;  // the group's levels from here on are kept
-            while (low > B && most[low - 1] <= kComposeMost) --low;
-            kept.push_back({T, low});
-            for (int q = low; q > B; --q) kept.push_back({q, q - 1});
-        }
-        reform = kept != groups;
-        groups = std::move(kept);
-        if (reform) {
-            comp_len = place_composites();
-            formed = xfer_len;
-        }
-    } else scratch.release();
     auto &m2l = h.m2l;
     m2l.clear();
     for (int f = 0; f < 2; ++f) {
@@ -1948,12 +1825,119 @@ void assemble_operators(Handle &h, double t0, DevBuf<double> &scratch) {
         if (p.rank > 0) p.ac_off = run(pad_ld(P.bcount[p.level][p.b]) * p.rank);
     }
     mo = align_up(mo, 32);
-    h.mat_len = std::max<int64_t>(mo, 32);
+    // composite transfers of the groups of several levels: per box c at T the blocks of all its ancestors of
+    // the group side by side (down), per box above T - 1 its descendants' blocks transposed (up; at T - 1
+    // that is the transfer itself)
+    auto groups = level_groups(h, nfam_lo, fam_on);
+    auto ancestor = [&](int c, int T, int j) { return c >> (P.dim * (T - j)); };
+    auto first_at = [&](int b, int j, int T) { return (int)((int64_t)b << (P.dim * (T - j))); };
+    auto rank_at = [&](int f, int b, int j, int T) {
+        int64_t R = 0;
+        for (int c = first_at(b, j, T); c < first_at(b + 1, j, T); ++c) R += h.fam[f][T].rank[c];
+        return R;
+    };
+    // room for the groups' blocks from `base` on; returns its length
+    auto place_composites = [&](int64_t base) {
+        mo = base;
+        for (auto [T, B] : groups)
+            for (int f = 0; f < 2 && B < T - 1; ++f) {
+                if (!fam_on[f]) continue;
+                FamLevel &ft = h.fam[f][T];
+                ft.c_off.assign(ft.nb, -1);
+                for (int c = 0; c < ft.nb; ++c) {
+                    int64_t n = 0;
+                    for (int j = T - 1; j >= std::max(B, nfam_lo[f]); --j) n += h.fam[f][j].rank[ancestor(c, T, j)];
+                    if (ft.rank[c] > 0 && n > 0) ft.c_off[c] = take(pad_ld(ft.rank[c]) * n);
+                }
+                for (int j = T - 2; j >= std::max(B, nfam_lo[f]); --j) {
+                    FamLevel &fl = h.fam[f][j];
+                    fl.ct_off.assign(fl.nb, -1);
+                    for (int b = 0; b < fl.nb; ++b) {
+                        const int64_t R = rank_at(f, b, j, T);
+                        if (fl.rank[b] > 0 && R > 0) fl.ct_off[b] = take(pad_ld(fl.rank[b]) * R);
+                    }
+                }
+            }
+        return mo - base;
+    };
+    // the blocks placed from `base` on (len elements) from the transfers in A, level by level away from T (block (c, a)
+    // from block (c, a's child)), with scratch at lo; returns the largest entry of every level
+    auto form_composites = [&](double *A, int64_t base, int64_t len, double *lo) {
+        std::vector<ComposeJob> jobs;
+        std::vector<std::array<int64_t, 3>> runs;  // level, its jobs
+        for (auto [T, B] : groups)
+            for (int j = T - 1; j >= B && B < T - 1; --j) {
+                const int64_t job0 = (int64_t)jobs.size();
+                for (int f = 0; f < 2; ++f) {
+                    if (!fam_on[f] || j < nfam_lo[f]) continue;
+                    const FamLevel &fl = h.fam[f][j], &ft = h.fam[f][T];
+                    for (int c = 0; c < ft.nb; ++c) {
+                        const int a = ancestor(c, T, j);
+                        if (ft.c_off[c] < 0 || fl.rank[a] == 0) continue;
+                        int64_t row = 0, col = 0;  // of the child's rows in a's transfer, of the block in c's run
+                        const int ch = ancestor(c, T, j + 1);
+                        for (int q = a * P.nchild; q < ch; ++q) row += h.fam[f][j + 1].rank[q];
+                        for (int i = T - 1; i > j; --i) col += h.fam[f][i].rank[ancestor(c, T, i)];
+                        const int kc = h.fam[f][j + 1].rank[ch];
+                        if (kc == 0) continue;
+                        ComposeJob J;
+                        J.m = ft.rank[c];
+                        J.n = fl.rank[a];
+                        J.ldd = (int32_t)pad_ld(J.m);
+                        J.d = ft.c_off[c] + col * J.ldd;
+                        J.dt = -1;
+                        J.ldt = (int32_t)pad_ld(J.n);
+                        J.pad = 0;
+                        J.lda = J.ldb = (int32_t)pad_ld((int64_t)fl.S[a].size());
+                        if (j == T - 1) {
+                            J.k = 0;
+                            J.a = fl.e_off[a] + row;
+                            J.b = 0;
+                        } else {
+                            J.k = kc;
+                            J.lda = J.ldd;
+                            J.a = J.d - (int64_t)kc * J.ldd;  // (c, ch), the block before
+                            J.b = fl.e_off[a] + row;
+                            J.dt = fl.ct_off[a] + (ft.o_off[c] - ft.o_off[first_at(a, j, T)]) * J.ldt;
+                        }
+                        jobs.push_back(J);
+                    }
+                }
+                runs.push_back({j, job0, (int64_t)jobs.size()});
+            }
+        // the blocks' low parts, the largest entry of each level, the jobs
+        const int64_t nj = (int64_t)(jobs.size() * sizeof(ComposeJob) / 8);
+        unsigned long long *dmost = reinterpret_cast<unsigned long long *>(lo + len);
+        ComposeJob *dj = reinterpret_cast<ComposeJob *>(dmost + P.nL + 1);
+        if (nj > 0) H2W_HIP(hipMemcpyAsync(dj, jobs.data(), (size_t)nj * 8, hipMemcpyHostToDevice, s));
+        // (a block across a box without a skeleton is never formed, but is a factor of the next level's: zero, low
+        // part included)
+        H2W_HIP(hipMemsetAsync(lo, 0, (len + P.nL + 1) * 8, s));
+        for (auto &r : runs)
+            launch_compose(dj + r[1], (int)(r[2] - r[1]), A, lo, base, dmost + r[0], s);
+        H2W_HIP(hipGetLastError());
+        std::vector<double> most(P.nL + 1);
+        H2W_HIP(hipMemcpyAsync(most.data(), dmost, (P.nL + 1) * 8, hipMemcpyDeviceToHost, s));
+        H2W_HIP(hipStreamSynchronize(s));
+        return most;
+    };
+    // Composites come last in the pool, once it is known which are used (kComposeMost): they are formed where the other
+    // blocks will be, or in scratch where that is too small.  Up to 2 MB is taken for them beforehand.
+    const int64_t pool_len = mo;
+    int64_t comp_len = place_composites(xfer_len);
+    const int64_t spare = std::min<int64_t>(comp_len, 1 << 18);
+    int64_t need = 2 * comp_len + P.nL + 1;  // blocks, low parts, largest entries, jobs
+    for (auto [T, B] : groups)
+        for (int f = 0; f < 2; ++f)
+            if (B < T - 1 && fam_on[f]) need += (int64_t)(T - B) * h.fam[f][T].nb * (int64_t)(sizeof(ComposeJob) / 8);
+    const bool inside = xfer_len + need <= pool_len;
+    if (comp_len == 0 || inside) scratch.release();
+    else scratch.ensure(xfer_len + need);
     h.memory = memory;
     // (complex kernels: pools of (re, im) pairs at the same element offsets)
     const int esz = h.cplx ? 2 : 1;
-    h.mat64.alloc(h.mat_len * esz);
-    H2W_HIP(hipMemsetAsync(h.mat64.p, 0, h.mat_len * esz * 8, s));
+    h.mat64.alloc(std::max<int64_t>(pool_len + spare, 32) * esz);
+    H2W_HIP(hipMemsetAsync(h.mat64.p, 0, h.mat64.n * 8, s));
     h.vec64.alloc(h.vec_len * esz);
     if (h.cplx) h.vec32.release();
     else h.vec32.alloc(h.vec_len);
@@ -1992,15 +1976,45 @@ void assemble_operators(Handle &h, double t0, DevBuf<double> &scratch) {
     }
 
     // ---- evaluate operators on the device
-    if (formed > 0) {
-        // (transfers, and composites if all are kept, as they are; else those that are, at their new places)
-        H2W_HIP(hipMemcpyAsync(h.mat64.p, scratch.p, formed * 8, hipMemcpyDeviceToDevice, s));
-        if (reform && comp_len > 0) form_composites(h.mat64.p, comp_len, 0);
+    form_transfers(h.mat64.p);
+    if (comp_len > 0) {
+        double *A = h.mat64.p;
+        if (!inside) {
+            A = scratch.p;
+            H2W_HIP(hipMemcpyAsync(A, h.mat64.p, xfer_len * 8, hipMemcpyDeviceToDevice, s));
+            H2W_HIP(hipMemsetAsync(A + xfer_len, 0, comp_len * 8, s));
+        }
+        const auto most = form_composites(A, xfer_len, comp_len, A + xfer_len + comp_len);
+        std::vector<std::pair<int, int>> kept;
+        for (auto [T, B] : groups) {
+            int low = T - 1;  // the group's levels from here on are kept
+            while (low > B && most[low - 1] <= kComposeMost) --low;
+            kept.push_back({T, low});
+            for (int q = low; q > B; --q) kept.push_back({q, q - 1});
+        }
+        const bool all = kept == groups;
+        const int64_t comp_trial = comp_len;
+        groups = std::move(kept);
+        comp_len = place_composites(pool_len);
+        if (comp_len > spare) {  // (not two pools at a time)
+            if (inside) {
+                scratch.ensure(xfer_len + need);
+                H2W_HIP(hipMemcpyAsync(scratch.p, A, (xfer_len + comp_trial) * 8, hipMemcpyDeviceToDevice, s));
+                A = scratch.p;
+            }
+            H2W_HIP(hipStreamSynchronize(s));
+            h.mat64.alloc(pool_len + comp_len);
+            H2W_HIP(hipMemsetAsync(h.mat64.p, 0, h.mat64.n * 8, s));
+            H2W_HIP(hipMemcpyAsync(h.mat64.p, A, xfer_len * 8, hipMemcpyDeviceToDevice, s));
+        }
+        double *M = h.mat64.p;
+        if (all) H2W_HIP(hipMemcpyAsync(M + pool_len, A + xfer_len, comp_len * 8, hipMemcpyDeviceToDevice, s));
+        else if (comp_len > 0) form_composites(M, pool_len, comp_len, A + xfer_len);
+        if (M == A) H2W_HIP(hipMemsetAsync(M + xfer_len, 0, need * 8, s));
         H2W_HIP(hipStreamSynchronize(s));
         scratch.release();
-    } else {
-        form_transfers(h.mat64.p);
     }
+    h.mat_len = std::max<int64_t>(pool_len + comp_len, 32);
     if (!h.pairs.empty()) {
         // semi-nested row factors
         std::vector<int32_t> idx;
