@@ -1320,7 +1320,7 @@ void build_inner(Handle &h, double irp) {
                 for (int b = 0; b < fl.nb; ++b) {
                     if (fl.ein_off[b] < 0) continue;
                     const int k = fl.kin[b];
-                    const int64_t lro = h.d_lr.p ? fl.lr[b] : lr.add(fl.Ir[b], fl.Ic[b], k);
+                    const int64_t lro = h.d_lr.p ? fl.lr[b] : lr.add(fl.Ir[b].data(), fl.Ic[b].data(), k);
                     const int64_t icq = (int64_t)idx.size();
                     idx.insert(idx.end(), fl.Ic[b].begin(), fl.Ic[b].begin() + k);
                     int64_t m = 0;
@@ -2313,12 +2313,12 @@ void assemble_operators(Handle &h, double t0, DevBuf<double> &scratch) {
 // y_tree = A x_tree inside the vector pool (x already at off_x)
 }  // namespace
 
-int64_t LrForm::add(const std::vector<int32_t> &Ir, const std::vector<int32_t> &Ic, int k) {
+int64_t LrForm::add(const int32_t *Ir, const int32_t *Ic, int k) {
     LrFormJob J;
     J.ir = (int64_t)idx.size();
-    idx.insert(idx.end(), Ir.begin(), Ir.begin() + k);
+    idx.insert(idx.end(), Ir, Ir + k);
     J.ic = (int64_t)idx.size();
-    idx.insert(idx.end(), Ic.begin(), Ic.begin() + k);
+    idx.insert(idx.end(), Ic, Ic + k);
     J.out = len;
     J.k = k;
     J.pad = 0;
@@ -2328,14 +2328,16 @@ int64_t LrForm::add(const std::vector<int32_t> &Ir, const std::vector<int32_t> &
 }
 void LrForm::run(const Handle &h) {
     if (jobs.empty()) return;
-    DevBuf<LrFormJob> dj;
-    DevBuf<int32_t> di;
-    dj.upload(jobs, h.stream);
-    di.upload(idx, h.stream);
+    d_jobs.upload(jobs, h.stream);
+    d_idx.upload(idx, h.stream);
     out.ensure(len);
-    launch_lr_form(dj.p, (int)jobs.size(), di.p, out.p, h.kp, h.stream);
+    launch_lr_form(d_jobs.p, (int)jobs.size(), d_idx.p, out.p, h.kp, h.stream);
     H2W_HIP(hipGetLastError());
-    H2W_HIP(hipStreamSynchronize(h.stream));
+}
+void LrForm::clear() {
+    jobs.clear();
+    idx.clear();
+    len = 0;
 }
 
 // operator phase of the assembly from skeletons already in the handle (loading a saved operator)

@@ -107,6 +107,63 @@ struct RelaxedCapture {
     ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
+// L and R of one skeleton of a level after another: formed on the device all at once, copied 4 MB (or one skeleton) at a
+// time, the next chunk while the host writes and hashes the one before.
+class FactorReader {
+    static constexpr int64_t kChunk = 1 << 19;
+    struct Chunk {
+        size_t end = 0;  // skeletons up to here
+        PinBuf host;
+        Event done;
+    };
+    const Handle &h;
+    LrForm form;
+    std::vector<int64_t> off{0};  // of every skeleton's factors, and their end
+    Chunk c[2];
+    size_t at = 0, first = 0;  // next skeleton; first of the present chunk
+    int cur = 0;
+    void issue(Chunk &k, size_t from) {
+        k.end = from;
+        while (k.end + 1 < off.size() && (off[k.end] == off[from] || off[k.end + 1] - off[from] <= kChunk)) ++k.end;
+        const int64_t len = off[k.end] - off[from];
+        if (len == 0) return;
+        size_t room = 4096;
+        while ((int64_t)room < len) room *= 2;
+        k.host.ensure(room);
+        H2W_HIP(hipMemcpyAsync(k.host.p, form.out.p + off[from], len * 8, hipMemcpyDeviceToHost, h.stream));
+        H2W_HIP(hipEventRecord(k.done, h.stream));
+    }
+
+public:
+    explicit FactorReader(const Handle &handle) : h(handle) {}
+    ~FactorReader() { (void)hipStreamSynchronize(h.stream); }  // (before the buffers go)
+    // a level: add() every skeleton, run(), then next() for every one
+    void clear() {
+        form.clear();
+        off.assign(1, 0);
+    }
+    void add(const std::vector<int32_t> &Ir, const std::vector<int32_t> &Ic, int rank) {
+        if (rank > 0) form.add(Ir.data(), Ic.data(), rank);
+        off.push_back(form.len);
+    }
+    void run() {
+        form.run(h);
+        at = first = 0;
+        cur = 1;
+        c[1].end = 0;
+        issue(c[0], 0);
+    }
+    const double *next() {
+        if (at == c[cur].end) {
+            cur ^= 1;
+            first = at;
+            if (off[c[cur].end] > off[first]) H2W_HIP(hipEventSynchronize(c[cur].done));
+            issue(c[cur ^ 1], c[cur].end);
+        }
+        return c[cur].host.p + (off[at++] - off[first]);
+    }
+};
+
 }  // namespace
 }  // namespace h2w
 
@@ -127,19 +184,7 @@ int h2w_save(const h2w_handle *h, const char *path) {
         // The caller, or another thread, may be capturing a graph: what follows concerns the handle's own stream only,
         // and must not end that capture.
         h2w::RelaxedCapture relaxed;
-        std::vector<double> lr;
-        auto fetch = [&](h2w::LrForm &form) {  // L and R of a level's skeletons
-            lr.resize(form.len);
-            if (lr.empty()) return;
-            form.run(*h);
-            H2W_HIP(hipMemcpyAsync(lr.data(), form.out.p, lr.size() * 8, hipMemcpyDeviceToHost, h->stream));
-            H2W_HIP(hipStreamSynchronize(h->stream));
-        };
-        int64_t at = 0;
-        auto put_lr = [&](int64_t r) {
-            w.raw(lr.data() + at, (size_t)(2 * r * r) * sizeof(double));
-            at += 2 * r * r;
-        };
+        h2w::FactorReader factors(*h);
         w.raw(h2w::kMagic, 8);
         const int32_t hdr[8] = {h->dim, h->variant, h->choice, h->tol_pow, h->n_max, P.nL, h->opts.compat, 0};
         w.raw(hdr, sizeof(hdr));
@@ -158,33 +203,29 @@ int h2w_save(const h2w_handle *h, const char *path) {
                 const h2w::FamLevel *fl = have ? &h->fam[f][j] : nullptr;
                 const int32_t nb = fl ? (int32_t)fl->rank.size() : 0;
                 w.put<int32_t>(nb);
-                h2w::LrForm form;
-                for (int b = 0; b < nb; ++b)
-                    if (fl->rank[b] > 0) form.add(fl->Ir[b], fl->Ic[b], fl->rank[b]);
-                fetch(form);
-                at = 0;
+                factors.clear();
+                for (int b = 0; b < nb; ++b) factors.add(fl->Ir[b], fl->Ic[b], fl->rank[b]);
+                factors.run();
                 for (int b = 0; b < nb; ++b) {
                     const int32_t r = fl->rank[b];
                     w.put<int32_t>(r);
                     w.vec(fl->Ir[b], r);
                     w.vec(fl->Ic[b], r);
-                    put_lr(r);
+                    w.raw(factors.next(), (size_t)(2LL * r * r) * sizeof(double));
                     w.put<int32_t>((int32_t)fl->hist[b].size());
                     w.vec(fl->hist[b], fl->hist[b].size());
                 }
             }
         w.put<int64_t>((int64_t)h->pairs.size());
-        h2w::LrForm form;
-        for (const auto &p : h->pairs)
-            if (p.rank > 0) form.add(p.Ir, p.Ic, p.rank);
-        fetch(form);
-        at = 0;
+        factors.clear();
+        for (const auto &p : h->pairs) factors.add(p.Ir, p.Ic, p.rank);
+        factors.run();
         for (const auto &p : h->pairs) {
             const int32_t v[4] = {p.level, p.b, p.v, p.rank};
             w.raw(v, sizeof(v));
             w.vec(p.Ir, p.rank);
             w.vec(p.Ic, p.rank);
-            put_lr(p.rank);
+            w.raw(factors.next(), (size_t)(2LL * p.rank * p.rank) * sizeof(double));
         }
         const uint64_t hash = w.hash;
         w.put<uint64_t>(hash);
