@@ -348,7 +348,7 @@ namespace h2w {
 using Handle = h2w_handle;
 
 // L and R of skeletons (or of their leading k pivots) formed from the pivots: add() returns the offset of L, R follows
-// at k^2, both k x k; run() queues their forming in out on the handle's stream, clear() (once that has run) starts again.
+// at k^2, both k x k; run() queues their forming in out on a stream, clear() (once that has run) starts again.
 struct LrForm {
     std::vector<LrFormJob> jobs;
     std::vector<int32_t> idx;
@@ -357,7 +357,7 @@ struct LrForm {
     DevBuf<int32_t> d_idx;
     DevBuf<double> out;
     int64_t add(const int32_t *Ir, const int32_t *Ic, int k);
-    void run(const Handle &h);
+    void run(const Handle &h, hipStream_t s);
     void clear();
 };
 

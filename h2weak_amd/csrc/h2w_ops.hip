@@ -1368,7 +1368,7 @@ void build_inner(Handle &h, double irp) {
         dxj.upload(xj, s);
         tmp.alloc(in_len);
         H2W_HIP(hipMemsetAsync(tmp.p, 0, in_len * 8, s));
-        lr.run(h);
+        lr.run(h, s);
         launch_xfer(dxj.p, (int)xj.size(), didx.p, h.d_lr.p ? h.d_lr.p : lr.out.p, tmp.p, h.kp, s);
         H2W_HIP(hipGetLastError());
         launch_to_fp32(tmp.p, h.mat32in.p, in_len, s);
@@ -2326,12 +2326,12 @@ int64_t LrForm::add(const int32_t *Ir, const int32_t *Ic, int k) {
     jobs.push_back(J);
     return J.out;
 }
-void LrForm::run(const Handle &h) {
+void LrForm::run(const Handle &h, hipStream_t s) {
     if (jobs.empty()) return;
-    d_jobs.upload(jobs, h.stream);
-    d_idx.upload(idx, h.stream);
+    d_jobs.upload(jobs, s);
+    d_idx.upload(idx, s);
     out.ensure(len);
-    launch_lr_form(d_jobs.p, (int)jobs.size(), d_idx.p, out.p, h.kp, h.stream);
+    launch_lr_form(d_jobs.p, (int)jobs.size(), d_idx.p, out.p, h.kp, s);
     H2W_HIP(hipGetLastError());
 }
 void LrForm::clear() {

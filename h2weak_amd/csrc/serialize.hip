@@ -108,7 +108,8 @@ struct RelaxedCapture {
 };
 
 // L and R of one skeleton of a level after another: formed on the device all at once, copied 4 MB (or one skeleton) at a
-// time, the next chunk while the host writes and hashes the one before.
+// time, the next chunk while the host writes and hashes the one before.  On a stream of its own: another thread may be
+// using the handle's, or capturing its product there.
 class FactorReader {
     static constexpr int64_t kChunk = 1 << 19;
     struct Chunk {
@@ -117,6 +118,7 @@ class FactorReader {
         Event done;
     };
     const Handle &h;
+    hipStream_t s = nullptr;
     LrForm form;
     std::vector<int64_t> off{0};  // of every skeleton's factors, and their end
     Chunk c[2];
@@ -130,13 +132,20 @@ class FactorReader {
         size_t room = 4096;
         while ((int64_t)room < len) room *= 2;
         k.host.ensure(room);
-        H2W_HIP(hipMemcpyAsync(k.host.p, form.out.p + off[from], len * 8, hipMemcpyDeviceToHost, h.stream));
-        H2W_HIP(hipEventRecord(k.done, h.stream));
+        H2W_HIP(hipMemcpyAsync(k.host.p, form.out.p + off[from], len * 8, hipMemcpyDeviceToHost, s));
+        H2W_HIP(hipEventRecord(k.done, s));
     }
 
 public:
-    explicit FactorReader(const Handle &handle) : h(handle) {}
-    ~FactorReader() { (void)hipStreamSynchronize(h.stream); }  // (before the buffers go)
+    explicit FactorReader(const Handle &handle) : h(handle) {
+        H2W_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+    }
+    ~FactorReader() {
+        (void)hipStreamSynchronize(s);  // (before the buffers go)
+        (void)hipStreamDestroy(s);
+    }
+    FactorReader(const FactorReader &) = delete;
+    FactorReader &operator=(const FactorReader &) = delete;
     // a level: add() every skeleton, run(), then next() for every one
     void clear() {
         form.clear();
@@ -147,7 +156,7 @@ public:
         off.push_back(form.len);
     }
     void run() {
-        form.run(h);
+        form.run(h, s);
         at = first = 0;
         cur = 1;
         c[1].end = 0;
@@ -181,8 +190,8 @@ int h2w_save(const h2w_handle *h, const char *path) {
         h2w::Writer w{fp.get()};
         const h2w::Plan &P = h->plan;
         H2W_HIP(hipSetDevice(h->opts.device));
-        // The caller, or another thread, may be capturing a graph: what follows concerns the handle's own stream only,
-        // and must not end that capture.
+        // The caller, or another thread, may be capturing a graph: what follows concerns a stream of its own, and must
+        // not end that capture.
         h2w::RelaxedCapture relaxed;
         h2w::FactorReader factors(*h);
         w.raw(h2w::kMagic, 8);
