@@ -1931,8 +1931,22 @@ void assemble_operators(Handle &h, double t0, DevBuf<double> &scratch) {
         for (int f = 0; f < 2; ++f)
             if (B < T - 1 && fam_on[f]) need += (int64_t)(T - B) * h.fam[f][T].nb * (int64_t)(sizeof(ComposeJob) / 8);
     const bool inside = xfer_len + need <= pool_len;
+    // scratch for them; where the device has none left, every level is a launch of its own instead
+    auto room = [&]() {
+        try {
+            scratch.ensure(xfer_len + need);
+            return true;
+        } catch (const Error &) {
+            (void)hipGetLastError();
+            std::vector<std::pair<int, int>> single;
+            for (int T = P.nL; T > 1; --T) single.push_back({T, T - 1});
+            groups = std::move(single);
+            comp_len = 0;
+            return false;
+        }
+    };
     if (comp_len == 0 || inside) scratch.release();
-    else scratch.ensure(xfer_len + need);
+    else room();
     h.memory = memory;
     // (complex kernels: pools of (re, im) pairs at the same element offsets)
     const int esz = h.cplx ? 2 : 1;
@@ -1996,9 +2010,8 @@ void assemble_operators(Handle &h, double t0, DevBuf<double> &scratch) {
         const int64_t comp_trial = comp_len;
         groups = std::move(kept);
         comp_len = place_composites(pool_len);
-        if (comp_len > spare) {  // (not two pools at a time)
+        if (comp_len > spare && (!inside || room())) {  // (not two pools at a time)
             if (inside) {
-                scratch.ensure(xfer_len + need);
                 H2W_HIP(hipMemcpyAsync(scratch.p, A, (xfer_len + comp_trial) * 8, hipMemcpyDeviceToDevice, s));
                 A = scratch.p;
             }
@@ -2008,7 +2021,7 @@ void assemble_operators(Handle &h, double t0, DevBuf<double> &scratch) {
             H2W_HIP(hipMemcpyAsync(h.mat64.p, A, xfer_len * 8, hipMemcpyDeviceToDevice, s));
         }
         double *M = h.mat64.p;
-        if (all) H2W_HIP(hipMemcpyAsync(M + pool_len, A + xfer_len, comp_len * 8, hipMemcpyDeviceToDevice, s));
+        if (all && comp_len > 0) H2W_HIP(hipMemcpyAsync(M + pool_len, A + xfer_len, comp_len * 8, hipMemcpyDeviceToDevice, s));
         else if (comp_len > 0) form_composites(M, pool_len, comp_len, A + xfer_len);
         if (M == A) H2W_HIP(hipMemsetAsync(M + xfer_len, 0, need * 8, s));
         H2W_HIP(hipStreamSynchronize(s));
